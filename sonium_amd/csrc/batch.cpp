@@ -559,6 +559,8 @@ sbh_status sbh_batch_set_problem(sbh_batch* b, const sbh_physics* physics, const
             }
         };
         build_families(b);  // sets in_family on the instances before they are uploaded
+        for (int i = 0; i < b->B; ++i)
+            b->inst[i].far_variant = far_variant(b->inst[i].k, b->meshes[i]->panel_radius, b->inst[i].beta[0]);
         put(b->d_inst, b->inst);
         put(b->d_col_inst, b->col_inst);
         put(b->d_col_q, b->col_q);

@@ -1,26 +1,27 @@
-"""Coefficients of the device sin/cos polynomials on |r| <= pi/2.
+"""Coefficients of the device sin/cos polynomials.
+
+Two pairs, both near-minimax: for |r| <= pi/2 (P and Q of degree 7, used after
+a reduction by pi and for moderate phase differences) and for |r| <= 0.32 (P of
+degree 4, Q of degree 3, for the phase differences inside one panel).
 
 sin r = r + r^3 P(r^2),   cos r = 1 - r^2/2 + r^4 Q(r^2),
 
-with P and Q of degree 7 interpolating (sin r - r)/r^3 and
-(cos r - 1 + r^2/2)/r^4 as functions of u = r^2 at the eight Chebyshev nodes
-of [0, (pi/2)^2] (Chebyshev interpolation, near-minimax for these entire
+with P and Q interpolating (sin r - r)/r^3 and
+(cos r - 1 + r^2/2)/r^4 as functions of u = r^2 at the Chebyshev nodes
+of [0, r_max^2] (Chebyshev interpolation, near-minimax for these entire
 functions), computed in 50-digit arithmetic with mpmath and rounded to double.
-The device reduces its argument by pi, so one sign flip finishes both values.
+After the reduction by pi one sign flip finishes both values.
 ``python gen_sincos_coefficients.py`` prints the constants and the maximum
 error of the polynomials with the rounded coefficients, measured against
-mpmath on 2001 points of [0, pi/2].
+mpmath on 2001 points of [0, r_max].
 """
 
 from __future__ import annotations
 
 import mpmath as mp
 
-DEGREE = 7
-
-
-def _half_range():
-    return mp.pi / 2  # evaluated at the working precision
+# r_max (evaluated at the working precision), degree of P, degree of Q
+RANGES = {"half period": (lambda: mp.pi / 2, 7, 7), "panel": (lambda: mp.mpf("0.32"), 4, 3)}
 
 
 def _g(u):
@@ -37,8 +38,8 @@ def _h(u):
     return (mp.cos(r) - 1 + u / 2) / u ** 2
 
 
-def _interpolate(f, degree):
-    upper = _half_range() ** 2
+def _interpolate(f, degree, r_max):
+    upper = r_max ** 2
     n = degree + 1
     nodes = [upper / 2 * (1 - mp.cos((2 * i + 1) * mp.pi / (2 * n))) for i in range(n)]
     vander = mp.matrix([[x ** j for j in range(n)] for x in nodes])
@@ -46,18 +47,20 @@ def _interpolate(f, degree):
     return [float(c) for c in mp.lu_solve(vander, values)]
 
 
-def coefficients():
+def coefficients(name="half period"):
     """(P, Q) as lists of doubles, lowest degree first."""
     with mp.workdps(50):
-        return _interpolate(_g, DEGREE), _interpolate(_h, DEGREE)
+        r_max, dp, dq = RANGES[name]
+        return _interpolate(_g, dp, r_max()), _interpolate(_h, dq, r_max())
 
 
-def max_errors(P, Q, samples=2001):
-    """Maximum |poly - exact| of sin and cos over [0, pi/2] with the given coefficients."""
+def max_errors(P, Q, name="half period", samples=2001):
+    """Maximum |poly - exact| of sin and cos over [0, r_max] with the given coefficients."""
     es = ec = mp.mpf(0)
     with mp.workdps(50):
+        r_max = RANGES[name][0]()
         for i in range(samples):
-            r = _half_range() * i / (samples - 1)
+            r = r_max * i / (samples - 1)
             u = r * r
             p = sum(mp.mpf(c) * u ** j for j, c in enumerate(P))
             q = sum(mp.mpf(c) * u ** j for j, c in enumerate(Q))
@@ -67,7 +70,9 @@ def max_errors(P, Q, samples=2001):
 
 
 if __name__ == "__main__":
-    P, Q = coefficients()
-    print("P =", ", ".join(repr(c) for c in P))
-    print("Q =", ", ".join(repr(c) for c in Q))
-    print("max error sin %.3e cos %.3e" % max_errors(P, Q))
+    for name in RANGES:
+        P, Q = coefficients(name)
+        print(name)
+        print("P =", ", ".join(repr(c) for c in P))
+        print("Q =", ", ".join(repr(c) for c in Q))
+        print("max error sin %.3e cos %.3e" % max_errors(P, Q, name))

@@ -173,6 +173,21 @@ struct PanelBc {
     double adm[2];
 };
 
+// Variants of the far loop (far_sums).  The phase of a rule point relative to
+// its panel's centre is at most k * POINT_RADIUS * panel_radius (POINT_RADIUS
+// bounds the rule's points against the farthest corner); below
+// PANEL_PHASE_MAX the short sine polynomials hold, up to half a period the
+// long ones without a reduction.  Both take lengths in units of 1/k and an
+// imaginary beta; any other k or beta takes the general form.
+enum FarVariant { FAR_GENERAL = 0, FAR_LONG = 1, FAR_SHORT = 2 };
+constexpr double PANEL_PHASE_MAX = 0.32;
+constexpr double POINT_RADIUS = 0.86;
+inline int far_variant(double k, double panel_radius, double beta_re) {
+    const double phase = k * panel_radius * POINT_RADIUS;
+    if (beta_re != 0.0 || !(phase > 1e-40)) return FAR_GENERAL;  // squares in units of 1/k must not underflow
+    return phase <= PANEL_PHASE_MAX ? FAR_SHORT : phase <= 1.57 ? FAR_LONG : FAR_GENERAL;
+}
+
 // One near pair: leaves [begin, begin+count) of the leaf-code array.
 struct NearPair {
     int32_t i, j;
@@ -201,7 +216,7 @@ struct BatchInstance {
     double sign;
     double beta[2];
     int32_t in_family;  // far entries written by the frequency-family kernel
-    int32_t pad2;
+    int32_t far_variant;
 };
 
 // Instances on one mesh whose wavenumbers are k0 + f dk (f < count): the far
@@ -286,6 +301,7 @@ struct sbh_mesh {
     std::vector<sbh::PanelGeom> geom;
     std::vector<sbh::PanelBc> bc;
     double diameter = 0.0;          // bounding-box diagonal of the nodes
+    double panel_radius = 0.0;      // largest distance of a corner from its panel's centre
     bool general = false;           // any pressure BC, admittance or nonzero BC value
     bool vertex_order_normals = false;  // keep (v1-v0)x(v2-v0) instead of orienting away from the origin
     std::vector<int32_t> nonzero_bc;  // panels whose BC value is nonzero (tbem.rs:1240-1242)

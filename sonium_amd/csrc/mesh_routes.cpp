@@ -281,8 +281,14 @@ void build_mesh_geometry(sbh_mesh* m) {
             nrm[2] = -nrm[2];
         }
         PanelGeom& g = m->geom[e];
-        for (int v = 0; v < 3; ++v)
-            for (int j = 0; j < 3; ++j) g.c[3 * v + j] = p[v][j];
+        for (int v = 0; v < 3; ++v) {
+            double r2 = 0.0;
+            for (int j = 0; j < 3; ++j) {
+                g.c[3 * v + j] = p[v][j];
+                r2 += (p[v][j] - cen[j]) * (p[v][j] - cen[j]);
+            }
+            m->panel_radius = std::max(m->panel_radius, std::sqrt(r2));
+        }
         // regular.rs:687-704: dx/ds = v1 - v0, dx/dt = v2 - v0, n = ds x dt, J = |n|
         double ds[3] = {p[1][0] - p[0][0], p[1][1] - p[0][1], p[1][2] - p[0][2]};
         double dt[3] = {p[2][0] - p[0][0], p[2][1] - p[0][1], p[2][2] - p[0][2]};

@@ -11,8 +11,7 @@
 //                panel in registers, the collocation point and normal are
 //                uniform (scalar loads), and 64 lanes store 1 KiB of a row.
 //                This is the FP64-VALU-bound kernel: 13 kernel evaluations
-//                per pair, each one rsqrt, one sincos (Cody–Waite reduction +
-//                Taylor polynomials) and ~75 FMA-class operations.
+//                per pair, each about 40 FP64 instructions (far_sums).
 //   near_kernel  overwrites the near pairs (level-0 ratio < 3) with the sum
 //                over their subdivision leaves; one wave per pair, lanes over
 //                (leaf, point), evaluated in the reference's operation order.
@@ -28,6 +27,7 @@
 // (incident.rs:807-834 with bem_solver.rs:5005-5034).
 
 #include <cmath>
+#include <type_traits>
 
 #include "internal.hpp"
 
@@ -88,19 +88,11 @@ __device__ __forceinline__ double fma_vvs(double a, double b, double c) {
     return d;
 }
 
-// sin and cos of x for |x| < 2^20.  Cody & Waite (1980) two-constant
-// reduction by pi with FMA, x = q pi + r, |r| <= pi/2; then
-// sin r = r + r^3 P(r^2) and cos r = 1 - r^2/2 + r^4 Q(r^2) with P, Q of
-// degree 7 interpolating at Chebyshev nodes in r^2 (gen_sincos_coefficients.py;
-// error below 3.6e-17 for sin and 1.6e-17 for cos), and both signs flipped
-// for odd q.
-__device__ __forceinline__ void sincos_red(double x, double* sp, double* cp) {
-    constexpr double ONE_OVER_PI = 0.3183098861837907;
-    constexpr double PI_HI = 3.141592653589793;
-    constexpr double PI_LO = 1.2246467991473532e-16;
-    const double q = __builtin_rint(x * ONE_OVER_PI);
-    double r = __builtin_fma(-q, PI_HI, x);
-    r = __builtin_fma(-q, PI_LO, r);
+// sin and cos of r for |r| <= pi/2: sin r = r + r^3 P(r^2) and
+// cos r = 1 - r^2/2 + r^4 Q(r^2) with P, Q of degree 7 interpolating at
+// Chebyshev nodes in r^2 (gen_sincos_coefficients.py; error below 3.6e-17 for
+// sin and 1.6e-17 for cos).
+__device__ __forceinline__ void sincos_half_period(double r, double* sp, double* cp) {
     const double r2 = r * r;
     constexpr double P0 = -0.16666666666666666, P1 = 0.008333333333333316, P2 = -0.00019841269841254974,
                      P3 = 2.7557319219163234e-06, P4 = -2.5052107616996182e-08, P5 = 1.6058977312464087e-10,
@@ -115,7 +107,7 @@ __device__ __forceinline__ void sincos_red(double x, double* sp, double* cp) {
     ps = fma_vvs(r2, ps, P2);
     ps = fma_vvs(r2, ps, P1);
     ps = fma_vvs(r2, ps, P0);
-    const double sr = __builtin_fma(r * r2, ps, r);
+    *sp = __builtin_fma(r * r2, ps, r);
     double pc = __builtin_fma(r2, Q7, Q6);
     pc = fma_vvs(r2, pc, Q5);
     pc = fma_vvs(r2, pc, Q4);
@@ -123,13 +115,46 @@ __device__ __forceinline__ void sincos_red(double x, double* sp, double* cp) {
     pc = fma_vvs(r2, pc, Q2);
     pc = fma_vvs(r2, pc, Q1);
     pc = fma_vvs(r2, pc, Q0);
-    const double cr = __builtin_fma(r2 * r2, pc, __builtin_fma(-0.5, r2, 1.0));
+    *cp = __builtin_fma(r2 * r2, pc, __builtin_fma(-0.5, r2, 1.0));
+}
+
+// The same for |r| <= 0.32 (PANEL_PHASE_MAX) with P of degree 4 and Q of
+// degree 3 ("panel" coefficients; error below 3e-19 for sin and 2e-17 for cos).
+__device__ __forceinline__ void sincos_panel(double r, double* sp, double* cp) {
+    const double r2 = r * r;
+    constexpr double SP0 = -0.16666666666666666, SP1 = 0.00833333333333161, SP2 = -0.0001984126982781413,
+                     SP3 = 2.7557282426861207e-06, SP4 = -2.501102979241046e-08;
+    constexpr double SQ0 = 0.041666666666664874, SQ1 = -0.001388888888329103, SQ2 = 2.4801559965701305e-05,
+                     SQ3 = -2.751459668586056e-07;
+    double ps = __builtin_fma(r2, SP4, SP3);
+    ps = fma_vvs(r2, ps, SP2);
+    ps = fma_vvs(r2, ps, SP1);
+    ps = fma_vvs(r2, ps, SP0);
+    *sp = __builtin_fma(r * r2, ps, r);
+    double pc = __builtin_fma(r2, SQ3, SQ2);
+    pc = fma_vvs(r2, pc, SQ1);
+    pc = fma_vvs(r2, pc, SQ0);
+    pc = __builtin_fma(r2, pc, -0.5);
+    *cp = __builtin_fma(r2, pc, 1.0);
+}
+
+// sin and cos of x for |x| < 2^20.  Cody & Waite (1980) two-constant
+// reduction by pi with FMA, x = q pi + r, |r| <= pi/2, and both signs
+// flipped for odd q.
+__device__ __forceinline__ void sincos_red(double x, double* sp, double* cp) {
+    constexpr double ONE_OVER_PI = 0.3183098861837907;
+    constexpr double PI_HI = 3.141592653589793;
+    constexpr double PI_LO = 1.2246467991473532e-16;
+    const double q = __builtin_rint(x * ONE_OVER_PI);
+    double r = __builtin_fma(-q, PI_HI, x);
+    r = __builtin_fma(-q, PI_LO, r);
+    double sr, cr;
+    sincos_half_period(r, &sr, &cr);
     // (-1)^q: bit 0 of q moved to the sign bit of both results
     const unsigned long long sign = (unsigned long long)((unsigned)(int)q & 1u) << 63;
     *sp = __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, sr) ^ sign);
     *cp = __builtin_bit_cast(double, __builtin_bit_cast(unsigned long long, cr) ^ sign);
 }
-
 // 1/sqrt(d2) to about 1 ulp: the hardware estimate (24 correct bits) and one
 // third-order (Householder) step, y1 = y0 (1 + e/2 + 3e^2/8) with
 // e = 1 - d2 y0^2, whose truncation error (5/16) e^3 is below 1e-22.
@@ -540,96 +565,257 @@ __device__ __forceinline__ FarPoints far_points(const FarPanel& P) {
     return f;
 }
 
-// 13-point sums of one (collocation point, field panel) pair.  MODE 0 needs only
-// H and E; MODE 1 also G and Ht.  With rel = v0 - x:
-//   |y_q - x|^2 = |rel|^2 + s_q (2 rel.e1 + s_q e1.e1 + 2 t_q e1.e2) + t_q (2 rel.e2 + t_q e2.e2)
-//   (y_q - x).n_y = rel.n_y                        (e1 and e2 lie in the panel plane)
-//   (y_q - x).n_x = rel.n_x + s_q e1.n_x + t_q e2.n_x
-// so the per-point geometry is five FMAs for the distance and one product for
-// each normal projection, after six dot products per pair.  Off the diagonal
-// (which the self-panel rule overwrites) the point-to-point distance is at
-// least a fraction of the panel size, so the expansion loses no accuracy.
+// 13-point sums of one (collocation point, field panel) pair: the matrix
+// factors cb = H tau + E beta and, in MODE 1, hb = G tau + Ht beta
+// (tbem.rs:1404-1417 with gamma = 1).
 //
-// The channel sums are grouped by powers of k, and the panel factor 0.5 J/(4 pi)
-// is applied once per pair.  With zg = w_q e^{ikr}/r, pn = r^.n_y,
-// qn = -r^.n_x, rq = pn qn and t = 3 rq + n_x.n_y:
-//   H  = sum zg (ik - 1/r) pn                       = -S1 + ik S2,
-//   Ht = sum zg (ik - 1/r) qn                       = -Q1 + ik Q2,
-//   E  = sum zg [(3/r^2 - k^2) rq + n_x.n_y/r^2 - ik t/r] = T1 - k^2 T2 - ik T3,
-// with S1 = sum zg pn/r, S2 = sum zg pn, Q1 = sum zg qn/r, Q2 = sum zg qn,
-// T1 = sum zg t/r^2, T2 = sum zg rq, T3 = sum zg t/r: per point one product
-// and two FMAs per sum instead of the complex kernel factors.
-template <int MODE>
-__device__ __forceinline__ void far_sums(const FarPanel& P, const FarPoints& F, const Source& src, double k,
-                                         double k2, double& hr, double& hi, double& er, double& ei, double& gr,
-                                         double& gi, double& tr, double& ti) {
-    const double rel0 = P.v0[0] - src.c[0];
-    const double rel1 = P.v0[1] - src.c[1];
-    const double rel2 = P.v0[2] - src.c[2];
-    const double nxny = src.n[0] * P.nf[0] + src.n[1] * P.nf[1] + src.n[2] * P.nf[2];
-    const double a = rel0 * rel0 + rel1 * rel1 + rel2 * rel2;
-    const double b1 = 2.0 * (rel0 * P.e1[0] + rel1 * P.e1[1] + rel2 * P.e1[2]);
-    const double b2 = 2.0 * (rel0 * P.e2[0] + rel1 * P.e2[1] + rel2 * P.e2[2]);
-    const double pr = rel0 * P.nf[0] + rel1 * P.nf[1] + rel2 * P.nf[2];
-    const double g0 = -(rel0 * src.n[0] + rel1 * src.n[1] + rel2 * src.n[2]);
-    const double g1 = -(P.e1[0] * src.n[0] + P.e1[1] * src.n[1] + P.e1[2] * src.n[2]);
-    const double g2 = -(P.e2[0] * src.n[0] + P.e2[1] * src.n[1] + P.e2[2] * src.n[2]);
-    double s1r = 0.0, s1i = 0.0, s2r = 0.0, s2i = 0.0;
-    double t1r = 0.0, t1i = 0.0, t2r = 0.0, t2i = 0.0, t3r = 0.0, t3i = 0.0;
-    double q1r = 0.0, q1i = 0.0, q2r = 0.0, q2i = 0.0;
-    gr = gi = 0.0;
-    // TR13 constants are uniform: scalar loads from constant memory.
-#pragma clang loop unroll_count(2)
-    for (int q = 0; q < 13; ++q) {
-        const double sq = kTrS[q], tq = kTrT[q];
-        const double u1 = __builtin_fma(tq, F.e12x2, __builtin_fma(sq, F.e11, b1));
-        const double u2 = __builtin_fma(tq, F.e22, b2);
-        // The diagonal is overwritten by the self-panel rule; keep it finite.
-        const double d2 = fmax(__builtin_fma(sq, u1, __builtin_fma(tq, u2, a)), 1e-300);
-        const double inv = rsqrt_nr(d2);
-        const double dis = d2 * inv;
-        const double pn = pr * inv;                                                  // r^.n_y
-        const double qn = __builtin_fma(sq, g1, __builtin_fma(tq, g2, g0)) * inv;    // -r^.n_x
-        double sn, cs;
-        sincos_red(k * dis, &sn, &cs);
-        const double re2 = kTrW[q] * inv;
-        const double zgr = cs * re2, zgi = sn * re2;
-        const double pi = pn * inv;
-        s1r = __builtin_fma(zgr, pi, s1r);
-        s1i = __builtin_fma(zgi, pi, s1i);
-        s2r = __builtin_fma(zgr, pn, s2r);
-        s2i = __builtin_fma(zgi, pn, s2i);
-        const double rq = pn * qn;
-        const double t = __builtin_fma(3.0, rq, nxny);
-        const double ti_ = t * inv;
-        const double ti2 = ti_ * inv;
-        t1r = __builtin_fma(zgr, ti2, t1r);
-        t1i = __builtin_fma(zgi, ti2, t1i);
-        t2r = __builtin_fma(zgr, rq, t2r);
-        t2i = __builtin_fma(zgi, rq, t2i);
-        t3r = __builtin_fma(zgr, ti_, t3r);
-        t3i = __builtin_fma(zgi, ti_, t3i);
-        if (MODE == 1) {
-            gr += zgr;
-            gi += zgi;
-            const double qi = qn * inv;
-            q1r = __builtin_fma(zgr, qi, q1r);
-            q1i = __builtin_fma(zgi, qi, q1i);
-            q2r = __builtin_fma(zgr, qn, q2r);
-            q2i = __builtin_fma(zgi, qn, q2i);
+// What bounds it is the FP64 VALU issue rate: 13 evaluations per pair, each a
+// square root, a sine and a cosine.  Everything that can be is moved out of
+// the evaluation:
+//  - Geometry from the panel centre.  With the corners at c + V_i (V_0 + V_1 +
+//    V_2 = 0) the rule's points are c, c + kappa V_i (two groups of three) and
+//    c + a V_i + b V_j + c V_k (the six permutations), so with A = |c - x|^2,
+//    D_i = (c - x).V_i:  |y - x|^2 = A + 2 kappa D_i + kappa^2 |V_i|^2, two FMAs
+//    (three in the group of six, whose |displacement|^2 is kept per panel),
+//    and the projection on n_x takes one or two.
+//  - Phase from the panel centre.  e^{ikr} = e^{ik r_c} e^{ik(r - r_c)}: the first
+//    factor multiplies the finished sums, and the difference stays below
+//    k times the panel radius, so sine and cosine need no reduction and, on
+//    a resolved mesh, a short polynomial (sincos_panel).  The centre point's
+//    own difference is zero.
+//  - Lengths in units of 1/k (FAR_LONG, FAR_SHORT), so that k is one.
+//  - One complex weight per point.  With y = 1/r, u = y^2, g = -(y_q - x).n_x,
+//    pr = (y_q - x).n_y (constant on a flat panel), rq = pr g u and
+//    t = 3 rq + n_x.n_y,
+//      H = sum z pr y (-y + ik),  E = sum z [(t u - k^2 rq) - ik t y],
+//      G = sum z,                 Ht = sum z g y (-y + ik),   z = w e^{ikr} y,
+//    so tau and an imaginary beta (the Burton-Miller factor i/k) enter the real
+//    and the imaginary part of one weight each, and cb takes four FMAs.
+//  - The rule's four weights multiply the sums of their groups.
+// Per evaluation this takes 41 FP64 instructions (529 a pair, pair work included)
+// where separate channel sums over a reduced sine took 68; the assembly of 20480
+// panels takes 9.2 ms instead of 13.3, of which this loop 7.9 instead of 12.2.
+//
+// Variants (far_variant): FAR_SHORT and FAR_LONG need a purely imaginary beta
+// and a phase difference within the range of their polynomials; FAR_GENERAL
+// takes any k and beta, with lengths as they are and a full reduction.
+constexpr double TR_A = 0.048690315425316, TR_B = 0.312865496004874, TR_C = 0.638444188569810;
+constexpr double TR_K1 = 0.479308067841920 - 0.260345966079040;  // first group of three: c + K1 V_i
+constexpr double TR_K2 = 0.869739794195568 - 0.065130102902216;  // second group of three
+constexpr double TR_W0 = -0.149570044467682, TR_W1 = 0.175615257433208, TR_W2 = 0.053347235608838,
+                 TR_W3 = 0.077113760890257;
+
+// Uniform values of a launch, in units of 1/s: s = k and kap = 1, or s = 1 and kap = k.
+struct FarUniform {
+    double s, kap, tau, br, bi;  // br + i bi = beta s
+};
+
+template <int VAR>
+__device__ __forceinline__ FarUniform far_uniform(double k, double tau, double2 beta) {
+    FarUniform u;
+    u.s = VAR == FAR_GENERAL ? 1.0 : k;
+    u.kap = VAR == FAR_GENERAL ? k : 1.0;
+    u.tau = tau;
+    u.br = beta.x * u.s;
+    u.bi = beta.y * u.s;
+    return u;
+}
+
+// A field panel as the far loop keeps it: corner 0 and centre offset (exact
+// lengths), V_1, V_2 and the squares below in units of 1/s.
+struct FarLane {
+    double v0[3], cv[3], V1[3], V2[3], nf[3];
+    double L[3];  // |V_i|^2
+    double Q[6];  // |displacement|^2 of the group of six
+    double wj;
+};
+
+__device__ __forceinline__ double dot3(const double* a, const double* b) {
+    return __builtin_fma(a[2], b[2], __builtin_fma(a[1], b[1], a[0] * b[0]));
+}
+
+__device__ __forceinline__ FarLane far_lane(const FarPanel& P, double s) {
+    FarLane f;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        f.v0[d] = P.v0[d];
+        f.cv[d] = (P.e1[d] + P.e2[d]) * (1.0 / 3.0);
+        f.V1[d] = s * (P.e1[d] - f.cv[d]);
+        f.V2[d] = s * (P.e2[d] - f.cv[d]);
+        f.nf[d] = P.nf[d];
+    }
+    const double V0[3] = {-(f.V1[0] + f.V2[0]), -(f.V1[1] + f.V2[1]), -(f.V1[2] + f.V2[2])};
+    f.L[0] = dot3(V0, V0);
+    f.L[1] = dot3(f.V1, f.V1);
+    f.L[2] = dot3(f.V2, f.V2);
+    // |a V_i + b V_j + c V_k|^2 = (a-b)(a-c)|V_i|^2 + (b-a)(b-c)|V_j|^2 + (c-a)(c-b)|V_k|^2, all terms
+    // with V_0 + V_1 + V_2 = 0
+    constexpr double qa = (TR_A - TR_B) * (TR_A - TR_C), qb = (TR_B - TR_A) * (TR_B - TR_C),
+                     qc = (TR_C - TR_A) * (TR_C - TR_B);
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+        const int i = m >> 1, j = (i + 1 + (m & 1)) % 3, k = 3 - i - j;  // a on corner i, b on j, c on k
+        f.Q[m] = __builtin_fma(qa, f.L[i], __builtin_fma(qb, f.L[j], qc * f.L[k]));
+    }
+    f.wj = P.wj;
+    return f;
+}
+
+template <int MODE, int VAR>
+__device__ __forceinline__ void far_sums(const FarLane& P, const Source& src, const FarUniform& K, double2& cb,
+                                         double2& hb) {
+    double x[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        x[d] = (P.v0[d] - src.c[d]) + P.cv[d];
+        if (VAR != FAR_GENERAL) x[d] *= K.s;
+    }
+    const double A = dot3(x, x);
+    const double D1 = dot3(x, P.V1), D2 = dot3(x, P.V2);
+    const double pr = dot3(x, P.nf);
+    const double nn = dot3(src.n, P.nf);
+    // g of the centre and its slopes; MODE 0 carries g pr (times beta, imaginary) instead
+    const double gm = MODE == 0 && VAR != FAR_GENERAL ? -K.bi * pr : VAR != FAR_GENERAL ? -K.bi : -1.0;
+    const double gc = gm * dot3(x, src.n);
+    const double g1 = gm * dot3(P.V1, src.n), g2 = gm * dot3(P.V2, src.n);
+    const double D[3] = {-(D1 + D2), D1, D2};
+    const double g[3] = {-(g1 + g2), g1, g2};
+    const double P1 = K.tau * pr;
+    const double N = VAR != FAR_GENERAL ? K.bi * nn : nn;
+    const double kap2 = K.kap * K.kap;
+    const double yc = rsqrt_nr(A);
+    const double rc = VAR == FAR_GENERAL ? K.kap * (A * yc) : A * yc;
+    struct Part {
+        double cr, ci, hr, hi;
+    };
+    // Orders the points: the next one's distance waits for this one's sums.  Left to itself the compiler
+    // interleaves all 13 (256 registers, one or two waves per SIMD).
+    double Ap = A;
+    auto after = [&](Part& a) {
+        if (MODE == 0)
+            asm volatile("" : "+v"(Ap), "+v"(a.cr), "+v"(a.ci));
+        else
+            asm volatile("" : "+v"(Ap), "+v"(a.cr), "+v"(a.ci), "+v"(a.hr), "+v"(a.hi));
+    };
+    // One point: distance d2, projection gq, added to a (phase difference zero at the centre).
+    auto point = [&](double d2, double gq, bool centre, Part& a) {
+        const double y = rsqrt_nr(d2);
+        const double u = y * y;
+        double sn = 0.0, cs = 1.0;
+        if (!centre) {
+            if (VAR == FAR_GENERAL)
+                sincos_red(__builtin_fma(K.kap, d2 * y, -rc), &sn, &cs);
+            else if (VAR == FAR_LONG)
+                sincos_half_period(__builtin_fma(d2, y, -rc), &sn, &cs);
+            else
+                sincos_panel(__builtin_fma(d2, y, -rc), &sn, &cs);
         }
+        double wr, wi;
+        if (VAR != FAR_GENERAL) {
+            const double R = (MODE == 0 ? gq : pr * gq) * u;  // beta rq
+            const double T = __builtin_fma(3.0, R, N);        // beta t
+            wr = u * __builtin_fma(-P1, y, T);
+            wi = __builtin_fma(y, __builtin_fma(T, u, -R), P1 * u);
+        } else {
+            const double rq = (pr * gq) * u;
+            const double t = __builtin_fma(3.0, rq, nn);
+            const double er = __builtin_fma(t, u, -kap2 * rq), ei = -K.kap * (t * y);
+            wr = y * (__builtin_fma(K.br, er, -K.bi * ei) - P1 * u);
+            wi = y * __builtin_fma(K.kap * P1, y, __builtin_fma(K.br, ei, K.bi * er));
+        }
+        a.cr = __builtin_fma(cs, wr, a.cr);
+        a.ci = __builtin_fma(cs, wi, a.ci);
+        if (!centre) {
+            a.cr = __builtin_fma(-sn, wi, a.cr);
+            a.ci = __builtin_fma(sn, wr, a.ci);
+        }
+        if (MODE == 1) {
+            double vr, vi;
+            if (VAR != FAR_GENERAL) {
+                vr = __builtin_fma(-gq, u, K.tau * y);  // y (tau - beta g y), imaginary beta
+                vi = -gq * (u * y);
+            } else {
+                const double hr = -u, hi = K.kap * y;  // y (-y + ik)
+                vr = y * __builtin_fma(gq, __builtin_fma(K.br, hr, -K.bi * hi), K.tau);
+                vi = y * (gq * __builtin_fma(K.br, hi, K.bi * hr));
+            }
+            a.hr = __builtin_fma(cs, vr, a.hr);
+            a.hi = __builtin_fma(cs, vi, a.hi);
+            if (!centre) {
+                a.hr = __builtin_fma(-sn, vi, a.hr);
+                a.hi = __builtin_fma(sn, vr, a.hi);
+            }
+        }
+        after(a);
+    };
+    Part tot = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](double w, const Part& a) {
+        tot.cr = __builtin_fma(w, a.cr, tot.cr);
+        tot.ci = __builtin_fma(w, a.ci, tot.ci);
+        if (MODE == 1) {
+            tot.hr = __builtin_fma(w, a.hr, tot.hr);
+            tot.hi = __builtin_fma(w, a.hi, tot.hi);
+        }
+    };
+    {
+        Part a = {0.0, 0.0, 0.0, 0.0};
+        point(A, gc, true, a);
+        add(TR_W0, a);
     }
-    const double w = P.wj;
-    hr = -w * __builtin_fma(k, s2i, s1r);
-    hi = w * __builtin_fma(k, s2r, -s1i);
-    er = w * __builtin_fma(k, t3i, __builtin_fma(-k2, t2r, t1r));
-    ei = w * __builtin_fma(-k, t3r, __builtin_fma(-k2, t2i, t1i));
-    if (MODE == 1) {
-        gr *= w;
-        gi *= w;
-        tr = -w * __builtin_fma(k, q2i, q1r);
-        ti = w * __builtin_fma(k, q2r, -q1i);
+    {
+        Part a = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            point(__builtin_fma(TR_K1 * TR_K1, P.L[i], __builtin_fma(2.0 * TR_K1, D[i], Ap)),
+                  __builtin_fma(TR_K1, g[i], gc), false, a);
+        add(TR_W1, a);
     }
+    {
+        Part a = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            point(__builtin_fma(TR_K2 * TR_K2, P.L[i], __builtin_fma(2.0 * TR_K2, D[i], Ap)),
+                  __builtin_fma(TR_K2, g[i], gc), false, a);
+        add(TR_W2, a);
+    }
+    {
+        Part a = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int m = 0; m < 6; ++m) {
+            // displacement (a - c) V_i + (b - c) V_j, c the weight of the third corner
+            const int i = m >> 1, j = (i + 1 + (m & 1)) % 3;
+            constexpr double ac = TR_A - TR_C, bc = TR_B - TR_C;
+            point(__builtin_fma(2.0 * ac, D[i], __builtin_fma(2.0 * bc, D[j], Ap + P.Q[m])),
+                  __builtin_fma(ac, g[i], __builtin_fma(bc, g[j], gc)), false, a);
+        }
+        add(TR_W3, a);
+    }
+    double sn, cs;
+    sincos_red(rc, &sn, &cs);
+    const double fh = P.wj * K.s, fc = fh * K.s;
+    cb = make_double2(fc * __builtin_fma(cs, tot.cr, -sn * tot.ci), fc * __builtin_fma(cs, tot.ci, sn * tot.cr));
+    if (MODE == 1)
+        hb = make_double2(fh * __builtin_fma(cs, tot.hr, -sn * tot.hi), fh * __builtin_fma(cs, tot.hi, sn * tot.hr));
+}
+
+// Matrix coefficient of a field panel from its two factors (tbem.rs:1404-1417).
+__device__ __forceinline__ double2 column_coefficient(double2 cb, double2 hb, const PanelBc& bc, double2 iwr) {
+    if (bc.type == 1) return make_double2(-hb.x, -hb.y);
+    double2 c = make_double2(0.0, 0.0);
+    if (bc.type == 0) {
+        c = cb;
+        if (bc.has_adm) c = csub(c, cmul(cmul(hb, make_double2(bc.adm[0], bc.adm[1])), iwr));
+    }
+    return c;
+}
+
+// Far entry of one pair.
+template <int MODE, int VAR>
+__device__ __forceinline__ double2 far_entry(const FarLane& P, const Source& S, const PanelBc& bc,
+                                             const FarUniform& K, double2 iwr) {
+    double2 cb, hb;
+    far_sums<MODE, VAR>(P, S, K, cb, hb);
+    return MODE == 0 ? cb : column_coefficient(cb, hb, bc, iwr);
 }
 
 // Rigid/vibrating coefficient (H * gamma) * tau + E * beta with gamma = 1.
@@ -651,7 +837,7 @@ __device__ __forceinline__ double2 velocity_coefficient(double hr, double hi, do
 // as bit patterns with an atomic max; the column-0 blocks clear that slot).
 constexpr int FAR_MAX_ROWS = 16;
 
-template <int MODE>
+template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void far_kernel(const FarPanel* __restrict__ panels,
                                                   const Source* __restrict__ sources,
                                                   const PanelBc* __restrict__ bcs, int64_t n,
@@ -665,11 +851,10 @@ __global__ __launch_bounds__(256) void far_kernel(const FarPanel* __restrict__ p
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool active = j < n;
     const int64_t jj = active ? j : n - 1;
-    const FarPanel P = panels[jj];
-    const FarPoints F = far_points(P);
+    const FarUniform K = far_uniform<VAR>(k, tau_r, beta);
+    const FarLane P = far_lane(panels[jj], K.s);
     PanelBc bc;
     if (MODE == 1) bc = bcs[jj];
-    const double k2 = k * k;
     const int64_t i0 = (int64_t)blockIdx.y * rows_per_block;
     const int64_t i1 = min(n, i0 + rows_per_block);
     const int64_t c0 = (int64_t)blockIdx.x * 256;
@@ -692,20 +877,7 @@ __global__ __launch_bounds__(256) void far_kernel(const FarPanel* __restrict__ p
         }
     }
     for (int64_t i = i0; i < i1; ++i) {
-        const Source src = sources[i];
-        double hr, hi, er, ei, gr, gi, tr, ti;
-        far_sums<MODE>(P, F, src, k, k2, hr, hi, er, ei, gr, gi, tr, ti);
-        double2 out;
-        if (MODE == 0) {
-            out = velocity_coefficient(hr, hi, er, ei, tau_r, beta);
-        } else {
-            Acc a;
-            a.g = make_double2(gr, gi);
-            a.h = make_double2(hr, hi);
-            a.ht = make_double2(tr, ti);
-            a.e = make_double2(er, ei);
-            out = coefficient(a, bc, make_double2(1.0, 0.0), make_double2(tau_r, 0.0), beta, iwr);
-        }
+        const double2 out = far_entry<MODE, VAR>(P, sources[i], bc, K, iwr);
         if (active) A[i * lda + j] = out;
         if (rowmax) smax[i - i0][threadIdx.x] = active ? fmax(fabs(out.x), fabs(out.y)) : 0.0;
     }
@@ -1431,18 +1603,27 @@ __global__ __launch_bounds__(256) void batch_assemble_kernel(BatchAssemblyArgs a
         const double2 beta = make_double2(I.beta[0], I.beta[1]);
         if (PHASE == 0) {
             const FarPanel* far = args.far + I.panel_off;
-            const double k2 = k * k;
-            // members of a frequency family got their far entries from batch_far_family_kernel
-            for (int64_t jc = 0; jc < (I.in_family ? 0 : n); jc += 256) {
-                const int64_t j = jc + threadIdx.x;
-                const bool active = j < n;
-                const FarPanel P = far[active ? j : n - 1];
-                const FarPoints F = far_points(P);
-                for (int64_t i = r0; i < r1; ++i) {
-                    double hr, hi, er, ei, gr, gi, tr, ti;
-                    far_sums<0>(P, F, src[i], k, k2, hr, hi, er, ei, gr, gi, tr, ti);
-                    if (active) A[i * n + j] = velocity_coefficient(hr, hi, er, ei, I.tau, beta);
+            auto fill = [&](auto variant) {
+                constexpr int VAR = decltype(variant)::value;
+                const FarUniform K = far_uniform<VAR>(k, I.tau, beta);
+                for (int64_t jc = 0; jc < n; jc += 256) {
+                    const int64_t j = jc + threadIdx.x;
+                    const bool active = j < n;
+                    const FarLane P = far_lane(far[active ? j : n - 1], K.s);
+                    for (int64_t i = r0; i < r1; ++i) {
+                        const double2 v = far_entry<0, VAR>(P, src[i], PanelBc(), K, make_double2(0.0, 0.0));
+                        if (active) A[i * n + j] = v;
+                    }
                 }
+            };
+            // members of a frequency family got their far entries from batch_far_family_kernel
+            if (!I.in_family) {
+                if (I.far_variant == FAR_SHORT)
+                    fill(std::integral_constant<int, FAR_SHORT>());
+                else if (I.far_variant == FAR_LONG)
+                    fill(std::integral_constant<int, FAR_LONG>());
+                else
+                    fill(std::integral_constant<int, FAR_GENERAL>());
             }
             const int64_t nr = (r1 - r0) * I.ncol;
             for (int64_t t = threadIdx.x; t < nr; t += 256) {
@@ -1489,54 +1670,43 @@ __global__ void reset_counters_kernel(unsigned* counter) { counter[threadIdx.x] 
 //                      order + self_i).
 constexpr int EXACT_ROWS = 4;
 
-template <int MODE>
-__device__ __forceinline__ double2 far_entry(const FarPanel& P, const FarPoints& F, const Source& S,
-                                             const PanelBc& bc, double k, double k2, double tau_r, double2 beta,
-                                             double2 iwr) {
-    double hr, hi, er, ei, gr, gi, tr, ti;
-    far_sums<MODE>(P, F, S, k, k2, hr, hi, er, ei, gr, gi, tr, ti);
-    if (MODE == 0) return velocity_coefficient(hr, hi, er, ei, tau_r, beta);
-    Acc a;
-    a.g = make_double2(gr, gi);
-    a.h = make_double2(hr, hi);
-    a.ht = make_double2(tr, ti);
-    a.e = make_double2(er, ei);
-    return coefficient(a, bc, make_double2(1.0, 0.0), make_double2(tau_r, 0.0), beta, iwr);
-}
-
-template <int MODE>
+template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void exact_far_kernel(const FarPanel* __restrict__ panels,
                                                         const Source* __restrict__ sources,
                                                         const PanelBc* __restrict__ bcs, int64_t n, double k,
                                                         double tau_r, double2 beta, double2 iwr,
                                                         const double2* __restrict__ x, double2* __restrict__ out) {
+    __shared__ double2 sums[EXACT_ROWS][256];  // each lane's row sums
     __shared__ double2 red[4][EXACT_ROWS];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int64_t i0 = (int64_t)blockIdx.x * EXACT_ROWS;
-    const double k2 = k * k;
-    // rows one after another, each over every column chunk in order (the
-    // panels are L2-resident), so one row's point loop is live at a time
+    const FarUniform K = far_uniform<VAR>(k, tau_r, beta);
+    for (int r = 0; r < EXACT_ROWS; ++r) sums[r][threadIdx.x] = make_double2(0.0, 0.0);
+    // a column chunk's panel constants serve all rows; the rows run one after
+    // another, so one row's points are live at a time
+    for (int64_t jc = 0; jc < n; jc += 256) {
+        const int64_t j = jc + threadIdx.x;
+        const bool active = j < n;
+        const int64_t jj = active ? j : n - 1;
+        const FarLane P = far_lane(panels[jj], K.s);
+        PanelBc bc;
+        if (MODE == 1) bc = bcs[jj];
+        const double2 xj = x[jj];
 #pragma clang loop unroll(disable)
-    for (int r = 0; r < EXACT_ROWS; ++r) {
-        const int64_t i = min(i0 + r, n - 1);  // rows past n are computed and dropped
-        const Source S = sources[i];
-        double2 acc = make_double2(0.0, 0.0);
-        for (int64_t jc = 0; jc < n; jc += 256) {
-            const int64_t j = jc + threadIdx.x;
-            const bool active = j < n;
-            const int64_t jj = active ? j : n - 1;
-            const FarPanel P = panels[jj];
-            const FarPoints F = far_points(P);
-            PanelBc bc;
-            if (MODE == 1) bc = bcs[jj];
-            const double2 xj = x[jj];
-            const double2 v = far_entry<MODE>(P, F, S, bc, k, k2, tau_r, beta, iwr);
+        for (int r = 0; r < EXACT_ROWS; ++r) {
+            const int64_t i = min(i0 + r, n - 1);  // rows past n are computed and dropped
+            const double2 v = far_entry<MODE, VAR>(P, sources[i], bc, K, iwr);
             if (active && j != i) {
+                double2 acc = sums[r][threadIdx.x];
                 acc.x += v.x * xj.x - v.y * xj.y;
                 acc.y += v.x * xj.y + v.y * xj.x;
+                sums[r][threadIdx.x] = acc;
             }
         }
+    }
+    for (int r = 0; r < EXACT_ROWS; ++r) {
+        double2 acc = sums[r][threadIdx.x];
         acc.x = wave_sum(acc.x);
         acc.y = wave_sum(acc.y);
         if (lane == 0) red[wave][r] = acc;
@@ -1549,7 +1719,7 @@ __global__ __launch_bounds__(256) void exact_far_kernel(const FarPanel* __restri
     }
 }
 
-template <int MODE>
+template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void exact_near_kernel(const NearPair* __restrict__ pairs, int64_t npairs,
                                                          const uint64_t* __restrict__ leaves,
                                                          const PanelGeom* __restrict__ geom,
@@ -1567,8 +1737,8 @@ __global__ __launch_bounds__(256) void exact_near_kernel(const NearPair* __restr
     const Source S = sources[np.i];
     const double2 v = near_entry(np, leaves, G, S, bc, k, wavruim, tau_r, beta, iwr, lane);
     if (lane == 0) {
-        const FarPanel P = panels[np.j];
-        const double2 f = far_entry<MODE>(P, far_points(P), S, bc, k, k * k, tau_r, beta, iwr);
+        const FarUniform K = far_uniform<VAR>(k, tau_r, beta);
+        const double2 f = far_entry<MODE, VAR>(far_lane(panels[np.j], K.s), S, bc, K, iwr);
         out[p] = cmul(csub(v, f), x[np.j]);
     }
 }
@@ -1815,6 +1985,23 @@ void upload_quadrature_tables(sbh_context* ctx) {
     (void)ctx;
 }
 
+// Calls launch(mode, variant) with the far loop's compile-time arguments.
+template <typename Launch>
+static void with_far_variant(int variant, int general, Launch&& launch) {
+    auto mode = [&](auto var) {
+        if (general)
+            launch(std::integral_constant<int, 1>(), var);
+        else
+            launch(std::integral_constant<int, 0>(), var);
+    };
+    if (variant == FAR_SHORT)
+        mode(std::integral_constant<int, FAR_SHORT>());
+    else if (variant == FAR_LONG)
+        mode(std::integral_constant<int, FAR_LONG>());
+    else
+        mode(std::integral_constant<int, FAR_GENERAL>());
+}
+
 void launch_assembly(sbh_workspace* ws, const sbh_physics& ph, sbh_c64 beta_c, sbh_system* sys) {
     injection_check(INJECT_LAUNCH);
     sbh_context* ctx = ws->ctx;
@@ -1843,14 +2030,11 @@ void launch_assembly(sbh_workspace* ws, const sbh_physics& ph, sbh_c64 beta_c, s
     double* rm = row_max ? sys->d_rowmax.ptr : nullptr;
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_ASSEMBLE_FAR, &ev);
-    if (general)
-        hipLaunchKernelGGL(far_kernel<1>, grid, dim3(256), 0, ctx->stream, m->d_far.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, n, sys->lda, rows_per_block, k, ph.tau, beta, iwr, sys->d_A.ptr,
-                           ws->d_row_ptr.ptr, ws->d_pairs.ptr, rm, nbx);
-    else
-        hipLaunchKernelGGL(far_kernel<0>, grid, dim3(256), 0, ctx->stream, m->d_far.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, n, sys->lda, rows_per_block, k, ph.tau, beta, iwr, sys->d_A.ptr,
-                           ws->d_row_ptr.ptr, ws->d_pairs.ptr, rm, nbx);
+    with_far_variant(far_variant(k, m->panel_radius, beta.x), general, [&](auto mode, auto var) {
+        hipLaunchKernelGGL((far_kernel<decltype(mode)::value, decltype(var)::value>), grid, dim3(256), 0, ctx->stream,
+                           m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, n, sys->lda, rows_per_block, k, ph.tau, beta, iwr,
+                           sys->d_A.ptr, ws->d_row_ptr.ptr, ws->d_pairs.ptr, rm, nbx);
+    });
     SBH_HIP(hipGetLastError());
     ctx->end_timed(SBH_KERNEL_ASSEMBLE_FAR, ev);
     if (ws->near_pairs > 0) {
@@ -2047,25 +2231,18 @@ void launch_exact_apply(const sbh_operator* op, const double2* x, double2* y) {
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_MATVEC, &ev);
     const dim3 far_grid((unsigned)((n + EXACT_ROWS - 1) / EXACT_ROWS));
-    if (general)
-        hipLaunchKernelGGL(exact_far_kernel<1>, far_grid, dim3(256), 0, ctx->stream, m->d_far.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, n, k, ph.tau, beta, iwr, x, op->d_far.ptr);
-    else
-        hipLaunchKernelGGL(exact_far_kernel<0>, far_grid, dim3(256), 0, ctx->stream, m->d_far.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, n, k, ph.tau, beta, iwr, x, op->d_far.ptr);
-    SBH_HIP(hipGetLastError());
-    if (ws->near_pairs > 0) {
-        const dim3 grid((unsigned)((ws->near_pairs + 3) / 4));
-        if (general)
-            hipLaunchKernelGGL(exact_near_kernel<1>, grid, dim3(256), 0, ctx->stream, ws->d_pairs.ptr, ws->near_pairs,
-                               ws->d_leaves.ptr, m->d_geom.ptr, m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, k, wavruim,
-                               ph.tau, beta, iwr, x, op->d_near.ptr);
-        else
-            hipLaunchKernelGGL(exact_near_kernel<0>, grid, dim3(256), 0, ctx->stream, ws->d_pairs.ptr, ws->near_pairs,
-                               ws->d_leaves.ptr, m->d_geom.ptr, m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, k, wavruim,
-                               ph.tau, beta, iwr, x, op->d_near.ptr);
+    with_far_variant(far_variant(k, m->panel_radius, beta.x), general, [&](auto mode, auto var) {
+        constexpr int MODE = decltype(mode)::value, VAR = decltype(var)::value;
+        hipLaunchKernelGGL((exact_far_kernel<MODE, VAR>), far_grid, dim3(256), 0, ctx->stream, m->d_far.ptr,
+                           m->d_src.ptr, m->d_bc.ptr, n, k, ph.tau, beta, iwr, x, op->d_far.ptr);
         SBH_HIP(hipGetLastError());
-    }
+        if (ws->near_pairs > 0)
+            hipLaunchKernelGGL((exact_near_kernel<MODE, VAR>), dim3((unsigned)((ws->near_pairs + 3) / 4)), dim3(256),
+                               0, ctx->stream, ws->d_pairs.ptr, ws->near_pairs, ws->d_leaves.ptr, m->d_geom.ptr,
+                               m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, k, wavruim, ph.tau, beta, iwr, x,
+                               op->d_near.ptr);
+    });
+    SBH_HIP(hipGetLastError());
     hipLaunchKernelGGL(exact_self_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, ctx->stream, m->d_geom.ptr,
                        m->d_src.ptr, m->d_bc.ptr, general, n, k, wavruim, ph.tau, beta, iwr, x, op->d_self.ptr);
     SBH_HIP(hipGetLastError());
