@@ -4,14 +4,16 @@
 // kernels and Adam on FP32 master weights.
 //
 // GEMM.  One kernel computes C = A B^T for row-major BF16 A (M x K) and B
-// (N x K): both operands are K-contiguous, so every MFMA operand is one
-// 16-byte load per lane.  The three products of a layer use it as
+// (N x K): both operands are K-contiguous.  The products of a layer use it as
 //   forward      H   = A_prev W^T          (A_prev: M x K_in,  W:  N_out x K_in)
 //   input grad   dA  = dZ (W^T)^T          (dZ:     M x N_out, W^T: K_in x N_out)
 //   weight grad  dW  = dZ^T (A_prev^T)^T   (dZ^T:   N_out x M, A_prev^T: K_in x M)
-// so the elementwise kernels write activations and their gradients in both
-// layouts, and the weight copy is kept as W and W^T.  Weight gradients reduce
-// over the M samples with split K (FP32 partials, summed in a fixed order).
+// and each product's elementwise work runs on its accumulators: bias, SiLU and
+// its derivative (forward), the derivative's product and the bias gradient's
+// partial sums (input gradient), the loss (output layer).  Activations and
+// their gradients are written in both layouts, and the weight copy is kept as
+// W and W^T.  Weight gradients reduce over the M samples with split K (FP32
+// partials, summed in a fixed order by the parameter update).
 //
 // Features of a sample (c centroid, n normal, d incident direction, k):
 //   c, n, d, k/12, d.n, d.c, then sin/cos(2^l pi q) for l = 0..5 and
@@ -40,186 +42,357 @@ constexpr int RAW = 10;  // c[3], n[3], d[3], k
 __device__ __forceinline__ u16 to_bf16(float f) { return Half<1>::from_float(f); }
 __device__ __forceinline__ float from_bf16(u16 v) { return Half<1>::to_float(v); }
 
-// C[z][M][N] = A[M, kz] B[N, kz]^T over the K slice z (tile 64 x 64, 4 waves of 32 x 32).
-__global__ __launch_bounds__(BLOCK) void mlp_gemm_kernel(const u16* __restrict__ A, int lda, const u16* __restrict__ B,
-                                                         int ldb, int M, int N, int kslice, float* __restrict__ C) {
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int m0 = blockIdx.x * 64 + 32 * (wave >> 1);
-    const int n0 = blockIdx.y * 64 + 32 * (wave & 1);
-    const int64_t k0 = (int64_t)blockIdx.z * kslice;
-    const int kq = (lane >> 5) * 8;
-    const u16* ap = A + (int64_t)(m0 + (lane & 31)) * lda + k0 + kq;
-    const u16* bp = B + (int64_t)(n0 + (lane & 31)) * ldb + k0 + kq;
-    f32x16 acc;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-    for (int k = 0; k < kslice; k += 16) {
-        const u32x4 a = *reinterpret_cast<const u32x4*>(ap + k);
-        const u32x4 b = *reinterpret_cast<const u32x4*>(bp + k);
-        acc = mfma32<1>(a, b, acc);
-    }
-    float* out = C + (int64_t)blockIdx.z * M * N;
-    const int col = n0 + (lane & 31);
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = m0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        out[(int64_t)row * N + col] = acc[v];
-    }
-}
-
-// The 64 features of one raw sample {c, n, d, k} (FEAT_USED used, zero padded).
-__device__ __forceinline__ void sample_features(const float* __restrict__ r, float* f) {
-    const float c0 = r[0], c1 = r[1], c2 = r[2], n0 = r[3], n1 = r[4], n2 = r[5], d0 = r[6], d1 = r[7], d2 = r[8];
-    const float kk = r[9] * (1.0f / 12.0f);
-    const float dc = d0 * c0 + d1 * c1 + d2 * c2;
-    const float dn = d0 * n0 + d1 * n1 + d2 * n2;
-    f[0] = c0; f[1] = c1; f[2] = c2;
-    f[3] = n0; f[4] = n1; f[5] = n2;
-    f[6] = d0; f[7] = d1; f[8] = d2;
-    f[9] = kk; f[10] = dn; f[11] = dc;
-    const float q[4] = {dc, dn, kk, kk * dc};
-    int o = 12;
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        float w = 3.14159265358979f;
-#pragma unroll
-        for (int l = 0; l < 6; ++l) {
-            f[o++] = sinf(w * q[a]);
-            f[o++] = cosf(w * q[a]);
-            w *= 2.0f;
-        }
-    }
-#pragma unroll
-    for (int j = FEAT_USED; j < FEAT; ++j) f[j] = 0.f;
-}
-
-// Features of samples idx[0..M) (or 0..M when idx is null) -> X (M x 64) and
-// X^T (64 x M; not written when XT is null, as in inference).
-__global__ void mlp_features_kernel(const float* __restrict__ raw, const int64_t* __restrict__ idx, int M,
-                                    u16* __restrict__ X, u16* __restrict__ XT) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= M) return;
-    float f[FEAT];
-    sample_features(raw + (idx ? idx[s] : s) * RAW, f);
-#pragma unroll
-    for (int j = 0; j < FEAT; ++j) {
-        const u16 h = to_bf16(f[j]);
-        X[(int64_t)s * FEAT + j] = h;
-        if (XT) XT[(int64_t)j * M + s] = h;
-    }
-}
-
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float silu_grad(float x) {
     const float sg = 1.0f / (1.0f + expf(-x));
     return sg * (1.0f + x * (1.0f - sg));
 }
 
-// H = sum of nsplit partials + bias (FP32, kept for the backward pass);
-// A = silu(H) in BF16, row-major and transposed (H and AT are null in
-// inference: only training reads them).
-__global__ void mlp_bias_act_kernel(const float* __restrict__ part, int nsplit, const float* __restrict__ bias, int M,
-                                    int N, float* __restrict__ H, u16* __restrict__ A, u16* __restrict__ AT) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)M * N) return;
-    const int m = (int)(t / N), j = (int)(t % N);
-    float h = bias[j];
-    for (int z = 0; z < nsplit; ++z) h += part[(int64_t)z * M * N + t];
-    if (H) H[t] = h;
-    const u16 a = to_bf16(silu(h));
-    A[t] = a;
-    if (AT) AT[(int64_t)j * M + m] = a;
-}
+// What a product does with its accumulators (EPI_*), and the arrays it takes.
+enum { EPI_PART, EPI_ACT, EPI_GRAD, EPI_OUT };
+struct GemmArgs {
+    const u16* A;
+    const u16* B;
+    int lda, ldb, M, N, K;
+    int kslice;          // K range of a block (a multiple of 64), blockIdx.z the slice
+    float* C;            // EPI_PART: partials, one M x N slab per slice
+    const float* bias;   // EPI_ACT, EPI_OUT
+    float* G;            // EPI_ACT: silu'(H), written; EPI_GRAD: the same, read (null: not kept)
+    u16* Y;              // EPI_ACT: silu(H); EPI_GRAD, EPI_OUT: dZ.  M x N
+    u16* YT;             // the same, N x M (null: not kept)
+    float* colsum;       // EPI_GRAD, EPI_OUT: sums of dZ over each 64 or 32 rows (half a row tile), [half tile][N]
+    const float* targets;
+    const int64_t* idx;  // EPI_OUT: sample of each row (null: the row)
+    float* out;          // EPI_OUT: M x 2
+    double* loss;        // EPI_OUT: one partial per block
+};
 
-// Output layer: Y = partial sum + bias (first 2 of 64 padded columns);
-// loss = sum (Y - T)^2 / (2 M); dZ = (Y - T) / M in BF16 (both layouts, zero
-// in the padded columns); loss partial per block.
-__global__ void mlp_output_kernel(const float* __restrict__ part, int nsplit, const float* __restrict__ bias, int M,
-                                  const float* __restrict__ targets, const int64_t* __restrict__ idx,
-                                  float* __restrict__ Y, u16* __restrict__ dZ, u16* __restrict__ dZT,
-                                  double* __restrict__ loss_part) {
-    __shared__ double sh[BLOCK];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double l = 0.0;
-    if (t < (int64_t)M * OUT_PAD) {
-        const int m = (int)(t / OUT_PAD), j = (int)(t % OUT_PAD);
-        u16 g = 0;
-        if (j < 2) {
-            float y = bias[j];
-            for (int z = 0; z < nsplit; ++z) y += part[(int64_t)z * M * OUT_PAD + t];
-            Y[(int64_t)m * 2 + j] = y;
-            if (targets) {
-                const float e = y - targets[(idx ? idx[m] : m) * 2 + j];
-                l = 0.5 * (double)e * (double)e;
-                g = to_bf16(e / (float)M);
+// C = A B^T on v_mfma_f32_32x32x16_bf16.  What bounds it at the training sizes
+// (16384 x 512 x 512: 8.6 GFLOP against 17 MB in and, with the FP32 derivative,
+// 67 MB out) is the epilogue's memory traffic; the tile keeps the MFMAs from
+// adding to it.  A block of four waves takes TM x TN outputs (2 x 2 waves), K in
+// stages of 64 through two LDS buffers, the next stage's pieces in registers
+// while one is multiplied.  LDS rows are 72 halves, so the 16-byte operand
+// reads of 16 consecutive lanes fall in distinct banks.  Every output
+// accumulates its products in order of k, 16 at a time, as the fused inference
+// kernel does.  Lane l holds column l % 32 and, per accumulator group, four
+// consecutive rows: the transposed copy is stored 8 bytes at a time.
+// At 16384 x 512 x 512 the product with its epilogue takes 26 us forward and 29 us
+// backward, where a product from global memory and separate elementwise passes
+// took 42 + 46 and 42 + 52; a weight gradient takes 21 us instead of 42.
+template <int TM, int TN, int EPI>
+__global__ __launch_bounds__(BLOCK, 2) void mlp_gemm_kernel(GemmArgs g) {
+    constexpr int LR = 64 + 8;
+    constexpr int WM = TM / 2, WN = TN / 2, MT = WM / 32, NT = WN / 32;
+    constexpr int AP = TM * 8 / BLOCK, BP = TN * 8 / BLOCK;  // 16-byte pieces per thread per stage
+    __shared__ __attribute__((aligned(16))) u16 As[2][TM * LR];
+    __shared__ __attribute__((aligned(16))) u16 Bs[2][TN * LR];
+    const int t = threadIdx.x;
+    const int lane = t & 63;
+    const int wm = t >> 7, wn = (t >> 6) & 1;
+    const int m0 = blockIdx.x * TM, n0 = blockIdx.y * TN;
+    const int kb = blockIdx.z * g.kslice, ke = min(g.K, kb + g.kslice);
+    const u16* ap = g.A + (int64_t)(m0 + (t >> 3)) * g.lda + (t & 7) * 8;
+    const u16* bp = g.B + (int64_t)(n0 + (t >> 3)) * g.ldb + (t & 7) * 8;
+    u32x4 ra[AP], rb[BP];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int i = 0; i < AP; ++i) ra[i] = *reinterpret_cast<const u32x4*>(ap + (int64_t)32 * i * g.lda + k);
+#pragma unroll
+        for (int i = 0; i < BP; ++i) rb[i] = *reinterpret_cast<const u32x4*>(bp + (int64_t)32 * i * g.ldb + k);
+    };
+    auto store = [&](int buf) {
+        const int o = (t >> 3) * LR + (t & 7) * 8;
+#pragma unroll
+        for (int i = 0; i < AP; ++i) *reinterpret_cast<u32x4*>(&As[buf][o + 32 * i * LR]) = ra[i];
+#pragma unroll
+        for (int i = 0; i < BP; ++i) *reinterpret_cast<u32x4*>(&Bs[buf][o + 32 * i * LR]) = rb[i];
+    };
+    f32x16 acc[MT][NT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
+    load(kb);
+    // the output layer's targets of this block's rows, gathered behind the product
+    __shared__ float2 tg[EPI == EPI_OUT ? TM : 1];
+    if (EPI == EPI_OUT && g.targets && t < TM) {
+        const int64_t at = g.idx ? g.idx[m0 + t] : m0 + t;
+        tg[t] = make_float2(g.targets[2 * at], g.targets[2 * at + 1]);
+    }
+    store(0);
+    int buf = 0;
+    for (int k = kb; k < ke; k += 64) {
+        __syncthreads();  // this stage is in LDS, and every wave is done with the other buffer
+        const bool more = k + 64 < ke;
+        if (more) load(k + 64);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int ko = 16 * s + 8 * (lane >> 5);
+            u32x4 av[MT], bv[NT];
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+                av[a] = *reinterpret_cast<const u32x4*>(&As[buf][(wm * WM + 32 * a + (lane & 31)) * LR + ko]);
+#pragma unroll
+            for (int b = 0; b < NT; ++b)
+                bv[b] = *reinterpret_cast<const u32x4*>(&Bs[buf][(wn * WN + 32 * b + (lane & 31)) * LR + ko]);
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int b = 0; b < NT; ++b) acc[a][b] = mfma32<1>(av[a], bv[b], acc[a][b]);
+        }
+        buf ^= 1;
+        if (more) store(buf);
+    }
+    // silu' of one 32 x 32 tile, loaded ahead of the stores of the tile before it
+    float gv[2][16];
+    auto load_grad = [&](int a, int b, float* v) {
+        const float* __restrict__ p = g.G + (int64_t)(m0 + wm * WM + 32 * a + 4 * (lane >> 5)) * g.N + n0 + wn * WN +
+                                      32 * b + (lane & 31);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[4 * q + r] = p[(int64_t)(8 * q + r) * g.N];
+    };
+    if (EPI == EPI_GRAD) load_grad(0, 0, gv[0]);
+    double loss = 0.0;
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+        const int col = n0 + wn * WN + 32 * b + (lane & 31);
+        const float bias = EPI == EPI_ACT || (EPI == EPI_OUT && col < 2) ? g.bias[col] : 0.f;
+        float sum = 0.f;
+#pragma unroll
+        for (int a = 0; a < MT; ++a) {
+            const int tile = b * MT + a;
+            if (EPI == EPI_GRAD && tile + 1 < MT * NT) load_grad((tile + 1) % MT, (tile + 1) / MT, gv[(tile + 1) & 1]);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int row = m0 + wm * WM + 32 * a + 8 * q + 4 * (lane >> 5);
+                u16 y[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float x = acc[a][b][4 * q + r];
+                    const int64_t o = (int64_t)(row + r) * g.N + col;
+                    if (EPI == EPI_PART) {
+                        g.C[(int64_t)blockIdx.z * g.M * g.N + o] = x;
+                    } else if (EPI == EPI_ACT) {
+                        const float h = bias + x;
+                        const float e = 1.0f + expf(-h);
+                        y[r] = to_bf16(h / e);
+                        g.Y[o] = y[r];
+                        if (g.G) {
+                            const float sg = 1.0f / e;
+                            g.G[o] = sg * (1.0f + h * (1.0f - sg));
+                        }
+                    } else if (EPI == EPI_GRAD) {
+                        y[r] = to_bf16(x * gv[tile & 1][4 * q + r]);
+                        g.Y[o] = y[r];
+                        sum += from_bf16(y[r]);
+                    } else {
+                        y[r] = 0;
+                        if (col < 2) {
+                            const float v = bias + x;
+                            g.out[(int64_t)(row + r) * 2 + col] = v;
+                            if (g.targets) {
+                                const float2 w = tg[row + r - m0];
+                                const float e = v - (col == 0 ? w.x : w.y);
+                                loss += 0.5 * (double)e * (double)e;
+                                y[r] = to_bf16(e / (float)g.M);
+                            }
+                        }
+                        if (g.Y) g.Y[o] = y[r];
+                        sum += from_bf16(y[r]);
+                    }
+                }
+                if (EPI != EPI_PART && g.YT) {
+                    const uint2 w = make_uint2((unsigned)y[0] | ((unsigned)y[1] << 16),
+                                               (unsigned)y[2] | ((unsigned)y[3] << 16));
+                    *reinterpret_cast<uint2*>(&g.YT[(int64_t)col * g.M + row]) = w;
+                }
             }
         }
-        if (dZ) {
-            dZ[t] = g;
-            dZT[(int64_t)j * M + m] = g;
+        if ((EPI == EPI_GRAD || EPI == EPI_OUT) && g.colsum) {
+            sum += __shfl_xor(sum, 32, 64);
+            if (lane < 32) g.colsum[(int64_t)(blockIdx.x * 2 + wm) * g.N + col] = sum;
         }
     }
-    sh[threadIdx.x] = l;
-    __syncthreads();
-    for (int s = BLOCK / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+    if (EPI == EPI_OUT && g.loss) {
+        __shared__ double part[4];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+        if (lane == 0) part[t >> 6] = loss;
         __syncthreads();
+        if (t == 0) g.loss[blockIdx.x] = (part[0] + part[1]) + (part[2] + part[3]);
     }
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = sh[0];
 }
 
-// dZ = dA * silu'(H) from the summed partials of dA; BF16 in both layouts.
-__global__ void mlp_act_grad_kernel(const float* __restrict__ part, int nsplit, const float* __restrict__ H, int M,
-                                    int N, u16* __restrict__ dZ, u16* __restrict__ dZT) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)M * N) return;
-    const int m = (int)(t / N), j = (int)(t % N);
-    float da = 0.f;
-    for (int z = 0; z < nsplit; ++z) da += part[(int64_t)z * M * N + t];
-    const u16 g = to_bf16(da * silu_grad(H[t]));
-    dZ[t] = g;
-    dZT[(int64_t)j * M + m] = g;
+// Features 2j and 2j + 1 (j < 32) of one raw sample {c, n, d, k}: FEAT_USED
+// used, zero padded.  The sums are explicit FMAs, so every kernel forms the
+// same bits.
+__device__ __forceinline__ float2 sample_feature_pair(const float* __restrict__ r, int j) {
+    if (j >= FEAT_USED / 2) return make_float2(0.f, 0.f);
+    const float kk = r[9] * (1.0f / 12.0f);
+    const float dc = fmaf(r[8], r[2], fmaf(r[7], r[1], r[6] * r[0]));
+    const float dn = fmaf(r[8], r[5], fmaf(r[7], r[4], r[6] * r[3]));
+    if (j < 4) return make_float2(r[2 * j], r[2 * j + 1]);
+    if (j == 4) return make_float2(r[8], kk);
+    if (j == 5) return make_float2(dn, dc);
+    const int a = (j - 6) / 6, l = (j - 6) % 6;
+    const float q = a == 0 ? dc : a == 1 ? dn : a == 2 ? kk : kk * dc;
+    const float x = (3.14159265358979f * (float)(1 << l)) * q;
+    return make_float2(sinf(x), cosf(x));
 }
 
-// out[t] = sum over the nsplit partial slabs (slab stride `stride`) for t < count;
-// count may be a prefix of the slab (the real rows of a padded layer).
-__global__ void mlp_sum_kernel(const float* __restrict__ part, int nsplit, int64_t stride, int64_t count,
-                               float* __restrict__ out) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    float s = 0.f;
-    for (int z = 0; z < nsplit; ++z) s += part[(int64_t)z * stride + t];
-    out[t] = s;
+__device__ __forceinline__ unsigned pack_bf16(float2 f) {
+    return (unsigned)to_bf16(f.x) | ((unsigned)to_bf16(f.y) << 16);
 }
 
-// Bias gradient: row sums of dZ^T (N x M), one block per row, fixed order.
-__global__ __launch_bounds__(BLOCK) void mlp_bias_grad_kernel(const u16* __restrict__ dZT, int M, float* __restrict__ out) {
-    __shared__ float sh[BLOCK];
-    const u16* row = dZT + (int64_t)blockIdx.x * M;
-    float s = 0.f;
-    for (int m = threadIdx.x; m < M; m += BLOCK) s += from_bf16(row[m]);
-    sh[threadIdx.x] = s;
+// Sample of row s of step `seed`: hash(seed, s) mod count.
+__device__ __forceinline__ int64_t sample_index(uint64_t seed, int s, int64_t count) {
+    uint64_t z = seed + 0x9E3779B97F4A7C15ull * (uint64_t)(s + 1);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    return (int64_t)(z % (uint64_t)count);
+}
+
+// Features of M rows -> X (M x 64) and X^T (64 x M; not written when XT is null,
+// as in inference).  With idx the rows are samples drawn by sample_index and
+// left in idx; without it row s is sample s.  A thread takes one feature pair
+// of a sample (32 threads a sample: one sine and cosine each), a block 64
+// samples, whose transposed copy leaves through LDS.
+constexpr int FEAT_ROWS = 64;
+__global__ __launch_bounds__(BLOCK) void mlp_features_kernel(const float* __restrict__ raw, int64_t* __restrict__ idx,
+                                                             uint64_t seed, int64_t count, int M,
+                                                             u16* __restrict__ X, u16* __restrict__ XT) {
+    __shared__ unsigned sh[FEAT_ROWS][33];
+    const int s0 = blockIdx.x * FEAT_ROWS;
+    const int j = threadIdx.x & 31;
+#pragma unroll
+    for (int i = 0; i < FEAT_ROWS * 32 / BLOCK; ++i) {
+        const int r = (threadIdx.x >> 5) + i * (BLOCK / 32);
+        const int s = s0 + r;
+        if (s >= M) break;
+        const int64_t at = idx ? sample_index(seed, s, count) : s;
+        if (idx && j == 0) idx[s] = at;
+        const unsigned w = pack_bf16(sample_feature_pair(raw + at * RAW, j));
+        reinterpret_cast<unsigned*>(X)[(int64_t)s * (FEAT / 2) + j] = w;
+        sh[r][j] = w;
+    }
+    if (!XT) return;
     __syncthreads();
-    for (int k = BLOCK / 2; k > 0; k >>= 1) {
-        if (threadIdx.x < k) sh[threadIdx.x] += sh[threadIdx.x + k];
-        __syncthreads();
+    // 8 samples of one feature per thread and pass
+#pragma unroll
+    for (int i = 0; i < FEAT * (FEAT_ROWS / 8) / BLOCK; ++i) {
+        const int e = threadIdx.x + i * BLOCK;
+        const int f = e >> 3, r0 = (e & 7) * 8;
+        if (s0 + r0 >= M) continue;  // M is a multiple of 8
+        u32x4 w;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const unsigned lo = sh[r0 + 2 * v][f >> 1], hi = sh[r0 + 2 * v + 1][f >> 1];
+            w[v] = (f & 1) ? (lo >> 16) | (hi & 0xffff0000u) : (lo & 0xffffu) | (hi << 16);
+        }
+        *reinterpret_cast<u32x4*>(&XT[(int64_t)f * M + s0 + r0]) = w;
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
 }
 
-// Adam on the FP32 master parameters (t = step number from 1).
-__global__ void mlp_adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m1,
-                                float* __restrict__ m2, int64_t count, float lr, float b1, float b2, float eps,
-                                float c1, float c2) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count) return;
-    const float gr = g[t];
-    const float a = b1 * m1[t] + (1.f - b1) * gr;
-    const float b = b2 * m2[t] + (1.f - b2) * gr * gr;
-    m1[t] = a;
-    m2[t] = b;
-    p[t] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
+// One layer of the parameter update, for every layer in one launch
+// (blockIdx.y): the gradient of each weight is the sum of its split-K partials
+// in slice order, that of each bias the sum of its column partials.  ADAM steps
+// the FP32 master parameters and refreshes the BF16 copies W and W^T; without it
+// the gradients are written out.  A block takes a 32 x 32 weight tile (the
+// transposed copy leaves through LDS) or, past the tiles, 32 biases.
+constexpr int kSplitW = 16;  // at most so many K slices (samples) of the weight-gradient products
+struct UpdateLayer {
+    const float* part;    // nsplit slabs of prow x cols
+    const float* colsum;  // nsum rows of prow
+    int rows, cols, prow, nsum;
+    int64_t w_off, b_off;
+    u16* W;
+    u16* WT;
+};
+struct UpdateArgs {
+    UpdateLayer layer[4];
+    int nsplit;
+    float *p, *m1, *m2, *grads;
+    float lr, b1, b2, eps, c1, c2;
+};
+
+__device__ __forceinline__ float adam_step(const UpdateArgs& u, int64_t t, float gr) {
+    const float a = u.b1 * u.m1[t] + (1.f - u.b1) * gr;
+    const float b = u.b2 * u.m2[t] + (1.f - u.b2) * gr * gr;
+    u.m1[t] = a;
+    u.m2[t] = b;
+    const float p = u.p[t] - u.lr * (a / u.c1) / (sqrtf(b / u.c2) + u.eps);
+    u.p[t] = p;
+    return p;
+}
+
+template <bool ADAM>
+__global__ __launch_bounds__(BLOCK) void mlp_update_kernel(UpdateArgs u) {
+    const UpdateLayer& l = u.layer[blockIdx.y];
+    const int tr = (l.rows + 31) / 32, tc = l.cols / 32;
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+    int b = blockIdx.x;
+    if (b < tr * tc) {
+        __shared__ u16 sh[32][34];
+        const int r0 = (b / tc) * 32, c = (b % tc) * 32 + x;
+        const int64_t slab = (int64_t)l.prow * l.cols;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + y + 8 * i;
+            if (r < l.rows) {
+                const int64_t o = (int64_t)r * l.cols + c;
+                float v[kSplitW];
+#pragma unroll
+                for (int z = 0; z < kSplitW; ++z) v[z] = z < u.nsplit ? l.part[z * slab + o] : 0.f;
+                float g = 0.f;
+#pragma unroll
+                for (int z = 0; z < kSplitW; ++z)
+                    if (z < u.nsplit) g += v[z];
+                if (ADAM) {
+                    const u16 h = to_bf16(adam_step(u, l.w_off + o, g));
+                    l.W[o] = h;
+                    sh[y + 8 * i][x] = h;
+                } else {
+                    u.grads[l.w_off + o] = g;
+                }
+            }
+        }
+        if (ADAM) {
+            __syncthreads();
+            const int r = r0 + x;
+            if (r < l.rows)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int cc = y + 8 * i;
+                    l.WT[(int64_t)((b % tc) * 32 + cc) * l.prow + r] = sh[x][cc];
+                }
+        }
+        return;
+    }
+    b -= tr * tc;
+    if (b >= tr) return;
+    __shared__ float bs[8][32];
+    const int col = b * 32 + x;
+    float s = 0.f;
+    if (col < l.rows)
+#pragma unroll 8
+        for (int z = y; z < l.nsum; z += 8) s += l.colsum[(int64_t)z * l.prow + col];
+    bs[y][x] = s;
+    __syncthreads();
+    if (y == 0 && col < l.rows) {
+        float g = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) g += bs[i][x];
+        if (ADAM)
+            (void)adam_step(u, l.b_off + col, g);
+        else
+            u.grads[l.b_off + col] = g;
+    }
 }
 
 // BF16 copies W (rows x cols, padded to prow rows) and W^T (cols x prow).
@@ -231,17 +404,6 @@ __global__ void mlp_cast_kernel(const float* __restrict__ w, int rows, int cols,
     const u16 h = r < rows ? to_bf16(w[(int64_t)r * cols + c]) : (u16)0;
     W[t] = h;
     WT[(int64_t)c * prow + r] = h;
-}
-
-// Sample indices for a step: idx[s] = hash(seed, step, s) mod count.
-__global__ void mlp_sample_kernel(int64_t* __restrict__ idx, int M, uint64_t seed, int64_t count) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= M) return;
-    uint64_t z = seed + 0x9E3779B97F4A7C15ull * (uint64_t)(s + 1);
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    idx[s] = (int64_t)(z % (uint64_t)count);
 }
 
 inline unsigned nb(int64_t n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
@@ -271,11 +433,10 @@ __global__ __launch_bounds__(BLOCK) void mlp_infer_kernel(const float* __restric
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int64_t s0 = (int64_t)blockIdx.x * INFER_ROWS;
-    if (threadIdx.x < INFER_ROWS) {
-        float f[FEAT];
-        sample_features(raw + (s0 + threadIdx.x) * RAW, f);
 #pragma unroll
-        for (int j = 0; j < FEAT; ++j) src[threadIdx.x * ldr + j] = to_bf16(f[j]);
+    for (int i = 0; i < INFER_ROWS * 32 / BLOCK; ++i) {
+        const int r = (threadIdx.x >> 5) + i * (BLOCK / 32), j = threadIdx.x & 31;
+        *reinterpret_cast<unsigned*>(&src[r * ldr + 2 * j]) = pack_bf16(sample_feature_pair(raw + (s0 + r) * RAW, j));
     }
     __syncthreads();
     for (int l = 0; l < 4; ++l) {
@@ -358,11 +519,12 @@ struct sbh_mlp {
     int64_t step = 0;
     // batch workspace (sized for max_batch samples)
     int max_batch = 0;
+    int max_train = 0;  // and the training arrays
     sbh::DeviceArray<uint16_t> X, XT;
-    std::vector<sbh::DeviceArray<float>> H;     // pre-activations per hidden layer
+    std::vector<sbh::DeviceArray<float>> G;     // silu' of the pre-activations per hidden layer
     std::vector<sbh::DeviceArray<uint16_t>> A, AT;  // activations per hidden layer
     sbh::DeviceArray<uint16_t> dZ, dZT, dZ2, dZ2T;
-    sbh::DeviceArray<float> part, Y;
+    sbh::DeviceArray<float> part, colsum, Y;  // per layer: weight-gradient and bias-gradient partials
     sbh::DeviceArray<double> loss_part;
     sbh::DeviceArray<int64_t> idx;
     sbh::DeviceArray<float> raw_ws;  // raw inputs of device-side predictions
@@ -378,40 +540,83 @@ inline sbh_context* ctx_of(const sbh_mlp* n) { return n ? n->ctx : nullptr; }
 namespace sbh {
 namespace {
 
-constexpr int kSplitW = 16;  // split K (samples) of the weight-gradient products
+constexpr int kLossSteps = 256;  // steps whose loss partials stay on the device between reads
 
-void gemm(sbh_context* ctx, const uint16_t* A, int lda, const uint16_t* B, int ldb, int M, int N, int K, int splits,
-          float* C) {
-    SBH_REQUIRE(M % 64 == 0 && N % 64 == 0 && K % (16 * splits) == 0, "MLP GEMM shape is not tile aligned");
-    dim3 grid(M / 64, N / 64, splits);
-    hipLaunchKernelGGL(mlp_gemm_kernel, grid, dim3(BLOCK), 0, ctx->stream, reinterpret_cast<const u16*>(A), lda,
-                       reinterpret_cast<const u16*>(B), ldb, M, N, K / splits, C);
+// K slices of the weight-gradient products over M samples: whole stages of 64.
+int weight_slice(int M) { return (M / 64 + kSplitW - 1) / kSplitW * 64; }
+int weight_splits(int M) { return (M + weight_slice(M) - 1) / weight_slice(M); }
+
+// The product's tile: 128 x 128, or 64 where a side is no multiple of 128 or the
+// larger tiles leave more than half of the 256 CUs without a block (batches
+// below 4096 at width 512).
+template <int EPI>
+int gemm(sbh_context* ctx, const GemmArgs& g) {
+    SBH_REQUIRE(g.M % 64 == 0 && g.N % 64 == 0 && g.K % 64 == 0 && g.kslice % 64 == 0,
+                "MLP GEMM shape is not tile aligned");
+    const int z = (g.K + g.kslice - 1) / g.kslice;
+    const bool small = (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * z < 192;
+    const bool m128 = g.M % 128 == 0 && !small, n128 = g.N % 128 == 0 && !small;
+    const dim3 grid(g.M / (m128 ? 128 : 64), g.N / (n128 ? 128 : 64), z);
+    if (m128 && n128)
+        hipLaunchKernelGGL((mlp_gemm_kernel<128, 128, EPI>), grid, dim3(BLOCK), 0, ctx->stream, g);
+    else if (m128)
+        hipLaunchKernelGGL((mlp_gemm_kernel<128, 64, EPI>), grid, dim3(BLOCK), 0, ctx->stream, g);
+    else if (n128)
+        hipLaunchKernelGGL((mlp_gemm_kernel<64, 128, EPI>), grid, dim3(BLOCK), 0, ctx->stream, g);
+    else
+        hipLaunchKernelGGL((mlp_gemm_kernel<64, 64, EPI>), grid, dim3(BLOCK), 0, ctx->stream, g);
     SBH_HIP(hipGetLastError());
+    return (int)grid.x;  // row tiles
 }
 
-void ensure_batch(sbh_mlp* net, int M) {
-    if (M <= net->max_batch) return;
+GemmArgs gemm_args(const uint16_t* A, int lda, const uint16_t* B, int ldb, int M, int N, int K, int kslice) {
+    GemmArgs g;
+    std::memset(&g, 0, sizeof(g));
+    g.A = reinterpret_cast<const u16*>(A);
+    g.B = reinterpret_cast<const u16*>(B);
+    g.lda = lda;
+    g.ldb = ldb;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.kslice = kslice;
+    return g;
+}
+
+void ensure_batch(sbh_mlp* net, int M, bool training) {
     const int W = net->width;
-    net->X.allocate((size_t)M * FEAT);
+    if (M > net->max_batch) {
+        net->max_batch = 0;  // a failed allocation below leaves no stale size
+        net->max_train = 0;
+        net->X.allocate((size_t)M * FEAT);
+        net->A.clear();
+        for (int l = 0; l < net->layers - 1; ++l) net->A.emplace_back((size_t)M * W);
+        net->Y.allocate((size_t)M * 2);
+        net->max_batch = M;
+    }
+    if (!training || M <= net->max_train) return;
+    net->max_train = 0;
     net->XT.allocate((size_t)M * FEAT);
-    net->H.clear();
-    net->A.clear();
+    net->G.clear();
     net->AT.clear();
     for (int l = 0; l < net->layers - 1; ++l) {
-        net->H.emplace_back((size_t)M * W);
-        net->A.emplace_back((size_t)M * W);
+        net->G.emplace_back((size_t)M * W);
         net->AT.emplace_back((size_t)M * W);
     }
     net->dZ.allocate((size_t)M * W);
     net->dZT.allocate((size_t)M * W);
     net->dZ2.allocate((size_t)M * W);
     net->dZ2T.allocate((size_t)M * W);
-    const size_t wpart = (size_t)kSplitW * W * W;
-    net->part.allocate(std::max<size_t>((size_t)M * W, wpart));
-    net->Y.allocate((size_t)M * 2);
-    net->loss_part.allocate(nb((int64_t)M * OUT_PAD));
+    size_t weights = 0, biases = 0;
+    for (const auto& ly : net->L) {
+        weights += (size_t)ly.prow * ly.cols;
+        biases += (size_t)ly.prow;
+    }
+    net->part.allocate((size_t)kSplitW * weights);
+    net->colsum.allocate((size_t)(M / 32) * biases);
+    net->loss_part.allocate((size_t)(M / 64) * kLossSteps);
     net->idx.allocate((size_t)M);
-    net->max_batch = M;
+    net->max_train = M;
 }
 
 void refresh_weights(sbh_mlp* net) {
@@ -425,72 +630,110 @@ void refresh_weights(sbh_mlp* net) {
     }
 }
 
-// Forward pass over M samples (inputs raw, optional gather idx); with targets
-// also the loss and the backward pass into net->grads.  Returns the loss
-// partials' block count (0 without targets).
-int forward_backward(sbh_mlp* net, const float* raw, const int64_t* idx, int M, const float* targets, bool backward) {
+// Forward pass over M samples; with targets also the loss partials (one per
+// row tile, at `loss`) and the backward pass, whose gradient partials are left
+// for `update`.  With draw, row s takes dataset sample sample_index(seed, s,
+// count).  Returns the number of loss partials (0 without targets).
+int forward_backward(sbh_mlp* net, const float* raw, bool draw, uint64_t seed, int64_t count, int M,
+                     const float* targets, double* loss, UpdateArgs* update) {
     sbh_context* ctx = net->ctx;
     const int W = net->width;
-    // the transposed activations, pre-activations and output gradients only
-    // feed the backward pass
+    const int last = net->layers - 1;
+    auto u = [](uint16_t* p) { return reinterpret_cast<u16*>(p); };
+    // the transposed activations, derivatives and output gradients only feed
+    // the backward pass
     const bool keep = targets != nullptr;
-    hipLaunchKernelGGL(mlp_features_kernel, dim3(nb(M)), dim3(BLOCK), 0, ctx->stream, raw, idx, M,
-                       reinterpret_cast<u16*>(net->X.ptr), keep ? reinterpret_cast<u16*>(net->XT.ptr) : nullptr);
+    hipLaunchKernelGGL(mlp_features_kernel, dim3((M + FEAT_ROWS - 1) / FEAT_ROWS), dim3(BLOCK), 0, ctx->stream, raw,
+                       draw ? net->idx.ptr : nullptr, seed, count, M, u(net->X.ptr), keep ? u(net->XT.ptr) : nullptr);
     SBH_HIP(hipGetLastError());
     const uint16_t* in = net->X.ptr;
     int in_dim = FEAT;
-    for (int l = 0; l < net->layers - 1; ++l) {
-        const mlp::Layer& ly = net->L[l];
-        gemm(ctx, in, in_dim, net->Wb.ptr + net->wb_off[l], in_dim, M, W, in_dim, 1, net->part.ptr);
-        hipLaunchKernelGGL(mlp_bias_act_kernel, dim3(nb((int64_t)M * W)), dim3(BLOCK), 0, ctx->stream, net->part.ptr,
-                           1, net->params.ptr + ly.b_off, M, W, keep ? net->H[l].ptr : nullptr,
-                           reinterpret_cast<u16*>(net->A[l].ptr),
-                           keep ? reinterpret_cast<u16*>(net->AT[l].ptr) : nullptr);
-        SBH_HIP(hipGetLastError());
+    for (int l = 0; l < last; ++l) {
+        GemmArgs g = gemm_args(in, in_dim, net->Wb.ptr + net->wb_off[l], in_dim, M, W, in_dim, in_dim);
+        g.bias = net->params.ptr + net->L[l].b_off;
+        g.G = keep ? net->G[l].ptr : nullptr;
+        g.Y = u(net->A[l].ptr);
+        g.YT = keep ? u(net->AT[l].ptr) : nullptr;
+        gemm<EPI_ACT>(ctx, g);
         in = net->A[l].ptr;
         in_dim = W;
     }
-    const mlp::Layer& lo = net->L[net->layers - 1];
-    gemm(ctx, in, W, net->Wb.ptr + net->wb_off[net->layers - 1], W, M, OUT_PAD, W, 1, net->part.ptr);
-    const int blocks = (int)nb((int64_t)M * OUT_PAD);
-    hipLaunchKernelGGL(mlp_output_kernel, dim3(blocks), dim3(BLOCK), 0, ctx->stream, net->part.ptr, 1,
-                       net->params.ptr + lo.b_off, M, targets, idx, net->Y.ptr,
-                       keep ? reinterpret_cast<u16*>(net->dZ.ptr) : nullptr,
-                       keep ? reinterpret_cast<u16*>(net->dZT.ptr) : nullptr, net->loss_part.ptr);
-    SBH_HIP(hipGetLastError());
-    if (!targets || !backward) return targets ? blocks : 0;
-    SBH_REQUIRE(M % (16 * kSplitW) == 0, "training batch must be a multiple of 256 samples");
-    // backward, last layer first; dZ/dZT hold the current layer's gradient, width = its output size
+    GemmArgs out = gemm_args(in, W, net->Wb.ptr + net->wb_off[last], W, M, OUT_PAD, W, W);
+    out.bias = net->params.ptr + net->L[last].b_off;
+    out.out = net->Y.ptr;
+    if (!keep) {
+        gemm<EPI_OUT>(ctx, out);
+        return 0;
+    }
+    SBH_REQUIRE(M % 256 == 0, "training batch must be a multiple of 256 samples");
+    const int splits = weight_splits(M);
+    std::memset(update, 0, sizeof(*update));
+    update->nsplit = splits;
+    float* part = net->part.ptr;
+    float* colsum = net->colsum.ptr;
+    for (int l = 0; l <= last; ++l) {
+        const mlp::Layer& ly = net->L[l];
+        UpdateLayer& ul = update->layer[l];
+        ul.part = part;
+        ul.colsum = colsum;
+        ul.rows = ly.rows;
+        ul.cols = ly.cols;
+        ul.prow = ly.prow;
+        ul.w_off = ly.w_off;
+        ul.b_off = ly.b_off;
+        ul.W = u(net->Wb.ptr + net->wb_off[l]);
+        ul.WT = u(net->WTb.ptr + net->wb_off[l]);
+        ul.nsum = 0;
+        part += (size_t)kSplitW * ly.prow * ly.cols;
+        colsum += (size_t)(M / 32) * ly.prow;
+    }
+    out.targets = targets;
+    out.idx = draw ? net->idx.ptr : nullptr;
+    out.Y = u(net->dZ.ptr);
+    out.YT = u(net->dZT.ptr);
+    out.colsum = const_cast<float*>(update->layer[last].colsum);
+    out.loss = loss;
+    const int blocks = gemm<EPI_OUT>(ctx, out);
+    update->layer[last].nsum = 2 * blocks;
+    // backward, last layer first; dz/dzt hold the current layer's gradient, width = its output size
     uint16_t* dz = net->dZ.ptr;
     uint16_t* dzt = net->dZT.ptr;
     uint16_t* dz_next = net->dZ2.ptr;
     uint16_t* dzt_next = net->dZ2T.ptr;
-    for (int l = net->layers - 1; l >= 0; --l) {
+    for (int l = last; l >= 0; --l) {
         const mlp::Layer& ly = net->L[l];
         const int out_dim = ly.prow;
         const int kin = ly.cols;
         const uint16_t* prevT = l == 0 ? net->XT.ptr : net->AT[l - 1].ptr;
-        // dW (out_dim x kin) = dZ^T prev ; rows >= ly.rows are padding
-        gemm(ctx, dzt, M, prevT, M, out_dim, kin, M, kSplitW, net->part.ptr);
-        // the padded rows are never read: rows x kin is a prefix of each out_dim x kin slab
-        hipLaunchKernelGGL(mlp_sum_kernel, dim3(nb((int64_t)ly.rows * kin)), dim3(BLOCK), 0, ctx->stream,
-                           net->part.ptr, kSplitW, (int64_t)out_dim * kin, (int64_t)ly.rows * kin,
-                           net->grads.ptr + ly.w_off);
-        SBH_HIP(hipGetLastError());
-        hipLaunchKernelGGL(mlp_bias_grad_kernel, dim3(ly.rows), dim3(BLOCK), 0, ctx->stream,
-                           reinterpret_cast<const u16*>(dzt), M, net->grads.ptr + ly.b_off);
-        SBH_HIP(hipGetLastError());
+        // dW (out_dim x kin) = dZ^T prev ; rows >= ly.rows are padding, never read
+        GemmArgs gw = gemm_args(dzt, M, prevT, M, out_dim, kin, M, weight_slice(M));
+        gw.C = const_cast<float*>(update->layer[l].part);
+        gemm<EPI_PART>(ctx, gw);
         if (l == 0) break;
         // dA_prev (M x kin) = dZ W  (W^T is kin x out_dim)
-        gemm(ctx, dz, out_dim, net->WTb.ptr + net->wb_off[l], out_dim, M, kin, out_dim, 1, net->part.ptr);
-        hipLaunchKernelGGL(mlp_act_grad_kernel, dim3(nb((int64_t)M * kin)), dim3(BLOCK), 0, ctx->stream,
-                           net->part.ptr, 1, net->H[l - 1].ptr, M, kin, reinterpret_cast<u16*>(dz_next),
-                           reinterpret_cast<u16*>(dzt_next));
-        SBH_HIP(hipGetLastError());
+        GemmArgs ga = gemm_args(dz, out_dim, net->WTb.ptr + net->wb_off[l], out_dim, M, kin, out_dim, out_dim);
+        ga.G = net->G[l - 1].ptr;
+        ga.Y = u(dz_next);
+        ga.YT = u(dzt_next);
+        ga.colsum = const_cast<float*>(update->layer[l - 1].colsum);
+        update->layer[l - 1].nsum = 2 * gemm<EPI_GRAD>(ctx, ga);
         std::swap(dz, dz_next);
         std::swap(dzt, dzt_next);
     }
     return blocks;
+}
+
+template <bool ADAM>
+void apply_update(sbh_mlp* net, UpdateArgs& u) {
+    u.p = net->params.ptr;
+    u.m1 = net->m1.ptr;
+    u.m2 = net->m2.ptr;
+    u.grads = net->grads.ptr;
+    const int W = net->width;
+    const unsigned blocks = (unsigned)(W / 32 * (W / 32) + W / 32);  // the widest layer's tiles and biases
+    hipLaunchKernelGGL(mlp_update_kernel<ADAM>, dim3(std::max(blocks, 64u), net->layers), dim3(BLOCK), 0,
+                       net->ctx->stream, u);
+    SBH_HIP(hipGetLastError());
 }
 
 // Predictions of Mp samples (a multiple of 256) into net->Y: the fused
@@ -499,8 +742,8 @@ int forward_backward(sbh_mlp* net, const float* raw, const int64_t* idx, int M, 
 void infer(sbh_mlp* net, const float* raw, int Mp) {
     const int W = net->width;
     if (W > 4 * INFER_MAX_TILES * 32) {
-        ensure_batch(net, Mp);
-        forward_backward(net, raw, nullptr, Mp, nullptr, false);
+        ensure_batch(net, Mp, false);
+        forward_backward(net, raw, false, 0, 0, Mp, nullptr, nullptr, nullptr);
         return;
     }
     if ((int64_t)net->Y.count < (int64_t)Mp * 2) net->Y.allocate((size_t)Mp * 2);
@@ -532,14 +775,15 @@ void infer(sbh_mlp* net, const float* raw, int Mp) {
     SBH_HIP(hipGetLastError());
 }
 
-double read_loss(sbh_mlp* net, int blocks) {
-    std::vector<double> h(blocks);
-    SBH_HIP(hipMemcpyAsync(h.data(), net->loss_part.ptr, blocks * sizeof(double), hipMemcpyDeviceToHost,
-                           net->ctx->stream));
-    SBH_HIP(hipStreamSynchronize(net->ctx->stream));
-    double s = 0.0;
-    for (double v : h) s += v;
-    return s;
+// Sums of `steps` steps' loss partials (blocks each, a step's at every `stride`), added in block order.
+void read_losses(sbh_mlp* net, int steps, int stride, int blocks, double* out) {
+    std::vector<double> h((size_t)(steps - 1) * stride + blocks);
+    copy_on_stream(net->ctx, h.data(), net->loss_part.ptr, h.size() * sizeof(double), hipMemcpyDeviceToHost);
+    for (int t = 0; t < steps; ++t) {
+        double s = 0.0;
+        for (int b = 0; b < blocks; ++b) s += h[(size_t)t * stride + b];
+        out[t] = s;
+    }
 }
 
 inline void use_device(sbh_context* ctx) { SBH_HIP(hipSetDevice(ctx->device)); }
@@ -660,14 +904,17 @@ sbh_status sbh_mlp_loss_and_gradients(sbh_mlp* net, const float* inputs, const f
         SBH_REQUIRE(net && inputs && targets, "null argument");
         SBH_REQUIRE(M > 0 && M % 256 == 0 && M <= (1 << 24), "M must be a positive multiple of 256");
         use_device(net->ctx);
-        ensure_batch(net, (int)M);
+        ensure_batch(net, (int)M, true);
         DeviceArray<float> din((size_t)M * RAW), dout((size_t)M * 2);
         copy_on_stream(net->ctx, din.ptr, inputs, din.bytes(), hipMemcpyHostToDevice);
         copy_on_stream(net->ctx, dout.ptr, targets, dout.bytes(), hipMemcpyHostToDevice);
-        SBH_HIP(hipMemsetAsync(net->grads.ptr, 0, net->grads.bytes(), net->ctx->stream));
-        const int blocks = forward_backward(net, din.ptr, nullptr, (int)M, dout.ptr, true);
-        const double l = read_loss(net, blocks) / (double)M;
-        if (loss) *loss = l;
+        UpdateArgs u;
+        const int blocks =
+            forward_backward(net, din.ptr, false, 0, 0, (int)M, dout.ptr, net->loss_part.ptr, &u);
+        apply_update<false>(net, u);
+        double l = 0.0;
+        read_losses(net, 1, blocks, blocks, &l);
+        if (loss) *loss = l / (double)M;
         if (grads) copy_on_stream(net->ctx, grads, net->grads.ptr, net->grads.bytes(), hipMemcpyDeviceToHost);
     });
 }
@@ -694,24 +941,35 @@ sbh_status sbh_mlp_train(sbh_mlp* net, int64_t steps, int64_t batch, double lr_m
         SBH_REQUIRE(steps >= 0, "steps must be >= 0");
         use_device(net->ctx);
         sbh_context* ctx = net->ctx;
-        ensure_batch(net, (int)batch);
+        ensure_batch(net, (int)batch, true);
         const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+        int pending = 0, blocks = 0;  // steps whose loss partials are still on the device
         for (int64_t s = 0; s < steps; ++s) {
-            hipLaunchKernelGGL(mlp_sample_kernel, dim3(nb(batch)), dim3(BLOCK), 0, ctx->stream, net->idx.ptr,
-                               (int)batch, seed * 0x100000001B3ull + (uint64_t)net->step, net->data_count);
-            SBH_HIP(hipGetLastError());
-            const int blocks =
-                forward_backward(net, net->data_in.ptr, net->idx.ptr, (int)batch, net->data_out.ptr, true);
-            if (losses) losses[s] = read_loss(net, blocks) / (double)batch;
+            UpdateArgs u;
+            blocks = forward_backward(net, net->data_in.ptr, true, seed * 0x100000001B3ull + (uint64_t)net->step,
+                                      net->data_count, (int)batch, net->data_out.ptr,
+                                      net->loss_part.ptr + (size_t)pending * (batch / 64), &u);
             net->step += 1;
             const double frac = steps > 1 ? (double)s / (double)(steps - 1) : 0.0;
             const double lr = lr_min + 0.5 * (lr_max - lr_min) * (1.0 + std::cos(M_PI * frac));
-            const float c1 = 1.f - std::pow(b1, (float)net->step);
-            const float c2 = 1.f - std::pow(b2, (float)net->step);
-            hipLaunchKernelGGL(mlp_adam_kernel, dim3(nb(net->nparams)), dim3(BLOCK), 0, ctx->stream, net->params.ptr,
-                               net->grads.ptr, net->m1.ptr, net->m2.ptr, net->nparams, (float)lr, b1, b2, eps, c1, c2);
-            SBH_HIP(hipGetLastError());
-            refresh_weights(net);
+            u.lr = (float)lr;
+            u.b1 = b1;
+            u.b2 = b2;
+            u.eps = eps;
+            u.c1 = 1.f - std::pow(b1, (float)net->step);
+            u.c2 = 1.f - std::pow(b2, (float)net->step);
+            apply_update<true>(net, u);
+            if (++pending == kLossSteps || s + 1 == steps) {
+                // the host reads the losses of a run of steps together
+                if (losses) {
+                    std::vector<double> l((size_t)pending);
+                    read_losses(net, pending, (int)(batch / 64), blocks, l.data());
+                    for (int t = 0; t < pending; ++t) losses[s + 1 - pending + t] = l[t] / (double)batch;
+                } else {
+                    SBH_HIP(hipStreamSynchronize(ctx->stream));  // bounds the queue
+                }
+                pending = 0;
+            }
         }
         SBH_HIP(hipStreamSynchronize(ctx->stream));
     });
@@ -723,12 +981,12 @@ sbh_status sbh_debug_mlp_predict_layered(sbh_mlp* net, const float* inputs, int6
         SBH_REQUIRE(M > 0 && M <= (1 << 24), "M out of range");
         use_device(net->ctx);
         const int Mp = (int)((M + 255) / 256 * 256);
-        ensure_batch(net, Mp);
+        ensure_batch(net, Mp, false);
         DeviceArray<float> din((size_t)Mp * RAW);
         SBH_HIP(hipMemsetAsync(din.ptr, 0, din.bytes(), net->ctx->stream));
         SBH_HIP(hipMemcpyAsync(din.ptr, inputs, (size_t)M * RAW * sizeof(float), hipMemcpyHostToDevice,
                                net->ctx->stream));
-        forward_backward(net, din.ptr, nullptr, Mp, nullptr, false);
+        forward_backward(net, din.ptr, false, 0, 0, Mp, nullptr, nullptr, nullptr);
         SBH_HIP(hipMemcpyAsync(out, net->Y.ptr, (size_t)M * 2 * sizeof(float), hipMemcpyDeviceToHost,
                                net->ctx->stream));
         SBH_HIP(hipStreamSynchronize(net->ctx->stream));

@@ -131,3 +131,67 @@ def test_learned_warm_start_lowers_iterations(ctx):
         learned.append(s2.iterations)
     print("final loss", losses[-1], "zero-guess iterations", np.mean(zero), "learned", np.mean(learned))
     assert np.mean(learned) < np.mean(zero)
+
+
+@pytest.mark.parametrize("width,m", [(64, 256), (192, 768), (128, 4352), (512, 256), (512, 12544), (1088, 512)])
+def test_gradients_match_oracle_at_tile_edges(ctx, width, m):
+    """Both product tiles (64 and 128 a side), mixed ones (a width of 64 times an
+    odd number), one K slice and a short last slice: bounds of test_gradients_match_oracle."""
+    net = ws.WarmStartMLP(ctx, width=width, seed=31)
+    rng = np.random.default_rng(width + m)
+    raw = _raw(rng, m)
+    t = rng.standard_normal((m, 2)).astype(np.float32)
+    loss, g = net.loss_and_gradients(raw, t)
+    loss_ref, g_ref, _ = omlp.loss_and_gradients(net.params().astype(np.float64), width, raw, t, bf16_storage=True)
+    assert abs(loss - loss_ref) <= 1e-4 * abs(loss_ref)
+    for off, cnt in _blocks(width):
+        assert rel_fro(g[off: off + cnt], g_ref[off: off + cnt]) < 2e-2, (off, cnt)
+
+
+def _sample_indices(seed, step, batch, count):
+    with np.errstate(over="ignore"):
+        z = np.uint64(seed * 0x100000001B3 + step) + np.uint64(0x9E3779B97F4A7C15) * np.arange(1, batch + 1,
+                                                                                              dtype=np.uint64)
+        z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        return ((z ^ (z >> np.uint64(31))) % np.uint64(count)).astype(np.int64)
+
+
+@pytest.mark.parametrize("width,batch", [(64, 256), (192, 1280), (512, 8192)])
+def test_training_steps_are_adam_on_the_drawn_samples(ctx, width, batch):
+    """Two one-step runs of train() against Adam in numpy on the gradients that
+    loss_and_gradients gives for the same samples at the network's own
+    parameters (so both round the same weights to BF16), and the refreshed
+    BF16 copies against those that set_params makes.  Bound: the FP32 value of
+    1 - 0.999^t is off by 6e-8 / 1e-3, 3e-5 of a step of lr; a few ulp of the
+    parameters."""
+    rng = np.random.default_rng(9)
+    raw, t = _raw(rng, 3000), rng.standard_normal((3000, 2)).astype(np.float32)
+    net = ws.WarmStartMLP(ctx, width=width, seed=8)
+    ref = ws.WarmStartMLP(ctx, width=width, seed=8)
+    net.set_dataset(raw, t)
+    m1 = m2 = 0.0
+    for step in range(2):
+        p = net.params()
+        losses = net.train(1, batch=batch, lr_max=1e-3, lr_min=1e-3, seed=4)
+        at = _sample_indices(4, step, batch, 3000)
+        ref.set_params(p)
+        loss, g = ref.loss_and_gradients(raw[at], t[at])
+        assert abs(losses[0] - loss) <= 1e-5 * loss
+        g = g.astype(np.float64)
+        m1, m2 = 0.9 * m1 + 0.1 * g, 0.999 * m2 + 0.001 * g * g
+        want = p - 1e-3 * (m1 / (1 - 0.9 ** (step + 1))) / (np.sqrt(m2 / (1 - 0.999 ** (step + 1))) + 1e-8)
+        q = net.params()
+        assert np.max(np.abs(q - want)) <= 1e-3 * 1e-4 + 4e-7 * np.max(np.abs(p))
+    ref.set_params(q)
+    assert np.array_equal(net.predict(raw[:700]), ref.predict(raw[:700]))
+
+
+def test_losses_of_long_runs_all_come_back(ctx):
+    """The loss partials stay on the device for a bounded run of steps between reads."""
+    rng = np.random.default_rng(10)
+    raw = _raw(rng, 2000)
+    net = ws.WarmStartMLP(ctx, width=64, seed=8)
+    net.set_dataset(raw, raw[:, 0:2])
+    losses = net.train(600, batch=512, seed=2)
+    assert np.all(losses > 0) and losses[-50:].mean() < 0.2 * losses[:5].mean()
