@@ -501,14 +501,12 @@ __device__ inline double2 h_block(const Acc& b, const DerivParams& P) {
 }
 
 // Matrix derivative of one pair for the field panel's BC (tbem.rs:1978-1995).
-__device__ inline double2 deriv_coefficient(const Acc& b, const Acc& d, const PanelBc& bc, const DerivParams& P) {
-    double2 d_cb, d_hb;
-    deriv_blocks(b, d, P, &d_cb, &d_hb);
+__device__ inline double2 deriv_from_blocks(double2 d_cb, double2 d_hb, double2 h_b, const PanelBc& bc,
+                                            const DerivParams& P) {
     if (bc.type == 0) {
         double2 v = cscale(d_cb, P.sign);
         if (bc.has_adm) {
             const double2 y = make_double2(bc.adm[0], bc.adm[1]);
-            const double2 h_b = h_block(b, P);
             v = csub(v, cmul(cscale(y, P.sign), cadd(cmul(d_hb, P.iwr), cmul(h_b, P.iwr_d))));
             v = csub(v, cmul(cmul(cscale(cscale(y, P.adm_scale), P.sign), h_b), P.iwr));
         }
@@ -516,6 +514,12 @@ __device__ inline double2 deriv_coefficient(const Acc& b, const Acc& d, const Pa
     }
     if (bc.type == 1) return cscale(d_hb, -P.sign);
     return make_double2(0.0, 0.0);
+}
+
+__device__ inline double2 deriv_coefficient(const Acc& b, const Acc& d, const PanelBc& bc, const DerivParams& P) {
+    double2 d_cb, d_hb;
+    deriv_blocks(b, d, P, &d_cb, &d_hb);
+    return deriv_from_blocks(d_cb, d_hb, h_block(b, P), bc, P);
 }
 
 // Right-hand-side derivative of a nonzero-BC field panel (tbem.rs:1998-2013).
@@ -551,14 +555,14 @@ __device__ inline void deriv_free_terms(const PanelBc& bc, const DerivParams& P,
 
 #pragma clang fp contract(on)
 
-// Per-panel constants of the TR13 points y_q = v0 + s_q e1 + t_q e2: the Gram
-// entries of the two edges.  Callers compute them once per field panel.
-struct FarPoints {
+// Per-panel constants of the TR13 points y_q = v0 + s_q e1 + t_q e2 of the
+// frequency-family kernel: the Gram entries of the two edges.
+struct FamilyPoints {
     double e11, e12x2, e22;  // e1.e1, 2 e1.e2, e2.e2
 };
 
-__device__ __forceinline__ FarPoints far_points(const FarPanel& P) {
-    FarPoints f;
+__device__ __forceinline__ FamilyPoints family_points(const FarPanel& P) {
+    FamilyPoints f;
     f.e11 = P.e1[0] * P.e1[0] + P.e1[1] * P.e1[1] + P.e1[2] * P.e1[2];
     f.e12x2 = 2.0 * (P.e1[0] * P.e2[0] + P.e1[1] * P.e2[1] + P.e1[2] * P.e2[2]);
     f.e22 = P.e2[0] * P.e2[0] + P.e2[1] * P.e2[1] + P.e2[2] * P.e2[2];
@@ -661,6 +665,57 @@ __device__ __forceinline__ FarLane far_lane(const FarPanel& P, double s) {
     return f;
 }
 
+// Calls point(d2, g, centre, sums) for the 13 points and add(weight, sums) for
+// each weight group.  Ap is A as the caller's ordering of the points left it.
+template <typename Part, typename Point, typename Add>
+__device__ __forceinline__ void far_points(const FarLane& P, double A, const double& Ap, const double* D, double gc,
+                                           const double* g, const Part& zero, Point&& point, Add&& add) {
+    {
+        Part a = zero;
+        point(A, gc, true, a);
+        add(TR_W0, a);
+    }
+    {
+        Part a = zero;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            point(__builtin_fma(TR_K1 * TR_K1, P.L[i], __builtin_fma(2.0 * TR_K1, D[i], Ap)),
+                  __builtin_fma(TR_K1, g[i], gc), false, a);
+        add(TR_W1, a);
+    }
+    {
+        Part a = zero;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            point(__builtin_fma(TR_K2 * TR_K2, P.L[i], __builtin_fma(2.0 * TR_K2, D[i], Ap)),
+                  __builtin_fma(TR_K2, g[i], gc), false, a);
+        add(TR_W2, a);
+    }
+    {
+        Part a = zero;
+#pragma unroll
+        for (int m = 0; m < 6; ++m) {
+            // displacement (a - c) V_i + (b - c) V_j, c the weight of the third corner
+            const int i = m >> 1, j = (i + 1 + (m & 1)) % 3;
+            constexpr double ac = TR_A - TR_C, bc = TR_B - TR_C;
+            point(__builtin_fma(2.0 * ac, D[i], __builtin_fma(2.0 * bc, D[j], Ap + P.Q[m])),
+                  __builtin_fma(ac, g[i], __builtin_fma(bc, g[j], gc)), false, a);
+        }
+        add(TR_W3, a);
+    }
+}
+
+// sin and cos of a phase difference in the variant's range (VAR's k times length).
+template <int VAR>
+__device__ __forceinline__ void sincos_difference(double x, double* sn, double* cs) {
+    if (VAR == FAR_GENERAL)
+        sincos_red(x, sn, cs);
+    else if (VAR == FAR_LONG)
+        sincos_half_period(x, sn, cs);
+    else
+        sincos_panel(x, sn, cs);
+}
+
 template <int MODE, int VAR>
 __device__ __forceinline__ void far_sums(const FarLane& P, const Source& src, const FarUniform& K, double2& cb,
                                          double2& hb) {
@@ -702,14 +757,9 @@ __device__ __forceinline__ void far_sums(const FarLane& P, const Source& src, co
         const double y = rsqrt_nr(d2);
         const double u = y * y;
         double sn = 0.0, cs = 1.0;
-        if (!centre) {
-            if (VAR == FAR_GENERAL)
-                sincos_red(__builtin_fma(K.kap, d2 * y, -rc), &sn, &cs);
-            else if (VAR == FAR_LONG)
-                sincos_half_period(__builtin_fma(d2, y, -rc), &sn, &cs);
-            else
-                sincos_panel(__builtin_fma(d2, y, -rc), &sn, &cs);
-        }
+        if (!centre)
+            sincos_difference<VAR>(VAR == FAR_GENERAL ? __builtin_fma(K.kap, d2 * y, -rc)
+                                                      : __builtin_fma(d2, y, -rc), &sn, &cs);
         double wr, wi;
         if (VAR != FAR_GENERAL) {
             const double R = (MODE == 0 ? gq : pr * gq) * u;  // beta rq
@@ -757,39 +807,7 @@ __device__ __forceinline__ void far_sums(const FarLane& P, const Source& src, co
             tot.hi = __builtin_fma(w, a.hi, tot.hi);
         }
     };
-    {
-        Part a = {0.0, 0.0, 0.0, 0.0};
-        point(A, gc, true, a);
-        add(TR_W0, a);
-    }
-    {
-        Part a = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            point(__builtin_fma(TR_K1 * TR_K1, P.L[i], __builtin_fma(2.0 * TR_K1, D[i], Ap)),
-                  __builtin_fma(TR_K1, g[i], gc), false, a);
-        add(TR_W1, a);
-    }
-    {
-        Part a = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            point(__builtin_fma(TR_K2 * TR_K2, P.L[i], __builtin_fma(2.0 * TR_K2, D[i], Ap)),
-                  __builtin_fma(TR_K2, g[i], gc), false, a);
-        add(TR_W2, a);
-    }
-    {
-        Part a = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int m = 0; m < 6; ++m) {
-            // displacement (a - c) V_i + (b - c) V_j, c the weight of the third corner
-            const int i = m >> 1, j = (i + 1 + (m & 1)) % 3;
-            constexpr double ac = TR_A - TR_C, bc = TR_B - TR_C;
-            point(__builtin_fma(2.0 * ac, D[i], __builtin_fma(2.0 * bc, D[j], Ap + P.Q[m])),
-                  __builtin_fma(ac, g[i], __builtin_fma(bc, g[j], gc)), false, a);
-        }
-        add(TR_W3, a);
-    }
+    far_points(P, A, Ap, D, gc, g, Part{0.0, 0.0, 0.0, 0.0}, point, add);
     double sn, cs;
     sincos_red(rc, &sn, &cs);
     const double fh = P.wj * K.s, fc = fh * K.s;
@@ -1038,97 +1056,137 @@ __global__ __launch_bounds__(256) void self_kernel(const PanelGeom* __restrict__
 // routes and launch structure as the value assembly, each pair producing its
 // values b and wavenumber derivatives d from one pass over its points.
 
-// Far sums with derivatives (fast arithmetic, harmonic factor +1), grouped by
-// powers of k as in far_sums.  With zg = w_q e^{ikr}/r, pn = r^.n_y,
-// qn = -r^.n_x, rq = pn qn, t = 3 rq + n_x.n_y, g = qn r (so that pn r = pr,
-// the pair constant (v0 - x).n_y of a flat panel), dG/dk = i r G and
-// d/dk[G (ik - 1/r)] = -k r G:
-//   E   = T1 - k^2 T2 - ik T3                 (T1 = sum zg t/r^2, T2 = sum zg rq, T3 = sum zg t/r)
-//   dH  = -k pr G                             (G = sum zg)
-//   dE  = sum [i r zg ef + zg def] = k (T2 + n_x.n_y G) - i k^2 U,  U = sum zg r rq,
-// where ef = t/r^2 - k^2 rq - ik t/r and def = -2k rq - i t/r (the i t/r
-// terms cancel); MODE 1 also G, Ht = -Q1 + ik Q2 (Q1 = sum zg qn/r, Q2 = sum zg qn),
-// dG = i D (D = sum zg r) and dHt = -k Q3 (Q3 = sum zg g).  MODE 0 (velocity
-// panels without admittance) needs E, dH, dE.  The panel factor is applied
-// once per pair.
-template <int MODE>
-// Same geometry as far_sums (distances from the edge Gram entries, normal
-// projections from per-pair dot products).
-__device__ __forceinline__ void far_sums_d(const FarPanel& P, const FarPoints& F, const Source& src, double k,
-                                           double k2, Acc& b, Acc& d) {
-    const double rel0 = P.v0[0] - src.c[0];
-    const double rel1 = P.v0[1] - src.c[1];
-    const double rel2 = P.v0[2] - src.c[2];
-    const double nxny = src.n[0] * P.nf[0] + src.n[1] * P.nf[1] + src.n[2] * P.nf[2];
-    const double a = rel0 * rel0 + rel1 * rel1 + rel2 * rel2;
-    const double b1 = 2.0 * (rel0 * P.e1[0] + rel1 * P.e1[1] + rel2 * P.e1[2]);
-    const double b2 = 2.0 * (rel0 * P.e2[0] + rel1 * P.e2[1] + rel2 * P.e2[2]);
-    const double pr = rel0 * P.nf[0] + rel1 * P.nf[1] + rel2 * P.nf[2];
-    const double g0 = -(rel0 * src.n[0] + rel1 * src.n[1] + rel2 * src.n[2]);
-    const double g1 = -(P.e1[0] * src.n[0] + P.e1[1] * src.n[1] + P.e1[2] * src.n[2]);
-    const double g2 = -(P.e2[0] * src.n[0] + P.e2[1] * src.n[1] + P.e2[2] * src.n[2]);
-    double gsr = 0.0, gsi = 0.0, t1r = 0.0, t1i = 0.0, t2r = 0.0, t2i = 0.0, t3r = 0.0, t3i = 0.0, ur = 0.0, ui = 0.0;
-    double q1r = 0.0, q1i = 0.0, q2r = 0.0, q2i = 0.0, q3r = 0.0, q3i = 0.0, dsr = 0.0, dsi = 0.0;
-#pragma unroll 2
-    for (int q = 0; q < 13; ++q) {
-        const double sq = kTrS[q], tq = kTrT[q];
-        const double u1 = __builtin_fma(tq, F.e12x2, __builtin_fma(sq, F.e11, b1));
-        const double u2 = __builtin_fma(tq, F.e22, b2);
-        const double d2 = fmax(__builtin_fma(sq, u1, __builtin_fma(tq, u2, a)), 1e-300);  // diagonal: overwritten later
-        const double inv = rsqrt_nr(d2);
-        const double dis = d2 * inv;
-        const double pn = pr * inv;
-        const double gq = __builtin_fma(sq, g1, __builtin_fma(tq, g2, g0));  // qn r
-        const double qn = gq * inv;
-        double sn, cs;
-        sincos_red(k * dis, &sn, &cs);
-        const double re2 = kTrW[q] * inv;
-        const double zgr = cs * re2, zgi = sn * re2;
-        gsr += zgr;
-        gsi += zgi;
-        const double rq = pn * qn;
-        const double t = __builtin_fma(3.0, rq, nxny);
-        const double ti1 = t * inv;
-        const double ti2 = ti1 * inv;
-        t1r = __builtin_fma(zgr, ti2, t1r);
-        t1i = __builtin_fma(zgi, ti2, t1i);
-        t2r = __builtin_fma(zgr, rq, t2r);
-        t2i = __builtin_fma(zgi, rq, t2i);
-        t3r = __builtin_fma(zgr, ti1, t3r);
-        t3i = __builtin_fma(zgi, ti1, t3i);
-        const double drq = dis * rq;
-        ur = __builtin_fma(zgr, drq, ur);
-        ui = __builtin_fma(zgi, drq, ui);
-        if (MODE == 1) {
-            const double qi = qn * inv;
-            q1r = __builtin_fma(zgr, qi, q1r);
-            q1i = __builtin_fma(zgi, qi, q1i);
-            q2r = __builtin_fma(zgr, qn, q2r);
-            q2i = __builtin_fma(zgi, qn, q2i);
-            q3r = __builtin_fma(zgr, gq, q3r);
-            q3i = __builtin_fma(zgi, gq, q3i);
-            dsr = __builtin_fma(zgr, dis, dsr);
-            dsi = __builtin_fma(zgi, dis, dsi);
-        }
+// Far sums with derivatives (harmonic factor +1), in the form of far_sums: one
+// complex weight per point for each of the factors that a column needs.  With
+// z = w e^{ikr} y, r = 1/y, dG/dk = i r G and d/dk[G (ik - 1/r)] = -k r G:
+//   dH  = -k pr sum z              dE  = sum z [k (rq + n_x.n_y) - i k^2 r rq]
+//   dG  = i sum z r                dHt = -k sum z g
+// (in dE the i t/r terms of dz ef and z def cancel), so with p = dk/dp and the
+// derivative beta' of beta
+//   d_cb = p (dH tau + dE beta) + E beta',  d_hb = p (dG tau + dHt beta) + Ht beta',
+//   hb   = G tau + Ht beta                  (tbem.rs:1972-1977).
+// MODE 0 (velocity panels without admittance) needs d_cb only.  The variants
+// are those of far_sums, chosen on the real parts of both beta and beta'.
+struct DerivUniform {
+    double s, kap, tau, wt;    // wt = p tau
+    double br, bi;             // beta s
+    double pbr, pbi, dbr, dbi; // p beta s and beta' s^2
+};
+
+template <int VAR>
+__device__ __forceinline__ DerivUniform deriv_uniform(const DerivParams& P) {
+    DerivUniform u;
+    u.s = VAR == FAR_GENERAL ? 1.0 : P.k;
+    u.kap = VAR == FAR_GENERAL ? P.k : 1.0;
+    u.tau = P.tau_r;
+    u.wt = P.ws * P.tau_r;
+    u.br = P.beta.x * u.s;
+    u.bi = P.beta.y * u.s;
+    u.pbr = P.ws * u.br;
+    u.pbi = P.ws * u.bi;
+    u.dbr = P.beta_d.x * (u.s * u.s);
+    u.dbi = P.beta_d.y * (u.s * u.s);
+    return u;
+}
+
+template <int MODE, int VAR>
+__device__ __forceinline__ void far_sums_d(const FarLane& P, const Source& src, const DerivUniform& K, double2& d_cb,
+                                           double2& d_hb, double2& hb) {
+    double x[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        x[d] = (P.v0[d] - src.c[d]) + P.cv[d];
+        if (VAR != FAR_GENERAL) x[d] *= K.s;
     }
-    const double w = P.wj;
-    b = acc_zero();
-    d = acc_zero();
-    b.e = make_double2(w * __builtin_fma(k, t3i, __builtin_fma(-k2, t2r, t1r)),
-                       w * __builtin_fma(-k, t3r, __builtin_fma(-k2, t2i, t1i)));
-    const double kpw = -k * pr * w;
-    d.h = make_double2(kpw * gsr, kpw * gsi);
-    d.e = make_double2(w * __builtin_fma(k, __builtin_fma(nxny, gsr, t2r), k2 * ui),
-                       w * __builtin_fma(k, __builtin_fma(nxny, gsi, t2i), -k2 * ur));
+    const double A = dot3(x, x);
+    const double D1 = dot3(x, P.V1), D2 = dot3(x, P.V2);
+    const double pr = dot3(x, P.nf);
+    const double nn = dot3(src.n, P.nf);
+    const double gm = MODE == 0 ? -pr : -1.0;  // MODE 0 carries g pr
+    const double gc = gm * dot3(x, src.n);
+    const double g1 = gm * dot3(P.V1, src.n), g2 = gm * dot3(P.V2, src.n);
+    const double D[3] = {-(D1 + D2), D1, D2};
+    const double g[3] = {-(g1 + g2), g1, g2};
+    const double kap2 = K.kap * K.kap;
+    const double yc = rsqrt_nr(A);
+    const double rc = A * yc;
+    const double c0 = -K.wt * K.kap * pr, bn = K.pbi * nn;
+    struct Part {
+        double cr, ci, hr, hi, vr, vi;
+    };
+    double Ap = A;
+    auto after = [&](Part& a) {  // one point at a time, as in far_sums
+        if (MODE == 0)
+            asm volatile("" : "+v"(Ap), "+v"(a.cr), "+v"(a.ci));
+        else
+            asm volatile("" : "+v"(Ap), "+v"(a.cr), "+v"(a.ci), "+v"(a.hr), "+v"(a.hi), "+v"(a.vr), "+v"(a.vi));
+    };
+    auto point = [&](double d2, double gq, bool centre, Part& a) {
+        const double y = rsqrt_nr(d2);
+        const double u = y * y;
+        const double r = d2 * y;
+        double sn = 0.0, cs = 1.0;
+        if (!centre) sincos_difference<VAR>(VAR == FAR_GENERAL ? K.kap * (r - rc) : r - rc, &sn, &cs);
+        const double rq = (MODE == 0 ? gq : pr * gq) * u;
+        const double t = __builtin_fma(3.0, rq, nn);
+        double wr, wi;
+        if (VAR != FAR_GENERAL) {
+            wr = y * __builtin_fma(K.dbi, t * y, __builtin_fma(K.pbi * r, rq, c0));
+            wi = y * __builtin_fma(K.dbi, __builtin_fma(t, u, -rq), __builtin_fma(K.pbi, rq, bn));
+        } else {
+            const double X = K.kap * (rq + nn), Z = -kap2 * (r * rq);
+            const double F = __builtin_fma(t, u, -kap2 * rq), H = -K.kap * (t * y);
+            wr = y * (c0 + __builtin_fma(K.pbr, X, -K.pbi * Z) + __builtin_fma(K.dbr, F, -K.dbi * H));
+            wi = y * (__builtin_fma(K.pbr, Z, K.pbi * X) + __builtin_fma(K.dbr, H, K.dbi * F));
+        }
+        auto put = [&](double vr, double vi, double& ar, double& ai) {
+            ar = __builtin_fma(cs, vr, ar);
+            ai = __builtin_fma(cs, vi, ai);
+            if (!centre) {
+                ar = __builtin_fma(-sn, vi, ar);
+                ai = __builtin_fma(sn, vr, ai);
+            }
+        };
+        put(wr, wi, a.cr, a.ci);
+        if (MODE == 1) {
+            if (VAR != FAR_GENERAL) {
+                const double gu = gq * u;  // g y times the y of z
+                put(-K.dbi * gu, y * __builtin_fma(-K.dbi, gu, __builtin_fma(-K.pbi, gq, K.wt * r)), a.hr, a.hi);
+                put(__builtin_fma(-K.bi, gu, K.tau * y), -K.bi * (gu * y), a.vr, a.vi);
+            } else {
+                const double kg = K.kap * gq, gy = gq * y;
+                put(y * (gy * __builtin_fma(-K.dbr, y, -K.dbi * K.kap) - K.pbr * kg),
+                    y * (__builtin_fma(K.wt, r, -K.pbi * kg) + gy * __builtin_fma(K.dbr, K.kap, -K.dbi * y)), a.hr,
+                    a.hi);
+                put(y * __builtin_fma(gy, __builtin_fma(-K.br, y, -K.bi * K.kap), K.tau),
+                    y * (gy * __builtin_fma(K.br, K.kap, -K.bi * y)), a.vr, a.vi);
+            }
+        }
+        after(a);
+    };
+    Part tot = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    auto add = [&](double w, const Part& a) {
+        tot.cr = __builtin_fma(w, a.cr, tot.cr);
+        tot.ci = __builtin_fma(w, a.ci, tot.ci);
+        if (MODE == 1) {
+            tot.hr = __builtin_fma(w, a.hr, tot.hr);
+            tot.hi = __builtin_fma(w, a.hi, tot.hi);
+            tot.vr = __builtin_fma(w, a.vr, tot.vr);
+            tot.vi = __builtin_fma(w, a.vi, tot.vi);
+        }
+    };
+    far_points(P, A, Ap, D, gc, g, Part{0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, point, add);
+    double sn, cs;
+    sincos_red(K.kap * rc, &sn, &cs);
+    const double f0 = P.wj, f1 = P.wj * K.s;
+    d_cb = make_double2(f1 * __builtin_fma(cs, tot.cr, -sn * tot.ci), f1 * __builtin_fma(cs, tot.ci, sn * tot.cr));
     if (MODE == 1) {
-        b.g = make_double2(w * gsr, w * gsi);
-        b.ht = make_double2(-w * __builtin_fma(k, q2i, q1r), w * __builtin_fma(k, q2r, -q1i));
-        d.g = make_double2(-w * dsi, w * dsr);
-        d.ht = make_double2(-k * w * q3r, -k * w * q3i);
+        d_hb = make_double2(f0 * __builtin_fma(cs, tot.hr, -sn * tot.hi), f0 * __builtin_fma(cs, tot.hi, sn * tot.hr));
+        hb = make_double2(f1 * __builtin_fma(cs, tot.vr, -sn * tot.vi), f1 * __builtin_fma(cs, tot.vi, sn * tot.vr));
     }
 }
 
-template <int MODE>
+template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void far_deriv_kernel(const FarPanel* __restrict__ panels,
                                                         const Source* __restrict__ sources,
                                                         const PanelBc* __restrict__ bcs, int64_t n, int64_t lda,
@@ -1137,17 +1195,15 @@ __global__ __launch_bounds__(256) void far_deriv_kernel(const FarPanel* __restri
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool active = j < n;
     const int64_t jj = active ? j : n - 1;
-    const FarPanel F = panels[jj];
-    const FarPoints FP = far_points(F);
+    const DerivUniform K = deriv_uniform<VAR>(P);
+    const FarLane F = far_lane(panels[jj], K.s);
     const PanelBc bc = MODE == 1 ? bcs[jj] : rigid_bc();
-    const double k2 = P.k * P.k;
     const int64_t i0 = (int64_t)blockIdx.y * rows_per_block;
     const int64_t i1 = min(n, i0 + rows_per_block);
     for (int64_t i = i0; i < i1; ++i) {
-        const Source src = sources[i];
-        Acc b, d;
-        far_sums_d<MODE>(F, FP, src, P.k, k2, b, d);
-        const double2 out = deriv_coefficient(b, d, bc, P);
+        double2 d_cb, d_hb = make_double2(0.0, 0.0), hb = make_double2(0.0, 0.0);
+        far_sums_d<MODE, VAR>(F, sources[i], K, d_cb, d_hb, hb);
+        const double2 out = deriv_from_blocks(d_cb, d_hb, hb, bc, P);
         if (active) A[i * lda + j] = out;
     }
 }
@@ -1385,7 +1441,7 @@ __global__ __launch_bounds__(256) void batch_far_family_kernel(const FreqFamily*
     const int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool active = j < n;
     const FarPanel P = far[fam.panel_off + (active ? j : n - 1)];
-    const FarPoints FP = far_points(P);
+    const FamilyPoints FP = family_points(P);
     const Source* src = sources + fam.panel_off;
     const double k0 = fam.k0, dk = fam.dk;
     const int64_t i1 = min(n, i0 + (int64_t)FAMILY_ROWS);
@@ -2108,12 +2164,12 @@ void launch_derivative_assembly(sbh_workspace* ws, const sbh_physics& ph, sbh_c6
     const dim3 grid((unsigned)((n + 255) / 256), (unsigned)((n + rows_per_block - 1) / rows_per_block));
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_ASSEMBLE_FAR, &ev);
-    if (general)
-        hipLaunchKernelGGL(far_deriv_kernel<1>, grid, dim3(256), 0, ctx->stream, m->d_far.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, n, sys->lda, rows_per_block, P, sys->d_A.ptr);
-    else
-        hipLaunchKernelGGL(far_deriv_kernel<0>, grid, dim3(256), 0, ctx->stream, m->d_far.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, n, sys->lda, rows_per_block, P, sys->d_A.ptr);
+    const int variant = far_variant(P.k, m->panel_radius, beta.re != 0.0 ? beta.re : beta_d.re);
+    with_far_variant(variant, general, [&](auto mode, auto var) {
+        hipLaunchKernelGGL((far_deriv_kernel<decltype(mode)::value, decltype(var)::value>), grid, dim3(256), 0,
+                           ctx->stream, m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, n, sys->lda, rows_per_block, P,
+                           sys->d_A.ptr);
+    });
     SBH_HIP(hipGetLastError());
     ctx->end_timed(SBH_KERNEL_ASSEMBLE_FAR, ev);
     if (ws->near_pairs > 0) {

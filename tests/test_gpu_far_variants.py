@@ -86,3 +86,24 @@ def test_batch_takes_the_single_system_variant(ctx, phase):
             ph = sa.PhysicsParams.from_wavenumber(k)
             beta = ph.burton_miller_beta() if betas is None else betas[i]
             assert np.array_equal(b.matrix(i), sa.build_tbem_system_with_beta(ctx, tm, ph, beta).matrix)
+
+
+@pytest.mark.parametrize("general", [False, True], ids=["rigid", "mixed"])
+@pytest.mark.parametrize("k,beta", list(_cases()))
+def test_far_derivatives_match_the_oracle(ctx, k, beta, general):
+    """d/dp with dk/dp = 0.7 and an unrelated beta derivative; the imaginary
+    beta of half the cases also meets a beta derivative with a real part,
+    which takes the general form."""
+    m = icosphere(1.0, 1)
+    bc = _mixed(m.num_elements) if general else {}
+    ph = sa.PhysicsParams.from_wavenumber(k)
+    ws = sa.TbemAssemblyWorkspace(ctx, sa.TbemMesh(ctx, m, **bc))
+    far = _far(m)
+    for beta_d in (-0.4j, 0.2 - 0.1j):
+        A = ws.assemble_parameter_derivative(ph, beta, beta_d, sign=-1.0, wavenumber_scale=0.7,
+                                             pressure_factor_derivative=3.0, admittance_scale=0.5).matrix
+        Ar, _ = oracle.build_tbem_derivative(m.nodes, m.triangles, k, beta, beta_d, sign=-1.0, wavenumber_scale=0.7,
+                                             pressure_factor_derivative=3.0,
+                                             admittance_scale=0.5, **bc)
+        assert rel_fro(A[far], Ar[far]) <= TOL
+        assert rel_fro(A, Ar) <= 1e-12
