@@ -1831,13 +1831,47 @@ __global__ void exact_combine_kernel(const double2* __restrict__ far, const doub
 // 1987-2044), constant basis on Tri3 panels:
 //   p(x) = sum_j sum_q [p_j G (-1/r + ik) (r.n_j)/r - v_j i rho omega G] J_j w_q
 // with r = y_q - x, G = e^{ikr}/(4 pi r) and the 7-point rule.  A workgroup
-// takes FIELD_ROWS points and one slice of the panels (lane per panel); each
-// quadrature point's position and weight are formed once per panel and used
-// for all the workgroup's points, whose coordinates are wave-uniform.  The
-// slices' partial sums are added per point in slice order.
+// takes FIELD_ROWS points and one slice of the panels (lane per panel); the
+// points' coordinates are wave-uniform.  The slices' partial sums are added per
+// point in slice order.
+//
+// FP64 VALU issue bounds it.  Distances come from the panel's corner offsets
+// and phases from its centre (far_sums): the rule's points are c, c + kappa V_i
+// and c + kappa' V_i, so an evaluation takes 29 FP64 instructions (42 with the
+// pair's share) where a difference per point and a reduced sine took 65, and
+// 5000 points x 10240 panels take 640 us instead of 904.  Within two panel
+// radii of a panel the expansion of the distance would lose digits, so there
+// the lanes take the differences directly (field_near), which also leaves out
+// a quadrature point that the evaluation point sits on.
 constexpr int FIELD_ROWS = 8;
+constexpr double TR7_K1 = 0.797426985353087 - 0.101286507323456;
+constexpr double TR7_K2 = 0.059715871789770 - 0.470142064105115;
+constexpr double TR7_W0 = 0.225, TR7_W1 = 0.125939180544827, TR7_W2 = 0.132394152788506;
 
-template <int HAS_V>
+// sum w z (-1/r + ik) dr/dn and sum w z of one pair without the panel factor.
+__device__ __forceinline__ void field_near(const FarPanel& P, const double* x, double k, double2* h, double2* g) {
+    const double pr = (P.v0[0] - x[0]) * P.nf[0] + (P.v0[1] - x[1]) * P.nf[1] + (P.v0[2] - x[2]) * P.nf[2];
+    *h = *g = make_double2(0.0, 0.0);
+#pragma clang loop unroll(disable)
+    for (int q = 0; q < 7; ++q) {
+        const double sq = kTr7S[q], tq = kTr7T[q];
+        double d[3];
+        for (int c = 0; c < 3; ++c) d[c] = __builtin_fma(sq, P.e1[c], __builtin_fma(tq, P.e2[c], P.v0[c])) - x[c];
+        const double d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+        if (!(d2 > 1e-30)) continue;  // a point within 1e-15 of the quadrature point contributes nothing
+        const double inv = rsqrt_nr(d2);
+        double sn, cs;
+        sincos_red(k * (d2 * inv), &sn, &cs);
+        const double zr = cs * (kTr7W[q] * inv), zi = sn * (kTr7W[q] * inv);
+        const double drdn = pr * inv;
+        h->x += (-zr * inv - zi * k) * drdn;
+        h->y += (zr * k - zi * inv) * drdn;
+        g->x += zr;
+        g->y += zi;
+    }
+}
+
+template <int HAS_V, int VAR>
 __global__ __launch_bounds__(256) void field_kernel(const FarPanel* __restrict__ panels, int64_t n,
                                                     const double* __restrict__ points, int64_t m,
                                                     const double2* __restrict__ p, const double2* __restrict__ v,
@@ -1849,56 +1883,119 @@ __global__ __launch_bounds__(256) void field_kernel(const FarPanel* __restrict__
     const int64_t i0 = (int64_t)blockIdx.x * FIELD_ROWS;
     const int64_t jbeg = (int64_t)blockIdx.y * panels_per_slice;
     const int64_t jend = min(n, jbeg + panels_per_slice);
-    double xs[FIELD_ROWS][3];
-#pragma unroll
-    for (int r = 0; r < FIELD_ROWS; ++r) {
-        const double* x = points + 3 * min(i0 + r, m - 1);  // rows past m are computed and dropped
-        xs[r][0] = x[0];
-        xs[r][1] = x[1];
-        xs[r][2] = x[2];
-    }
+    const double s = VAR == FAR_GENERAL ? 1.0 : k, kap = VAR == FAR_GENERAL ? k : 1.0;
     double2 acc[FIELD_ROWS];
 #pragma unroll
     for (int r = 0; r < FIELD_ROWS; ++r) acc[r] = make_double2(0.0, 0.0);
     for (int64_t jc = jbeg; jc < jend; jc += 256) {
         const int64_t j = jc + threadIdx.x;
         const bool active = j < jend;
-        const FarPanel P = panels[active ? j : n - 1];
+        const FarPanel& P = panels[active ? j : n - 1];
         const double2 pj = p[active ? j : n - 1];
         const double2 vj = HAS_V ? v[active ? j : n - 1] : make_double2(0.0, 0.0);
-        const double scale = (active && P.wj > 0.0) ? P.wj : 0.0;  // w J / (4 pi), times 0.5 for the rule
-        // (y_q - x).n_y = (v0 - x).n_y for every point y_q of the flat panel
-        double pr[FIELD_ROWS];
+        const FarLane F = far_lane(P, s);
+        const double scale = (active && F.wj > 0.0) ? F.wj : 0.0;  // w J / (4 pi), times 0.5 for the rule
+        const double reach = 4.0 * fmax(F.L[0], fmax(F.L[1], F.L[2]));
+        unsigned close = 0;  // rows within reach of this lane's panel
+        // p_j h - i pf v_j g
+        auto term = [&](double2 h, double2 g) {
+            double2 t = make_double2(scale * __builtin_fma(pj.x, h.x, -pj.y * h.y),
+                                     scale * __builtin_fma(pj.x, h.y, pj.y * h.x));
+            if (HAS_V) {
+                const double sp = scale * pf;
+                t.x = __builtin_fma(sp, __builtin_fma(vj.x, g.y, vj.y * g.x), t.x);
+                t.y = __builtin_fma(sp, __builtin_fma(vj.y, g.y, -vj.x * g.x), t.y);
+            }
+            return t;
+        };
 #pragma unroll
-        for (int r = 0; r < FIELD_ROWS; ++r)
-            pr[r] = (P.v0[0] - xs[r][0]) * P.nf[0] + (P.v0[1] - xs[r][1]) * P.nf[1] + (P.v0[2] - xs[r][2]) * P.nf[2];
+        for (int r = 0; r < FIELD_ROWS; ++r) {
+            const double* xr = points + 3 * min(i0 + r, m - 1);  // rows past m are computed and dropped
+            double x[3];
 #pragma unroll
-        for (int q = 0; q < 7; ++q) {
-            const double sq = kTr7S[q], tq = kTr7T[q];
-            const double y0 = __builtin_fma(sq, P.e1[0], __builtin_fma(tq, P.e2[0], P.v0[0]));
-            const double y1 = __builtin_fma(sq, P.e1[1], __builtin_fma(tq, P.e2[1], P.v0[1]));
-            const double y2 = __builtin_fma(sq, P.e1[2], __builtin_fma(tq, P.e2[2], P.v0[2]));
-            const double wq = kTr7W[q] * scale;
-#pragma unroll
-            for (int r = 0; r < FIELD_ROWS; ++r) {
-                const double dx = y0 - xs[r][0], dy = y1 - xs[r][1], dz = y2 - xs[r][2];
-                const double d2 = dx * dx + dy * dy + dz * dz;
-                // a point within 1e-15 of the quadrature point contributes nothing
-                const double inv = rsqrt_nr(fmax(d2, 1e-30));
-                double sn, cs;
-                sincos_red(k * (d2 * inv), &sn, &cs);
-                const double wt = d2 > 1e-30 ? wq * inv : 0.0;
-                const double zgr = cs * wt, zgi = sn * wt;
-                const double drdn = pr[r] * inv;
-                // p_j * zg * (-1/r + ik) * drdn
-                const double ar = (-zgr * inv - zgi * k) * drdn, ai = (zgr * k - zgi * inv) * drdn;
-                acc[r].x = __builtin_fma(pj.x, ar, __builtin_fma(-pj.y, ai, acc[r].x));
-                acc[r].y = __builtin_fma(pj.x, ai, __builtin_fma(pj.y, ar, acc[r].y));
+            for (int d = 0; d < 3; ++d) {
+                x[d] = (F.v0[d] - xr[d]) + F.cv[d];
+                if (VAR != FAR_GENERAL) x[d] *= s;
+            }
+            const double A = dot3(x, x);
+            const double D1 = dot3(x, F.V1), D2 = dot3(x, F.V2);
+            const double D[3] = {-(D1 + D2), D1, D2};
+            const double pr = dot3(x, F.nf);
+            const double yc = rsqrt_nr(A);
+            const double rc = A * yc;
+            struct Part {
+                double hr, hi, gr, gi;
+            };
+            double Ap = A;
+            auto point = [&](double d2, bool centre, Part& a) {
+                const double y = rsqrt_nr(d2);
+                const double u = y * y;
+                const double uy = u * y;
+                double sn = 0.0, cs = 1.0;
+                if (!centre)
+                    sincos_difference<VAR>(VAR == FAR_GENERAL ? kap * __builtin_fma(d2, y, -rc)
+                                                              : __builtin_fma(d2, y, -rc), &sn, &cs);
+                const double ku = VAR == FAR_GENERAL ? kap * u : u;
+                a.hr = __builtin_fma(-cs, uy, a.hr);
+                a.hi = __builtin_fma(cs, ku, a.hi);
+                if (!centre) {
+                    a.hr = __builtin_fma(-sn, ku, a.hr);
+                    a.hi = __builtin_fma(-sn, uy, a.hi);
+                }
                 if (HAS_V) {
-                    // - v_j * (i pf) * zg = v_j * pf * (zgi - i zgr)
-                    const double br = pf * zgi, bi = -pf * zgr;
-                    acc[r].x = __builtin_fma(vj.x, br, __builtin_fma(-vj.y, bi, acc[r].x));
-                    acc[r].y = __builtin_fma(vj.x, bi, __builtin_fma(vj.y, br, acc[r].y));
+                    a.gr = __builtin_fma(cs, y, a.gr);
+                    if (!centre) a.gi = __builtin_fma(sn, y, a.gi);
+                    asm volatile("" : "+v"(Ap), "+v"(a.hr), "+v"(a.hi), "+v"(a.gr), "+v"(a.gi));
+                } else {
+                    asm volatile("" : "+v"(Ap), "+v"(a.hr), "+v"(a.hi));  // one point at a time, as in far_sums
+                }
+            };
+            Part tot = {0.0, 0.0, 0.0, 0.0};
+            auto add = [&](double w, const Part& a) {
+                tot.hr = __builtin_fma(w, a.hr, tot.hr);
+                tot.hi = __builtin_fma(w, a.hi, tot.hi);
+                if (HAS_V) {
+                    tot.gr = __builtin_fma(w, a.gr, tot.gr);
+                    tot.gi = __builtin_fma(w, a.gi, tot.gi);
+                }
+            };
+            Part a0 = {0.0, 0.0, 0.0, 0.0}, a1 = a0, a2 = a0;
+            point(A, true, a0);
+            add(TR7_W0, a0);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                point(__builtin_fma(TR7_K1 * TR7_K1, F.L[i], __builtin_fma(2.0 * TR7_K1, D[i], Ap)), false, a1);
+            add(TR7_W1, a1);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                point(__builtin_fma(TR7_K2 * TR7_K2, F.L[i], __builtin_fma(2.0 * TR7_K2, D[i], Ap)), false, a2);
+            add(TR7_W2, a2);
+            double sn, cs;
+            sincos_red(VAR == FAR_GENERAL ? kap * rc : rc, &sn, &cs);
+            const double fh = (s * s) * pr;
+            double2 h = make_double2(fh * __builtin_fma(cs, tot.hr, -sn * tot.hi),
+                                     fh * __builtin_fma(cs, tot.hi, sn * tot.hr));
+            double2 g = make_double2(0.0, 0.0);
+            if (HAS_V)
+                g = make_double2(s * __builtin_fma(cs, tot.gr, -sn * tot.gi),
+                                 s * __builtin_fma(cs, tot.gi, sn * tot.gr));
+            const double2 t = term(h, g);
+            const bool far = A > reach;
+            if (!far) close |= 1u << r;
+            acc[r].x += far ? t.x : 0.0;
+            acc[r].y += far ? t.y : 0.0;
+        }
+        if (__any(close != 0u)) {
+#pragma clang loop unroll(disable)
+            for (int r = 0; r < FIELD_ROWS; ++r) {
+                if (!((close >> r) & 1u)) continue;
+                double2 h, g;
+                field_near(P, points + 3 * min(i0 + r, m - 1), k, &h, &g);
+                const double2 t = term(h, g);
+#pragma unroll
+                for (int q = 0; q < FIELD_ROWS; ++q) {
+                    acc[q].x += q == r ? t.x : 0.0;
+                    acc[q].y += q == r ? t.y : 0.0;
                 }
             }
         }
@@ -2335,12 +2432,10 @@ void launch_field(sbh_context* ctx, const sbh_mesh* m, const sbh_physics& ph, co
     const dim3 grid((unsigned)row_blocks, (unsigned)slices);
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_FIELD, &ev);
-    if (v)
-        hipLaunchKernelGGL(field_kernel<1>, grid, dim3(256), 0, ctx->stream, m->d_far.ptr, n, d_points, npts, p, v,
-                           hf * k, pf, per_slice, part.ptr);
-    else
-        hipLaunchKernelGGL(field_kernel<0>, grid, dim3(256), 0, ctx->stream, m->d_far.ptr, n, d_points, npts, p, v,
-                           hf * k, pf, per_slice, part.ptr);
+    with_far_variant(far_variant(hf * k, m->panel_radius, 0.0), v ? 1 : 0, [&](auto has_v, auto var) {
+        hipLaunchKernelGGL((field_kernel<decltype(has_v)::value, decltype(var)::value>), grid, dim3(256), 0,
+                           ctx->stream, m->d_far.ptr, n, d_points, npts, p, v, hf * k, pf, per_slice, part.ptr);
+    });
     SBH_HIP(hipGetLastError());
     ctx->end_timed(SBH_KERNEL_FIELD, ev);
     hipLaunchKernelGGL(field_finish_kernel, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, ctx->stream, part.ptr,

@@ -200,3 +200,30 @@ def test_plane_waves_through_the_source_api(ctx):
     fa = sa.compute_total_field(pts, tm, x, a, ph)
     fb = sa.compute_total_field(pts, tm, x, b, ph)
     assert np.array_equal(fa.p_total, fb.p_total)
+
+
+@pytest.mark.parametrize("velocity", [False, True])
+@pytest.mark.parametrize("phase", [0.05, 0.319, 0.321, 1.569, 1.571, 4.0])
+def test_field_variants_and_points_close_to_panels(ctx, phase, velocity):
+    """Both sides of the ranges of the short and long sine polynomials (the
+    phase inside a panel), and points that take the direct differences: on a
+    quadrature point, over a panel at 1e-3 to 2.2 panel radii (the switch is
+    at 2).  A distance d from the surface carries its position's rounding,
+    2^-52 / d <= 2e-13 relative, twice in 1/r^2."""
+    m = icosphere(1.0, 2)
+    n = m.num_elements
+    p = m.nodes[m.triangles]
+    radius = np.max(np.linalg.norm(p - p.mean(axis=1, keepdims=True), axis=2))
+    k = phase / 0.86 / radius
+    c, nn, _ = m.element_geometry()
+    rng = np.random.default_rng(41)
+    sol = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    vel = 1e-3 * (rng.standard_normal(n) + 1j * rng.standard_normal(n)) if velocity else None
+    s, t = 0.797426985353087, 0.101286507323456
+    on = [c[3], p[7, 0] + s * (p[7, 1] - p[7, 0]) + t * (p[7, 2] - p[7, 0])]
+    over = [c[j] + e * radius * nn[j] for j in (0, 11, 200) for e in (1e-3, 0.3, 1.0, 1.95, 2.05, 2.2)]
+    pts = np.concatenate([on, over, _points(rng, 45, 1.5, 3.0)])
+    tm = sa.TbemMesh(ctx, m)
+    got = sa.compute_scattered_field(pts, tm, sol, sa.PhysicsParams.from_wavenumber(k), surface_velocity=vel)
+    ref = oracle.field(pts, m.nodes, m.triangles, sol, k, v_surf=vel)
+    assert np.max(np.abs(got - ref) / np.abs(ref)) <= 1e-12 * max(1.0, np.max(np.abs(sol)) / np.min(np.abs(ref)))
