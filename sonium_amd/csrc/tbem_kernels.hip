@@ -13,8 +13,7 @@
 //                This is the FP64-VALU-bound kernel: 13 kernel evaluations
 //                per pair, each about 40 FP64 instructions (far_sums).
 //   near_kernel  overwrites the near pairs (level-0 ratio < 3) with the sum
-//                over their subdivision leaves; one wave per pair, lanes over
-//                (leaf, point), evaluated in the reference's operation order.
+//                over their subdivision leaves; one lane per leaf.
 //   self_kernel  overwrites the diagonal: Stokes edge integral of the
 //                hypersingular kernel plus Duffy-collapsed Gauss–Legendre on
 //                the 3 x nsec2 sub-triangles (singular.rs:297-578), the
@@ -598,7 +597,7 @@ __device__ __forceinline__ FamilyPoints family_points(const FarPanel& P) {
 //  - The rule's four weights multiply the sums of their groups.
 // Per evaluation this takes 41 FP64 instructions (529 a pair, pair work included)
 // where separate channel sums over a reduced sine took 68; the assembly of 20480
-// panels takes 9.2 ms instead of 13.3, of which this loop 7.9 instead of 12.2.
+// panels takes 8.0 ms instead of 13.2, of which this loop 7.8 instead of 12.0.
 //
 // Variants (far_variant): FAR_SHORT and FAR_LONG need a purely imaginary beta
 // and a phase difference within the range of their polynomials; FAR_GENERAL
@@ -638,16 +637,8 @@ __device__ __forceinline__ double dot3(const double* a, const double* b) {
     return __builtin_fma(a[2], b[2], __builtin_fma(a[1], b[1], a[0] * b[0]));
 }
 
-__device__ __forceinline__ FarLane far_lane(const FarPanel& P, double s) {
-    FarLane f;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        f.v0[d] = P.v0[d];
-        f.cv[d] = (P.e1[d] + P.e2[d]) * (1.0 / 3.0);
-        f.V1[d] = s * (P.e1[d] - f.cv[d]);
-        f.V2[d] = s * (P.e2[d] - f.cv[d]);
-        f.nf[d] = P.nf[d];
-    }
+// The squares of a lane's corner offsets and of its group of six.
+__device__ __forceinline__ void lane_squares(FarLane& f) {
     const double V0[3] = {-(f.V1[0] + f.V2[0]), -(f.V1[1] + f.V2[1]), -(f.V1[2] + f.V2[2])};
     f.L[0] = dot3(V0, V0);
     f.L[1] = dot3(f.V1, f.V1);
@@ -661,6 +652,19 @@ __device__ __forceinline__ FarLane far_lane(const FarPanel& P, double s) {
         const int i = m >> 1, j = (i + 1 + (m & 1)) % 3, k = 3 - i - j;  // a on corner i, b on j, c on k
         f.Q[m] = __builtin_fma(qa, f.L[i], __builtin_fma(qb, f.L[j], qc * f.L[k]));
     }
+}
+
+__device__ __forceinline__ FarLane far_lane(const FarPanel& P, double s) {
+    FarLane f;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        f.v0[d] = P.v0[d];
+        f.cv[d] = (P.e1[d] + P.e2[d]) * (1.0 / 3.0);
+        f.V1[d] = s * (P.e1[d] - f.cv[d]);
+        f.V2[d] = s * (P.e2[d] - f.cv[d]);
+        f.nf[d] = P.nf[d];
+    }
+    lane_squares(f);
     f.wj = P.wj;
     return f;
 }
@@ -945,22 +949,91 @@ __device__ __forceinline__ void fold_row_max(double* slot, double2 v) {
     if (m == m) atomicMax(reinterpret_cast<unsigned long long*>(slot), (unsigned long long)__double_as_longlong(m));
 }
 
-// Coefficient of one near pair, summed over its leaves by one wave (lanes
-// over (leaf, point)); every lane returns the total.
-__device__ __forceinline__ double2 near_entry(const NearPair& np, const uint64_t* __restrict__ leaves,
-                                              const PanelGeom& G, const Source& src, const PanelBc& bc,
-                                              double k, double wavruim, double tau_r, double2 beta, double2 iwr,
-                                              int lane) {
-    const double k2 = k * k;
-    Acc a = acc_zero();
-    const int total = np.count * 13;
-    for (int t = lane; t < total; t += 64) {
-        int leaf = t / 13;
-        int q = t - leaf * 13;
-        near_point(G, leaves[np.begin + leaf], q, src.c, src.n, wavruim, k2, a);
+// Near pairs.  A subdivision leaf is a triangle similar to its panel: centre c +
+// offset and corners at +-2^-depth V_i from it (the centre child of a cell is
+// turned around, and the labels of a cell's corners rotate, which a symmetric
+// rule does not see).  Every leaf is at least three of its sizes away, so its 13
+// points take the far loop's evaluation, and one lane takes one leaf.
+// What bounded the former wave per pair was everything but the evaluation: each
+// lane decoded the leaf of its point, interpolated a position, and eight channel
+// sums crossed the wave; 577620 pairs with 4.71 million leaves (20480 panels)
+// took 1.13 ms, and take 0.18.
+__device__ __forceinline__ FarLane leaf_lane(const FarPanel& P, uint64_t code, double s) {
+    const int depth = (int)(code >> LEAF_DEPTH_SHIFT);
+    double w0 = 0.0, w1 = 0.0, w2 = 0.0, size = 1.0;
+    int rot = 0;  // corner m of the cell points along V_{(m + rot) % 3}
+    for (int l = 0; l < depth; ++l) {
+        const int ch = (int)((code >> (2 * l)) & 3u);
+        const int d = ch + rot >= 3 ? ch + rot - 3 : ch + rot;
+        size *= 0.5;
+        if (ch == 3) {
+            size = -size;
+            rot = rot == 0 ? 2 : rot - 1;
+        } else {
+            w0 += d == 0 ? size : 0.0;
+            w1 += d == 1 ? size : 0.0;
+            w2 += d == 2 ? size : 0.0;
+            rot = d;
+        }
     }
-    wave_sum_acc(a);
-    return coefficient(a, bc, make_double2(1.0, 0.0), make_double2(tau_r, 0.0), beta, iwr);
+    FarLane f;
+    const double a1 = w1 - w0, a2 = w2 - w0, ss = s * size;  // V_0 = -V_1 - V_2
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const double cv = (P.e1[d] + P.e2[d]) * (1.0 / 3.0);
+        const double V1 = P.e1[d] - cv, V2 = P.e2[d] - cv;
+        f.v0[d] = P.v0[d];
+        f.cv[d] = __builtin_fma(a1, V1, __builtin_fma(a2, V2, cv));
+        f.V1[d] = ss * V1;
+        f.V2[d] = ss * V2;
+        f.nf[d] = P.nf[d];
+    }
+    lane_squares(f);
+    f.wj = P.wj * (size * size);  // the leaf's share of the panel's area
+    return f;
+}
+
+// Sums over the leaves of pairs [p0, p0 + np) (np <= 256), by the whole
+// workgroup: lane per leaf, 256 leaves at a time; each pair's leaves are added
+// in order by one thread, so the sum depends on the pair alone.
+// eval(pair, code) gives a leaf's double2; put(t, pair, sum) takes pair p0 + t's sum
+// on thread t.
+template <typename Eval, typename Put>
+__device__ __forceinline__ void near_pairs(const NearPair* __restrict__ pairs, int64_t p0, int np,
+                                           const uint64_t* __restrict__ leaves, Eval&& eval, Put&& put) {
+    __shared__ int off[257];
+    __shared__ double2 res[256];
+    const int t = threadIdx.x;
+    const NearPair mine = pairs[p0 + min(t, np - 1)];
+    __syncthreads();  // the previous call's sums have been taken
+    off[t + 1] = t < np ? mine.count : 0;
+    if (t == 0) off[0] = 0;
+    for (int d = 1; d < 256; d <<= 1) {  // inclusive scan
+        __syncthreads();
+        const int v = t >= d ? off[t + 1 - d] : 0;
+        __syncthreads();
+        off[t + 1] += v;
+    }
+    __syncthreads();
+    const int total = off[np];
+    const int b = off[t], e = off[t + 1];
+    double2 sum = make_double2(0.0, 0.0);
+    for (int base = 0; base < total; base += 256) {
+        const int l = base + t;
+        if (l < total) {
+            int lo = 0, hi = np - 1;  // the last pair whose leaves start at or before l
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (off[mid] <= l) lo = mid; else hi = mid - 1;
+            }
+            const NearPair np_l = pairs[p0 + lo];
+            res[t] = eval(np_l, leaves[np_l.begin + (l - off[lo])]);
+        }
+        __syncthreads();
+        for (int q = max(b, base); q < min(e, base + 256); ++q) sum = cadd(sum, res[q - base]);
+        __syncthreads();
+    }
+    if (t < np) put(t, mine, sum);
 }
 
 // Diagonal entry and BC free-term right-hand side of panel G (self integral
@@ -1005,28 +1078,29 @@ __device__ __forceinline__ PanelBc rigid_bc() {
     return bc;
 }
 
-// One wave per near pair; lanes over (leaf, point).
+// pairs_per_block near pairs per workgroup.
+template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void near_kernel(const NearPair* __restrict__ pairs, int64_t npairs,
-                                                   const uint64_t* __restrict__ leaves,
-                                                   const PanelGeom* __restrict__ geom,
+                                                   int pairs_per_block, const uint64_t* __restrict__ leaves,
+                                                   const FarPanel* __restrict__ panels,
                                                    const Source* __restrict__ sources,
-                                                   const PanelBc* __restrict__ bcs, int general,
-                                                   int64_t lda, double k, double wavruim,
+                                                   const PanelBc* __restrict__ bcs, int64_t lda, double k,
                                                    double tau_r, double2 beta, double2 iwr,
                                                    double2* __restrict__ A, double* __restrict__ rowmax,
                                                    int64_t nbx) {
-    const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (p >= npairs) return;
-    const NearPair np = pairs[p];
-    const PanelBc bc = general ? bcs[np.j] : rigid_bc();
-    const PanelGeom G = geom[np.j];  // constant indexing only: lives in registers
-    const Source S = sources[np.i];
-    const double2 v = near_entry(np, leaves, G, S, bc, k, wavruim, tau_r, beta, iwr, lane);
-    if (lane == 0) {
-        A[(int64_t)np.i * lda + np.j] = v;
-        if (rowmax) fold_row_max(rowmax + (int64_t)np.i * nbx + nbx - 1, v);
-    }
+    const int64_t p0 = (int64_t)blockIdx.x * pairs_per_block;
+    const FarUniform K = far_uniform<VAR>(k, tau_r, beta);
+    near_pairs(
+        pairs, p0, (int)min((int64_t)pairs_per_block, npairs - p0), leaves,
+        [&](const NearPair& np, uint64_t code) {
+            PanelBc bc;
+            if (MODE == 1) bc = bcs[np.j];
+            return far_entry<MODE, VAR>(leaf_lane(panels[np.j], code, K.s), sources[np.i], bc, K, iwr);
+        },
+        [&](int, const NearPair& np, double2 v) {
+            A[(int64_t)np.i * lda + np.j] = v;
+            if (rowmax) fold_row_max(rowmax + (int64_t)np.i * nbx + nbx - 1, v);
+        });
 }
 
 // One wave per panel: self integrals, free terms, BC free-term RHS.
@@ -1208,30 +1282,24 @@ __global__ __launch_bounds__(256) void far_deriv_kernel(const FarPanel* __restri
     }
 }
 
-// One wave per near pair; lanes over (leaf, point); reference operation order.
+// pairs_per_block near pairs per workgroup, lane per leaf as in near_kernel.
+template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void near_deriv_kernel(const NearPair* __restrict__ pairs, int64_t npairs,
-                                                         const uint64_t* __restrict__ leaves,
-                                                         const PanelGeom* __restrict__ geom,
+                                                         int pairs_per_block, const uint64_t* __restrict__ leaves,
+                                                         const FarPanel* __restrict__ panels,
                                                          const Source* __restrict__ sources,
-                                                         const PanelBc* __restrict__ bcs, int general, int64_t lda,
+                                                         const PanelBc* __restrict__ bcs, int64_t lda,
                                                          DerivParams P, double2* __restrict__ A) {
-    const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (p >= npairs) return;
-    const NearPair np = pairs[p];
-    const PanelBc bc = general ? bcs[np.j] : rigid_bc();
-    const PanelGeom G = geom[np.j];
-    const Source S = sources[np.i];
-    const double k2 = P.k * P.k;
-    Acc b = acc_zero(), d = acc_zero();
-    const int total = np.count * 13;
-    for (int t = lane; t < total; t += 64) {
-        const int leaf = t / 13;
-        near_point_t<true>(G, leaves[np.begin + leaf], t - leaf * 13, S.c, S.n, P.wavruim, k2, P.k, P.hf, b, d);
-    }
-    wave_sum_acc(b);
-    wave_sum_acc(d);
-    if (lane == 0) A[(int64_t)np.i * lda + np.j] = deriv_coefficient(b, d, bc, P);
+    const int64_t p0 = (int64_t)blockIdx.x * pairs_per_block;
+    const DerivUniform K = deriv_uniform<VAR>(P);
+    near_pairs(
+        pairs, p0, (int)min((int64_t)pairs_per_block, npairs - p0), leaves,
+        [&](const NearPair& np, uint64_t code) {
+            double2 d_cb, d_hb = make_double2(0.0, 0.0), hb = make_double2(0.0, 0.0);
+            far_sums_d<MODE, VAR>(leaf_lane(panels[np.j], code, K.s), sources[np.i], K, d_cb, d_hb, hb);
+            return deriv_from_blocks(d_cb, d_hb, hb, MODE == 1 ? bcs[np.j] : rigid_bc(), P);
+        },
+        [&](int, const NearPair& np, double2 v) { A[(int64_t)np.i * lda + np.j] = v; });
 }
 
 // One wave per panel: self-integral derivatives, free terms, BC free-term RHS.
@@ -1690,18 +1758,29 @@ __global__ __launch_bounds__(256) void batch_assemble_kernel(BatchAssemblyArgs a
             }
         } else {
             const PanelGeom* geom = args.geom + I.panel_off;
+            const FarPanel* far = args.far + I.panel_off;
             const PanelBc bc = rigid_bc();
             const double2 iwr = make_double2(0.0, 0.0);  // no admittance on rigid panels
-            // members of a frequency family got their near entries from batch_near_family_kernel
+            // members of a frequency family got their near pairs from batch_near_family_kernel
             const int64_t pb = args.row_ptr[I.panel_off + r0];
             const int64_t pe = I.in_family ? pb : args.row_ptr[I.panel_off + r1];
-            for (int64_t p = pb + wave; p < pe; p += 4) {
-                const NearPair np = args.pairs[p];
-                const PanelGeom G = geom[np.j];
-                const Source S = src[np.i];
-                const double2 v = near_entry(np, args.leaves, G, S, bc, k, k, I.tau, beta, iwr, lane);
-                if (lane == 0) A[(int64_t)np.i * n + np.j] = v;
-            }
+            auto fill = [&](auto variant) {
+                constexpr int VAR = decltype(variant)::value;
+                const FarUniform K = far_uniform<VAR>(k, I.tau, beta);
+                for (int64_t p = pb; p < pe; p += 256)
+                    near_pairs(
+                        args.pairs, p, (int)min((int64_t)256, pe - p), args.leaves,
+                        [&](const NearPair& np, uint64_t code) {
+                            return far_entry<0, VAR>(leaf_lane(far[np.j], code, K.s), src[np.i], bc, K, iwr);
+                        },
+                        [&](int, const NearPair& np, double2 v) { A[(int64_t)np.i * n + np.j] = v; });
+            };
+            if (I.far_variant == FAR_SHORT)
+                fill(std::integral_constant<int, FAR_SHORT>());
+            else if (I.far_variant == FAR_LONG)
+                fill(std::integral_constant<int, FAR_LONG>());
+            else
+                fill(std::integral_constant<int, FAR_GENERAL>());
             for (int64_t i = r0 + wave; i < r1; i += 4) {
                 double2 diag, unused;
                 self_entry(geom[i], src[i], bc, k, k, I.tau, beta, iwr, lane, &diag, &unused);
@@ -1777,26 +1856,27 @@ __global__ __launch_bounds__(256) void exact_far_kernel(const FarPanel* __restri
 
 template <int MODE, int VAR>
 __global__ __launch_bounds__(256) void exact_near_kernel(const NearPair* __restrict__ pairs, int64_t npairs,
-                                                         const uint64_t* __restrict__ leaves,
-                                                         const PanelGeom* __restrict__ geom,
+                                                         int pairs_per_block, const uint64_t* __restrict__ leaves,
                                                          const FarPanel* __restrict__ panels,
                                                          const Source* __restrict__ sources,
-                                                         const PanelBc* __restrict__ bcs, double k, double wavruim,
-                                                         double tau_r, double2 beta, double2 iwr,
-                                                         const double2* __restrict__ x, double2* __restrict__ out) {
-    const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
-    if (p >= npairs) return;
-    const NearPair np = pairs[p];
-    const PanelBc bc = MODE == 1 ? bcs[np.j] : rigid_bc();
-    const PanelGeom G = geom[np.j];
-    const Source S = sources[np.i];
-    const double2 v = near_entry(np, leaves, G, S, bc, k, wavruim, tau_r, beta, iwr, lane);
-    if (lane == 0) {
-        const FarUniform K = far_uniform<VAR>(k, tau_r, beta);
-        const double2 f = far_entry<MODE, VAR>(far_lane(panels[np.j], K.s), S, bc, K, iwr);
-        out[p] = cmul(csub(v, f), x[np.j]);
-    }
+                                                         const PanelBc* __restrict__ bcs, double k, double tau_r,
+                                                         double2 beta, double2 iwr, const double2* __restrict__ x,
+                                                         double2* __restrict__ out) {
+    const int64_t p0 = (int64_t)blockIdx.x * pairs_per_block;
+    const FarUniform K = far_uniform<VAR>(k, tau_r, beta);
+    near_pairs(
+        pairs, p0, (int)min((int64_t)pairs_per_block, npairs - p0), leaves,
+        [&](const NearPair& np, uint64_t code) {
+            PanelBc bc;
+            if (MODE == 1) bc = bcs[np.j];
+            return far_entry<MODE, VAR>(leaf_lane(panels[np.j], code, K.s), sources[np.i], bc, K, iwr);
+        },
+        [&](int t, const NearPair& np, double2 v) {
+            PanelBc bc;
+            if (MODE == 1) bc = bcs[np.j];
+            const double2 f = far_entry<MODE, VAR>(far_lane(panels[np.j], K.s), sources[np.i], bc, K, iwr);
+            out[p0 + t] = cmul(csub(v, f), x[np.j]);
+        });
 }
 
 __global__ __launch_bounds__(256) void exact_self_kernel(const PanelGeom* __restrict__ geom,
@@ -2155,6 +2235,15 @@ static void with_far_variant(int variant, int general, Launch&& launch) {
         mode(std::integral_constant<int, FAR_GENERAL>());
 }
 
+// Near pairs per workgroup: 256 fill the lanes of its leaf passes best (8 leaves
+// a pair on average, a partial pass per workgroup); fewer where that would
+// leave less than two workgroups per CU.
+static int near_pairs_per_block(int64_t npairs) {
+    int per = 256;
+    while (per > 32 && npairs / per < 512) per /= 2;
+    return per;
+}
+
 void launch_assembly(sbh_workspace* ws, const sbh_physics& ph, sbh_c64 beta_c, sbh_system* sys) {
     injection_check(INJECT_LAUNCH);
     sbh_context* ctx = ws->ctx;
@@ -2192,10 +2281,13 @@ void launch_assembly(sbh_workspace* ws, const sbh_physics& ph, sbh_c64 beta_c, s
     ctx->end_timed(SBH_KERNEL_ASSEMBLE_FAR, ev);
     if (ws->near_pairs > 0) {
         ctx->begin_timed(SBH_KERNEL_ASSEMBLE_NEAR, &ev);
-        hipLaunchKernelGGL(near_kernel, dim3((unsigned)((ws->near_pairs + 3) / 4)), dim3(256), 0,
-                           ctx->stream, ws->d_pairs.ptr, ws->near_pairs, ws->d_leaves.ptr,
-                           m->d_geom.ptr, m->d_src.ptr, m->d_bc.ptr, general, sys->lda, k, wavruim,
-                           ph.tau, beta, iwr, sys->d_A.ptr, rm, nbx);
+        const int per = near_pairs_per_block(ws->near_pairs);
+        with_far_variant(far_variant(k, m->panel_radius, beta.x), general, [&](auto mode, auto var) {
+            hipLaunchKernelGGL((near_kernel<decltype(mode)::value, decltype(var)::value>),
+                               dim3((unsigned)((ws->near_pairs + per - 1) / per)), dim3(256), 0, ctx->stream,
+                               ws->d_pairs.ptr, ws->near_pairs, per, ws->d_leaves.ptr, m->d_far.ptr, m->d_src.ptr,
+                               m->d_bc.ptr, sys->lda, k, ph.tau, beta, iwr, sys->d_A.ptr, rm, nbx);
+        });
         SBH_HIP(hipGetLastError());
         ctx->end_timed(SBH_KERNEL_ASSEMBLE_NEAR, ev);
     }
@@ -2271,9 +2363,13 @@ void launch_derivative_assembly(sbh_workspace* ws, const sbh_physics& ph, sbh_c6
     ctx->end_timed(SBH_KERNEL_ASSEMBLE_FAR, ev);
     if (ws->near_pairs > 0) {
         ctx->begin_timed(SBH_KERNEL_ASSEMBLE_NEAR, &ev);
-        hipLaunchKernelGGL(near_deriv_kernel, dim3((unsigned)((ws->near_pairs + 3) / 4)), dim3(256), 0, ctx->stream,
-                           ws->d_pairs.ptr, ws->near_pairs, ws->d_leaves.ptr, m->d_geom.ptr, m->d_src.ptr,
-                           m->d_bc.ptr, general, sys->lda, P, sys->d_A.ptr);
+        const int per = near_pairs_per_block(ws->near_pairs);
+        with_far_variant(variant, general, [&](auto mode, auto var) {
+            hipLaunchKernelGGL((near_deriv_kernel<decltype(mode)::value, decltype(var)::value>),
+                               dim3((unsigned)((ws->near_pairs + per - 1) / per)), dim3(256), 0, ctx->stream,
+                               ws->d_pairs.ptr, ws->near_pairs, per, ws->d_leaves.ptr, m->d_far.ptr, m->d_src.ptr,
+                               m->d_bc.ptr, sys->lda, P, sys->d_A.ptr);
+        });
         SBH_HIP(hipGetLastError());
         ctx->end_timed(SBH_KERNEL_ASSEMBLE_NEAR, ev);
     }
@@ -2384,16 +2480,16 @@ void launch_exact_apply(const sbh_operator* op, const double2* x, double2* y) {
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_MATVEC, &ev);
     const dim3 far_grid((unsigned)((n + EXACT_ROWS - 1) / EXACT_ROWS));
+    const int per = near_pairs_per_block(ws->near_pairs);
     with_far_variant(far_variant(k, m->panel_radius, beta.x), general, [&](auto mode, auto var) {
         constexpr int MODE = decltype(mode)::value, VAR = decltype(var)::value;
         hipLaunchKernelGGL((exact_far_kernel<MODE, VAR>), far_grid, dim3(256), 0, ctx->stream, m->d_far.ptr,
                            m->d_src.ptr, m->d_bc.ptr, n, k, ph.tau, beta, iwr, x, op->d_far.ptr);
         SBH_HIP(hipGetLastError());
         if (ws->near_pairs > 0)
-            hipLaunchKernelGGL((exact_near_kernel<MODE, VAR>), dim3((unsigned)((ws->near_pairs + 3) / 4)), dim3(256),
-                               0, ctx->stream, ws->d_pairs.ptr, ws->near_pairs, ws->d_leaves.ptr, m->d_geom.ptr,
-                               m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, k, wavruim, ph.tau, beta, iwr, x,
-                               op->d_near.ptr);
+            hipLaunchKernelGGL((exact_near_kernel<MODE, VAR>), dim3((unsigned)((ws->near_pairs + per - 1) / per)),
+                               dim3(256), 0, ctx->stream, ws->d_pairs.ptr, ws->near_pairs, per, ws->d_leaves.ptr,
+                               m->d_far.ptr, m->d_src.ptr, m->d_bc.ptr, k, ph.tau, beta, iwr, x, op->d_near.ptr);
     });
     SBH_HIP(hipGetLastError());
     hipLaunchKernelGGL(exact_self_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, ctx->stream, m->d_geom.ptr,

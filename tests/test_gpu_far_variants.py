@@ -107,3 +107,26 @@ def test_far_derivatives_match_the_oracle(ctx, k, beta, general):
                                              admittance_scale=0.5, **bc)
         assert rel_fro(A[far], Ar[far]) <= TOL
         assert rel_fro(A, Ar) <= 1e-12
+
+
+@pytest.mark.parametrize("derivative", [False, True])
+@pytest.mark.parametrize("axes,level,k", [((1.0, 1.0, 1.0), 0, 0.7), ((1.0, 1.0, 1.0), 2, 2.0),
+                                          ((1.4, 0.35, 0.3), 2, 3.0), ((1.4, 0.35, 0.3), 3, 40.0)])
+def test_near_entries_match_the_oracle(ctx, axes, level, k, derivative):
+    """Subdivided pairs alone: one workgroup's worth of pairs and many, panels
+    of aspect up to 5 (deep trees, up to the 110-leaf cap), the general form.
+    The oracle forms positions before subtracting: 2^-53 * 1.4 over a leaf
+    distance of at least 0.02, up to three powers of 1/r: 3e-14."""
+    m = ellipsoid(axes, level)
+    near = ~_far(m) & ~np.eye(m.num_elements, dtype=bool)
+    ph = sa.PhysicsParams.from_wavenumber(k)
+    for general in (False, True):
+        bc = _mixed(m.num_elements) if general else {}
+        ws = sa.TbemAssemblyWorkspace(ctx, sa.TbemMesh(ctx, m, **bc))
+        if derivative:
+            A = ws.assemble_parameter_derivative(ph, 1j / k, -1j / k ** 2).matrix
+            Ar, _ = oracle.build_tbem_derivative(m.nodes, m.triangles, k, 1j / k, -1j / k ** 2, **bc)
+        else:
+            A = ws.assemble(ph, 1j / k).matrix
+            Ar, _ = oracle.build_tbem_system(m.nodes, m.triangles, k, 1j / k, **bc)
+        assert rel_fro(A[near], Ar[near]) <= 1e-13
