@@ -402,11 +402,12 @@ __global__ void lp_reduce_kernel(const float* __restrict__ Ypart, int64_t n, int
 // Block: 4 waves over BM = 128 rows x 16*NT real columns; wave w owns rows
 // 32w..32w+31 (2 x NT tiles of 16 x 16). Stages of 8 complex (16 real) columns
 // of A go through LDS, transposed so that MFMA operand reads are contiguous.
-// The K range is split in ZG_SPLIT slices (slice = blockIdx % ZG_SPLIT, one per
-// XCD); partials go to Ypart[slice][row][16*NT] and zgemm_reduce_kernel sums
-// them in slice order.
+// The K range is split in slices (slice = blockIdx % splits, zgemm_plan);
+// partials go to Ypart[slice][row][16*NT] and zgemm_reduce_kernel sums them in
+// slice order.
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-constexpr int ZG_SPLIT = 8;
+constexpr int ZG_SPLIT = 8;          // slices the fixed scratch is sized for
+constexpr int ZG_MAX_SPLIT = 16;
 constexpr int ZG_BM = 128;
 constexpr int ZG_BKC = 16;           // complex columns of A per stage
 constexpr int ZG_AROW = ZG_BM + 2;   // LDS row of the transposed A stage (doubles)
@@ -414,15 +415,15 @@ constexpr int ZG_AROW = ZG_BM + 2;   // LDS row of the transposed A stage (doubl
 template <int NT>
 __global__ __launch_bounds__(BLOCK) void zgemm_f64_kernel(const double2* __restrict__ A, int64_t lda, int64_t n,
                                                           const double2* __restrict__ X, int64_t ldx, int kc,
-                                                          int64_t kslice, double* __restrict__ Ypart) {
+                                                          int64_t kslice, int splits, double* __restrict__ Ypart) {
     constexpr int NR = 16 * NT;  // real output columns
     __shared__ double As[2 * ZG_BKC][ZG_AROW];
     __shared__ __attribute__((aligned(16))) double Xs[2 * ZG_BKC][NR];
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int w = t >> 6;
-    const int split = blockIdx.x % ZG_SPLIT;
-    const int64_t row0 = (int64_t)(blockIdx.x / ZG_SPLIT) * ZG_BM;
+    const int split = blockIdx.x % splits;
+    const int64_t row0 = (int64_t)(blockIdx.x / splits) * ZG_BM;
     const int64_t kbeg = (int64_t)split * kslice;
     const int64_t kend = min(n, kbeg + kslice);
     f64x4 acc[2][NT];
@@ -503,19 +504,24 @@ __global__ __launch_bounds__(BLOCK) void zgemm_f64_kernel(const double2* __restr
 }
 
 // Y[r, c] = sum over slices of the partials (complex columns c < kc), slice order fixed
-__global__ void zgemm_reduce_kernel(const double* __restrict__ Ypart, int64_t n, int nr, int kc,
+__global__ void zgemm_reduce_kernel(const double* __restrict__ Ypart, int splits, int64_t n, int nr, int kc,
                                     double2* __restrict__ Y, int64_t ldy) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n * kc) return;
     const int64_t r = e / kc;
     const int c = (int)(e % kc);
+    double2 p[ZG_MAX_SPLIT];  // all loads in flight before the additions
+#pragma unroll
+    for (int s = 0; s < ZG_MAX_SPLIT; ++s)
+        p[s] = s < splits ? *reinterpret_cast<const double2*>(Ypart + ((size_t)s * n + r) * nr + 2 * c)
+                          : make_double2(0.0, 0.0);
     double sr = 0.0, si = 0.0;
 #pragma unroll
-    for (int s = 0; s < ZG_SPLIT; ++s) {
-        const double2 p = *reinterpret_cast<const double2*>(Ypart + ((size_t)s * n + r) * nr + 2 * c);
-        sr += p.x;
-        si += p.y;
-    }
+    for (int s = 0; s < ZG_MAX_SPLIT; ++s)
+        if (s < splits) {
+            sr += p[s].x;
+            si += p[s].y;
+        }
     Y[r * ldy + c] = make_double2(sr, si);
 }
 
@@ -879,11 +885,51 @@ SBH_LOWP_PRODUCTS(double2)
 SBH_LOWP_PRODUCTS(float2)
 #undef SBH_LOWP_PRODUCTS
 
-// Split-K partials of one 64-column chunk: ZG_SPLIT x n x nr doubles.
+// Doubles that the fixed scratch must hold for a shape to be accepted there:
+// ZG_SPLIT slices of the next power of two of 8-column tiles.
 static size_t zgemm_partial_doubles(int64_t n, int64_t k) {
     const int kc = (int)std::min<int64_t>(64, k);
     const int nt = kc <= 8 ? 1 : kc <= 16 ? 2 : kc <= 32 ? 4 : 8;
     return (size_t)ZG_SPLIT * (size_t)n * (size_t)(16 * nt);
+}
+
+// Column tiles and K slices of one chunk of kc columns.  The chip holds 512
+// workgroups of this kernel (two per CU) and they all cost the same, so what
+// counts is the last round: 10240 rows make 80 row tiles, whose 640 workgroups
+// at 8 slices took two rounds, 1.15 ms at 64 columns, and whose 480 at 6 take one,
+// 0.89 ms; 24 columns on 5056 rows take 124 us instead of 219.  The
+// slice count is the one with the least rounds x stages per workgroup, plus
+// the partials' traffic (a slice writes and reads n x 16 nt doubles; in stages
+// of 7 us, n nt / 1e5 with the reduction).  Shapes that the fixed scratch takes
+// use no more slices than fit there, so both entry points do the same work.
+struct ZgemmPlan {
+    int nt, splits;
+    int64_t kslice;
+};
+
+static ZgemmPlan zgemm_plan(int64_t n, int kc) {
+    ZgemmPlan p;
+    p.nt = (kc + 7) / 8;
+    const int64_t row_tiles = (n + ZG_BM - 1) / ZG_BM;
+    const int64_t stages = (n + ZG_BKC - 1) / ZG_BKC;
+    const size_t slab = (size_t)n * (size_t)(16 * p.nt);
+    int limit = ZG_MAX_SPLIT;
+    if (zgemm_partial_doubles(n, kc) <= NOALLOC_SCRATCH_DOUBLES)
+        limit = (int)std::min<size_t>(limit, NOALLOC_SCRATCH_DOUBLES / slab);
+    p.splits = 1;
+    double best = 0.0;
+    for (int s = 1; s <= limit && s <= stages; ++s) {
+        const int64_t per = (stages + s - 1) / s;
+        if ((stages + per - 1) / per != s) continue;  // some slice would be empty
+        const double cost = (double)((row_tiles * s + 511) / 512) * (double)(per + 2) * (double)p.nt / 8.0 +
+                            (double)s * (double)n * (double)p.nt / 1.0e5;
+        if (s == 1 || cost < best) {
+            best = cost;
+            p.splits = s;
+            p.kslice = per * ZG_BKC;
+        }
+    }
+    return p;
 }
 
 // Y = A X in 64-column chunks; part (null: the context's scratch, grown on
@@ -891,26 +937,34 @@ static size_t zgemm_partial_doubles(int64_t n, int64_t k) {
 // every chunk.
 static void zgemm_f64_into(sbh_context* ctx, const double2* A, int64_t lda, int64_t n, const double2* X, int64_t k,
                            double2* Y, double* part) {
-    const int64_t kslice = ((n + ZG_SPLIT - 1) / ZG_SPLIT + ZG_BKC - 1) / ZG_BKC * ZG_BKC;
     const int64_t row_tiles = (n + ZG_BM - 1) / ZG_BM;
-    SBH_REQUIRE(row_tiles * ZG_SPLIT < ((int64_t)1 << 31), "block product too large");
+    SBH_REQUIRE(row_tiles * ZG_MAX_SPLIT < ((int64_t)1 << 31), "block product too large");
     for (int64_t c0 = 0; c0 < k; c0 += 64) {
         const int kc = (int)std::min<int64_t>(64, k - c0);
-        const int nt = kc <= 8 ? 1 : kc <= 16 ? 2 : kc <= 32 ? 4 : 8;
-        const int nr = 16 * nt;
-        double* chunk_part = part ? part : reinterpret_cast<double*>(ctx->device_scratch((size_t)ZG_SPLIT * n * nr / 2));
-        const dim3 grid((unsigned)(row_tiles * ZG_SPLIT));
+        const ZgemmPlan p = zgemm_plan(n, kc);
+        const int nr = 16 * p.nt;
+        double* chunk_part =
+            part ? part : reinterpret_cast<double*>(ctx->device_scratch((size_t)p.splits * n * nr / 2));
+        const dim3 grid((unsigned)(row_tiles * p.splits));
 #define SBH_ZG(NT_)                                                                                           \
-    hipLaunchKernelGGL(zgemm_f64_kernel<NT_>, grid, dim3(BLOCK), 0, ctx->stream, A, lda, n, X + c0, k, kc, kslice, \
-                       chunk_part)
-        if (nt == 1) SBH_ZG(1);
-        else if (nt == 2) SBH_ZG(2);
-        else if (nt == 4) SBH_ZG(4);
-        else SBH_ZG(8);
+    case NT_:                                                                                                 \
+        hipLaunchKernelGGL(zgemm_f64_kernel<NT_>, grid, dim3(BLOCK), 0, ctx->stream, A, lda, n, X + c0, k, kc, \
+                           p.kslice, p.splits, chunk_part);                                                   \
+        break
+        switch (p.nt) {
+            SBH_ZG(1);
+            SBH_ZG(2);
+            SBH_ZG(3);
+            SBH_ZG(4);
+            SBH_ZG(5);
+            SBH_ZG(6);
+            SBH_ZG(7);
+            SBH_ZG(8);
+        }
 #undef SBH_ZG
         SBH_HIP(hipGetLastError());
-        hipLaunchKernelGGL(zgemm_reduce_kernel, dim3(nblocks(n * kc)), dim3(BLOCK), 0, ctx->stream, chunk_part, n, nr,
-                           kc, Y + c0, k);
+        hipLaunchKernelGGL(zgemm_reduce_kernel, dim3(nblocks(n * kc)), dim3(BLOCK), 0, ctx->stream, chunk_part,
+                           p.splits, n, nr, kc, Y + c0, k);
         SBH_HIP(hipGetLastError());
     }
 }

@@ -182,3 +182,28 @@ def test_block_gmres_checked_boundary(sphere1280):
         sa.block_gmres_preconditioned_with_guess(op, B, None, X0)
     assert "initial guess" in str(e.value)
     op.close()
+
+
+@pytest.mark.parametrize("n_theta,n_phi", [(5, 3), (5, 17), (9, 40), (21, 61)])
+@pytest.mark.parametrize("k", [1, 8, 9, 24, 33, 41, 56, 57, 64, 70])
+def test_block_product_tiles_and_slices(ctx, n_theta, n_phi, k):
+    """Every column tile count (8 columns each, the last ragged, two chunks at
+    70) on 24 to 2440 panels, one to 16 K slices with a short last one; FP64 sums
+    in another order: 1e-14 of |A| |X|, and the allocation-free entry point's
+    bits."""
+    from sonium_amd.mesh import fibonacci_sphere
+
+    m = fibonacci_sphere(1.0, n_theta, n_phi)
+    n = m.num_elements
+    ph = sa.PhysicsParams.from_wavenumber(1.0)
+    system = sa.build_tbem_system(ctx, sa.TbemMesh(ctx, m), ph)
+    op = sa.DenseMatrixOperator(system)
+    rng = np.random.default_rng(n + k)
+    X = rng.standard_normal((n, k)) + 1j * rng.standard_normal((n, k))
+    Y = op.apply_block(X)
+    A = system.matrix
+    assert np.max(np.abs(Y - A @ X) / (np.abs(A) @ np.abs(X))) <= 1e-14
+    x, y = sa.DeviceVector(ctx, n * k), sa.DeviceVector(ctx, n * k)
+    x.upload(X)
+    op.apply_block_noalloc(x, y, k)
+    assert np.array_equal(y.download().reshape(n, k), Y)
