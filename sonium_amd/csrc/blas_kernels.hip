@@ -211,6 +211,95 @@ __global__ __launch_bounds__(BLOCK) void project_norm_kernel(const double2* __re
     if (threadIdx.x == 0) norm_out[blockIdx.x] = t;
 }
 
+// One Gram–Schmidt step in one workgroup, for vectors of at most ARNOLDI_MAX_N:
+// classical Gram–Schmidt of w against v_0 .. v_{nvec-1}, a second pass when the
+// norm falls below 0.707 of the first (cgs_orth.rs:180-301), and the normalised
+// next basis vector, all without the host.  out (pinned host memory) gets the
+// nvec summed coefficients, then ||w|| and 1.0 if the second pass ran.
+//
+// It is latency that bounds a step at these sizes: the separate dot, sum,
+// projection and copy launches with a host read per pass take 53 us a step at 320
+// panels, most of it in the two round trips; this kernel takes 9 us there and
+// the host reads it behind the next step (a step is 18 us).  w stays in LDS; a wave takes every
+// 16th dot product, a thread one element of the projection.  Above
+// ARNOLDI_MAX_N one CU's share of the L2 is the slower way.
+constexpr int ARNOLDI_THREADS = 1024;
+
+__global__ __launch_bounds__(ARNOLDI_THREADS) void arnoldi_small_kernel(const double2* __restrict__ V, int64_t ldv,
+                                                                        int nvec, const double2* __restrict__ w,
+                                                                        int n, double2* __restrict__ vnext,
+                                                                        double* __restrict__ out) {
+    __shared__ double2 ws[ARNOLDI_MAX_N];
+    __shared__ double2 coef[ARNOLDI_MAX_BASIS], total[ARNOLDI_MAX_BASIS];
+    __shared__ double red[ARNOLDI_THREADS / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    auto norm = [&](double v) {  // sqrt of the block's sum, on every thread
+        v = wave_sum(v);
+        __syncthreads();
+        if (lane == 0) red[wave] = v;
+        __syncthreads();
+        double sum = 0.0;
+#pragma unroll
+        for (int q = 0; q < ARNOLDI_THREADS / 64; ++q) sum += red[q];
+        return sqrt(sum);
+    };
+    double nr = 0.0;
+    for (int k = t; k < n; k += ARNOLDI_THREADS) {
+        const double2 v = w[k];
+        ws[k] = v;
+        nr += v.x * v.x + v.y * v.y;
+    }
+    const double before = norm(nr);  // also orders ws
+    double after = before;
+    bool again = false;
+    for (int pass = 0; pass < 2; ++pass) {
+        for (int i = wave; i < nvec; i += ARNOLDI_THREADS / 64) {
+            const double2* __restrict__ v = V + (int64_t)i * ldv;
+            double sr = 0.0, si = 0.0;
+#pragma unroll 4
+            for (int k = lane; k < n; k += 64) {
+                const double2 p = cmulc(v[k], ws[k]);
+                sr += p.x;
+                si += p.y;
+            }
+            sr = wave_sum(sr);
+            si = wave_sum(si);
+            if (lane == 0) {
+                coef[i] = make_double2(sr, si);
+                total[i] = pass == 0 ? coef[i] : make_double2(total[i].x + sr, total[i].y + si);
+            }
+        }
+        __syncthreads();
+        nr = 0.0;
+        for (int k = t; k < n; k += ARNOLDI_THREADS) {
+            double sr = 0.0, si = 0.0;
+#pragma unroll 8
+            for (int i = 0; i < nvec; ++i) {
+                const double2 p = cmul(coef[i], V[(int64_t)i * ldv + k]);
+                sr += p.x;
+                si += p.y;
+            }
+            const double2 v = make_double2(ws[k].x - sr, ws[k].y - si);
+            ws[k] = v;
+            nr += v.x * v.x + v.y * v.y;
+        }
+        after = norm(nr);
+        if (pass == 1 || !(after < 0.707 * before)) break;
+        again = true;
+    }
+    for (int i = t; i < nvec; i += ARNOLDI_THREADS) {
+        out[2 * i] = total[i].x;
+        out[2 * i + 1] = total[i].y;
+    }
+    if (t == 0) {
+        out[2 * nvec] = after;
+        out[2 * nvec + 1] = again ? 1.0 : 0.0;
+    }
+    if (after < 1e-20) return;  // breakdown: the host forms no further vector
+    const double alpha = 1.0 / after;
+    for (int k = t; k < n; k += ARNOLDI_THREADS) vnext[k] = make_double2(ws[k].x * alpha, ws[k].y * alpha);
+}
+
 __global__ void basis_update_kernel(const double2* __restrict__ V, int64_t ldv, int nvec,
                                     const double2* __restrict__ c, double2* __restrict__ x, int64_t n) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -294,26 +383,27 @@ int reduction_chunks(int64_t n) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(c, 64));
 }
 
+// Four rows a wave reuse each element of x; up to 4096 rows that makes fewer
+// workgroups than CUs and a row a wave is faster (320 rows: 3.8 instead of 4.6 us).
+// A row's sum is the same either way.
+static void zgemv_n_strided(sbh_context* ctx, const double2* A, int64_t lda, int64_t rows,
+                            int64_t cols, const double2* x, int64_t incx, double2* y, int64_t incy) {
+    if (rows <= 4096)
+        hipLaunchKernelGGL(zgemv_n_kernel<1>, dim3(blocks_for(rows, BLOCK / 64)), dim3(BLOCK), 0, ctx->stream, A, lda,
+                           rows, cols, x, incx, y, incy);
+    else
+        hipLaunchKernelGGL(zgemv_n_kernel<4>, dim3(blocks_for((rows + 3) / 4, BLOCK / 64)), dim3(BLOCK), 0,
+                           ctx->stream, A, lda, rows, cols, x, incx, y, incy);
+    SBH_HIP(hipGetLastError());
+}
+
 void zgemv_n(sbh_context* ctx, const double2* A, int64_t lda, int64_t rows, int64_t cols,
              const double2* x, double2* y) {
     if (rows == 0) return;
-    constexpr int ROWS = 4;
-    const int64_t waves = (rows + ROWS - 1) / ROWS;
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_MATVEC, &ev);
-    hipLaunchKernelGGL(zgemv_n_kernel<ROWS>, dim3(blocks_for(waves, BLOCK / 64)), dim3(BLOCK), 0,
-                       ctx->stream, A, lda, rows, cols, x, (int64_t)1, y, (int64_t)1);
-    SBH_HIP(hipGetLastError());
+    zgemv_n_strided(ctx, A, lda, rows, cols, x, 1, y, 1);
     ctx->end_timed(SBH_KERNEL_MATVEC, ev);
-}
-
-static void zgemv_n_strided(sbh_context* ctx, const double2* A, int64_t lda, int64_t rows,
-                            int64_t cols, const double2* x, int64_t incx, double2* y, int64_t incy) {
-    constexpr int ROWS = 4;
-    const int64_t waves = (rows + ROWS - 1) / ROWS;
-    hipLaunchKernelGGL(zgemv_n_kernel<ROWS>, dim3(blocks_for(waves, BLOCK / 64)), dim3(BLOCK), 0,
-                       ctx->stream, A, lda, rows, cols, x, incx, y, incy);
-    SBH_HIP(hipGetLastError());
 }
 
 void zgemv_n_untimed(sbh_context* ctx, const double2* A, int64_t lda, int64_t rows, int64_t cols,
@@ -398,6 +488,17 @@ void basis_update(sbh_context* ctx, const double2* V, int64_t ldv, int nvec, con
     ctx->begin_timed(SBH_KERNEL_KRYLOV_VECTOR, &ev);
     hipLaunchKernelGGL(basis_update_kernel, dim3(blocks_for(n)), dim3(BLOCK), 0, ctx->stream, V, ldv,
                        nvec, c, x, n);
+    SBH_HIP(hipGetLastError());
+    ctx->end_timed(SBH_KERNEL_KRYLOV_VECTOR, ev);
+}
+
+void arnoldi_small(sbh_context* ctx, const double2* V, int64_t ldv, int nvec, const double2* w, int64_t n,
+                   double2* vnext, double* out) {
+    SBH_REQUIRE(n <= ARNOLDI_MAX_N && nvec <= ARNOLDI_MAX_BASIS, "one-workgroup Gram-Schmidt step out of range");
+    hipEvent_t ev;
+    ctx->begin_timed(SBH_KERNEL_KRYLOV_VECTOR, &ev);
+    hipLaunchKernelGGL(arnoldi_small_kernel, dim3(1), dim3(ARNOLDI_THREADS), 0, ctx->stream, V, ldv, nvec, w, (int)n,
+                       vnext, out);
     SBH_HIP(hipGetLastError());
     ctx->end_timed(SBH_KERNEL_KRYLOV_VECTOR, ev);
 }

@@ -12,6 +12,8 @@
 // The Krylov basis, the iterate and every vector operation stay on the
 // device; only the (j+1) Gram–Schmidt coefficients and norms come back to the
 // host each step, where the small Hessenberg recurrence runs in FP64.
+// Small dense systems (Krylov::small_steps) take a step's whole orthogonalisation
+// in one launch and keep one step in flight while the host works on the last.
 
 #include <algorithm>
 #include <cmath>
@@ -73,6 +75,7 @@ sbh_status run_gmres(sbh_operator* op, sbh_precond* M, const double2* d_b, const
     K.precond(d_b, w.ptr);
     const double raw_pb = (!M || M->kind == 0) ? raw_b : K.norm(w.ptr);
     int64_t total = 0, restarts = 0, reorth = 0, exact_checks = 0;
+    const bool small = K.small_steps(alloc_m);
     auto done = [&]() {
         sol->spmv_count = K.spmv;
         sol->reorthogonalizations = reorth;
@@ -140,27 +143,39 @@ sbh_status run_gmres(sbh_operator* op, sbh_precond* M, const double2* d_b, const
         g[0] = cplx(beta, 0.0);
         bool inner_converged = false;
         bool restart_now = false;
+        if (small) K.queue_step(V.ptr, 0, w.ptr, opb.ptr);
         for (int j = 0; j < m; ++j) {
             total += 1;
-            if (!M || M->kind == 0) {
-                K.apply(vec(j), w.ptr);
+            double wn;
+            if (small) {
+                // step j + 1 needs nothing of the host: it is queued before
+                // step j is read (and left unused when step j ends the cycle)
+                if (j + 1 < m) K.queue_step(V.ptr, j + 1, w.ptr, opb.ptr);
+                bool again = false;
+                wn = K.wait_step(j, coeffs, &again);
+                for (int i = 0; i <= j; ++i) h(i, j) = coeffs[i];
+                if (again) reorth += 1;
             } else {
-                K.apply(vec(j), opb.ptr);
-                K.precond(opb.ptr, w.ptr);
-            }
-            double wnb = 0.0;
-            double wn = K.dots_project(V.ptr, j + 1, w.ptr, coeffs, &wnb);
-            for (int i = 0; i <= j; ++i) h(i, j) = coeffs[i];
-            if (wn < 0.707 * wnb) {
-                reorth += 1;
-                double unused = 0.0;
-                wn = K.dots_project(V.ptr, j + 1, w.ptr, re, &unused);
-                for (int i = 0; i <= j; ++i) h(i, j) += re[i];
+                if (!M || M->kind == 0) {
+                    K.apply(vec(j), w.ptr);
+                } else {
+                    K.apply(vec(j), opb.ptr);
+                    K.precond(opb.ptr, w.ptr);
+                }
+                double wnb = 0.0;
+                wn = K.dots_project(V.ptr, j + 1, w.ptr, coeffs, &wnb);
+                for (int i = 0; i <= j; ++i) h(i, j) = coeffs[i];
+                if (wn < 0.707 * wnb) {
+                    reorth += 1;
+                    double unused = 0.0;
+                    wn = K.dots_project(V.ptr, j + 1, w.ptr, re, &unused);
+                    for (int i = 0; i <= j; ++i) h(i, j) += re[i];
+                }
             }
             h(j + 1, j) = cplx(wn, 0.0);
             if (wn < 1e-20) {
                 inner_converged = true;
-            } else {
+            } else if (!small) {
                 scale_copy(ctx, w.ptr, 1.0 / wn, vec(j + 1), n);
             }
             for (int i = 0; i < j; ++i) {

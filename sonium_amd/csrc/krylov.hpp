@@ -41,7 +41,48 @@ struct Krylov {
         size_t need = std::max<size_t>((size_t)(m + 2) * chunks, (size_t)((n + 255) / 256)) + 8;
         part.allocate(need);
         coeff.allocate((size_t)m + 2);
-        host = ctx->pinned_rw(need * 2);
+        // after the reductions' staging: two slots for steps in flight
+        slot_stride = 2 * ((size_t)m + 4);
+        host = ctx->pinned_rw(need * 2 + 2 * slot_stride);
+        slots = host + need * 2;
+    }
+    ~Krylov() {
+        for (hipEvent_t e : done)
+            if (e) (void)hipEventDestroy(e);
+    }
+    Krylov(const Krylov&) = delete;
+    Krylov& operator=(const Krylov&) = delete;
+
+    // Steps j of a cycle on arnoldi_small: `queue_step` enqueues one (its
+    // results go to slot j % 2), `wait_step` waits for it alone, so the next
+    // step runs while the host works on this one.
+    double* slots = nullptr;
+    size_t slot_stride = 0;
+    hipEvent_t done[2] = {nullptr, nullptr};
+    bool small_steps(int m) const {
+        return op->dense() && n <= ARNOLDI_MAX_N && m <= ARNOLDI_MAX_BASIS && (!M || M->kind <= 1);
+    }
+    void queue_step(double2* V, int j, double2* w, double2* tmp) {
+        if (!M || M->kind == 0) {
+            operator_apply_device(op, V + (size_t)j * n, w);
+        } else {
+            operator_apply_device(op, V + (size_t)j * n, tmp);
+            precond(tmp, w);
+        }
+        arnoldi_small(ctx, V, n, j + 1, w, n, V + (size_t)(j + 1) * n, slots + (j & 1) * slot_stride);
+        hipEvent_t& e = done[j & 1];
+        if (!e) SBH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        SBH_HIP(hipEventRecord(e, ctx->stream));
+    }
+    // Returns ||w|| after the step; coefficients in out.
+    double wait_step(int j, std::vector<cplx>& out, bool* again) {
+        SBH_HIP(hipEventSynchronize(done[j & 1]));
+        spmv += 1;
+        const double* r = slots + (j & 1) * slot_stride;
+        out.resize((size_t)j + 1);
+        for (int i = 0; i <= j; ++i) out[i] = cplx(r[2 * i], r[2 * i + 1]);
+        *again = r[2 * (j + 1) + 1] != 0.0;
+        return r[2 * (j + 1)];
     }
 
     void apply(const double2* x, double2* y) {

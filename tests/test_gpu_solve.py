@@ -184,3 +184,34 @@ def test_gmres_rejects_negative_options(c1):
     op = sa.DenseMatrixOperator(c1["sys"])
     sol = sa.gmres(op, c1["b"], sa.GmresConfig(10, 10, 1e-8, convergence_check_interval=-1))
     assert sol.status == "numerical_error" and sol.iterations == 0
+
+
+@pytest.mark.parametrize("n_theta,n_phi,restart,jacobi", [
+    (5, 3, 50, False),       # 24 panels: the basis can fill the space
+    (9, 20, 4, True),        # restarts, left preconditioning
+    (9, 20, 256, False),     # the longest basis of the one-workgroup step
+    (9, 20, 257, False),     # and the first that takes the general steps
+    (33, 32, 30, False),     # 2048 panels: its largest vectors
+    (33, 33, 30, True),      # 2112: the general steps
+])
+def test_gmres_steps_at_the_edges_of_the_small_path(ctx, n_theta, n_phi, restart, jacobi):
+    """Step counts, reorthogonalisations and solutions of the oracle on both
+    sides of every limit of the one-workgroup Gram-Schmidt step."""
+    from sonium_amd.mesh import fibonacci_sphere
+
+    m = fibonacci_sphere(1.0, n_theta, n_phi)
+    k = 1.5
+    ph = sa.PhysicsParams.from_wavenumber(k)
+    tm = sa.TbemMesh(ctx, m)
+    beta = ph.burton_miller_beta()
+    system = sa.build_tbem_system_with_beta(ctx, tm, ph, beta)
+    b = sa.IncidentField.plane_wave_z().compute_rhs_with_beta(tm, ph, beta)
+    op = sa.DenseMatrixOperator(system)
+    pre = sa.JacobiPreconditioner(op) if jacobi else None
+    sol = sa.gmres_preconditioned(op, pre, b, sa.GmresConfig(max_iterations=60, restart=restart, tolerance=1e-8))
+    xr, st = oracle.gmres(system.matrix, b, restart=restart, max_iterations=60, tol=1e-8, jacobi=jacobi)
+    assert sol.converged and sol.residual <= 1e-8
+    assert sol.iterations == st["iterations"] and sol.restarts == st["restarts"]
+    # the same steps in another summation order
+    assert np.linalg.norm(sol.x - xr) <= 1e-10 * np.linalg.norm(xr)
+    assert np.linalg.norm(b - op.apply(sol.x)) <= 1.01e-8 * np.linalg.norm(b)
