@@ -40,7 +40,7 @@ void require_dense(const sbh_operator* op, const char* what) {
 
 // Device copy of a host or device input vector.
 struct DeviceInput {
-    DeviceArray<double2> owned;
+    WorkArray<double2> owned;
     const double2* ptr = nullptr;
     DeviceInput(sbh_context* ctx, const sbh_c64* p, size_t n, int memory) {
         if (memory == SBH_MEM_DEVICE) {
@@ -55,7 +55,7 @@ struct DeviceInput {
 };
 
 struct DeviceOutput {
-    DeviceArray<double2> owned;
+    WorkArray<double2> owned;
     double2* ptr = nullptr;
     sbh_c64* host = nullptr;
     size_t n = 0;
@@ -126,6 +126,107 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 thread_local sbh_context* g_current_ctx = nullptr;
 std::atomic<int64_t> g_live_device_bytes{0};
 
+namespace {
+struct WorkPool {
+    std::mutex mu;
+    std::vector<WorkBlock> idle;  // oldest first
+    size_t bytes = 0;
+};
+// never destroyed: arrays may outlive the library's static objects
+WorkPool& work_pool() {
+    static WorkPool* pool = new WorkPool;
+    return *pool;
+}
+
+void work_free(const WorkBlock& b) {
+    if (b.pinned)
+        (void)hipHostFree(b.ptr);
+    else
+        (void)hipFree(b.ptr);
+}
+}  // namespace
+
+void work_trim() {
+    WorkPool& pool = work_pool();
+    std::vector<WorkBlock> idle;
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        idle.swap(pool.idle);
+        pool.bytes = 0;
+    }
+    for (const WorkBlock& b : idle) work_free(b);
+}
+
+void* device_malloc(size_t bytes) {
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // clear it
+        work_trim();
+        e = hipMalloc(&p, bytes);
+    }
+    SBH_HIP(e);
+    return p;
+}
+
+WorkBlock work_take(size_t bytes, bool pinned) {
+    WorkBlock b;
+    b.bytes = (bytes + 255) / 256 * 256;
+    b.pinned = pinned;
+    SBH_HIP(hipGetDevice(&b.device));
+    {
+        // the smallest idle block that fits without wasting more than a quarter
+        WorkPool& pool = work_pool();
+        std::lock_guard<std::mutex> lk(pool.mu);
+        size_t best = pool.idle.size();
+        for (size_t i = 0; i < pool.idle.size(); ++i) {
+            const WorkBlock& c = pool.idle[i];
+            if (c.device == b.device && c.pinned == pinned && c.bytes >= b.bytes &&
+                c.bytes <= b.bytes + b.bytes / 4 + 65536 && (best == pool.idle.size() || c.bytes < pool.idle[best].bytes))
+                best = i;
+        }
+        if (best < pool.idle.size()) {
+            b = pool.idle[best];
+            pool.idle.erase(pool.idle.begin() + (std::ptrdiff_t)best);
+            pool.bytes -= b.bytes;
+            return b;
+        }
+    }
+    if (pinned)
+        SBH_HIP(hipHostMalloc(&b.ptr, b.bytes, hipHostMallocDefault));
+    else
+        b.ptr = device_malloc(b.bytes);
+    return b;
+}
+
+void work_give(const WorkBlock& b) {
+    // hipFree's order: nothing on the device uses the block any more, whatever
+    // stream it was on
+    int device = -1;
+    if (b.bytes > WORK_BLOCK_LIMIT || hipGetDevice(&device) != hipSuccess || device != b.device ||
+        hipDeviceSynchronize() != hipSuccess) {
+        work_free(b);
+        return;
+    }
+    WorkPool& pool = work_pool();
+    {
+        std::lock_guard<std::mutex> lk(pool.mu);
+        pool.idle.push_back(b);
+        pool.bytes += b.bytes;
+    }
+    for (;;) {
+        WorkBlock oldest;
+        {
+            std::lock_guard<std::mutex> lk(pool.mu);
+            if (pool.bytes <= WORK_IDLE_LIMIT && pool.idle.size() <= WORK_IDLE_BLOCKS) return;
+            oldest = pool.idle.front();
+            pool.idle.erase(pool.idle.begin());
+            pool.bytes -= oldest.bytes;
+        }
+        work_free(oldest);
+    }
+}
+
 void injection_check(int point) {
     sbh_context* ctx = g_current_ctx;
     if (!ctx) return;
@@ -155,6 +256,10 @@ void admit_device(sbh_context* ctx, int64_t bytes, const char* what, bool reserv
                                                std::to_string(budget) + " with " + std::to_string(held) + " held");
     size_t free_b = 0, total_b = 0;
     SBH_HIP(hipMemGetInfo(&free_b, &total_b));
+    if ((uint64_t)bytes > (uint64_t)free_b) {  // idle work blocks do not count
+        work_trim();
+        SBH_HIP(hipMemGetInfo(&free_b, &total_b));
+    }
     if ((uint64_t)bytes > (uint64_t)free_b)
         throw Error(SBH_ERR_OUT_OF_MEMORY, std::string("admission refused: ") + what + " needs " +
                                                std::to_string(bytes) + " device bytes; the device has " +
@@ -182,6 +287,7 @@ void context_release(sbh_context* ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
+    work_trim();
 }
 
 }  // namespace sbh
@@ -205,7 +311,7 @@ double2* sbh_context::device_scratch(size_t count) {
         if (scratch) (void)hipFree(scratch);
         scratch = nullptr;
         scratch_count = 0;
-        SBH_HIP(hipMalloc(reinterpret_cast<void**>(&scratch), count * sizeof(double2)));
+        scratch = static_cast<double2*>(device_malloc(count * sizeof(double2)));
         scratch_count = count;
     }
     return scratch;
@@ -845,8 +951,8 @@ sbh_status sbh_incident_plane_wave_rhs(sbh_context* ctx, const sbh_mesh* mesh, c
                 dirs[3 * c + 2] = -1.0;
             }
         }
-        DeviceArray<double> d_dirs(3 * num_rhs);
-        DeviceArray<double2> d_amps(num_rhs);
+        WorkArray<double> d_dirs(3 * num_rhs);
+        WorkArray<double2> d_amps(num_rhs);
         SBH_HIP(hipMemcpyAsync(d_dirs.ptr, dirs.data(), d_dirs.bytes(), hipMemcpyHostToDevice, ctx->stream));
         SBH_HIP(hipMemcpyAsync(d_amps.ptr, amplitudes, d_amps.bytes(), hipMemcpyHostToDevice, ctx->stream));
         const size_t total = (size_t)mesh->n * (size_t)num_rhs;
@@ -855,7 +961,7 @@ sbh_status sbh_incident_plane_wave_rhs(sbh_context* ctx, const sbh_mesh* mesh, c
                                 reinterpret_cast<double2*>(rhs), accumulate != 0);
             SBH_HIP(hipStreamSynchronize(ctx->stream));
         } else {
-            DeviceArray<double2> tmp(total);
+            WorkArray<double2> tmp(total);
             if (accumulate)
                 SBH_HIP(hipMemcpyAsync(tmp.ptr, rhs, tmp.bytes(), hipMemcpyHostToDevice, ctx->stream));
             launch_incident_rhs(ctx, mesh, *ph, beta, sign, d_dirs.ptr, d_amps.ptr, num_rhs, tmp.ptr,
@@ -934,7 +1040,7 @@ static void field_pressure_impl(sbh_context* ctx, const sbh_mesh* mesh, const sb
             if (!std::isfinite(h[j].re) || !std::isfinite(h[j].im))
                 throw Error(SBH_ERR_INVALID_ARGUMENT, "surface sample " + std::to_string(j) + " is not finite");
     }
-    DeviceArray<IncidentSource> d_src(sources.size());
+    WorkArray<IncidentSource> d_src(sources.size());
     if (!sources.empty())
         SBH_HIP(hipMemcpyAsync(d_src.ptr, sources.data(), d_src.bytes(), hipMemcpyHostToDevice, ctx->stream));
     const double2* d_sol = reinterpret_cast<const double2*>(solution);
@@ -942,8 +1048,8 @@ static void field_pressure_impl(sbh_context* ctx, const sbh_mesh* mesh, const sb
     const double* d_pts = points;
     double2* outs[3] = {reinterpret_cast<double2*>(scattered), reinterpret_cast<double2*>(incident),
                         reinterpret_cast<double2*>(total)};
-    DeviceArray<double2> h_sol, h_vel, h_out[3];
-    DeviceArray<double> h_pts;
+    WorkArray<double2> h_sol, h_vel, h_out[3];
+    WorkArray<double> h_pts;
     if (memory == SBH_MEM_HOST) {
         h_sol.allocate((size_t)n);
         h_pts.allocate((size_t)(3 * num_points));
@@ -1027,7 +1133,7 @@ sbh_status sbh_incident_rhs(sbh_context* ctx, const sbh_mesh* mesh, const sbh_ph
                             std::isfinite(s[w].amp[0]) && std::isfinite(s[w].amp[1]),
                         "incident sources must be finite");
         }
-        DeviceArray<IncidentSource> d_src((size_t)num_sources);
+        WorkArray<IncidentSource> d_src((size_t)num_sources);
         if (num_sources)
             SBH_HIP(hipMemcpyAsync(d_src.ptr, s, d_src.bytes(), hipMemcpyHostToDevice, ctx->stream));
         if (memory == SBH_MEM_DEVICE) {
@@ -1035,7 +1141,7 @@ sbh_status sbh_incident_rhs(sbh_context* ctx, const sbh_mesh* mesh, const sbh_ph
                               accumulate != 0);
             SBH_HIP(hipStreamSynchronize(ctx->stream));
         } else {
-            DeviceArray<double2> tmp((size_t)mesh->n);
+            WorkArray<double2> tmp((size_t)mesh->n);
             if (accumulate) SBH_HIP(hipMemcpyAsync(tmp.ptr, rhs, tmp.bytes(), hipMemcpyHostToDevice, ctx->stream));
             launch_source_rhs(ctx, mesh, *ph, beta, sign, d_src.ptr, num_sources, tmp.ptr, accumulate != 0);
             SBH_HIP(hipMemcpyAsync(rhs, tmp.ptr, tmp.bytes(), hipMemcpyDeviceToHost, ctx->stream));
@@ -1144,7 +1250,7 @@ sbh_status sbh_operator_apply_block(sbh_operator* op, const sbh_c64* X, sbh_c64*
             operator_apply_device(op, in.ptr, outv.ptr);
         } else if (!op->dense()) {
             // column by column (the trait's default apply_block): strided gather, product, scatter
-            DeviceArray<double2> xc((size_t)n), yc((size_t)n);
+            WorkArray<double2> xc((size_t)n), yc((size_t)n);
             for (int64_t c = 0; c < k; ++c) {
                 SBH_HIP(hipMemcpy2DAsync(xc.ptr, sizeof(double2), in.ptr + c, sizeof(double2) * k, sizeof(double2),
                                          n, hipMemcpyDeviceToDevice, op->ctx->stream));
@@ -1358,7 +1464,7 @@ sbh_status sbh_block_gmres(sbh_operator* op, sbh_precond* precond, const sbh_c64
         if (memory == SBH_MEM_DEVICE) {
             // device inputs: the same finiteness checks through one norm each
             // (bk_frob_partials writes at most 256 partials)
-            DeviceArray<double> part(256 + 16);
+            WorkArray<double> part(256 + 16);
             auto finite_norm = [&](const double2* v) {
                 const int chunks = bk_frob_partials(op->ctx, v, n * k, part.ptr);
                 std::vector<double> h((size_t)chunks);
@@ -1447,7 +1553,7 @@ sbh_status sbh_gcro_dr(sbh_operator* op, sbh_precond* precond, const sbh_c64* b,
         if (x0) dx0.reset(new DeviceInput(op->ctx, x0, (size_t)n, memory));
         DeviceOutput dx(op->ctx, x, (size_t)n, memory);
         if (memory == SBH_MEM_DEVICE) {
-            DeviceArray<double> part(256 + 16);
+            WorkArray<double> part(256 + 16);
             auto finite_norm = [&](const double2* v) {
                 const int chunks = bk_frob_partials(op->ctx, v, n, part.ptr);
                 std::vector<double> h((size_t)chunks);

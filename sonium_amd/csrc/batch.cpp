@@ -774,7 +774,7 @@ sbh_status sbh_batch_apply(sbh_batch* b, int format, const sbh_c64* X, sbh_c64* 
         const size_t L = (size_t)b->L;
         for (size_t i = 0; i < L; ++i)
             SBH_REQUIRE(std::isfinite(X[i].re) && std::isfinite(X[i].im), "X is not finite");
-        DeviceArray<double2> dx(L), dy(L);
+        WorkArray<double2> dx(L), dy(L);
         DeviceArray<int> active((size_t)b->B);
         fill_int(b->ctx, active, 1);
         copy_on_stream(b->ctx, dx.ptr, X, L * sizeof(double2), hipMemcpyHostToDevice);
@@ -1043,15 +1043,15 @@ sbh_status sbh_batch_autotune(sbh_batch* b, double* table, int max_entries, int*
         // chunk size: one Gram-Schmidt pass (dots + projection) over 16 basis vectors
         best_ms = INFINITY;
         const int nvec = 16;
-        DeviceArray<double2> V((size_t)(nvec + 1) * b->L);
+        WorkArray<double2> V((size_t)(nvec + 1) * b->L);
         SBH_HIP(hipMemsetAsync(V.ptr, 0, V.bytes(), ctx->stream));
         DeviceArray<int> flag((size_t)b->B);
         fill_int(ctx, flag, 1);
         for (int ce : {2048, 4096, 8192, 16384}) {
             b->tuning.chunk_elems = ce;
             build_chunks(b);
-            DeviceArray<double2> part((size_t)b->nchunks * (nvec + 2) * kMaxCol);
-            DeviceArray<double2> coef((size_t)b->C * (nvec + 2));
+            WorkArray<double2> part((size_t)b->nchunks * (nvec + 2) * kMaxCol);
+            WorkArray<double2> coef((size_t)b->C * (nvec + 2));
             SBH_HIP(hipMemsetAsync(coef.ptr, 0, coef.bytes(), ctx->stream));
             RaggedLayout lay;
             lay.B = b->B;

@@ -179,10 +179,10 @@ class BatchedGmres {
     int64_t n_;
     int k_, m_;
     bool flexible_;
-    DeviceArray<T> V_, Z_, W_, R_;
-    DeviceArray<double2> part_, C_, scratch_, gs_;
-    DeviceArray<double> alpha_;
-    PinnedArray<double> down_, up_coef_, up_alpha_;
+    WorkArray<T> V_, Z_, W_, R_;
+    WorkArray<double2> part_, C_, scratch_, gs_;
+    WorkArray<double> alpha_;
+    WorkArray<double, true> down_, up_coef_, up_alpha_;
     double* pinned_ = nullptr;  // download region
 
     T* vec(int i) { return V_.ptr + (size_t)i * n_ * k_; }
@@ -566,7 +566,7 @@ struct InnerGmresPreconditioner : BlockPreconditioner {
     std::vector<int64_t> inner_iterations;
     sbh_context* ctx;
     int64_t n;
-    DeviceArray<float2> V32, Z32;
+    WorkArray<float2> V32, Z32;
     InnerGmresPreconditioner(BlockOperatorT<float2>& op, int64_t nn, int k, int max_inner, double tol)
         : A(op), engine(op.ctx, nn, k, max_inner, false), inner_iterations(k, 0), ctx(op.ctx), n(nn) {
         V32.allocate((size_t)nn * k);

@@ -291,12 +291,12 @@ class BlockGmresEngine {
     int s_;
     const double2* dinv_;
     int max_steps_ = 0, max_basis_ = 0;
-    DeviceArray<double2> V_, W_, Rcm_, Xc_, AX_, Vrm_, Yrm_, gram_, qpart_, dl_dev_;
-    DeviceArray<double> gpart_, npart_, small_;
-    DeviceArray<int> flag_;
-    PinnedArray<double> dl_host_, small_host_;
-    DeviceArray<double2> qg_;     // sj x sj Gram matrix of the block being factored
-    PinnedArray<double> qg_host_;  // its host copy
+    WorkArray<double2> V_, W_, Rcm_, Xc_, AX_, Vrm_, Yrm_, gram_, qpart_, dl_dev_;
+    WorkArray<double> gpart_, npart_, small_;
+    WorkArray<int> flag_;
+    WorkArray<double, true> dl_host_, small_host_;
+    WorkArray<double2> qg_;        // sj x sj Gram matrix of the block being factored
+    WorkArray<double, true> qg_host_;  // its host copy
     HostQrState qrh_;              // outcome of the block QR, whichever way it ran
     int64_t cholqr_blocks_ = 0, chain_blocks_ = 0;
     size_t hacc_off_ = 0, qr_off_ = 0, dl_bytes_ = 0;

@@ -297,13 +297,13 @@ sbh_status run_gcro_dr(sbh_operator* op, sbh_precond* M, const double2* d_b, con
     Krylov K(ctx, op, M, n, std::max(m, kmax));
     admit_device(ctx, (int64_t)sizeof(double2) * ((int64_t)(m + 1 + 2 * kmax + 3) * n),
                  "the GCRO-DR Krylov basis and recycled vectors", false);
-    DeviceArray<double2> V((size_t)(m + 1) * n), w(n), opb(n);
-    DeviceArray<double2> C((size_t)std::max(kmax, 1) * n), Unew((size_t)std::max(kmax, 1) * n);
+    WorkArray<double2> V((size_t)(m + 1) * n), w(n), opb(n);
+    WorkArray<double2> C((size_t)std::max(kmax, 1) * n), Unew((size_t)std::max(kmax, 1) * n);
     if (d_x0)
         SBH_HIP(hipMemcpyAsync(d_x, d_x0, sizeof(double2) * n, hipMemcpyDeviceToDevice, ctx->stream));
     else
         SBH_HIP(hipMemsetAsync(d_x, 0, sizeof(double2) * n, ctx->stream));
-    auto vec = [&](const DeviceArray<double2>& A, int i) { return A.ptr + (size_t)i * n; };
+    auto vec = [&](const WorkArray<double2>& A, int i) { return A.ptr + (size_t)i * n; };
     int64_t total = 0, restarts = 0, reorth = 0, exact_checks = 0;
     auto finish = [&](double res, double est, bool conv, int status) {
         sol->iterations = total;

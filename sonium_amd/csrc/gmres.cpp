@@ -49,7 +49,7 @@ sbh_status run_gmres(sbh_operator* op, sbh_precond* M, const double2* d_b, const
     const int64_t check_every = std::max<int64_t>(1, cfg.convergence_check_interval);
     Krylov K(ctx, op, M, n, alloc_m);
     admit_device(ctx, (int64_t)sizeof(double2) * ((int64_t)(alloc_m + 1) * n + 2 * n), "the GMRES Krylov basis", false);
-    DeviceArray<double2> V((size_t)(alloc_m + 1) * n), w(n), opb(n);
+    WorkArray<double2> V((size_t)(alloc_m + 1) * n), w(n), opb(n);
     // Initial guess.
     if (d_x0)
         SBH_HIP(hipMemcpyAsync(d_x, d_x0, sizeof(double2) * n, hipMemcpyDeviceToDevice, ctx->stream));

@@ -30,8 +30,8 @@ struct Krylov {
     sbh_operator* op;
     sbh_precond* M;
     int64_t n;
-    DeviceArray<double2> part;   // reduction partials
-    DeviceArray<double2> coeff;  // (m+1) coefficients
+    WorkArray<double2> part;   // reduction partials
+    WorkArray<double2> coeff;  // (m+1) coefficients
     double* host = nullptr;      // pinned
     int64_t spmv = 0;
 

@@ -520,16 +520,16 @@ struct sbh_mlp {
     // batch workspace (sized for max_batch samples)
     int max_batch = 0;
     int max_train = 0;  // and the training arrays
-    sbh::DeviceArray<uint16_t> X, XT;
-    std::vector<sbh::DeviceArray<float>> G;     // silu' of the pre-activations per hidden layer
-    std::vector<sbh::DeviceArray<uint16_t>> A, AT;  // activations per hidden layer
-    sbh::DeviceArray<uint16_t> dZ, dZT, dZ2, dZ2T;
-    sbh::DeviceArray<float> part, colsum, Y;  // per layer: weight-gradient and bias-gradient partials
-    sbh::DeviceArray<double> loss_part;
-    sbh::DeviceArray<int64_t> idx;
-    sbh::DeviceArray<float> raw_ws;  // raw inputs of device-side predictions
+    sbh::WorkArray<uint16_t> X, XT;
+    std::vector<sbh::WorkArray<float>> G;     // silu' of the pre-activations per hidden layer
+    std::vector<sbh::WorkArray<uint16_t>> A, AT;  // activations per hidden layer
+    sbh::WorkArray<uint16_t> dZ, dZT, dZ2, dZ2T;
+    sbh::WorkArray<float> part, colsum, Y;  // per layer: weight-gradient and bias-gradient partials
+    sbh::WorkArray<double> loss_part;
+    sbh::WorkArray<int64_t> idx;
+    sbh::WorkArray<float> raw_ws;  // raw inputs of device-side predictions
     // dataset
-    sbh::DeviceArray<float> data_in, data_out;
+    sbh::WorkArray<float> data_in, data_out;
     int64_t data_count = 0;
 };
 
@@ -905,7 +905,7 @@ sbh_status sbh_mlp_loss_and_gradients(sbh_mlp* net, const float* inputs, const f
         SBH_REQUIRE(M > 0 && M % 256 == 0 && M <= (1 << 24), "M must be a positive multiple of 256");
         use_device(net->ctx);
         ensure_batch(net, (int)M, true);
-        DeviceArray<float> din((size_t)M * RAW), dout((size_t)M * 2);
+        WorkArray<float> din((size_t)M * RAW), dout((size_t)M * 2);
         copy_on_stream(net->ctx, din.ptr, inputs, din.bytes(), hipMemcpyHostToDevice);
         copy_on_stream(net->ctx, dout.ptr, targets, dout.bytes(), hipMemcpyHostToDevice);
         UpdateArgs u;
@@ -982,7 +982,7 @@ sbh_status sbh_debug_mlp_predict_layered(sbh_mlp* net, const float* inputs, int6
         use_device(net->ctx);
         const int Mp = (int)((M + 255) / 256 * 256);
         ensure_batch(net, Mp, false);
-        DeviceArray<float> din((size_t)Mp * RAW);
+        WorkArray<float> din((size_t)Mp * RAW);
         SBH_HIP(hipMemsetAsync(din.ptr, 0, din.bytes(), net->ctx->stream));
         SBH_HIP(hipMemcpyAsync(din.ptr, inputs, (size_t)M * RAW * sizeof(float), hipMemcpyHostToDevice,
                                net->ctx->stream));
@@ -999,7 +999,7 @@ sbh_status sbh_mlp_predict(sbh_mlp* net, const float* inputs, int64_t M, float* 
         SBH_REQUIRE(M > 0 && M <= (1 << 24), "M out of range");
         use_device(net->ctx);
         const int Mp = (int)((M + 255) / 256 * 256);
-        DeviceArray<float> din((size_t)Mp * RAW);
+        WorkArray<float> din((size_t)Mp * RAW);
         SBH_HIP(hipMemsetAsync(din.ptr, 0, din.bytes(), net->ctx->stream));
         SBH_HIP(hipMemcpyAsync(din.ptr, inputs, (size_t)M * RAW * sizeof(float),
                                memory == SBH_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,

@@ -2508,7 +2508,7 @@ void launch_field(sbh_context* ctx, const sbh_mesh* m, const sbh_physics& ph, co
     if (npts == 0) return;
     const double k = ph.wave_number, hf = ph.harmonic_factor, pf = ph.pressure_factor;
     const double2* p = sol;
-    DeviceArray<double2> pe, ve;
+    WorkArray<double2> pe, ve;
     if (!v && m->general) {
         pe.allocate((size_t)n);
         ve.allocate((size_t)n);
@@ -2524,7 +2524,7 @@ void launch_field(sbh_context* ctx, const sbh_mesh* m, const sbh_physics& ph, co
     const int64_t chunks = (n + 255) / 256;
     const int64_t slices = std::max<int64_t>(1, std::min<int64_t>({chunks, 2048 / row_blocks, 65535}));
     const int64_t per_slice = (chunks + slices - 1) / slices * 256;
-    DeviceArray<double2> part((size_t)(slices * npts));
+    WorkArray<double2> part((size_t)(slices * npts));
     const dim3 grid((unsigned)row_blocks, (unsigned)slices);
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_FIELD, &ev);
