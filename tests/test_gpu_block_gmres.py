@@ -207,3 +207,33 @@ def test_block_product_tiles_and_slices(ctx, n_theta, n_phi, k):
     x.upload(X)
     op.apply_block_noalloc(x, y, k)
     assert np.array_equal(y.download().reshape(n, k), Y)
+
+
+@pytest.mark.parametrize("n_theta,n_phi", [(5, 3), (5, 17), (9, 40), (21, 61)])
+@pytest.mark.parametrize("s", [1, 2, 8, 9, 17, 24, 25, 33, 49, 64])
+def test_block_gmres_tiles(ctx, n_theta, n_phi, s):
+    """Every tile width of the block products and of the Cholesky QR (16 and 32
+    basis vectors, 16 to 128 real columns, ragged) on 24 to 2440 rows, with
+    blocks as wide as the space itself, against the oracle's steps.  The reported
+    residuals are those of the returned solution to 1e-6, and to 1e-13 where
+    rounding of A x is all that is left of them; an error of a solution is at
+    most cond(A) times its residual."""
+    from sonium_amd.mesh import fibonacci_sphere
+
+    m = fibonacci_sphere(1.0, n_theta, n_phi)
+    n = m.num_elements
+    system = sa.build_tbem_system(ctx, sa.TbemMesh(ctx, m), sa.PhysicsParams.from_wavenumber(1.0))
+    op = sa.DenseMatrixOperator(system)
+    rng = np.random.default_rng(n + s)
+    B = rng.standard_normal((n, s)) + 1j * rng.standard_normal((n, s))
+    A = system.matrix
+    sol = sa.block_gmres(op, B, sa.BlockGmresConfig(max_iterations=20, restart=30, tolerance=1e-8))
+    ref, st = oracle.block_gmres(A, B, restart=30, max_iterations=20, tol=1e-8)
+    assert sol.converged and st["converged"]
+    assert abs(sol.iterations - st["iterations"]) <= 1
+    norm = np.linalg.norm(B, axis=0)
+    residual = np.linalg.norm(B - A @ sol.x, axis=0) / norm
+    np.testing.assert_allclose(sol.true_residuals, residual, rtol=1e-6, atol=1e-13)
+    smallest = np.linalg.svd(A, compute_uv=False)[-1]
+    exact = np.linalg.solve(A, B)
+    assert np.all(np.linalg.norm(sol.x - exact, axis=0) <= 1.01 * (residual + 1e-13) * norm / smallest)
