@@ -38,12 +38,10 @@ int64_t batched_scratch_elems(int64_t n, int k, int max_vec);
 // Block vectors of complex FP64 (double2) or FP32 (float2) entries; the
 // reductions return FP64 values for both.
 #define SBH_DECLARE_VECTOR_OPS(T)                                                                                 \
-    void lowp_gemm(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format, const double* row_inv, \
-                   const T* X, int k, uint16_t* XT, unsigned* colmax, double* col_inv, float* Ypart, T* Y);       \
     void bdots(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const T* W, int64_t n, int k,                 \
-               double2* scratch, double2* out);                                                                   \
+               double2* scratch, double2* out, double2* host);                                                    \
     void bproject(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const double2* C, T* W, int64_t n, int k,   \
-                  double* scratch, double* out);                                                                  \
+                  double* scratch, double* out, double* host, uint64_t live, double* alpha);                      \
     void bresidual(sbh_context* ctx, const T* B, T* R, int64_t n, int k, double* scratch, double* out);           \
     void bupdate(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const double2* Yc, T* X, int64_t n, int k); \
     void bscale(sbh_context* ctx, const T* X, const double* alpha, T* Y, int64_t n, int k);                       \
@@ -51,6 +49,10 @@ int64_t batched_scratch_elems(int64_t n, int k, int max_vec);
 SBH_DECLARE_VECTOR_OPS(double2)
 SBH_DECLARE_VECTOR_OPS(float2)
 #undef SBH_DECLARE_VECTOR_OPS
+void lowp_operand(sbh_context* ctx, int64_t ld, int64_t n, int format, const float2* X, int k, uint16_t* XT,
+                  unsigned* colmax, double* col_inv);
+void lowp_multiply(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format, const double* row_inv, int k,
+                   const uint16_t* XT, const double* col_inv, float* Ypart, float2* Y);
 void convert_block(sbh_context* ctx, const double2* X, float2* Y, int64_t count);
 void convert_block(sbh_context* ctx, const float2* X, double2* Y, int64_t count);
 
@@ -77,6 +79,12 @@ struct BlockOperatorT {
     int64_t n = 0;
     int64_t applies = 0;
     virtual void apply(const T* X, T* Y, int k) = 0;
+    // The same in two parts: what X alone takes, then the product with it.
+    virtual void prepare(const T* X, int k) {
+        (void)X;
+        (void)k;
+    }
+    virtual void multiply(const T* X, T* Y, int k) { apply(X, Y, k); }
     virtual ~BlockOperatorT() = default;
 };
 using BlockOperator = BlockOperatorT<double2>;
@@ -96,17 +104,23 @@ struct DenseBlockOperator : BlockOperator {
     }
 };
 
-template <typename T>
-struct LowpBlockOperator : BlockOperatorT<T> {
+struct LowpBlockOperator : BlockOperatorT<float2> {
     sbh_lowp_matrix* lp;
     explicit LowpBlockOperator(sbh_lowp_matrix* m) : lp(m) {
-        this->ctx = m->ctx;
-        this->n = m->n;
+        ctx = m->ctx;
+        n = m->n;
     }
-    void apply(const T* X, T* Y, int k) override {
-        lowp_gemm(this->ctx, lp->d_A.ptr, lp->ld, this->n, lp->format, lp->d_row_inv.ptr, X, k, lp->d_XT.ptr,
-                  lp->d_colmax.ptr, lp->d_colinv.ptr, lp->d_ypart.ptr, Y);
-        this->applies += 1;
+    void apply(const float2* X, float2* Y, int k) override {
+        prepare(X, k);
+        multiply(X, Y, k);
+    }
+    void prepare(const float2* X, int k) override {
+        lowp_operand(ctx, lp->ld, n, lp->format, X, k, lp->d_XT.ptr, lp->d_colmax.ptr, lp->d_colinv.ptr);
+    }
+    void multiply(const float2*, float2* Y, int k) override {
+        lowp_multiply(ctx, lp->d_A.ptr, lp->ld, n, lp->format, lp->d_row_inv.ptr, k, lp->d_XT.ptr, lp->d_colinv.ptr,
+                      lp->d_ypart.ptr, Y);
+        applies += 1;
     }
 };
 
@@ -131,7 +145,10 @@ struct BatchedParams {
     // Unconditional two-pass classical Gram-Schmidt whose coefficients go from
     // the dot products straight into the projection on the device, as the
     // reference's inner solve does (gmres_inner, gmres_ir.rs:360-394: h = d1 + d2,
-    // then the norm after the second pass); one host read per Arnoldi step.
+    // then the norm after the second pass).  The device scales the next vector
+    // and prepares its product before the host has read the step: the read and
+    // the rotations of 64 columns leave the device idle for 60 us a step
+    // otherwise, a sixth of it at 10240 rows.
     // Otherwise: one pass plus the DGKS pass when ||w|| < 0.707 ||w0|| (gmres_core).
     bool cgs2 = false;
 };
@@ -169,7 +186,13 @@ class BatchedGmres {
         up_coef_.allocate((size_t)(m + 1) * k * 2 + 16);
         up_alpha_.allocate((size_t)k + 16);
         pinned_ = down_.ptr;
+        SBH_HIP(hipEventCreateWithFlags(&step_done_, hipEventDisableTiming));
     }
+    ~BatchedGmres() {
+        if (step_done_) (void)hipEventDestroy(step_done_);
+    }
+    BatchedGmres(const BatchedGmres&) = delete;
+    BatchedGmres& operator=(const BatchedGmres&) = delete;
 
     void run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, const T* B, T* X, const BatchedParams& p,
              std::vector<ColumnResult>& out);
@@ -184,6 +207,7 @@ class BatchedGmres {
     WorkArray<double> alpha_;
     WorkArray<double, true> down_, up_coef_, up_alpha_;
     double* pinned_ = nullptr;  // download region
+    hipEvent_t step_done_ = nullptr;
 
     T* vec(int i) { return V_.ptr + (size_t)i * n_ * k_; }
     T* zvec(int i) { return Z_.ptr + (size_t)i * n_ * k_; }
@@ -215,7 +239,7 @@ class BatchedGmres {
     }
     // coefficients <v_i, w> for i < nvec (per column) and ||w||
     void dots(int nvec, const T* Wd, std::vector<std::vector<cplx>>& coef, std::vector<double>& wn) {
-        bdots(ctx_, V_.ptr, n_ * k_, nvec, Wd, n_, k_, scratch_.ptr, part_.ptr);
+        bdots(ctx_, V_.ptr, n_ * k_, nvec, Wd, n_, k_, scratch_.ptr, part_.ptr, nullptr);
         fetch(part_.ptr, (size_t)(nvec + 1) * k_ * 2);
         coef.assign(k_, std::vector<cplx>(nvec));
         wn.assign(k_, 0.0);
@@ -260,7 +284,8 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
     };
     // invalid_gmres_input (gmres.rs:252-275)
     std::vector<double> bn = norms(B);
-    std::vector<double> xn = norms(X);
+    std::vector<double> xn(k, 0.0);
+    if (!p.x_zero) xn = norms(X);
     const bool bad_cfg = p.max_iterations <= 0 || p.restart <= 0 || !std::isfinite(p.tol) || p.tol <= 0.0;
     std::vector<double> true_b(k), pb(k);
     for (int c = 0; c < k; ++c) {
@@ -287,13 +312,14 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
     auto refresh_residual = [&]() {
         if (r_version == x_version) return;
         if (x_version == 0 && p.x_zero) {
-            zero_fill(ctx_, R_.ptr, n_ * k_);
+            SBH_HIP(hipMemcpyAsync(R_.ptr, B, sizeof(T) * n_ * k_, hipMemcpyDeviceToDevice, ctx_->stream));
             std::fill(ax_abs.begin(), ax_abs.end(), 0.0);
+            r_abs = bn;
         } else {
             A.apply(X, R_.ptr, k);
             if (p.finalize) ax_abs = norms(R_.ptr);
+            r_abs = residual_norms(B, R_.ptr);
         }
-        r_abs = residual_norms(B, R_.ptr);
         r_version = x_version;
     };
 
@@ -360,6 +386,7 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
         if (!anycyc) continue;
         upload_alpha(alpha);
         bscale(ctx_, R_.ptr, alpha_.ptr, vec(0), n_, k);
+        if (p.cgs2) A.prepare(vec(0), k);
         std::vector<char> end_of_cycle(k, 0);
         for (int j = 0; j < m; ++j) {
             bool live = false;
@@ -372,7 +399,10 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
                 M->apply(vec(j), zvec(j), k);
                 zj = zvec(j);
             }
-            A.apply(zj, W_.ptr, k);
+            if (p.cgs2)
+                A.multiply(zj, W_.ptr, k);
+            else
+                A.apply(zj, W_.ptr, k);
             if (p.cgs2) {
                 // pass 1 and pass 2 of CGS2 with device-side coefficients; a column that has
                 // stopped has zero vectors from here on, so projecting it changes nothing
@@ -381,11 +411,20 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
                 double2* d2 = gs_.ptr + region;
                 double* nrm = reinterpret_cast<double*>(gs_.ptr + 2 * region);
                 double* scratch = reinterpret_cast<double*>(scratch_.ptr);
-                bdots(ctx_, V_.ptr, n_ * k_, j + 1, W_.ptr, n_, k, scratch_.ptr, d1);
-                bproject(ctx_, V_.ptr, n_ * k_, j + 1, d1, W_.ptr, n_, k, scratch, nullptr);
-                bdots(ctx_, V_.ptr, n_ * k_, j + 1, W_.ptr, n_, k, scratch_.ptr, d2);
-                bproject(ctx_, V_.ptr, n_ * k_, j + 1, d2, W_.ptr, n_, k, scratch, nrm);
-                fetch(gs_.ptr, 2 * region * 2 + k);
+                double2* h1_out = reinterpret_cast<double2*>(pinned_);
+                uint64_t live_columns = 0;
+                for (int c = 0; c < k; ++c) live_columns |= (uint64_t)(cycling[c] ? 1 : 0) << c;
+                bdots(ctx_, V_.ptr, n_ * k_, j + 1, W_.ptr, n_, k, scratch_.ptr, d1, h1_out);
+                bproject(ctx_, V_.ptr, n_ * k_, j + 1, d1, W_.ptr, n_, k, scratch, nullptr, nullptr, 0, nullptr);
+                bdots(ctx_, V_.ptr, n_ * k_, j + 1, W_.ptr, n_, k, scratch_.ptr, d2, h1_out + region);
+                bproject(ctx_, V_.ptr, n_ * k_, j + 1, d2, W_.ptr, n_, k, scratch, nrm, pinned_ + 4 * region,
+                         live_columns, alpha_.ptr);
+                SBH_HIP(hipEventRecord(step_done_, ctx_->stream));
+                if (j + 1 < m) {
+                    bscale(ctx_, W_.ptr, alpha_.ptr, vec(j + 1), n_, k);
+                    A.prepare(vec(j + 1), k);
+                }
+                SBH_HIP(hipEventSynchronize(step_done_));
                 const double* h1 = pinned_;
                 const double* h2 = pinned_ + 2 * region;
                 const double* hn = pinned_ + 4 * region;
@@ -405,7 +444,7 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
                     for (int i = 0; i <= j; ++i) h(c, i, j) = coef[c][i];
             upload_coeffs(coef, j + 1, cycling);
             bproject(ctx_, V_.ptr, n_ * k_, j + 1, C_.ptr, W_.ptr, n_, k, reinterpret_cast<double*>(scratch_.ptr),
-                     reinterpret_cast<double*>(part_.ptr));
+                     reinterpret_cast<double*>(part_.ptr), nullptr, 0, nullptr);
             column_sums(wn);
             for (auto& v : wn) v = std::sqrt(v);
             std::vector<char> reo(k, 0);
@@ -425,7 +464,7 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
                     }
                 upload_coeffs(re, j + 1, reo);
                 bproject(ctx_, V_.ptr, n_ * k_, j + 1, C_.ptr, W_.ptr, n_, k, reinterpret_cast<double*>(scratch_.ptr),
-                         reinterpret_cast<double*>(part_.ptr));
+                         reinterpret_cast<double*>(part_.ptr), nullptr, 0, nullptr);
                 column_sums(wn2);
                 for (int c = 0; c < k; ++c)
                     if (reo[c]) wn[c] = std::sqrt(wn2[c]);
@@ -440,8 +479,10 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
                 else
                     alpha[c] = 1.0 / wn[c];
             }
-            upload_alpha(alpha);
-            bscale(ctx_, W_.ptr, alpha_.ptr, vec(j + 1), n_, k);
+            if (!p.cgs2) {
+                upload_alpha(alpha);
+                bscale(ctx_, W_.ptr, alpha_.ptr, vec(j + 1), n_, k);
+            }
             std::vector<char> fin(k, 0), conv(k, 0);
             std::vector<double> rrel(k, 0.0);
             bool anyfin = false;
@@ -620,7 +661,7 @@ sbh_status run_gmres_block(sbh_operator* op, const double2* d_B, double2* d_X, i
 sbh_status run_gmres_ir(sbh_operator* op, sbh_lowp_matrix* lp, const double2* d_B, double2* d_X, int k,
                         const sbh_gmres_ir_config& cfg, sbh_gmres_ir_status* st) {
     DenseBlockOperator A(op->sys);
-    LowpBlockOperator<float2> Alp(lp);
+    LowpBlockOperator Alp(lp);
     const int64_t n = op->sys->n;
     const int max_outer = (int)std::max<int64_t>(1, cfg.max_outer_iterations);
     const int restart = (int)std::max<int64_t>(1, cfg.restart_size > 0 ? std::min<int64_t>(cfg.restart_size, max_outer)

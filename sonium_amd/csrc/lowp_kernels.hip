@@ -543,77 +543,69 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 b) {
 // flight (one per row it owns) instead of one dependent load at a time.
 constexpr int BT = 8;
 
-
 // out[(chunk * (nvec + 1) + vec) * k + c] = sum conj(V_vec[:,c]) W[:,c]; vec == nvec -> ||W[:,c]||^2.
-// Block (chunk, group) takes vectors group*BV .. group*BV + BV - 1 for its rows
+// Block (chunk, group) takes vectors group*NV .. group*NV + NV - 1 for its rows
 // together: per row pass it issues the loads of all of them, keeps one
-// partial per vector in registers, and reduces the BV partials in one tree.
-// Its W values stay in registers when the chunk is one pass (S * BT rows),
-// which is the usual case.  Per vector a thread adds its rows in row order.
-constexpr int BV = 8;
-template <typename T>
+// partial per vector in registers, and reduces the NV partials in one tree.
+// Per vector a thread adds its rows in row order.  The bytes of V bound it;
+// what it needs is enough of them in flight, so the vectors are spread over
+// workgroups (NV down to 1) before the rows are: the chunks of one row range
+// run on one XCD, whose L2 then serves W, and 64 chunks keep the sums to one
+// pass.  Chunks of 32 rows with 8 vectors each, 320 to 640 workgroups and two
+// sums after them, took 20.5 + 9 us at 10240 rows, 64 columns and 8 vectors on
+// average (42 MB); now 10.5 + 5.
+template <typename T, int NV>
 __global__ __launch_bounds__(BLOCK) void bdots_kernel(const T* __restrict__ V, int64_t ldv, int nvec,
                                                       const T* __restrict__ W, int64_t n, int k,
                                                       int64_t chunk_len, double2* __restrict__ out) {
-    __shared__ double2 sh[BV * BLOCK];
+    __shared__ double2 sh[NV * BLOCK];
     const int S = BLOCK / k;
     const int c = threadIdx.x % k;
     const int sub = threadIdx.x / k;
     const int64_t b = (int64_t)blockIdx.x * chunk_len;
     const int64_t e = min(n, b + chunk_len);
-    const bool one_pass = e - b <= (int64_t)S * BT;
-    const int vec0 = (int)blockIdx.y * BV;
-    const int nv = min(nvec + 1, vec0 + BV) - vec0;
-    double2 w[BT];
-    if (one_pass && sub < S) {
+    const int vec0 = (int)blockIdx.y * NV;
+    const int nv = min(nvec + 1, vec0 + NV) - vec0;
+    double2 s[NV];
 #pragma unroll
-        for (int t = 0; t < BT; ++t) {
-            const int64_t r = b + sub + (int64_t)S * t;
-            w[t] = r < e ? ld2(W[r * k + c]) : make_double2(0.0, 0.0);
-        }
-    }
-    double2 s[BV];
-#pragma unroll
-    for (int v = 0; v < BV; ++v) s[v] = make_double2(0.0, 0.0);
+    for (int v = 0; v < NV; ++v) s[v] = make_double2(0.0, 0.0);
     if (sub < S) {
         for (int64_t g = b + sub; g < e; g += (int64_t)S * BT) {
-            if (!one_pass) {
+            // rows past the end repeat the last one and are left out of the sums
+            int64_t at[BT];
+            bool in[BT];
+            double2 w[BT];
 #pragma unroll
-                for (int t = 0; t < BT; ++t) {
-                    const int64_t r = g + (int64_t)S * t;
-                    w[t] = r < e ? ld2(W[r * k + c]) : make_double2(0.0, 0.0);
-                }
+            for (int t = 0; t < BT; ++t) {
+                const int64_t r = g + (int64_t)S * t;
+                in[t] = r < e;
+                at[t] = min(r, e - 1) * k + c;
+                w[t] = ld2(W[at[t]]);
             }
 #pragma unroll
-            for (int v = 0; v < BV; ++v) {
+            for (int v = 0; v < NV; ++v) {
                 if (v >= nv) break;
                 const int vec = vec0 + v;
                 if (vec < nvec) {
                     const T* __restrict__ vp = V + (int64_t)vec * ldv;
                     double2 x[BT];
 #pragma unroll
-                    for (int t = 0; t < BT; ++t) {
-                        const int64_t r = g + (int64_t)S * t;
-                        x[t] = r < e ? ld2(vp[r * k + c]) : make_double2(0.0, 0.0);
-                    }
+                    for (int t = 0; t < BT; ++t) x[t] = ld2(vp[at[t]]);
 #pragma unroll
                     for (int t = 0; t < BT; ++t) {
-                        if (g + (int64_t)S * t < e) {
-                            const double2 p = cmulc(x[t], w[t]);
-                            s[v].x += p.x;
-                            s[v].y += p.y;
-                        }
+                        const double2 p = cmulc(x[t], w[t]);
+                        s[v].x += in[t] ? p.x : 0.0;
+                        s[v].y += in[t] ? p.y : 0.0;
                     }
                 } else {
 #pragma unroll
-                    for (int t = 0; t < BT; ++t)
-                        if (g + (int64_t)S * t < e) s[v].x += w[t].x * w[t].x + w[t].y * w[t].y;
+                    for (int t = 0; t < BT; ++t) s[v].x += in[t] ? w[t].x * w[t].x + w[t].y * w[t].y : 0.0;
                 }
             }
         }
     }
 #pragma unroll
-    for (int v = 0; v < BV; ++v)
+    for (int v = 0; v < NV; ++v)
         if (v < nv) sh[v * BLOCK + threadIdx.x] = s[v];
     column_tree_multi(sh, S, k, sub, c, nv);
     if (threadIdx.x < k)
@@ -623,9 +615,10 @@ __global__ __launch_bounds__(BLOCK) void bdots_kernel(const T* __restrict__ V, i
 
 // W[:,c] -= sum_i C[i*k+c] V_i[:,c]; norm partials per column into out[chunk*k + c].
 // Per element the sum over i runs in order before the subtraction.  A thread
-// owns R rows per pass and unrolls the vector loop by U: R = 8, U = 1 for wide
-// blocks; R = 2, U = 4 for short chunks (at most 2 rows per thread), where the
-// loads of four vectors are in flight together.  Both give the same sums.
+// owns R rows per pass and unrolls the vector loop by U, so that R U loads are in
+// flight: <4, 4> where that leaves 512 workgroups, else <2, 4> or <1, 8>.  All
+// give the same sums.  10240 rows, 64 columns and 8 vectors on average (52 MB):
+// 21.5 us with 8 rows and one vector at a time, 320 workgroups, now 10.3.
 template <typename T, int R, int U>
 __global__ __launch_bounds__(BLOCK) void bproject_kernel(const T* __restrict__ V, int64_t ldv, int nvec,
                                                          const double2* __restrict__ C, T* __restrict__ W,
@@ -649,10 +642,7 @@ __global__ __launch_bounds__(BLOCK) void bproject_kernel(const T* __restrict__ V
                 const T* __restrict__ v = V + (int64_t)i * ldv;
                 double2 x[R];
 #pragma unroll
-                for (int t = 0; t < R; ++t) {
-                    const int64_t r = g + (int64_t)S * t;
-                    x[t] = r < e ? ld2(v[r * k + c]) : make_double2(0.0, 0.0);
-                }
+                for (int t = 0; t < R; ++t) x[t] = ld2(v[min(g + (int64_t)S * t, e - 1) * k + c]);
 #pragma unroll
                 for (int t = 0; t < R; ++t) {
                     const double2 p = cmul(coef, x[t]);
@@ -709,35 +699,52 @@ __global__ __launch_bounds__(BLOCK) void bresidual_kernel(const T* __restrict__ 
     if (threadIdx.x < k) out[(int64_t)blockIdx.x * k + threadIdx.x] = sh[threadIdx.x];
 }
 
-// Column sums of chunk partials in two coalesced passes with a fixed order:
-// group g of G adds part[q * nout + o] over q = g, g + G, ...; then
-// out[o] = sum over g of the group sums.
-constexpr int BSUM_GROUPS = 64;
+// Chunks of the dot products, and so terms of their sums
+constexpr int BSUM_CHUNKS = 64;
 
-__global__ void bsum_groups_kernel(const double* __restrict__ part, int chunks, int64_t nout,
-                                   double* __restrict__ tmp) {
+// out[o] = sum over the chunks of part[q * nout + o], in chunk order; all loads
+// are issued before the additions.  host (may be null): a second copy, in
+// pinned memory.
+__global__ __launch_bounds__(64) void bsum_kernel(const double* __restrict__ part, int64_t nout, int chunks,
+                                                  double* __restrict__ out, double* __restrict__ host) {
     const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (o >= nout) return;
+    double v[BSUM_CHUNKS];
+#pragma unroll
+    for (int g = 0; g < BSUM_CHUNKS; ++g) v[g] = g < chunks ? part[(int64_t)g * nout + o] : 0.0;
     double s = 0.0;
-#pragma unroll 8
-    for (int q = blockIdx.y; q < chunks; q += BSUM_GROUPS) s += part[(int64_t)q * nout + o];
-    tmp[(int64_t)blockIdx.y * nout + o] = s;
+#pragma unroll
+    for (int g = 0; g < BSUM_CHUNKS; ++g)
+        if (g < chunks) s += v[g];
+    out[o] = s;
+    if (host) host[o] = s;
 }
 
-// out[o] = sum over g < groups (at most BSUM_GROUPS) of tmp[g * nout + o], in
-// g order; all loads are issued before the additions.
-__global__ __launch_bounds__(BLOCK) void bsum_small_kernel(const double* __restrict__ tmp, int64_t nout, int groups,
-                                                          double* __restrict__ out) {
-    const int64_t o = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= nout) return;
-    double v[BSUM_GROUPS];
-#pragma unroll
-    for (int g = 0; g < BSUM_GROUPS; ++g) v[g] = g < groups ? tmp[(int64_t)g * nout + o] : 0.0;
+// out[c] = sum over the chunks of part[q * k + c], one column per workgroup:
+// each thread its chunks in order, then a fixed tree.  alpha (may be null):
+// 1 / sqrt(out[c]) for the columns of `live`, 0 for the others and below the
+// threshold where a column's Krylov space is taken to be exhausted.
+__global__ __launch_bounds__(BLOCK) void bnorm_sum_kernel(const double* __restrict__ part, int chunks, int k,
+                                                          double* __restrict__ out, double* __restrict__ host,
+                                                          uint64_t live, double* __restrict__ alpha) {
+    __shared__ double sh[BLOCK];
+    const int c = blockIdx.x;
     double s = 0.0;
-#pragma unroll
-    for (int g = 0; g < BSUM_GROUPS; ++g)
-        if (g < groups) s += v[g];
-    out[o] = s;
+    for (int q = threadIdx.x; q < chunks; q += BLOCK) s += part[(int64_t)q * k + c];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = BLOCK / 2; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        out[c] = sh[0];
+        if (host) host[c] = sh[0];
+        if (alpha) {
+            const double norm = sqrt(sh[0]);
+            alpha[c] = (live >> c & 1) == 0 || norm < 1e-20 ? 0.0 : 1.0 / norm;
+        }
+    }
 }
 
 // X[:,c] += sum_i Yc[i*k+c] V_i[:,c]
@@ -814,11 +821,11 @@ void lowp_convert(sbh_context* ctx, const double2* A, int64_t lda, int64_t n, in
     SBH_HIP(hipGetLastError());
 }
 
-// Y = A X for k in 1..64 columns (k = 1 on lp_gemv_kernel).  Rows k..32*ntr-1 of XT (left from a wider
-// product or zero) feed only output columns that lp_reduce_kernel discards.
+// X (n x k, k in 1..64) as the operand of the product: its columns scaled and
+// rounded to the format in XT, and the scales in col_inv.
 template <typename T>
-static void lowp_gemm_t(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format, const double* row_inv,
-                        const T* X, int k, uint16_t* XT, unsigned* colmax, double* col_inv, float* Ypart, T* Y) {
+static void lowp_operand_t(sbh_context* ctx, int64_t ld, int64_t n, int format, const T* X, int k, uint16_t* XT,
+                           unsigned* colmax, double* col_inv) {
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, colmax, k, 0u);
     {
         const int64_t rpb = std::max<int64_t>(1, 4096 / k);
@@ -832,6 +839,13 @@ static void lowp_gemm_t(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t
         hipLaunchKernelGGL((x_to_lp_kernel<1, T>), dim3(nblocks(n * k)), dim3(BLOCK), 0, ctx->stream, X, n, k, ld,
                            colmax, XT, col_inv);
     SBH_HIP(hipGetLastError());
+}
+
+// Y = A X from that operand (k = 1 on lp_gemv_kernel).  Rows k..32*ntr-1 of XT (left from a wider
+// product or zero) feed only output columns that lp_reduce_kernel discards.
+template <typename T>
+static void lowp_multiply_t(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format,
+                            const double* row_inv, int k, const uint16_t* XT, const double* col_inv, float* Ypart, T* Y) {
     const int ntr = (k + 31) / 32;  // 32-column tiles of the real part (the imaginary part has as many)
     const int64_t n_tiles = (n + 31) / 32;
     if (k == 1) {
@@ -876,14 +890,20 @@ static void lowp_gemm_t(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t
     ctx->end_timed(SBH_KERNEL_LOWP, ev);
 }
 
-#define SBH_LOWP_PRODUCTS(T)                                                                                         \
-    void lowp_gemm(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format, const double* row_inv,    \
-                   const T* X, int k, uint16_t* XT, unsigned* colmax, double* col_inv, float* Ypart, T* Y) {         \
-        lowp_gemm_t(ctx, A, ld, n, format, row_inv, X, k, XT, colmax, col_inv, Ypart, Y);                            \
-    }
-SBH_LOWP_PRODUCTS(double2)
-SBH_LOWP_PRODUCTS(float2)
-#undef SBH_LOWP_PRODUCTS
+void lowp_gemm(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format, const double* row_inv,
+               const double2* X, int k, uint16_t* XT, unsigned* colmax, double* col_inv, float* Ypart, double2* Y) {
+    lowp_operand_t(ctx, ld, n, format, X, k, XT, colmax, col_inv);
+    lowp_multiply_t(ctx, A, ld, n, format, row_inv, k, XT, col_inv, Ypart, Y);
+}
+// The two parts for FP32 vectors
+void lowp_operand(sbh_context* ctx, int64_t ld, int64_t n, int format, const float2* X, int k, uint16_t* XT,
+                  unsigned* colmax, double* col_inv) {
+    lowp_operand_t(ctx, ld, n, format, X, k, XT, colmax, col_inv);
+}
+void lowp_multiply(sbh_context* ctx, const uint16_t* A, int64_t ld, int64_t n, int format, const double* row_inv, int k,
+                   const uint16_t* XT, const double* col_inv, float* Ypart, float2* Y) {
+    lowp_multiply_t(ctx, A, ld, n, format, row_inv, k, XT, col_inv, Ypart, Y);
+}
 
 // Doubles that the fixed scratch must hold for a shape to be accepted there:
 // ZG_SPLIT slices of the next power of two of 8-column tiles.
@@ -1014,87 +1034,97 @@ void zgemm_f64_noalloc(sbh_context* ctx, const double2* A, int64_t lda, int64_t 
     zgemm_f64_into(ctx, A, lda, n, X, k, Y, ptr);
 }
 
-// Rows per block of the column-batched reductions: one pass of BT rows per
-// thread (S * BT rows, S = BLOCK / k threads per column), at most 4096 blocks.
-static int batched_chunks(int64_t n, int k, int64_t* len) {
-    const int64_t rpb = (int64_t)(BLOCK / k) * BT;
-    int64_t chunks = (n + rpb - 1) / rpb;
-    // few columns: shorter chunks (down to one row per thread) for more
-    // workgroups, up to the count whose sums still take one pass
-    if (chunks < BSUM_GROUPS) chunks = std::min<int64_t>(BSUM_GROUPS, (n + BLOCK / k - 1) / (BLOCK / k));
-    chunks = std::max<int64_t>(1, std::min<int64_t>(chunks, 4096));
+// Workgroups of the reductions over rows that keep R rows per thread (S =
+// BLOCK / k threads per column), at most 4096.
+constexpr int64_t BMAX_CHUNKS = 4096;
+static int row_chunks(int64_t n, int k, int R, int64_t* len) {
+    const int64_t rows = (int64_t)(BLOCK / k) * R;
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((n + rows - 1) / rows, BMAX_CHUNKS));
     *len = (n + chunks - 1) / chunks;
     return (int)chunks;
 }
 
-// out[o] = sum over the chunks of part[q * nout + o]; the group sums go right
-// after the partials in the same scratch buffer.
-static void column_sums(sbh_context* ctx, double* part, int chunks, int64_t nout, double* out) {
-    if (chunks <= BSUM_GROUPS) {
-        // one pass in chunk order: the same sums as the two passes, whose groups then hold one chunk each
-        hipLaunchKernelGGL(bsum_small_kernel, dim3(nblocks(nout)), dim3(BLOCK), 0, ctx->stream, part, nout, chunks,
-                           out);
-        SBH_HIP(hipGetLastError());
-        return;
-    }
-    double* tmp = part + (int64_t)chunks * nout;
-    hipLaunchKernelGGL(bsum_groups_kernel, dim3(nblocks(nout), BSUM_GROUPS), dim3(BLOCK), 0, ctx->stream, part,
-                       chunks, nout, tmp);
-    SBH_HIP(hipGetLastError());
-    hipLaunchKernelGGL(bsum_small_kernel, dim3(nblocks(nout)), dim3(BLOCK), 0, ctx->stream, tmp, nout, BSUM_GROUPS,
-                       out);
-    SBH_HIP(hipGetLastError());
+// Rows per thread of a pass over n rows: as many as leave 512 workgroups, two
+// to a CU, of 4, 2 and 1.
+static int pass_rows(int64_t n, int k) {
+    int64_t len;
+    for (int R = 4; R > 1; R /= 2)
+        if (row_chunks(n, k, R, &len) >= 512) return R;
+    return 1;
 }
 
 // The wrappers below exist for double2 (FP64 vectors) and float2 (FP32
 // vectors); the partial sums and reduced values are FP64 either way.
 
 // Partials land in `scratch` (chunks x (nvec+1) x k complex); the reduced
-// (nvec+1) x k complex values land in `out`.
+// (nvec+1) x k complex values land in `out` and, if given, in pinned `host`.
 template <typename T>
 static void bdots_t(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const T* W, int64_t n, int k,
-                    double2* scratch, double2* out) {
-    int64_t len;
-    const int chunks = batched_chunks(n, k, &len);
-    hipLaunchKernelGGL(bdots_kernel<T>, dim3((unsigned)chunks, (unsigned)((nvec + BV) / BV)), dim3(BLOCK), 0,
-                       ctx->stream, V, ldv, nvec, W, n, k, len, scratch);
+                    double2* scratch, double2* out, double2* host) {
+    const int64_t S = BLOCK / k;
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(BSUM_CHUNKS, (n + S - 1) / S));
+    const int64_t len = (n + chunks - 1) / chunks;
+    int nv = 8;  // vectors per workgroup: as many as leave 512 workgroups
+    while (nv > 1 && chunks * ((nvec + nv) / nv) < 512) nv /= 2;
+    const dim3 grid((unsigned)chunks, (unsigned)((nvec + nv) / nv));
+#define SBH_BD(NV_) \
+    hipLaunchKernelGGL((bdots_kernel<T, NV_>), grid, dim3(BLOCK), 0, ctx->stream, V, ldv, nvec, W, n, k, len, scratch)
+    if (nv == 8) SBH_BD(8);
+    else if (nv == 4) SBH_BD(4);
+    else if (nv == 2) SBH_BD(2);
+    else SBH_BD(1);
+#undef SBH_BD
     SBH_HIP(hipGetLastError());
-    column_sums(ctx, reinterpret_cast<double*>(scratch), chunks, (int64_t)(nvec + 1) * k * 2,
-                reinterpret_cast<double*>(out));
+    const int64_t nout = (int64_t)(nvec + 1) * k * 2;
+    hipLaunchKernelGGL(bsum_kernel, dim3(nblocks(nout, 64)), dim3(64), 0, ctx->stream,
+                       reinterpret_cast<const double*>(scratch), nout, (int)chunks, reinterpret_cast<double*>(out),
+                       reinterpret_cast<double*>(host));
+    SBH_HIP(hipGetLastError());
 }
 
-// W -= sum C_i V_i per column; the reduced k squared norms land in `out`
-// (out == nullptr: no norms wanted, and their sums are not launched).
+// k column sums of chunk partials
+static void bnorm_sums(sbh_context* ctx, const double* part, int chunks, int k, double* out, double* host,
+                       uint64_t live, double* alpha) {
+    hipLaunchKernelGGL(bnorm_sum_kernel, dim3((unsigned)k), dim3(BLOCK), 0, ctx->stream, part, chunks, k, out, host,
+                       live, alpha);
+    SBH_HIP(hipGetLastError());
+}
+
+// W -= sum C_i V_i per column; the reduced k squared norms land in `out` and,
+// if given, in pinned `host`, their reciprocal roots in `alpha` (see
+// bnorm_sum_kernel); out == nullptr: no norms wanted.
 template <typename T>
 static void bproject_t(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const double2* C, T* W, int64_t n, int k,
-                       double* scratch, double* out) {
+                       double* scratch, double* out, double* host, uint64_t live, double* alpha) {
+    const int R = pass_rows(n, k);
     int64_t len;
-    const int chunks = batched_chunks(n, k, &len);
-    if (len <= 2 * (int64_t)(BLOCK / k))
-        hipLaunchKernelGGL((bproject_kernel<T, 2, 4>), dim3((unsigned)chunks), dim3(BLOCK), 0, ctx->stream, V, ldv,
-                           nvec, C, W, n, k, len, scratch);
-    else
-        hipLaunchKernelGGL((bproject_kernel<T, BT, 1>), dim3((unsigned)chunks), dim3(BLOCK), 0, ctx->stream, V, ldv,
-                           nvec, C, W, n, k, len, scratch);
+    const int chunks = row_chunks(n, k, R, &len);
+#define SBH_BP(R_, U_)                                                                                             \
+    hipLaunchKernelGGL((bproject_kernel<T, R_, U_>), dim3((unsigned)chunks), dim3(BLOCK), 0, ctx->stream, V, ldv,  \
+                       nvec, C, W, n, k, len, scratch)
+    if (R == 4) SBH_BP(4, 4);
+    else if (R == 2) SBH_BP(2, 4);
+    else SBH_BP(1, 8);
+#undef SBH_BP
     SBH_HIP(hipGetLastError());
-    if (out) column_sums(ctx, scratch, chunks, (int64_t)k, out);
+    if (out) bnorm_sums(ctx, scratch, chunks, k, out, host, live, alpha);
 }
 
 // R = B - R (B may be null: norms only); the reduced k squared norms land in `out`.
 template <typename T>
 static void bresidual_t(sbh_context* ctx, const T* B, T* R, int64_t n, int k, double* scratch, double* out) {
     int64_t len;
-    const int chunks = batched_chunks(n, k, &len);
+    const int chunks = row_chunks(n, k, pass_rows(n, k), &len);
     hipLaunchKernelGGL(bresidual_kernel<T>, dim3((unsigned)chunks), dim3(BLOCK), 0, ctx->stream, B, R, n, k, len,
                        scratch);
     SBH_HIP(hipGetLastError());
-    column_sums(ctx, scratch, chunks, (int64_t)k, out);
+    bnorm_sums(ctx, scratch, chunks, k, out, nullptr, 0, nullptr);
 }
 
+// Complex elements of the partials of any of them, with up to max_vec vectors
 int64_t batched_scratch_elems(int64_t n, int k, int max_vec) {
     int64_t len;
-    const int chunks = batched_chunks(n, k, &len);
-    return (int64_t)(chunks + BSUM_GROUPS) * (max_vec + 1) * k;  // complex elements: partials + group sums
+    return std::max<int64_t>((int64_t)BSUM_CHUNKS * (max_vec + 1) * k, ((int64_t)row_chunks(n, k, 1, &len) * k + 1) / 2);
 }
 
 template <typename T>
@@ -1119,12 +1149,12 @@ static void zero_fill_t(sbh_context* ctx, T* X, int64_t count) {
 
 #define SBH_VECTOR_OPS(T)                                                                                       \
     void bdots(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const T* W, int64_t n, int k,               \
-               double2* scratch, double2* out) {                                                                \
-        bdots_t(ctx, V, ldv, nvec, W, n, k, scratch, out);                                                      \
+               double2* scratch, double2* out, double2* host) {                                                 \
+        bdots_t(ctx, V, ldv, nvec, W, n, k, scratch, out, host);                                                \
     }                                                                                                           \
     void bproject(sbh_context* ctx, const T* V, int64_t ldv, int nvec, const double2* C, T* W, int64_t n, int k, \
-                  double* scratch, double* out) {                                                               \
-        bproject_t(ctx, V, ldv, nvec, C, W, n, k, scratch, out);                                                \
+                  double* scratch, double* out, double* host, uint64_t live, double* alpha) {                   \
+        bproject_t(ctx, V, ldv, nvec, C, W, n, k, scratch, out, host, live, alpha);                             \
     }                                                                                                           \
     void bresidual(sbh_context* ctx, const T* B, T* R, int64_t n, int k, double* scratch, double* out) {        \
         bresidual_t(ctx, B, R, n, k, scratch, out);                                                             \

@@ -338,3 +338,32 @@ def test_block_gmres_initial_guess_matches_single(c1_block):
     Xe = np.linalg.solve(A, B)
     _, sols = sa.gmres_block(op, B, cfg, X0=Xe)
     assert all(s.converged and s.iterations == 0 for s in sols)
+
+
+@pytest.mark.parametrize("n_theta,n_phi,k", [(5, 3, 1), (5, 3, 24), (5, 17, 64), (9, 40, 3), (21, 61, 13),
+                                             (33, 70, 64), (33, 130, 64), (33, 130, 5)])
+def test_refinement_row_and_vector_splits(ctx, n_theta, n_phi, k):
+    """Every split of the batched dot products and projections over rows and
+    vectors: fewer rows than threads, one, two and four rows per thread, one to
+    eight vectors per workgroup.  The refinement and the block GMRES end at
+    their tolerance, by a residual formed apart from them (rounding of A x: 1e-13
+    of the right-hand side), and repeat their bits."""
+    from sonium_amd.mesh import fibonacci_sphere
+
+    m = fibonacci_sphere(1.0, n_theta, n_phi)
+    n = m.num_elements
+    system = sa.build_tbem_system(ctx, sa.TbemMesh(ctx, m), sa.PhysicsParams.from_wavenumber(1.0))
+    op = sa.DenseMatrixOperator(system)
+    lp = sa.LowpMatrix(system, "fp16")
+    rng = np.random.default_rng(n + k)
+    B = rng.standard_normal((n, k)) + 1j * rng.standard_normal((n, k))
+    norm = np.linalg.norm(B, axis=0)
+    X, st = sa.gmres_ir(op, lp, B, sa.GmresIrConfig(max_outer_iterations=20, outer_tolerance=1e-9,
+                                                    max_inner_iterations=50))
+    residual = np.linalg.norm(B - op.apply_block(X), axis=0) / norm
+    assert all(s.converged for s in st) and residual.max() <= 1e-9 + 1e-13
+    assert np.array_equal(sa.gmres_ir(op, lp, B, sa.GmresIrConfig(max_outer_iterations=20, outer_tolerance=1e-9,
+                                                                  max_inner_iterations=50))[0], X)
+    X, st = sa.gmres_block(op, B, sa.GmresConfig(max_iterations=20, restart=50, tolerance=1e-9))
+    residual = np.linalg.norm(B - op.apply_block(X), axis=0) / norm
+    assert all(s.converged for s in st) and residual.max() <= 1e-9 + 1e-13
