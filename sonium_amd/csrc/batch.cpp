@@ -89,7 +89,7 @@ struct sbh_batch {
     struct Solver {
         int m = 0, MV = 0;
         sbh::DeviceArray<double2> V, W, R, H, cs, sn, g, coef, part;
-        sbh::DeviceArray<double> wn0, wn, est, bnorm, rnorm, scale, tol_abs;
+        sbh::DeviceArray<double> wn0, est, bnorm, rnorm, scale, tol_abs;
         sbh::DeviceArray<int> active, reorth, done, jlen, inst_active, inst_reorth, inst_pending;
         sbh::DeviceArray<int64_t> iters, cycles, reorth_count;
         sbh::DeviceArray<unsigned long long> t_done;
@@ -288,7 +288,7 @@ void ensure_solver(sbh_batch* b, int m) {
     s.g.allocate(C * (m + 1));
     s.coef.allocate(C * s.MV);
     s.part.allocate((size_t)b->nchunks * s.MV * kMaxCol);
-    for (auto* a : {&s.wn0, &s.wn, &s.est, &s.bnorm, &s.rnorm, &s.scale, &s.tol_abs}) a->allocate(C);
+    for (auto* a : {&s.wn0, &s.est, &s.bnorm, &s.rnorm, &s.scale, &s.tol_abs}) a->allocate(C);
     for (auto* a : {&s.active, &s.reorth, &s.done, &s.jlen}) a->allocate(C);
     for (auto* a : {&s.inst_active, &s.inst_reorth, &s.inst_pending}) a->allocate((size_t)b->B);
     for (auto* a : {&s.iters, &s.cycles, &s.reorth_count}) a->allocate(C);
@@ -316,20 +316,16 @@ void cycle(sbh_batch* b, int format, double tol, double inner_tol) {
         ragged_sum_dots(ctx, lay, s.part.ptr, j + 1, j, s.active.ptr, s.reorth.ptr, 0, s.H.ptr, s.coef.ptr,
                         s.wn0.ptr);
         ragged_project(ctx, lay, s.inst_active.ptr, s.V.ptr, j + 1, s.coef.ptr, s.W.ptr, s.part.ptr);
-        ragged_norm(ctx, lay, s.part.ptr, s.active.ptr, s.wn0.ptr, 0, s.wn.ptr, s.reorth.ptr, s.reorth_count.ptr);
-        ragged_flags(ctx, lay, s.active.ptr, s.reorth.ptr, s.done.ptr, s.inst_active.ptr, s.inst_reorth.ptr,
-                     s.inst_pending.ptr);
+        ragged_norm(ctx, lay, s.part.ptr, s.active.ptr, s.wn0.ptr, s.reorth.ptr, s.reorth_count.ptr,
+                    s.inst_reorth.ptr);
         ragged_dots(ctx, lay, s.inst_reorth.ptr, s.V.ptr, j + 1, s.W.ptr, s.part.ptr);
         ragged_sum_dots(ctx, lay, s.part.ptr, j + 1, j, s.active.ptr, s.reorth.ptr, 1, s.H.ptr, s.coef.ptr,
                         s.wn0.ptr);
         ragged_project(ctx, lay, s.inst_reorth.ptr, s.V.ptr, j + 1, s.coef.ptr, s.W.ptr, s.part.ptr);
-        ragged_norm(ctx, lay, s.part.ptr, s.active.ptr, s.wn0.ptr, 1, s.wn.ptr, s.reorth.ptr, s.reorth_count.ptr);
-        ragged_givens(ctx, lay, j, s.active.ptr, s.wn.ptr, s.H.ptr, s.cs.ptr, s.sn.ptr, s.g.ptr, s.tol_abs.ptr,
-                      s.est.ptr, s.jlen.ptr, s.iters.ptr, s.scale.ptr);
+        ragged_step(ctx, lay, s.part.ptr, j, s.active.ptr, s.H.ptr, s.cs.ptr, s.sn.ptr, s.g.ptr, s.tol_abs.ptr,
+                    s.est.ptr, s.jlen.ptr, s.iters.ptr, s.scale.ptr, s.inst_active.ptr);
         if (j + 1 < m)
             ragged_scale(ctx, lay, s.inst_active.ptr, s.scale.ptr, s.W.ptr, Vj(j + 1));
-        ragged_flags(ctx, lay, s.active.ptr, s.reorth.ptr, s.done.ptr, s.inst_active.ptr, s.inst_reorth.ptr,
-                     s.inst_pending.ptr);
     }
     ragged_solve(ctx, lay, s.H.ptr, s.g.ptr, s.jlen.ptr, s.coef.ptr);
     ragged_update(ctx, lay, s.inst_pending.ptr, s.V.ptr, s.jlen.ptr, s.coef.ptr, b->d_x.ptr);

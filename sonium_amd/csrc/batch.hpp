@@ -37,12 +37,12 @@ void ragged_sum_dots(sbh_context* ctx, const RaggedLayout& lay, const double2* p
 void ragged_project(sbh_context* ctx, const RaggedLayout& lay, const int* flag, const double2* V, int nvec,
                     const double2* coef, double2* W, double2* part);
 void ragged_norm(sbh_context* ctx, const RaggedLayout& lay, const double2* part, const int* active, const double* wn0,
-                 int pass, double* wn, int* reorth, int64_t* reorth_count);
+                 int* reorth, int64_t* reorth_count, int* inst_reorth);
 void ragged_flags(sbh_context* ctx, const RaggedLayout& lay, const int* active, const int* reorth, const int* done,
                   int* inst_active, int* inst_reorth, int* inst_pending);
-void ragged_givens(sbh_context* ctx, const RaggedLayout& lay, int j, int* active, const double* wn, double2* H,
-                   double2* cs, double2* sn, double2* g, const double* tol_abs, double* est, int* jlen, int64_t* iters,
-                   double* scale);
+void ragged_step(sbh_context* ctx, const RaggedLayout& lay, const double2* part, int j, int* active, double2* H,
+                 double2* cs, double2* sn, double2* g, const double* tol_abs, double* est, int* jlen, int64_t* iters,
+                 double* scale, int* inst_active);
 void ragged_solve(sbh_context* ctx, const RaggedLayout& lay, const double2* H, const double2* g, const int* jlen,
                   double2* coef);
 void ragged_update(sbh_context* ctx, const RaggedLayout& lay, const int* flag, const double2* V, const int* jlen,

@@ -322,6 +322,7 @@ __global__ void rsum_dots_kernel(int C, const int* __restrict__ col_inst, const 
     if (take) {
         const int2 r = chunk_range[col_inst[c]];
         const int q = col_q[c];
+#pragma unroll 4
         for (int ch = r.x; ch < r.y; ++ch) {
             const double2 p = part[((int64_t)ch * MV + slot) * MAXCOL + q];
             s.x += p.x;
@@ -339,12 +340,21 @@ __global__ void rsum_dots_kernel(int C, const int* __restrict__ col_inst, const 
     }
 }
 
-// W -= sum_{s < nvec} coef[c][s] V_s per column; ||W||^2 partials into slot 0.
+// Workgroups of a chunk in the projection, each with its own partial slot
+inline int project_parts(int MV) { return std::min(4, MV); }
+
+// W -= sum_{s < nvec} coef[c][s] V_s per column; ||W||^2 partials of the
+// chunk's parts (gridDim.y) into slots 0, 1, ...  Per element the sum over
+// vectors runs in order before the subtraction.  The bytes of V bound it; four
+// rows and four vectors of loads are in flight per thread, and a quarter of a
+// chunk goes to a workgroup: 457 000 rows times columns and 16 vectors on
+// average (132 MB) took 32 us in 112 workgroups, now 20.
 __global__ __launch_bounds__(BLOCK) void rproject_kernel(const VecChunk* __restrict__ chunks,
                                                          const BatchInstance* __restrict__ inst,
                                                          const int* __restrict__ flag, const double2* __restrict__ V,
                                                          int64_t L, int nvec, const double2* __restrict__ coef, int MV,
                                                          double2* __restrict__ W, double2* __restrict__ part) {
+    constexpr int R = 4;
     __shared__ double sh[BLOCK];
     const VecChunk ch = chunks[blockIdx.x];
     if (!flag[ch.inst]) return;
@@ -353,41 +363,43 @@ __global__ __launch_bounds__(BLOCK) void rproject_kernel(const VecChunk* __restr
     const int S = BLOCK / kb;
     const int c = threadIdx.x % kb;
     const int sub = threadIdx.x / kb;
+    const int share = (ch.rows + (int)gridDim.y - 1) / (int)gridDim.y;
+    const int rbeg = (int)blockIdx.y * share;
+    const int rend = min(ch.rows, rbeg + share);
     const int64_t base = I.vec_off + ch.r0 * kb + c;
     const double2* cf = coef + (int64_t)(I.col_off + c) * MV;
     double nr = 0.0;
     if (sub < S) {
-        // RB rows per pass: per vector their RB loads are issued together; per
-        // element the sum over vectors runs in order before the subtraction
-        for (int r0 = sub; r0 < ch.rows; r0 += S * RB) {
-            double sr[RB], si[RB];
+        for (int r0 = rbeg + sub; r0 < rend; r0 += S * R) {
+            // rows past the end repeat the last one and are not stored
+            int64_t at[R];
+            double sr[R], si[R];
 #pragma unroll
-            for (int t = 0; t < RB; ++t) sr[t] = si[t] = 0.0;
+            for (int t = 0; t < R; ++t) {
+                at[t] = base + (int64_t)min(r0 + S * t, rend - 1) * kb;
+                sr[t] = si[t] = 0.0;
+            }
+#pragma unroll 4
             for (int s = 0; s < nvec; ++s) {
                 const double2 cs = cf[s];
                 const double2* v = V + (int64_t)s * L;
-                double2 x[RB];
+                double2 x[R];
 #pragma unroll
-                for (int t = 0; t < RB; ++t) {
-                    const int r = r0 + S * t;
-                    x[t] = r < ch.rows ? v[base + (int64_t)r * kb] : make_double2(0.0, 0.0);
-                }
+                for (int t = 0; t < R; ++t) x[t] = v[at[t]];
 #pragma unroll
-                for (int t = 0; t < RB; ++t) {
+                for (int t = 0; t < R; ++t) {
                     const double2 p = cmul(cs, x[t]);
                     sr[t] += p.x;
                     si[t] += p.y;
                 }
             }
 #pragma unroll
-            for (int t = 0; t < RB; ++t) {
-                const int r = r0 + S * t;
-                if (r < ch.rows) {
-                    const int64_t idx = base + (int64_t)r * kb;
-                    double2 w = W[idx];
+            for (int t = 0; t < R; ++t) {
+                if (r0 + S * t < rend) {
+                    double2 w = W[at[t]];
                     w.x -= sr[t];
                     w.y -= si[t];
-                    W[idx] = w;
+                    W[at[t]] = w;
                     nr += w.x * w.x + w.y * w.y;
                 }
             }
@@ -395,33 +407,48 @@ __global__ __launch_bounds__(BLOCK) void rproject_kernel(const VecChunk* __restr
     }
     sh[threadIdx.x] = nr;
     column_tree(sh, S, kb, sub, c);
-    if (threadIdx.x < kb) part[((int64_t)blockIdx.x * MV) * MAXCOL + threadIdx.x] = make_double2(sh[threadIdx.x], 0.0);
+    if (threadIdx.x < kb)
+        part[((int64_t)blockIdx.x * MV + blockIdx.y) * MAXCOL + threadIdx.x] = make_double2(sh[threadIdx.x], 0.0);
 }
 
-// ||W|| per column from slot 0 of the partials; pass 0 also flags the
-// columns whose norm dropped below 0.707 of the norm before projection
-// (the reorthogonalisation test of the single-system GMRES).
-__global__ void rnorm_kernel(int C, const int* __restrict__ col_inst, const int* __restrict__ col_q,
-                             const int2* __restrict__ chunk_range, const double2* __restrict__ part, int MV,
-                             const int* __restrict__ active, const double* __restrict__ wn0, int pass,
-                             double* __restrict__ wn, int* __restrict__ reorth, int64_t* __restrict__ reorth_count) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    if (!active[c]) {
-        if (pass == 0) reorth[c] = 0;
-        return;
-    }
-    const int2 r = chunk_range[col_inst[c]];
-    const int q = col_q[c];
+// ||W|| of a column from the projection's partials, in chunk and part order
+__device__ double projected_norm(const int2 range, int parts, int MV, int q, const double2* __restrict__ part) {
     double s = 0.0;
-    for (int ch = r.x; ch < r.y; ++ch) s += part[((int64_t)ch * MV) * MAXCOL + q].x;
-    const double v = sqrt(s);
-    wn[c] = v;
-    if (pass == 0) {
-        const int f = v < 0.707 * wn0[c] ? 1 : 0;
+    for (int ch = range.x; ch < range.y; ++ch) {
+        double v[4];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) v[p] = part[((int64_t)ch * MV + min(p, parts - 1)) * MAXCOL + q].x;
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+            if (p < parts) s += v[p];
+    }
+    return sqrt(s);
+}
+
+// After the first projection, one workgroup per instance: ||W|| per column,
+// the columns whose norm dropped below 0.707 of the norm before it (the
+// reorthogonalisation test of the single-system GMRES), and whether the
+// instance has any.  The kernels between the products cost their launches:
+// with the norms, flags and rotations of a step in two instead of five, 24 us
+// a step became 14.
+__global__ __launch_bounds__(64) void rnorm_kernel(const BatchInstance* __restrict__ inst,
+                                                   const int2* __restrict__ chunk_range,
+                                                   const double2* __restrict__ part, int parts, int MV,
+                                                   const int* __restrict__ active, const double* __restrict__ wn0,
+                                                   int* __restrict__ reorth, int64_t* __restrict__ reorth_count,
+                                                   int* __restrict__ inst_reorth) {
+    const int b = blockIdx.x;
+    const BatchInstance& I = inst[b];
+    const int q = threadIdx.x;
+    int f = 0;
+    if (q < I.ncol) {
+        const int c = I.col_off + q;
+        if (active[c]) f = projected_norm(chunk_range[b], parts, MV, q, part) < 0.707 * wn0[c] ? 1 : 0;
         reorth[c] = f;
         reorth_count[c] += f;
     }
+    const bool any = __ballot(f) != 0;
+    if (q == 0) inst_reorth[b] = any ? 1 : 0;
 }
 
 // Instance flags: any column active / flagged / not yet converged.
@@ -448,21 +475,14 @@ __global__ void rflags_kernel(int B, const BatchInstance* __restrict__ inst, con
 // estimate.  A column freezes (jlen = j + 1) when the estimate drops below
 // its threshold, when ||w|| < 1e-20 (happy breakdown) or at the end of the
 // cycle.  scale = 1/||w|| for the next basis vector (0 once frozen).
-__global__ void rgivens_kernel(int C, int j, int m, int* __restrict__ active, const double* __restrict__ wn,
-                               double2* __restrict__ H, double2* __restrict__ cs, double2* __restrict__ sn,
-                               double2* __restrict__ g, const double* __restrict__ tol_abs, double* __restrict__ est,
-                               int* __restrict__ jlen, int64_t* __restrict__ iters, double* __restrict__ scale) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
-    if (!active[c]) {
-        scale[c] = 0.0;
-        return;
-    }
+__device__ void rotate_column(int c, int j, int m, double w, int* __restrict__ active, double2* __restrict__ H,
+                              double2* __restrict__ cs, double2* __restrict__ sn, double2* __restrict__ g,
+                              const double* __restrict__ tol_abs, double* __restrict__ est, int* __restrict__ jlen,
+                              int64_t* __restrict__ iters, double* __restrict__ scale) {
     double2* h = H + ((int64_t)c * m + j) * (m + 1);
     double2* C_ = cs + (int64_t)c * m;
     double2* S_ = sn + (int64_t)c * m;
     double2* gc = g + (int64_t)c * (m + 1);
-    const double w = wn[c];
     h[j + 1] = make_double2(w, 0.0);
     const bool breakdown = w < 1e-20;
     for (int i = 0; i < j; ++i) {
@@ -501,6 +521,36 @@ __global__ void rgivens_kernel(int C, int j, int m, int* __restrict__ active, co
     } else {
         scale[c] = 1.0 / w;
     }
+}
+
+// After the second projection, one workgroup per instance: ||W|| (the first
+// projection's where the second was not needed), the recurrence of each active
+// column, and whether the instance still has any.
+__global__ __launch_bounds__(64) void rstep_kernel(const BatchInstance* __restrict__ inst,
+                                                   const int2* __restrict__ chunk_range,
+                                                   const double2* __restrict__ part, int parts, int MV, int j, int m,
+                                                   int* __restrict__ active, double2* __restrict__ H,
+                                                   double2* __restrict__ cs, double2* __restrict__ sn,
+                                                   double2* __restrict__ g, const double* __restrict__ tol_abs,
+                                                   double* __restrict__ est, int* __restrict__ jlen,
+                                                   int64_t* __restrict__ iters, double* __restrict__ scale,
+                                                   int* __restrict__ inst_active) {
+    const int b = blockIdx.x;
+    const BatchInstance& I = inst[b];
+    const int q = threadIdx.x;
+    int still = 0;
+    if (q < I.ncol) {
+        const int c = I.col_off + q;
+        if (active[c]) {
+            const double w = projected_norm(chunk_range[b], parts, MV, q, part);
+            rotate_column(c, j, m, w, active, H, cs, sn, g, tol_abs, est, jlen, iters, scale);
+            still = active[c];
+        } else {
+            scale[c] = 0.0;
+        }
+    }
+    const bool any = __ballot(still) != 0;
+    if (q == 0) inst_active[b] = any ? 1 : 0;
 }
 
 // Back substitution y = R^{-1} g over the column's jlen steps (gmres.rs
@@ -857,7 +907,7 @@ void ragged_dots(sbh_context* ctx, const RaggedLayout& lay, const int* flag, con
 
 void ragged_sum_dots(sbh_context* ctx, const RaggedLayout& lay, const double2* part, int nvec, int j,
                      const int* active, const int* reorth, int pass, double2* H, double2* coef, double* wn0) {
-    hipLaunchKernelGGL(rsum_dots_kernel, dim3(nb((int64_t)lay.C * (nvec + 1))), dim3(BLOCK), 0, ctx->stream, lay.C,
+    hipLaunchKernelGGL(rsum_dots_kernel, dim3(nb((int64_t)lay.C * (nvec + 1), 64)), dim3(64), 0, ctx->stream, lay.C,
                        lay.col_inst, lay.col_q, lay.chunk_range, part, lay.MV, nvec, j, lay.m, active, reorth, pass, H,
                        coef, wn0);
     SBH_HIP(hipGetLastError());
@@ -865,15 +915,15 @@ void ragged_sum_dots(sbh_context* ctx, const RaggedLayout& lay, const double2* p
 
 void ragged_project(sbh_context* ctx, const RaggedLayout& lay, const int* flag, const double2* V, int nvec,
                     const double2* coef, double2* W, double2* part) {
-    hipLaunchKernelGGL(rproject_kernel, dim3((unsigned)lay.nchunks), dim3(BLOCK), 0, ctx->stream, lay.chunks, lay.inst,
+    hipLaunchKernelGGL(rproject_kernel, dim3((unsigned)lay.nchunks, (unsigned)project_parts(lay.MV)), dim3(BLOCK), 0, ctx->stream, lay.chunks, lay.inst,
                        flag, V, lay.L, nvec, coef, lay.MV, W, part);
     SBH_HIP(hipGetLastError());
 }
 
 void ragged_norm(sbh_context* ctx, const RaggedLayout& lay, const double2* part, const int* active, const double* wn0,
-                 int pass, double* wn, int* reorth, int64_t* reorth_count) {
-    hipLaunchKernelGGL(rnorm_kernel, dim3(nb(lay.C)), dim3(BLOCK), 0, ctx->stream, lay.C, lay.col_inst, lay.col_q,
-                       lay.chunk_range, part, lay.MV, active, wn0, pass, wn, reorth, reorth_count);
+                 int* reorth, int64_t* reorth_count, int* inst_reorth) {
+    hipLaunchKernelGGL(rnorm_kernel, dim3((unsigned)lay.B), dim3(64), 0, ctx->stream, lay.inst, lay.chunk_range, part,
+                       project_parts(lay.MV), lay.MV, active, wn0, reorth, reorth_count, inst_reorth);
     SBH_HIP(hipGetLastError());
 }
 
@@ -884,11 +934,12 @@ void ragged_flags(sbh_context* ctx, const RaggedLayout& lay, const int* active, 
     SBH_HIP(hipGetLastError());
 }
 
-void ragged_givens(sbh_context* ctx, const RaggedLayout& lay, int j, int* active, const double* wn, double2* H,
-                   double2* cs, double2* sn, double2* g, const double* tol_abs, double* est, int* jlen, int64_t* iters,
-                   double* scale) {
-    hipLaunchKernelGGL(rgivens_kernel, dim3(nb(lay.C)), dim3(BLOCK), 0, ctx->stream, lay.C, j, lay.m, active, wn, H,
-                       cs, sn, g, tol_abs, est, jlen, iters, scale);
+void ragged_step(sbh_context* ctx, const RaggedLayout& lay, const double2* part, int j, int* active, double2* H,
+                 double2* cs, double2* sn, double2* g, const double* tol_abs, double* est, int* jlen, int64_t* iters,
+                 double* scale, int* inst_active) {
+    hipLaunchKernelGGL(rstep_kernel, dim3((unsigned)lay.B), dim3(64), 0, ctx->stream, lay.inst, lay.chunk_range, part,
+                       project_parts(lay.MV), lay.MV, j, lay.m, active, H, cs, sn, g, tol_abs, est, jlen, iters, scale,
+                       inst_active);
     SBH_HIP(hipGetLastError());
 }
 

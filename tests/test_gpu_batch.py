@@ -427,3 +427,34 @@ def test_frequency_family_matches_single_system(ctx):
     b2.close()
     ws.close()
     tm.close()
+
+
+@pytest.mark.parametrize("restart", [1, 2, 3, 30])
+@pytest.mark.parametrize("chunk", [256, 4096, 65536])
+def test_batch_projection_parts(ctx, restart, chunk):
+    """One to four partial norms per chunk (as many as a cycle has slots for),
+    chunks shorter than the parts and whole instances, 1 to 16 columns: the
+    reported residual is that of the returned solution (rounding of A x: 1e-12
+    of the right-hand side), graph and direct launches give the same bits, and
+    cycles of 30 steps converge."""
+    rng = np.random.default_rng(restart)
+    meshes = [ellipsoid(rng.uniform(0.7, 1.3, size=3), level) for level in (0, 1, 2)]
+    b = sa.Batch(ctx, [sa.TbemMesh(ctx, m) for m in meshes])
+    b.set_problem([1.0, 1.5, 2.0], [uniform_directions(rng, q) for q in (1, 16, 5)])
+    tuning = b.tuning()
+    b.set_tuning(tuning["rows_per_item"], tuning["blocks_per_cu"], chunk)
+    b.assemble()
+    sts = b.solve("fp64", restart=restart, max_cycles=6, tolerance=1e-8, use_graph=False)
+    direct = [b.solution(i).copy() for i in range(3)]
+    for i, X in enumerate(direct):
+        A, B = b.matrix(i), b.rhs(i)
+        first = sum((1, 16, 5)[:i])
+        for q in range(B.shape[1]):
+            res = np.linalg.norm(B[:, q] - A @ X[:, q]) / np.linalg.norm(B[:, q])
+            assert abs(sts[first + q].residual - res) <= 1e-6 * res + 1e-12
+            assert restart < 30 or sts[first + q].converged
+    for _ in range(2):
+        b.solve("fp64", restart=restart, max_cycles=6, tolerance=1e-8)
+        for i, X in enumerate(direct):
+            assert np.array_equal(b.solution(i), X)
+    b.close()
