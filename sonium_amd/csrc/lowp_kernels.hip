@@ -223,11 +223,16 @@ __global__ void x_to_lp_kernel(const T* __restrict__ X, int64_t n, int k, int64_
 // for the real-part columns and NTR for the imaginary-part columns (operand
 // derived in registers).  Partial sums go to Ypart[slab][row][col] (real part
 // at col, imaginary part at NTR * 32 + col) and lp_reduce_kernel adds the
-// slabs in a fixed order.
+// slabs in a fixed order.  The bytes of A bound it if the CUs are full: one holds
+// 12 waves of the 64-column form, so three blocks of 4 waves, but one of 8, and
+// 10240 rows took two rounds of the latter, 101 us, where the 640 blocks of 4
+// waves take 90 (62 at the rate of a plain read; half the CUs get three blocks,
+// half two).  Blocks of 5 waves, which would spread evenly, do not fit twice: two
+// of their waves share a SIMD (119 us).
 constexpr int LP_SPLIT = 8;
 constexpr int LP_BK = 128;
 constexpr int LP_LDS_ROW = LP_BK + 8;
-constexpr int LP_WAVES = 8;
+constexpr int LP_WAVES = 4;
 constexpr int LP_THREADS = LP_WAVES * 64;
 
 __device__ __forceinline__ u32x4 imag_operand(u32x4 b) {  // [xr, -xi] -> [xi, xr] per 32-bit word
@@ -238,7 +243,7 @@ __device__ __forceinline__ u32x4 imag_operand(u32x4 b) {  // [xr, -xi] -> [xi, x
 }
 
 template <int FMT, int NTR>
-__global__ __launch_bounds__(LP_THREADS) void lp_gemm_kernel(const u16* __restrict__ A, int64_t ld, int64_t n,
+__global__ __launch_bounds__(LP_THREADS, 3) void lp_gemm_kernel(const u16* __restrict__ A, int64_t ld, int64_t n,
                                                              const u16* __restrict__ XT, float* __restrict__ Ypart) {
     constexpr int BN = 2 * NTR * 32;
     __shared__ __attribute__((aligned(16))) u16 Bs[NTR * 32 * LP_LDS_ROW];
