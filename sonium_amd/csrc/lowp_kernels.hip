@@ -213,7 +213,7 @@ __global__ void x_to_lp_kernel(const T* __restrict__ X, int64_t n, int k, int64_
     re_row[2 * j + 1] = nxi;
 }
 
-// Split-K MFMA product with FP32 accumulation.  Block = LP_WAVES waves, each
+// Split-K MFMA product with FP32 accumulation.  Block = WAVES waves, each
 // owning one 32-row tile, and one of LP_SPLIT K slabs; slab = blockIdx %
 // LP_SPLIT, so on the 8-XCD part every XCD streams one slab of the block
 // operand, which stays in that XCD's L2.  A wave loads its A fragments for a
@@ -223,17 +223,24 @@ __global__ void x_to_lp_kernel(const T* __restrict__ X, int64_t n, int k, int64_
 // for the real-part columns and NTR for the imaginary-part columns (operand
 // derived in registers).  Partial sums go to Ypart[slab][row][col] (real part
 // at col, imaginary part at NTR * 32 + col) and lp_reduce_kernel adds the
-// slabs in a fixed order.  The bytes of A bound it if the CUs are full: one holds
-// 12 waves of the 64-column form, so three blocks of 4 waves, but one of 8, and
-// 10240 rows took two rounds of the latter, 101 us, where the 640 blocks of 4
-// waves take 90 (62 at the rate of a plain read; half the CUs get three blocks,
-// half two).  Blocks of 5 waves, which would spread evenly, do not fit twice: two
-// of their waves share a SIMD (119 us).
+// slabs in a fixed order.  The bytes of A bound it where every CU has its
+// share of them: lp_waves.
 constexpr int LP_SPLIT = 8;
 constexpr int LP_BK = 128;
 constexpr int LP_LDS_ROW = LP_BK + 8;
-constexpr int LP_WAVES = 4;
-constexpr int LP_THREADS = LP_WAVES * 64;
+
+// Waves of a block.  Up to 32 columns 4: measured faster or equal at every size
+// (2440 rows 10 against 13 us, 10240 80 against 85, 40960 1.06 against 1.08 ms).
+// The 64-column form fits a CU three times with 4 waves and once with 8, which
+// load XT half as often, 7 % of the time; what decides is the waves of the
+// fullest of 256 CUs.  us with 8 and with 4 waves: 2440 rows 17, 15; 5056 31,
+// 34; 10240 99, 87; 15232 172, 199; 20480 319, 306; 40960 1122, 1181 (10240 rows:
+// 62 us at the rate of a plain read).  Blocks of 5 waves do not fit a CU twice,
+// since two of their waves share a SIMD: 119 us at 10240 rows.
+inline int lp_waves(int64_t n_tiles, int ntr) {
+    auto fullest = [&](int waves) { return ((n_tiles + waves - 1) / waves * LP_SPLIT + 255) / 256 * waves; };
+    return ntr == 1 || 1.07 * (double)fullest(4) < (double)fullest(8) ? 4 : 8;
+}
 
 __device__ __forceinline__ u32x4 imag_operand(u32x4 b) {  // [xr, -xi] -> [xi, xr] per 32-bit word
     u32x4 r;
@@ -242,23 +249,24 @@ __device__ __forceinline__ u32x4 imag_operand(u32x4 b) {  // [xr, -xi] -> [xi, x
     return r;
 }
 
-template <int FMT, int NTR>
-__global__ __launch_bounds__(LP_THREADS, 3) void lp_gemm_kernel(const u16* __restrict__ A, int64_t ld, int64_t n,
+template <int FMT, int NTR, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 3) void lp_gemm_kernel(const u16* __restrict__ A, int64_t ld, int64_t n,
                                                              const u16* __restrict__ XT, float* __restrict__ Ypart) {
     constexpr int BN = 2 * NTR * 32;
+    constexpr int THREADS = WAVES * 64;
     __shared__ __attribute__((aligned(16))) u16 Bs[NTR * 32 * LP_LDS_ROW];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int split = blockIdx.x % LP_SPLIT;
     const int64_t n_tiles = (n + 31) / 32;
-    const int64_t rt = (int64_t)(blockIdx.x / LP_SPLIT) * LP_WAVES + wave;
+    const int64_t rt = (int64_t)(blockIdx.x / LP_SPLIT) * WAVES + wave;
     const bool live = rt < n_tiles;
     const int64_t slab = (2 * ld) / LP_SPLIT;  // a multiple of LP_BK (ld is a multiple of 512)
     const int64_t k_begin = split * slab;
     const int64_t k_end = k_begin + slab;
     const u32x4* __restrict__ afrag = reinterpret_cast<const u32x4*>(A) + (live ? rt : 0) * (ld / 8) * 64 + lane;
     constexpr int AS = LP_BK / 16;                                // fragments per stage
-    constexpr int BR = (NTR * 32 * (LP_BK / 8)) / LP_THREADS;     // 16-byte XT pieces per thread per stage
+    constexpr int BR = (NTR * 32 * (LP_BK / 8)) / THREADS;     // 16-byte XT pieces per thread per stage
     u32x4 ra[AS], rb[BR];
     auto load = [&](int64_t kc) {
         if (live) {
@@ -268,7 +276,7 @@ __global__ __launch_bounds__(LP_THREADS, 3) void lp_gemm_kernel(const u16* __res
         }
 #pragma unroll
         for (int i = 0; i < BR; ++i) {
-            const int e = threadIdx.x + i * LP_THREADS;
+            const int e = threadIdx.x + i * THREADS;
             rb[i] = *reinterpret_cast<const u32x4*>(XT + (int64_t)(e >> 4) * 2 * ld + kc + (e & 15) * 8);
         }
     };
@@ -285,7 +293,7 @@ __global__ __launch_bounds__(LP_THREADS, 3) void lp_gemm_kernel(const u16* __res
         for (int i = 0; i < AS; ++i) ca[i] = ra[i];
 #pragma unroll
         for (int i = 0; i < BR; ++i) {
-            const int e = threadIdx.x + i * LP_THREADS;
+            const int e = threadIdx.x + i * THREADS;
             *reinterpret_cast<u32x4*>(&Bs[(e >> 4) * LP_LDS_ROW + (e & 15) * 8]) = rb[i];
         }
         __syncthreads();
@@ -872,20 +880,23 @@ static void lowp_multiply_t(sbh_context* ctx, const uint16_t* A, int64_t ld, int
         return;
     }
     const int bn = 2 * ntr * 32;
-    const int64_t row_blocks = (n_tiles + LP_WAVES - 1) / LP_WAVES;
+    const int waves = lp_waves(n_tiles, ntr);
+    const int64_t row_blocks = (n_tiles + waves - 1) / waves;
     SBH_REQUIRE(row_blocks * LP_SPLIT < ((int64_t)1 << 31), "low-precision product too large");
     const unsigned grid = (unsigned)(row_blocks * LP_SPLIT);
     hipEvent_t ev;
     ctx->begin_timed(SBH_KERNEL_LOWP, &ev);
-#define SBH_LP_GEMM(F, NTV)                                                                                          \
-    hipLaunchKernelGGL((lp_gemm_kernel<F, NTV>), dim3(grid), dim3(LP_THREADS), 0, ctx->stream,                       \
+#define SBH_LP_GEMM(F, NTV, W)                                                                                       \
+    hipLaunchKernelGGL((lp_gemm_kernel<F, NTV, W>), dim3(grid), dim3(W * 64), 0, ctx->stream,                        \
                        reinterpret_cast<const u16*>(A), ld, n, reinterpret_cast<const u16*>(XT), Ypart)
     if (format == 0) {
-        if (ntr == 1) SBH_LP_GEMM(0, 1);
-        else SBH_LP_GEMM(0, 2);
+        if (ntr == 1) SBH_LP_GEMM(0, 1, 4);
+        else if (waves == 4) SBH_LP_GEMM(0, 2, 4);
+        else SBH_LP_GEMM(0, 2, 8);
     } else {
-        if (ntr == 1) SBH_LP_GEMM(1, 1);
-        else SBH_LP_GEMM(1, 2);
+        if (ntr == 1) SBH_LP_GEMM(1, 1, 4);
+        else if (waves == 4) SBH_LP_GEMM(1, 2, 4);
+        else SBH_LP_GEMM(1, 2, 8);
     }
 #undef SBH_LP_GEMM
     SBH_HIP(hipGetLastError());

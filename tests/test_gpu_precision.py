@@ -367,3 +367,24 @@ def test_refinement_row_and_vector_splits(ctx, n_theta, n_phi, k):
     X, st = sa.gmres_block(op, B, sa.GmresConfig(max_iterations=20, restart=50, tolerance=1e-9))
     residual = np.linalg.norm(B - op.apply_block(X), axis=0) / norm
     assert all(s.converged for s in st) and residual.max() <= 1e-9 + 1e-13
+
+
+@pytest.mark.parametrize("n_theta,n_phi", [(5, 3), (9, 8), (9, 40), (21, 61), (33, 79), (41, 90)])
+@pytest.mark.parametrize("k", [2, 32, 33, 64])
+def test_block_product_waves(ctx, n_theta, n_phi, k):
+    """Blocks of four and of eight waves, the last ones part empty, one and two
+    column tiles.  FP16 rounds an entry of A and of X to 2^-11 of the row's and
+    column's largest, and the FP32 sums of 2 n products add n 2^-23 of them."""
+    from sonium_amd.mesh import fibonacci_sphere
+
+    m = fibonacci_sphere(1.0, n_theta, n_phi)
+    n = m.num_elements
+    system = sa.build_tbem_system(ctx, sa.TbemMesh(ctx, m), sa.PhysicsParams.from_wavenumber(1.0))
+    lp = sa.LowpMatrix(system, "fp16")
+    rng = np.random.default_rng(n + k)
+    X = rng.standard_normal((n, k)) + 1j * rng.standard_normal((n, k))
+    A = system.matrix
+    top = np.max(np.abs(A), axis=1, keepdims=True) * np.max(np.abs(X), axis=0)
+    scale = np.abs(A) @ np.abs(X)
+    bound = 2.0 ** -9 * scale + n * 2.0 ** -22 * scale + 2.0 ** -20 * n * top
+    assert np.all(np.abs(lp.apply(X) - A @ X) <= bound)
