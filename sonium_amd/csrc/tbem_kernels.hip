@@ -212,6 +212,31 @@ __device__ __forceinline__ void wave_sum_acc(Acc& a) {
     a.e.x = wave_sum(a.e.x); a.e.y = wave_sum(a.e.y);
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_read(double v) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo);
+}
+
+// Sum over the 16 lanes of a DPP row; every lane of the row gets a total.
+__device__ __forceinline__ double row16_sum(double v) {
+    v += dpp_read<0xB1>(v);   // quad_perm [1,0,3,2]
+    v += dpp_read<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += dpp_read<0x141>(v);  // row_half_mirror: lane i <- 7 - i within each half row
+    v += dpp_read<0x140>(v);  // row_mirror: lane i <- 15 - i
+    return v;
+}
+
+// The same over the 16 lanes of each row.
+__device__ __forceinline__ void row16_sum_acc(Acc& a) {
+    a.g.x = row16_sum(a.g.x); a.g.y = row16_sum(a.g.y);
+    a.h.x = row16_sum(a.h.x); a.h.y = row16_sum(a.h.y);
+    a.ht.x = row16_sum(a.ht.x); a.ht.y = row16_sum(a.ht.y);
+    a.e.x = row16_sum(a.e.x); a.e.y = row16_sum(a.e.y);
+}
+
 // ---------------------------------------------------------------------------
 // One quadrature point of the regular kernel, regular.rs:214-281.  DERIV also
 // accumulates the analytic wavenumber derivative of every channel into dr
@@ -1330,7 +1355,7 @@ __global__ __launch_bounds__(256) void self_deriv_kernel(const PanelGeom* __rest
 }
 
 // Block per row: right-hand-side derivative over the nonzero-BC columns in a
-// fixed order, as bc_rhs_kernel.
+// fixed order, as bc_rhs_kernel (4378 panels, 164 -> 81 us).
 __global__ __launch_bounds__(256) void bc_rhs_deriv_kernel(const int32_t* __restrict__ cols, int64_t ncols,
                                                            const NearPair* __restrict__ pairs,
                                                            const int64_t* __restrict__ row_ptr,
@@ -1339,22 +1364,22 @@ __global__ __launch_bounds__(256) void bc_rhs_deriv_kernel(const int32_t* __rest
                                                            const Source* __restrict__ sources,
                                                            const PanelBc* __restrict__ bcs, DerivParams P,
                                                            double2* __restrict__ rhs) {
-    __shared__ double part[4][2];
+    __shared__ double part[16][2];
     const int64_t i = blockIdx.x;
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
+    const int group = threadIdx.x >> 4;
+    const int lane = threadIdx.x & 15;
     const Source src = sources[i];
     const double k2 = P.k * P.k;
     double2 sum = make_double2(0.0, 0.0);
     const int64_t pb = row_ptr[i], pe = row_ptr[i + 1];
-    for (int64_t c = wave; c < ncols; c += 4) {
+    for (int64_t c = group; c < ncols; c += 16) {
         const int32_t j = cols[c];
         const PanelGeom G = geom[j];
         Acc b = acc_zero(), d = acc_zero();
         if (j == i) {
             const SelfTier t = tier_for(P.k * G.size);
             const int ns = self_samples(t);
-            for (int s = lane; s < ns; s += 64)
+            for (int s = lane; s < ns; s += 16)
                 self_sample_t<true>(G, t, s, src.c, src.n, P.wavruim, k2, P.k, P.hf, b, d);
         } else {
             int64_t lo = pb, hi = pe;
@@ -1365,7 +1390,7 @@ __global__ __launch_bounds__(256) void bc_rhs_deriv_kernel(const int32_t* __rest
             if (lo < pe && pairs[lo].j == j) {
                 const NearPair np = pairs[lo];
                 const int total = np.count * 13;
-                for (int t = lane; t < total; t += 64) {
+                for (int t = lane; t < total; t += 16) {
                     const int leaf = t / 13;
                     near_point_t<true>(G, leaves[np.begin + leaf], t - leaf * 13, src.c, src.n, P.wavruim, k2, P.k,
                                        P.hf, b, d);
@@ -1374,24 +1399,26 @@ __global__ __launch_bounds__(256) void bc_rhs_deriv_kernel(const int32_t* __rest
                 full_point_t<true>(G, lane, src.c, src.n, P.wavruim, k2, P.k, P.hf, b, d);
             }
         }
-        wave_sum_acc(b);
-        wave_sum_acc(d);
+        row16_sum_acc(b);
+        row16_sum_acc(d);
         sum = cadd(sum, deriv_bc_contribution(b, d, bcs[j], P));
     }
     if (lane == 0) {
-        part[wave][0] = sum.x;
-        part[wave][1] = sum.y;
+        part[group][0] = sum.x;
+        part[group][1] = sum.y;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         double2 t = rhs[i];
-        for (int w = 0; w < 4; ++w) t = cadd(t, make_double2(part[w][0], part[w][1]));
+        for (int w = 0; w < 16; ++w) t = cadd(t, make_double2(part[w][0], part[w][1]));
         rhs[i] = t;
     }
 }
 
 // Block per row: sum over nonzero-BC columns of tbem.rs:1419-1435, in a
-// fixed order (wave w takes columns w, w+4, ...; waves summed 0..3).
+// fixed order (sixteen lanes take columns g, g+16, ...; the groups summed in
+// order).  FP64 issue bounds it: the rule's 13 points on 16 lanes leave 3 idle,
+// on a wave 51 (4378 panels, 139 -> 82 us).
 __global__ __launch_bounds__(256) void bc_rhs_kernel(const int32_t* __restrict__ cols, int64_t ncols,
                                                      const NearPair* __restrict__ pairs,
                                                      const int64_t* __restrict__ row_ptr,
@@ -1401,24 +1428,24 @@ __global__ __launch_bounds__(256) void bc_rhs_kernel(const int32_t* __restrict__
                                                      const PanelBc* __restrict__ bcs, double k,
                                                      double wavruim, double tau_r, double2 beta,
                                                      double2 iwr, double2* __restrict__ rhs) {
-    __shared__ double part[4][2];
+    __shared__ double part[16][2];
     const int64_t i = blockIdx.x;
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
+    const int group = threadIdx.x >> 4;
+    const int lane = threadIdx.x & 15;
     const Source src = sources[i];
     const double k2 = k * k;
     const double2 gamma = make_double2(1.0, 0.0);
     const double2 tau = make_double2(tau_r, 0.0);
     double2 sum = make_double2(0.0, 0.0);
     const int64_t pb = row_ptr[i], pe = row_ptr[i + 1];
-    for (int64_t c = wave; c < ncols; c += 4) {
+    for (int64_t c = group; c < ncols; c += 16) {
         const int32_t j = cols[c];
         const PanelGeom G = geom[j];
         Acc a = acc_zero();
         if (j == i) {
             const SelfTier t = tier_for(k * G.size);
             const int ns = self_samples(t);
-            for (int s = lane; s < ns; s += 64) self_sample(G, t, s, src.c, src.n, wavruim, k2, a);
+            for (int s = lane; s < ns; s += 16) self_sample(G, t, s, src.c, src.n, wavruim, k2, a);
         } else {
             int64_t lo = pb, hi = pe;  // pairs of row i are sorted by column
             while (lo < hi) {
@@ -1428,7 +1455,7 @@ __global__ __launch_bounds__(256) void bc_rhs_kernel(const int32_t* __restrict__
             if (lo < pe && pairs[lo].j == j) {
                 const NearPair np = pairs[lo];
                 const int total = np.count * 13;
-                for (int t = lane; t < total; t += 64) {
+                for (int t = lane; t < total; t += 16) {
                     int leaf = t / 13;
                     near_point(G, leaves[np.begin + leaf], t - leaf * 13, src.c, src.n, wavruim, k2, a);
                 }
@@ -1436,17 +1463,17 @@ __global__ __launch_bounds__(256) void bc_rhs_kernel(const int32_t* __restrict__
                 full_point(G, lane, src.c, src.n, wavruim, k2, a);
             }
         }
-        wave_sum_acc(a);
+        row16_sum_acc(a);
         sum = cadd(sum, bc_contribution(a, bcs[j], gamma, tau, beta, iwr));
     }
     if (lane == 0) {
-        part[wave][0] = sum.x;
-        part[wave][1] = sum.y;
+        part[group][0] = sum.x;
+        part[group][1] = sum.y;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         double2 t = rhs[i];
-        for (int w = 0; w < 4; ++w) t = cadd(t, make_double2(part[w][0], part[w][1]));
+        for (int w = 0; w < 16; ++w) t = cadd(t, make_double2(part[w][0], part[w][1]));
         rhs[i] = t;
     }
 }
@@ -1589,23 +1616,6 @@ __global__ __launch_bounds__(256) void batch_far_family_kernel(const FreqFamily*
 // phase by one complex product.  Rigid panels need the H and E channels
 // only; the 16-lane sums use row DPP, and lane f writes member f's entry.
 constexpr int NEAR_FAMILY_LANES = 16;
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_read(double v) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
-    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo);
-}
-
-// Sum over the 16 lanes of a DPP row; every lane of the row gets a total.
-__device__ __forceinline__ double row16_sum(double v) {
-    v += dpp_read<0xB1>(v);   // quad_perm [1,0,3,2]
-    v += dpp_read<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp_read<0x141>(v);  // row_half_mirror: lane i <- 7 - i within each half row
-    v += dpp_read<0x140>(v);  // row_mirror: lane i <- 15 - i
-    return v;
-}
 
 template <int F>
 __global__ __launch_bounds__(256) void batch_near_family_kernel(const FreqFamily* __restrict__ families,

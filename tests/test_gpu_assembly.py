@@ -92,6 +92,20 @@ def test_pressure_and_admittance_columns_match_oracle(ctx):
     assert rel_fro(b, br) <= TOL
 
 
+@pytest.mark.parametrize("driven", [1, 15, 16, 17, 33, 80])
+def test_driven_columns_in_groups(ctx, driven):
+    """Fewer driven panels than the sixteen groups of a row's sum, as many, one
+    more and all: the right-hand side of every row, near, far and own panels."""
+    m = icosphere(1.0, 1)
+    rng = np.random.default_rng(driven)
+    bv = np.zeros(m.num_elements, dtype=np.complex128)
+    at = rng.permutation(m.num_elements)[:driven]
+    bv[at] = rng.standard_normal(driven) + 1j * rng.standard_normal(driven)
+    b = _assemble_gpu(ctx, m, 2.0, 0.5j, bc_value=bv)[1]
+    br = _assemble_cpu(m, 2.0, 0.5j, bc_value=bv)[1]
+    assert rel_fro(b, br) <= TOL
+
+
 @pytest.mark.parametrize("k", [0.5, 4.0, 8.0])
 def test_self_panel_tiers_on_coarse_mesh(ctx, k):
     """80-panel icosphere: k*sqrt(area) spans the 4 QuadratureParams::for_ka tiers (singular.rs:51-85)."""
