@@ -1417,8 +1417,10 @@ void BlockLeastSquares::reset(const double2* c0, int s1) {
 }
 
 void BlockLeastSquares::add(const void* chol, const void* chain, const double2* hacc, int sj) {
-    SBH_REQUIRE(sj >= 1 && sj <= s_ && (size_t)done_ + 1 < steps_.count && cols_ + sj <= ldg_ - s_,
-                "block least-squares step");
+    SBH_REQUIRE(sj >= 1 && sj <= s_, "block least-squares step");
+    // more directions than the space has: the rank-drop test saw no numbers
+    if ((size_t)done_ + 1 >= steps_.count || cols_ + sj > ldg_ - s_)
+        throw Error(SBH_ERR_NUMERICAL, "block GMRES generated NaN or infinity in its basis");
     hipEvent_t ev;
     ctx_->begin_timed(SBH_KERNEL_KRYLOV_VECTOR, &ev);
     const LsState st = ls_state(steps_.ptr, refl_.ptr, qh_.ptr, R_.ptr, window_.ptr, g_.ptr, ldg_, host_.ptr);

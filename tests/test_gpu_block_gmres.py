@@ -237,3 +237,19 @@ def test_block_gmres_tiles(ctx, n_theta, n_phi, s):
     smallest = np.linalg.svd(A, compute_uv=False)[-1]
     exact = np.linalg.solve(A, B)
     assert np.all(np.linalg.norm(sol.x - exact, axis=0) <= 1.01 * (residual + 1e-13) * norm / smallest)
+
+
+@pytest.mark.parametrize("s", [1, 8, 40])
+def test_block_gmres_at_the_ends_of_the_range(ctx, s):
+    """Squares that still fit (1e150), that overflow (1e160) and that vanish
+    (1e-170): solved, refused as numerical, and zero to the norms, with a block
+    wider than the 20-panel space among them."""
+    system = sa.build_tbem_system(ctx, sa.TbemMesh(ctx, icosphere(1.0, 0)), sa.PhysicsParams.from_wavenumber(1.0))
+    op = sa.DenseMatrixOperator(system)
+    rng = np.random.default_rng(s)
+    B = rng.standard_normal((op.num_rows(), s)) + 1j * rng.standard_normal((op.num_rows(), s))
+    cfg = sa.BlockGmresConfig(max_iterations=5, restart=30, tolerance=1e-8)
+    assert sa.block_gmres(op, 1e150 * B, cfg).converged
+    with pytest.raises(sa.SbhError, match="NaN or infinity"):
+        sa.block_gmres(op, 1e160 * B, cfg)
+    assert sa.block_gmres(op, 1e-170 * B, cfg).iterations == 0
