@@ -78,8 +78,7 @@ class BlockGmresEngine {
     BlockGmresEngine(sbh_operator* op, const sbh_precond* M, int s, int64_t restart)
         : op_(op), ctx_(op->ctx), n_(op->n), s_(s), dinv_(M && M->kind == 1 ? M->d_dinv.ptr : nullptr),
           max_steps_((int)std::max<int64_t>(1, restart)), max_basis_((max_steps_ + 1) * s),
-          // the rank-drop test keeps the basis within the space, and a step adds to it or ends the cycle
-          ls_(ctx_, s, (int)std::min<int64_t>(max_basis_, n_ + 2 * s), (int)std::min<int64_t>(max_steps_, n_ + 1)) {
+          ls_(ctx_, n_, s, max_basis_, max_steps_) {
         const size_t blk = (size_t)n_ * s;
         admit_device(ctx_, (int64_t)(sizeof(double2) * ((size_t)(max_basis_ + s) * n_ + 6 * blk)),
                      "the shared block Krylov basis", false);

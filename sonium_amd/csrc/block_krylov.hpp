@@ -14,10 +14,16 @@ struct BlockStep {
     double tail[64];   // residual norms of the right-hand sides
 };
 
-// min ||g - H y|| over the block Hessenberg columns added so far.
+// min ||g - H y|| over the block Hessenberg columns added so far, at most
+// max_basis in max_steps steps.  A basis of an n-dimensional space has n
+// directions as long as the numbers are good, so the arrays start with room for
+// n + 2 s of them in n + 1 steps and grow when a step needs more: the rank-drop
+// test measures a column against its norm after the projection, and once the
+// basis fills the space (or the operator's range) the rounding errors left of a
+// step pass it as new directions.
 class BlockLeastSquares {
    public:
-    BlockLeastSquares(sbh_context* ctx, int s, int max_basis, int max_steps);
+    BlockLeastSquares(sbh_context* ctx, int64_t n, int s, int max_basis, int max_steps);
 
     // Queues the outcome of a block QR of sj columns (chain null: the Cholesky one's).
     void report(const void* chol, const void* chain, int sj);
@@ -37,9 +43,13 @@ class BlockLeastSquares {
     const BlockStep& host() const { return *host_.ptr; }  // after a synchronization
 
    private:
+    void make_room(int steps, int cols);
+
     sbh_context* ctx_;
     int s_, done_ = 0, cols_ = 0;
-    int64_t ldg_;
+    int max_basis_, max_steps_;            // limits of a cycle
+    int room_cols_ = 0, room_steps_ = 0;   // what the arrays hold
+    int64_t ldg_ = 0;
     WorkArray<int2> steps_;
     WorkArray<double2> refl_, qh_, R_, window_, g_, work_;
     WorkArray<BlockStep, true> host_;

@@ -1382,17 +1382,39 @@ void bk_block_qr(sbh_context* ctx, double2* W, double2* Q, int64_t n, int sj, in
 
 size_t bk_ls_window(int s) { return s <= 32 ? 64 : 128; }
 
-BlockLeastSquares::BlockLeastSquares(sbh_context* ctx, int s, int max_basis, int max_steps)
-    : ctx_(ctx), s_(s), ldg_(max_basis + s) {
+BlockLeastSquares::BlockLeastSquares(sbh_context* ctx, int64_t n, int s, int max_basis, int max_steps)
+    : ctx_(ctx), s_(s), max_basis_(max_basis), max_steps_(max_steps) {
     const size_t window = bk_ls_window(s);
-    steps_.allocate((size_t)max_steps + 1);
     refl_.allocate((size_t)s * window);
-    qh_.allocate((size_t)max_steps * window * window);
-    R_.allocate((size_t)max_basis * (max_basis + 1) / 2);
     window_.allocate((size_t)s * window);
-    g_.allocate((size_t)ldg_ * s);
-    work_.allocate((size_t)ldg_ * s);
     host_.allocate(1);
+    make_room((int)std::min<int64_t>(max_steps, n + 1), (int)std::min<int64_t>(max_basis, n + 2 * s));
+}
+
+// Arrays for `steps` steps with `cols` columns; the columns added so far are kept.
+void BlockLeastSquares::make_room(int steps, int cols) {
+    const size_t window = bk_ls_window(s_);
+    const int64_t ldg = cols + s_;
+    WorkArray<int2> steps_new((size_t)steps + 1);
+    WorkArray<double2> qh((size_t)steps * window * window), R((size_t)cols * (cols + 1) / 2), g((size_t)ldg * s_),
+        work((size_t)ldg * s_);
+    auto keep = [&](void* to, const void* from, size_t bytes) {
+        if (bytes) SBH_HIP(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, ctx_->stream));
+    };
+    keep(steps_new.ptr, steps_.ptr, sizeof(int2) * done_);
+    keep(qh.ptr, qh_.ptr, sizeof(double2) * done_ * window * window);
+    keep(R.ptr, R_.ptr, sizeof(double2) * ((size_t)cols_ * (cols_ + 1) / 2));
+    if (ldg_)
+        SBH_HIP(hipMemcpy2DAsync(g.ptr, sizeof(double2) * ldg, g_.ptr, sizeof(double2) * ldg_, sizeof(double2) * ldg_,
+                                 s_, hipMemcpyDeviceToDevice, ctx_->stream));
+    steps_.swap(steps_new);
+    qh_.swap(qh);
+    R_.swap(R);
+    g_.swap(g);
+    work_.swap(work);
+    ldg_ = ldg;
+    room_cols_ = cols;
+    room_steps_ = steps;
 }
 
 namespace {
@@ -1417,10 +1439,17 @@ void BlockLeastSquares::reset(const double2* c0, int s1) {
 }
 
 void BlockLeastSquares::add(const void* chol, const void* chain, const double2* hacc, int sj) {
-    SBH_REQUIRE(sj >= 1 && sj <= s_, "block least-squares step");
-    // more directions than the space has: the rank-drop test saw no numbers
-    if ((size_t)done_ + 1 >= steps_.count || cols_ + sj > ldg_ - s_)
-        throw Error(SBH_ERR_NUMERICAL, "block GMRES generated NaN or infinity in its basis");
+    SBH_REQUIRE(sj >= 1 && sj <= s_ && done_ < max_steps_ && cols_ + sj <= max_basis_, "block least-squares step");
+    if (done_ + 1 > room_steps_ || cols_ + sj > room_cols_) {
+        // without numbers the solve ends as a numerical error however long it goes on
+        for (int c = 0; c < s_ && done_ > 0; ++c)
+            if (!std::isfinite(host_.ptr->tail[c]))
+                throw Error(SBH_ERR_NUMERICAL, "block GMRES generated NaN or infinity in its basis");
+        auto grown = [](int room, int need, int most) {
+            return need <= room ? room : (int)std::min<int64_t>(most, std::max<int64_t>(need, 2 * (int64_t)room));
+        };
+        make_room(grown(room_steps_, done_ + 1, max_steps_), grown(room_cols_, cols_ + sj, max_basis_));
+    }
     hipEvent_t ev;
     ctx_->begin_timed(SBH_KERNEL_KRYLOV_VECTOR, &ev);
     const LsState st = ls_state(steps_.ptr, refl_.ptr, qh_.ptr, R_.ptr, window_.ptr, g_.ptr, ldg_, host_.ptr);

@@ -112,6 +112,11 @@ struct WorkArray {
         o.count = 0;
     }
     ~WorkArray() { release(); }
+    void swap(WorkArray& o) noexcept {
+        std::swap(ptr, o.ptr);
+        std::swap(count, o.count);
+        std::swap(block_, o.block_);
+    }
     void allocate(size_t n) {
         release();
         if (n == 0) return;

@@ -253,3 +253,24 @@ def test_block_gmres_at_the_ends_of_the_range(ctx, s):
     with pytest.raises(sa.SbhError, match="NaN or infinity"):
         sa.block_gmres(op, 1e160 * B, cfg)
     assert sa.block_gmres(op, 1e-170 * B, cfg).iterations == 0
+
+
+@pytest.mark.parametrize("n,s,restart", [(48, 1, 200), (60, 12, 20), (60, 24, 20), (80, 40, 20), (200, 64, 9)])
+def test_block_gmres_basis_beyond_the_space(ctx, n, s, restart):
+    """An operator of rank n / 2 and a tolerance out of reach: once the basis
+    fills the space, what rounding leaves of a step passes the rank-drop test, and
+    two whole cycles run to an unconverged end with finite results, as in the
+    oracle, on more directions than n + 2 s (and, with one column, more steps than
+    n + 1)."""
+    rng = np.random.default_rng(n + s)
+    c = lambda *shape: rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    A, B = c(n, n // 2) @ c(n // 2, n) / n, c(n, s)
+    _, st = oracle.block_gmres(A, B, restart=restart, max_iterations=2, tol=1e-30)
+    assert st["iterations"] == 2 * restart and not st["converged"] and np.all(np.isfinite(st["true_residuals"]))
+    op = sa.CallbackOperator(ctx, n, lambda x: A @ x)
+    sol = sa.block_gmres(op, B, sa.BlockGmresConfig(max_iterations=2, restart=restart, tolerance=1e-30))
+    assert sol.iterations == 2 * restart and sol.restart_cycles == 2 and sol.max_basis > n + 2 * s
+    assert not sol.converged and sol.status == "max_iterations"
+    assert np.all(np.isfinite(sol.x)) and np.all(np.isfinite(sol.true_residuals))
+    assert np.all(sol.residuals == 0.0)  # as the reference reports a spent budget
+    op.close()
