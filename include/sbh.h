@@ -350,7 +350,8 @@ int64_t sbh_live_device_bytes(void);
  * parts follow the reference's conservative estimate (dense operator n*n*16,
  * right-hand sides n*rhs*16 per frequency, scratch n*(4*16 + 8)); device_bytes
  * is this library's allocation for the same work (system, right-hand sides
- * and solutions, GMRES(restart) basis; the shared block basis for rhs > 1).
+ * and solutions, GMRES(restart) basis; for rhs > 1 the shared block basis and
+ * its least squares).
  * Errors: a zero request -> SBH_ERR_INVALID_ARGUMENT (InvalidRequest);
  * overflow -> SBH_ERR_INVALID_ARGUMENT (ArithmeticOverflow); over a limit
  * -> SBH_ERR_OUT_OF_MEMORY (LimitExceeded, the message names the resource);

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <memory>
 
+#include "block_krylov.hpp"
 #include "internal.hpp"
 
 namespace sbh {
@@ -467,13 +468,14 @@ sbh_status sbh_admission_estimate(int64_t n, int64_t rhs, int64_t freq, int64_t 
         e.host_bytes = sum({e.operator_bytes, e.rhs_bytes, e.scratch_bytes}, "peak host allocation");
         // this library: system (matrix, one right-hand side, row maxima of the
         // assembly), right-hand sides and solutions, Krylov basis (shared
-        // block basis for rhs > 1)
+        // block basis for rhs > 1, with its least squares; at most 64 columns a solve)
         const int64_t basis_vectors = rhs == 1 ? sum({restart, 3}, "basis size")
                                                : prod({sum({restart, 2}, "basis size"), rhs}, "basis size");
         e.device_bytes = sum({e.operator_bytes, prod({n, C}, "rhs"), prod({n, (n + 255) / 256 + 1, 8}, "row maxima"),
                               prod({2, rhs_bytes}, "blocks"),
                               prod({basis_vectors, n, C}, "Krylov basis"),
-                              prod({6, rhs_bytes}, "block scratch")},
+                              prod({6, rhs_bytes}, "block scratch"),
+                              rhs == 1 ? 0 : BlockLeastSquares::device_bytes(n, (int)std::min<int64_t>(rhs, 64), restart)},
                              "peak device allocation");
         *out = e;
     });

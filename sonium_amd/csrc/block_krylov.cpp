@@ -80,8 +80,11 @@ class BlockGmresEngine {
           max_steps_((int)std::max<int64_t>(1, restart)), max_basis_((max_steps_ + 1) * s),
           ls_(ctx_, n_, s, max_basis_, max_steps_) {
         const size_t blk = (size_t)n_ * s;
-        admit_device(ctx_, (int64_t)(sizeof(double2) * ((size_t)(max_basis_ + s) * n_ + 6 * blk)),
+        admit_device(ctx_,
+                     (int64_t)(sizeof(double2) * ((size_t)(max_basis_ + s) * n_ + 6 * blk)) +
+                         BlockLeastSquares::device_bytes(n_, s, max_steps_),
                      "the shared block Krylov basis", false);
+        ls_.allocate();
         V_.allocate((size_t)(max_basis_ + s) * n_);
         W_.allocate(blk);
         Rcm_.allocate(blk);

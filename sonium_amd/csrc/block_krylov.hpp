@@ -24,6 +24,9 @@ struct BlockStep {
 class BlockLeastSquares {
    public:
     BlockLeastSquares(sbh_context* ctx, int64_t n, int s, int max_basis, int max_steps);
+    // Device bytes that allocate() takes in a solve of s columns on n rows.
+    static int64_t device_bytes(int64_t n, int s, int64_t restart);
+    void allocate();
 
     // Queues the outcome of a block QR of sj columns (chain null: the Cholesky one's).
     void report(const void* chol, const void* chain, int sj);
@@ -43,9 +46,11 @@ class BlockLeastSquares {
     const BlockStep& host() const { return *host_.ptr; }  // after a synchronization
 
    private:
+    static int64_t room_bytes(int s, int64_t steps, int64_t cols);
     void make_room(int steps, int cols);
 
     sbh_context* ctx_;
+    int64_t n_;
     int s_, done_ = 0, cols_ = 0;
     int max_basis_, max_steps_;            // limits of a cycle
     int room_cols_ = 0, room_steps_ = 0;   // what the arrays hold

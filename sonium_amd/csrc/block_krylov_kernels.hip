@@ -1383,12 +1383,26 @@ void bk_block_qr(sbh_context* ctx, double2* W, double2* Q, int64_t n, int sj, in
 size_t bk_ls_window(int s) { return s <= 32 ? 64 : 128; }
 
 BlockLeastSquares::BlockLeastSquares(sbh_context* ctx, int64_t n, int s, int max_basis, int max_steps)
-    : ctx_(ctx), s_(s), max_basis_(max_basis), max_steps_(max_steps) {
-    const size_t window = bk_ls_window(s);
-    refl_.allocate((size_t)s * window);
-    window_.allocate((size_t)s * window);
+    : ctx_(ctx), n_(n), s_(s), max_basis_(max_basis), max_steps_(max_steps) {}
+
+void BlockLeastSquares::allocate() {
+    const size_t window = bk_ls_window(s_);
+    refl_.allocate((size_t)s_ * window);
+    window_.allocate((size_t)s_ * window);
     host_.allocate(1);
-    make_room((int)std::min<int64_t>(max_steps, n + 1), (int)std::min<int64_t>(max_basis, n + 2 * s));
+    make_room((int)std::min<int64_t>(max_steps_, n_ + 1), (int)std::min<int64_t>(max_basis_, n_ + 2 * s_));
+}
+
+int64_t BlockLeastSquares::room_bytes(int s, int64_t steps, int64_t cols) {
+    const int64_t window = (int64_t)bk_ls_window(s);
+    return (int64_t)sizeof(int2) * (steps + 1) +
+           (int64_t)sizeof(double2) * (steps * window * window + cols * (cols + 1) / 2 + 2 * (cols + s) * s);
+}
+
+int64_t BlockLeastSquares::device_bytes(int64_t n, int s, int64_t restart) {
+    const int64_t steps = std::min(restart, n + 1);
+    const int64_t cols = std::min((steps + 1) * s, n + 2 * s);
+    return room_bytes(s, steps, cols) + (int64_t)sizeof(double2) * 2 * s * (int64_t)bk_ls_window(s);
 }
 
 // Arrays for `steps` steps with `cols` columns; the columns added so far are kept.
@@ -1448,7 +1462,9 @@ void BlockLeastSquares::add(const void* chol, const void* chain, const double2* 
         auto grown = [](int room, int need, int most) {
             return need <= room ? room : (int)std::min<int64_t>(most, std::max<int64_t>(need, 2 * (int64_t)room));
         };
-        make_room(grown(room_steps_, done_ + 1, max_steps_), grown(room_cols_, cols_ + sj, max_basis_));
+        const int steps = grown(room_steps_, done_ + 1, max_steps_), cols = grown(room_cols_, cols_ + sj, max_basis_);
+        admit_device(ctx_, room_bytes(s_, steps, cols), "the block least squares", false);
+        make_room(steps, cols);
     }
     hipEvent_t ev;
     ctx_->begin_timed(SBH_KERNEL_KRYLOV_VECTOR, &ev);

@@ -56,3 +56,14 @@ def test_device_estimate_covers_the_dense_path():
     assert e["device_bytes"] >= 16 * n * n + 16 * n * 101
     e64 = sa.admission_estimate(40960, 64, 1, 100)
     assert e64["device_bytes"] >= 16 * 40960 ** 2 + 16 * 40960 * 102 * 64
+
+
+@pytest.mark.parametrize("n,rhs,restart", [(10240, 64, 200), (5056, 24, 30), (80, 40, 500)])
+def test_device_estimate_covers_the_block_least_squares(n, rhs, restart):
+    # the shared basis of restart + 2 blocks, blocks and their scratch, and the
+    # triangle of the least squares over as many directions as the space has
+    e = sa.admission_estimate(n, rhs, 1, restart)
+    blocks = 16 * n * (n + 1) + 8 * n * ((n + 255) // 256 + 1) + 16 * n * rhs * (restart + 2 + 8)
+    m = min((restart + 1) * rhs, n + 2 * rhs)
+    assert e["device_bytes"] >= blocks + 8 * m * m
+    assert sa.admission_admit(e["host_bytes"], e["device_bytes"], rhs, n, rhs, 1, restart) == e

@@ -48,3 +48,29 @@ def test_device_budget_refuses_before_allocating():
         sa.TbemSystem(ctx, 300000)
     assert e.value.status == 4 and "free of" in str(e.value)
     ctx.close()
+
+
+@pytest.mark.parametrize("s,restart", [(8, 50), (40, 12)])
+def test_block_solve_admits_its_least_squares(s, restart):
+    """The refusal counts the least squares with the basis, and a budget of the
+    estimate admits the solve."""
+    c = sa.Context(0)
+    n = 1280
+    estimate = sa.admission_estimate(n, s, 1, restart)["device_bytes"]
+    tm = sa.TbemMesh(c, icosphere(1.0, 3))
+    ph = sa.PhysicsParams.from_wavenumber(2.0)
+    ws = sa.TbemAssemblyWorkspace(c, tm)
+    system = ws.assemble(ph, ph.burton_miller_beta())
+    held = c.device_budget()[1]
+    op = sa.DenseMatrixOperator(system)
+    B = np.ones((n, s), dtype=np.complex128) + np.eye(n, s)
+    cfg = sa.BlockGmresConfig(max_iterations=1, restart=restart, tolerance=1e-8)
+    basis = 16 * n * s * (restart + 2 + 6)
+    c.set_device_budget(held + basis)
+    with pytest.raises(sa.SbhError) as e:
+        sa.block_gmres(op, B, cfg)
+    assert e.value.status == 4 and "block Krylov basis" in str(e.value)
+    c.set_device_budget(estimate)
+    assert sa.block_gmres(op, B, cfg).iterations >= 1
+    for o in (op, ws, system, tm, c):
+        o.close()
