@@ -127,107 +127,6 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 thread_local sbh_context* g_current_ctx = nullptr;
 std::atomic<int64_t> g_live_device_bytes{0};
 
-namespace {
-struct WorkPool {
-    std::mutex mu;
-    std::vector<WorkBlock> idle;  // oldest first
-    size_t bytes = 0;
-};
-// never destroyed: arrays may outlive the library's static objects
-WorkPool& work_pool() {
-    static WorkPool* pool = new WorkPool;
-    return *pool;
-}
-
-void work_free(const WorkBlock& b) {
-    if (b.pinned)
-        (void)hipHostFree(b.ptr);
-    else
-        (void)hipFree(b.ptr);
-}
-}  // namespace
-
-void work_trim() {
-    WorkPool& pool = work_pool();
-    std::vector<WorkBlock> idle;
-    {
-        std::lock_guard<std::mutex> lk(pool.mu);
-        idle.swap(pool.idle);
-        pool.bytes = 0;
-    }
-    for (const WorkBlock& b : idle) work_free(b);
-}
-
-void* device_malloc(size_t bytes) {
-    void* p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();  // clear it
-        work_trim();
-        e = hipMalloc(&p, bytes);
-    }
-    SBH_HIP(e);
-    return p;
-}
-
-WorkBlock work_take(size_t bytes, bool pinned) {
-    WorkBlock b;
-    b.bytes = (bytes + 255) / 256 * 256;
-    b.pinned = pinned;
-    SBH_HIP(hipGetDevice(&b.device));
-    {
-        // the smallest idle block that fits without wasting more than a quarter
-        WorkPool& pool = work_pool();
-        std::lock_guard<std::mutex> lk(pool.mu);
-        size_t best = pool.idle.size();
-        for (size_t i = 0; i < pool.idle.size(); ++i) {
-            const WorkBlock& c = pool.idle[i];
-            if (c.device == b.device && c.pinned == pinned && c.bytes >= b.bytes &&
-                c.bytes <= b.bytes + b.bytes / 4 + 65536 && (best == pool.idle.size() || c.bytes < pool.idle[best].bytes))
-                best = i;
-        }
-        if (best < pool.idle.size()) {
-            b = pool.idle[best];
-            pool.idle.erase(pool.idle.begin() + (std::ptrdiff_t)best);
-            pool.bytes -= b.bytes;
-            return b;
-        }
-    }
-    if (pinned)
-        SBH_HIP(hipHostMalloc(&b.ptr, b.bytes, hipHostMallocDefault));
-    else
-        b.ptr = device_malloc(b.bytes);
-    return b;
-}
-
-void work_give(const WorkBlock& b) {
-    // hipFree's order: nothing on the device uses the block any more, whatever
-    // stream it was on
-    int device = -1;
-    if (b.bytes > WORK_BLOCK_LIMIT || hipGetDevice(&device) != hipSuccess || device != b.device ||
-        hipDeviceSynchronize() != hipSuccess) {
-        work_free(b);
-        return;
-    }
-    WorkPool& pool = work_pool();
-    {
-        std::lock_guard<std::mutex> lk(pool.mu);
-        pool.idle.push_back(b);
-        pool.bytes += b.bytes;
-    }
-    for (;;) {
-        WorkBlock oldest;
-        {
-            std::lock_guard<std::mutex> lk(pool.mu);
-            if (pool.bytes <= WORK_IDLE_LIMIT && pool.idle.size() <= WORK_IDLE_BLOCKS) return;
-            oldest = pool.idle.front();
-            pool.idle.erase(pool.idle.begin());
-            pool.bytes -= oldest.bytes;
-        }
-        work_free(oldest);
-    }
-}
-
 void injection_check(int point) {
     sbh_context* ctx = g_current_ctx;
     if (!ctx) return;
@@ -300,7 +199,7 @@ double* sbh_context::pinned_rw(size_t count) {
         if (pinned) (void)hipHostFree(pinned);
         pinned = nullptr;
         pinned_count = 0;
-        SBH_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), count * sizeof(double), hipHostMallocDefault));
+        pinned = static_cast<double*>(pinned_malloc(count * sizeof(double)));
         pinned_count = count;
     }
     return pinned;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <mutex>
@@ -70,8 +71,9 @@ extern std::atomic<int64_t> g_live_device_bytes;
         if (!(cond)) throw ::sbh::Error(SBH_ERR_INVALID_ARGUMENT, (msg));   \
     } while (0)
 
-// hipMalloc that gives the idle work blocks back before it fails.
+// hipMalloc and hipHostMalloc that give the idle work blocks back before they fail.
 void* device_malloc(size_t bytes);
+void* pinned_malloc(size_t bytes);
 
 // Work blocks of the solvers.  A solve needs its Krylov basis and staging for
 // the length of one call; hipMalloc and hipFree of those cost 15 us each for
@@ -79,14 +81,16 @@ void* device_malloc(size_t bytes);
 // gigabyte in 14 blocks; with the blocks kept the refinement takes 26.4 instead
 // of 30.4 ms, a 5056-panel solve of 24 columns 14.9 instead of 16.2, and 40
 // training steps with 16384 samples 13.6 instead of 18.4).  Blocks given back
-// stay idle for the next call: at most WORK_IDLE_LIMIT bytes in
-// WORK_IDLE_BLOCKS, none above WORK_BLOCK_LIMIT, the oldest freed first; all
-// are freed when a context is destroyed and when an allocation or an admission
-// would fail.  Giving a block back waits for the device, as hipFree does, so a
+// stay idle for the next call: at most WORK_IDLE_LIMIT bytes of device and
+// WORK_IDLE_PINNED_LIMIT of pinned memory (a solve of 64 columns with a restart
+// of 1000 pins 6 MB) in WORK_IDLE_BLOCKS, none above WORK_BLOCK_LIMIT, the
+// oldest freed first; all are freed when a context is destroyed and when an
+// allocation or an admission would fail.  Giving a block back waits for the device, as hipFree does, so a
 // block may go to any thread, context or stream next.  Contents are undefined,
 // as hipMalloc's.
 constexpr size_t WORK_BLOCK_LIMIT = (size_t)2 << 30;
 constexpr size_t WORK_IDLE_LIMIT = (size_t)4 << 30;
+constexpr size_t WORK_IDLE_PINNED_LIMIT = (size_t)64 << 20;
 constexpr size_t WORK_IDLE_BLOCKS = 128;
 struct WorkBlock {
     void* ptr = nullptr;
