@@ -342,6 +342,11 @@ typedef enum {
 sbh_status sbh_context_inject_failure(sbh_context* ctx, int point);
 /* Bytes held by the library's device allocations in this process. */
 int64_t sbh_live_device_bytes(void);
+/* Solves keep their work memory for the next call (at most 4 GiB on the
+ * devices and 64 MiB of pinned host memory in this process, which the figure
+ * above does not count).  This gives it back, for other allocators of the
+ * process; the outputs (may be null) are the bytes given back. */
+sbh_status sbh_trim_idle_memory(int64_t* device_bytes, int64_t* pinned_bytes);
 
 /* ---------------------------------------------------------------------------
  * Resource admission — BemResourceBudget / BemResourceRequest::estimate /
@@ -382,7 +387,8 @@ sbh_status sbh_admission_admit(const sbh_resource_budget* budget, int64_t active
  * workspaces) is refused with SBH_ERR_OUT_OF_MEMORY before it is made when the
  * bytes held by the context's objects plus the request exceed it; requests
  * beyond the device's free memory are refused the same way with or without a
- * budget.  0 removes the budget. */
+ * budget.  Idle work memory is given back where it would exceed the budget
+ * with them.  0 removes the budget. */
 sbh_status sbh_context_set_device_budget(sbh_context* ctx, int64_t max_device_bytes);
 sbh_status sbh_context_device_budget(sbh_context* ctx, int64_t* max_device_bytes, int64_t* held_bytes);
 

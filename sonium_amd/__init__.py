@@ -54,6 +54,13 @@ def live_device_bytes() -> int:
     return int(_lib().sbh_live_device_bytes())
 
 
+def trim_idle_memory():
+    """Gives back the work memory that solves keep for the next call: (device, pinned) bytes."""
+    d, p = ctypes.c_int64(), ctypes.c_int64()
+    _check(_lib().sbh_trim_idle_memory(ctypes.byref(d), ctypes.byref(p)))
+    return int(d.value), int(p.value)
+
+
 def _lib():
     return _ffi.load()
 

@@ -157,6 +157,7 @@ SIGNATURES = {
                                    ctypes.POINTER(resource_estimate_t)]),
     "sbh_context_inject_failure": (_int, [_vp, _int]),
     "sbh_live_device_bytes": (_i64, []),
+    "sbh_trim_idle_memory": (_int, [ctypes.POINTER(_i64), ctypes.POINTER(_i64)]),
     "sbh_context_kernel_stats": (_int, [_vp, _int, ctypes.POINTER(_i64), _dp]),
     "sbh_context_reset_stats": (_int, [_vp]),
     "sbh_vector_create": (_int, [_vp, _i64, _pp]),

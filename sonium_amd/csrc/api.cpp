@@ -154,6 +154,7 @@ void admit_device(sbh_context* ctx, int64_t bytes, const char* what, bool reserv
         throw Error(SBH_ERR_OUT_OF_MEMORY, std::string("admission refused: ") + what + " needs " +
                                                std::to_string(bytes) + " device bytes; the context's budget is " +
                                                std::to_string(budget) + " with " + std::to_string(held) + " held");
+    if (budget > 0 && held + bytes + work_idle_bytes(ctx->device) > budget) work_trim();
     size_t free_b = 0, total_b = 0;
     SBH_HIP(hipMemGetInfo(&free_b, &total_b));
     if ((uint64_t)bytes > (uint64_t)free_b) {  // idle work blocks do not count
@@ -406,6 +407,7 @@ sbh_status sbh_context_set_device_budget(sbh_context* ctx, int64_t bytes) {
         SBH_REQUIRE(ctx, "ctx is null");
         SBH_REQUIRE(bytes >= 0, "the device budget must be >= 0");
         ctx->device_budget = bytes;
+        if (bytes > 0 && ctx->device_reserved.load() + work_idle_bytes(ctx->device) > bytes) work_trim();
     });
 }
 
@@ -426,6 +428,14 @@ sbh_status sbh_context_inject_failure(sbh_context* ctx, int point) {
 }
 
 int64_t sbh_live_device_bytes(void) { return g_live_device_bytes.load(); }
+
+sbh_status sbh_trim_idle_memory(int64_t* device_bytes, int64_t* pinned_bytes) {
+    return guard([&] {
+        const IdleBytes freed = work_trim();
+        if (device_bytes) *device_bytes = freed.device;
+        if (pinned_bytes) *pinned_bytes = freed.pinned;
+    });
+}
 
 sbh_status sbh_context_set_profiling(sbh_context* ctx, int enabled) {
     return guard_on(ctx_of(ctx), [&] {

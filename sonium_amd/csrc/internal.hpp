@@ -84,8 +84,9 @@ void* pinned_malloc(size_t bytes);
 // stay idle for the next call: at most WORK_IDLE_LIMIT bytes of device and
 // WORK_IDLE_PINNED_LIMIT of pinned memory (a solve of 64 columns with a restart
 // of 1000 pins 6 MB) in WORK_IDLE_BLOCKS, none above WORK_BLOCK_LIMIT, the
-// oldest freed first; all are freed when a context is destroyed and when an
-// allocation or an admission would fail.  Giving a block back waits for the device, as hipFree does, so a
+// oldest freed first; all are freed when a context is destroyed, when an
+// allocation or an admission would fail or idle blocks would exceed a context's
+// device budget, and by sbh_trim_idle_memory.  Giving a block back waits for the device, as hipFree does, so a
 // block may go to any thread, context or stream next.  Contents are undefined,
 // as hipMalloc's.
 constexpr size_t WORK_BLOCK_LIMIT = (size_t)2 << 30;
@@ -100,7 +101,11 @@ struct WorkBlock {
 };
 WorkBlock work_take(size_t bytes, bool pinned);
 void work_give(const WorkBlock& b);
-void work_trim();
+struct IdleBytes {
+    int64_t device = 0, pinned = 0;
+};
+IdleBytes work_trim();                // frees every idle block: the bytes freed
+int64_t work_idle_bytes(int device);  // device memory of the idle blocks
 
 // Owning block from the work pool: device memory, or pinned host memory.
 template <typename T, bool PINNED = false>

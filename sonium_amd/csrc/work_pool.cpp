@@ -55,17 +55,28 @@ void* with_trim(Alloc&& alloc) {
 
 }  // namespace
 
-void work_trim() {
+IdleBytes work_trim() {
     WorkPool& pool = work_pool();
+    IdleBytes freed;
     for (;;) {
         WorkBlock b;
         {
             std::lock_guard<std::mutex> lk(pool.mu);
-            if (pool.idle.empty()) return;
+            if (pool.idle.empty()) return freed;
             b = pool.take(pool.idle.size() - 1);
         }
+        (b.pinned ? freed.pinned : freed.device) += (int64_t)b.bytes;
         work_free(b);
     }
+}
+
+int64_t work_idle_bytes(int device) {
+    WorkPool& pool = work_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    int64_t sum = 0;
+    for (const WorkBlock& b : pool.idle)
+        if (!b.pinned && b.device == device) sum += (int64_t)b.bytes;
+    return sum;
 }
 
 void* device_malloc(size_t bytes) {

@@ -93,8 +93,11 @@ int main() {
     const WorkBlock big = work_take(WORK_IDLE_PINNED_LIMIT + 1, true);
     work_give(big);
     check(live.find(big.ptr) == live.end(), "a pinned block above the limit is not kept");
-    work_trim();
-    check(live.empty(), "trim");
+    const size_t device = held(false), pinned = held(true);
+    check(work_idle_bytes(0) == (int64_t)device && work_idle_bytes(1) == 0, "idle bytes of a device");
+    const IdleBytes freed = work_trim();
+    check(live.empty() && work_idle_bytes(0) == 0, "trim");
+    check(freed.device == (int64_t)device && freed.pinned == (int64_t)pinned, "bytes given back");
     // an allocation of either kind that finds the memory full of idle blocks
     capacity = 100 * MB;
     for (bool pinned : {false, true}) {

@@ -73,3 +73,22 @@ def test_threads_that_exchange_blocks_match_serial_bits():
         for run in runs:
             for x, y in zip(run, ref):
                 assert np.array_equal(x, y)
+
+
+def test_idle_blocks_are_given_back():
+    p = Problem(2)
+    want = p.answers()
+    device, pinned = sa.trim_idle_memory()
+    assert device > 0 and pinned > 0
+    assert sa.trim_idle_memory() == (0, 0)
+    for x, y in zip(p.answers(), want):
+        assert np.array_equal(x, y)
+    # a budget that idle blocks would exceed
+    p.ctx.set_device_budget(p.ctx.device_budget()[1] + 1024)
+    assert sa.trim_idle_memory()[0] == 0
+    p.ctx.set_device_budget(0)
+    p.answers()
+    with pytest.raises(sa.SbhError, match="budget"):
+        p.ctx.set_device_budget(p.ctx.device_budget()[1] + 1024)
+        sa.TbemSystem(p.ctx, 1000)
+    assert sa.trim_idle_memory()[0] == 0
