@@ -80,6 +80,8 @@ struct BlockOperatorT {
     int64_t applies = 0;
     virtual void apply(const T* X, T* Y, int k) = 0;
     // The same in two parts: what X alone takes, then the product with it.
+    // The operand stands in the operator's own memory: between the two neither
+    // X changes nor does another apply or prepare run on the operator.
     virtual void prepare(const T* X, int k) {
         (void)X;
         (void)k;
@@ -148,7 +150,9 @@ struct BatchedParams {
     // then the norm after the second pass).  The device scales the next vector
     // and prepares its product before the host has read the step: the read and
     // the rotations of 64 columns leave the device idle for 60 us a step
-    // otherwise, a sixth of it at 10240 rows.
+    // otherwise, a sixth of it at 10240 rows.  Not with exact_checks, whose
+    // product in the middle of a cycle would replace the prepared operand, nor
+    // in a flexible engine, whose product takes the preconditioned vector.
     // Otherwise: one pass plus the DGKS pass when ||w|| < 0.707 ||w0|| (gmres_core).
     bool cgs2 = false;
 };
@@ -272,6 +276,7 @@ void BatchedGmres<T>::run(BlockOperatorT<T>& A, BlockPreconditionerT<T>* M, cons
                           const BatchedParams& p, std::vector<ColumnResult>& out) {
     const int k = k_;
     const int m = m_;
+    SBH_REQUIRE(!p.cgs2 || (!flexible_ && !p.exact_checks), "a prepared operand must not be replaced");
     out.assign(k, ColumnResult{});
     std::vector<char> done(k, 0);
     auto finish = [&](int c, double res, double est, double bw, bool conv, int status) {
