@@ -75,6 +75,42 @@ def _cptr(a: np.ndarray):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+def _handle_of(obj, kind):
+    """The library handle of obj, which has to be a ``kind``: the library takes
+    the address for one, so any other object's would be read as something it is not."""
+    if not isinstance(obj, kind):
+        raise TypeError(f"expected a {kind.__name__.lstrip('_')}, got {type(obj).__name__}")
+    return obj._h
+
+
+def _ctx_h(ctx):
+    return _handle_of(ctx, Context)
+
+
+def _mesh_h(mesh):
+    return _handle_of(mesh, TbemMesh)
+
+
+def _system_h(system):
+    return _handle_of(system, TbemSystem)
+
+
+def _op_h(op):
+    return _handle_of(op, DenseMatrixOperator)
+
+
+def _precond_h(precond):
+    return None if precond is None else _handle_of(precond, _Precond)
+
+
+def _subspace_h(subspace):
+    return _handle_of(subspace, GcroDrSubspace)
+
+
+def _lowp_h(lp):
+    return _handle_of(lp, LowpMatrix)
+
+
 def _c128(a, n=None) -> np.ndarray:
     arr = np.ascontiguousarray(a, dtype=np.complex128)
     if n is not None and arr.size != n:
@@ -189,7 +225,7 @@ class DeviceVector:
     def __init__(self, ctx: Context, length: int):
         self.ctx = ctx
         h = ctypes.c_void_p()
-        _check(_lib().sbh_vector_create(ctx.handle, int(length), ctypes.byref(h)))
+        _check(_lib().sbh_vector_create(_ctx_h(ctx), int(length), ctypes.byref(h)))
         self._h = h
         self.length = int(length)
 
@@ -247,7 +283,7 @@ class TbemMesh:
         rule = {"outward": 0, "vertex_order": 1}[normals]
         h = ctypes.c_void_p()
         _check(_lib().sbh_mesh_create_oriented(
-            ctx.handle, _cptr(mesh.nodes), mesh.nodes.shape[0], _cptr(mesh.triangles), n,
+            _ctx_h(ctx), _cptr(mesh.nodes), mesh.nodes.shape[0], _cptr(mesh.triangles), n,
             None if bt is None else _cptr(bt), None if bv is None else _cptr(bv),
             None if ad is None else _cptr(ad), None if has is None else _cptr(has), rule, ctypes.byref(h)))
         self._h = h
@@ -283,7 +319,7 @@ class TbemSystem:
         self.ctx = ctx
         self.num_dofs = int(num_dofs)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_system_create(ctx.handle, self.num_dofs, ctypes.byref(h)))
+        _check(_lib().sbh_system_create(_ctx_h(ctx), self.num_dofs, ctypes.byref(h)))
         self._h = h
 
     @property
@@ -341,7 +377,7 @@ class TbemAssemblyWorkspace:
         self.ctx = ctx
         self.mesh = mesh
         h = ctypes.c_void_p()
-        _check(_lib().sbh_workspace_create(ctx.handle, mesh.handle, route_threads, ctypes.byref(h)))
+        _check(_lib().sbh_workspace_create(_ctx_h(ctx), _mesh_h(mesh), route_threads, ctypes.byref(h)))
         self._h = h
 
     @property
@@ -363,7 +399,7 @@ class TbemAssemblyWorkspace:
         if system is None:
             system = TbemSystem(self.ctx, self.mesh.num_elements)
         b = _ffi.c64(complex(beta).real, complex(beta).imag)
-        _check(_lib().sbh_workspace_assemble(self._h, ctypes.byref(physics._p), b, system.handle))
+        _check(_lib().sbh_workspace_assemble(self._h, ctypes.byref(physics._p), b, _system_h(system)))
         return system
 
     def assemble_parameter_derivative(self, physics: PhysicsParams, beta: complex, beta_derivative: complex, *,
@@ -384,7 +420,7 @@ class TbemAssemblyWorkspace:
         bd = _ffi.c64(complex(beta_derivative).real, complex(beta_derivative).imag)
         _check(_lib().sbh_workspace_assemble_derivative(
             self._h, ctypes.byref(physics._p), b, bd, float(sign), float(wavenumber_scale),
-            float(pressure_factor_derivative), float(admittance_scale), system.handle))
+            float(pressure_factor_derivative), float(admittance_scale), _system_h(system)))
         return system
 
     def _derivative(self, physics, sign, beta_scale, ws, pfd, adm, system):
@@ -529,7 +565,7 @@ class IncidentField:
             col = np.zeros(mesh.num_elements, dtype=np.complex128)
             b = _ffi.c64(complex(beta).real, complex(beta).imag)
             for i in range(self.num_rhs):
-                _check(_lib().sbh_incident_rhs(mesh.ctx.handle, mesh.handle, ctypes.byref(physics._p), b, float(sign),
+                _check(_lib().sbh_incident_rhs(mesh.ctx.handle, _mesh_h(mesh), ctypes.byref(physics._p), b, float(sign),
                                                ctypes.byref(src[i]), 1, _cptr(col), MEM_HOST, 0))
                 out[:, i] = col
         return out if self.num_rhs > 1 else out[:, 0]
@@ -554,13 +590,13 @@ class IncidentField:
             raise ValueError("device right-hand sides with point sources take one source per column")
         b = _ffi.c64(complex(beta).real, complex(beta).imag)
         src = self.source_array()
-        _check(_lib().sbh_incident_rhs(mesh.ctx.handle, mesh.handle, ctypes.byref(physics._p), b, float(sign), src, 1,
+        _check(_lib().sbh_incident_rhs(mesh.ctx.handle, _mesh_h(mesh), ctypes.byref(physics._p), b, float(sign), src, 1,
                                        ptr, MEM_DEVICE, int(accumulate)))
 
     def _launch(self, mesh, physics, beta, sign, ptr, memory, accumulate):
         b = _ffi.c64(complex(beta).real, complex(beta).imag)
         _check(_lib().sbh_incident_plane_wave_rhs(
-            mesh.ctx.handle, mesh.handle, ctypes.byref(physics._p), b, float(sign), _cptr(self.directions),
+            mesh.ctx.handle, _mesh_h(mesh), ctypes.byref(physics._p), b, float(sign), _cptr(self.directions),
             _cptr(self.amplitudes), self.num_rhs, ptr, memory, int(accumulate)))
 
 
@@ -578,12 +614,12 @@ def _field(mesh, solution, surface_velocity, physics, incident, points, with_inc
             MEM_HOST)
     if incident is None or incident._plane_only:
         _check(_lib().sbh_field_pressure(
-            mesh.ctx.handle, mesh.handle, ctypes.byref(physics._p), _cptr(sol), None if vel is None else _cptr(vel),
+            mesh.ctx.handle, _mesh_h(mesh), ctypes.byref(physics._p), _cptr(sol), None if vel is None else _cptr(vel),
             None if incident is None else _cptr(incident.directions),
             None if incident is None else _cptr(incident.amplitudes), nw, *outs))
     else:
         _check(_lib().sbh_field_pressure_sources(
-            mesh.ctx.handle, mesh.handle, ctypes.byref(physics._p), _cptr(sol), None if vel is None else _cptr(vel),
+            mesh.ctx.handle, _mesh_h(mesh), ctypes.byref(physics._p), _cptr(sol), None if vel is None else _cptr(vel),
             incident.source_array(), nw, *outs))
     return pts, scat, inc, tot
 
@@ -650,7 +686,7 @@ class DenseMatrixOperator:
         self.system = system
         self.ctx = system.ctx
         h = ctypes.c_void_p()
-        _check(_lib().sbh_dense_operator_create(system.handle, ctypes.byref(h)))
+        _check(_lib().sbh_dense_operator_create(_system_h(system), ctypes.byref(h)))
         self._h = h
 
     @property
@@ -737,7 +773,7 @@ class TbemExactOperator(DenseMatrixOperator):
         self.ctx = workspace.ctx
         bv = physics.burton_miller_beta() if beta is None else complex(beta)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_exact_operator_create(workspace.handle, ctypes.byref(physics._p),
+        _check(_lib().sbh_exact_operator_create(_handle_of(workspace, TbemAssemblyWorkspace), ctypes.byref(physics._p),
                                                 _ffi.c64(bv.real, bv.imag), float(sign), ctypes.byref(h)))
         self._h = h
 
@@ -774,7 +810,7 @@ class CallbackOperator(DenseMatrixOperator):
         self.ctx = ctx
         self._cb = _host_callback(fn)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_operator_create_callback(ctx.handle, int(n), self._cb, None, MEM_HOST, ctypes.byref(h)))
+        _check(_lib().sbh_operator_create_callback(_ctx_h(ctx), int(n), self._cb, None, MEM_HOST, ctypes.byref(h)))
         self._h = h
 
 
@@ -804,7 +840,7 @@ class CallbackPreconditioner(_Precond):
         self.n = int(n)
         self._cb = _host_callback(fn)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_precond_create_callback(ctx.handle, self.n, self._cb, None, MEM_HOST, ctypes.byref(h)))
+        _check(_lib().sbh_precond_create_callback(_ctx_h(ctx), self.n, self._cb, None, MEM_HOST, ctypes.byref(h)))
         self._h = h
 
 
@@ -812,7 +848,7 @@ class IdentityPreconditioner(_Precond):
     def __init__(self, ctx: Context, n: int):
         self.n = int(n)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_precond_identity(ctx.handle, self.n, ctypes.byref(h)))
+        _check(_lib().sbh_precond_identity(_ctx_h(ctx), self.n, ctypes.byref(h)))
         self._h = h
 
 
@@ -822,7 +858,7 @@ class JacobiPreconditioner(_Precond):
     def __init__(self, op: DenseMatrixOperator):
         self.n = op.num_rows()
         h = ctypes.c_void_p()
-        _check(_lib().sbh_precond_jacobi(op.handle, ctypes.byref(h)))
+        _check(_lib().sbh_precond_jacobi(_op_h(op), ctypes.byref(h)))
         self._h = h
 
 
@@ -890,7 +926,7 @@ def gmres_preconditioned_with_guess(op: DenseMatrixOperator, precond, b, x0, con
     x = np.zeros(n, dtype=np.complex128)
     raw = _ffi.gmres_solution_t()
     cfg = config._c()
-    _check(_lib().sbh_gmres(op.handle, None if precond is None else precond._h, _cptr(bv),
+    _check(_lib().sbh_gmres(_op_h(op), _precond_h(precond), _cptr(bv),
                             None if x0v is None else _cptr(x0v), ctypes.byref(cfg), _cptr(x), MEM_HOST,
                             ctypes.byref(raw)))
     return _solution(raw, x)
@@ -916,7 +952,7 @@ def gmres_device(op: DenseMatrixOperator, b_ptr: int, x: DeviceVector, config: G
     """GMRES on device-resident b (device pointer) and x; the solution stays in HBM."""
     raw = _ffi.gmres_solution_t()
     cfg = config._c()
-    _check(_lib().sbh_gmres(op.handle, None if precond is None else precond._h, ctypes.c_void_p(b_ptr),
+    _check(_lib().sbh_gmres(_op_h(op), _precond_h(precond), ctypes.c_void_p(b_ptr),
                             None if x0 is None else ctypes.c_void_p(x0.ptr), ctypes.byref(cfg),
                             ctypes.c_void_p(x.ptr), MEM_DEVICE, ctypes.byref(raw)))
     return _solution(raw, None)
@@ -948,7 +984,7 @@ class GcroDrSubspace:
         self.n = int(n)
         self.k = int(k)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_gcro_subspace_create(ctx.handle, self.n, self.k, ctypes.byref(h)))
+        _check(_lib().sbh_gcro_subspace_create(_ctx_h(ctx), self.n, self.k, ctypes.byref(h)))
         self._h = h
 
     @property
@@ -995,8 +1031,8 @@ def gcro_dr_preconditioned(op: DenseMatrixOperator, precond, b, x0, subspace: Gc
     x = np.zeros(n, dtype=np.complex128)
     raw = _ffi.gmres_solution_t()
     cfg = config._c()
-    _check(_lib().sbh_gcro_dr(op.handle, None if precond is None else precond._h, _cptr(bv),
-                              None if x0v is None else _cptr(x0v), subspace.handle, ctypes.byref(cfg), _cptr(x),
+    _check(_lib().sbh_gcro_dr(_op_h(op), _precond_h(precond), _cptr(bv),
+                              None if x0v is None else _cptr(x0v), _subspace_h(subspace), ctypes.byref(cfg), _cptr(x),
                               MEM_HOST, ctypes.byref(raw)))
     return _solution(raw, x)
 
@@ -1011,8 +1047,8 @@ def gcro_dr_device(op: DenseMatrixOperator, b_ptr: int, x: DeviceVector, subspac
     """GCRO-DR on device-resident b (device pointer) and x."""
     raw = _ffi.gmres_solution_t()
     cfg = config._c()
-    _check(_lib().sbh_gcro_dr(op.handle, None if precond is None else precond._h, ctypes.c_void_p(b_ptr),
-                              None if x0 is None else ctypes.c_void_p(x0.ptr), subspace.handle, ctypes.byref(cfg),
+    _check(_lib().sbh_gcro_dr(_op_h(op), _precond_h(precond), ctypes.c_void_p(b_ptr),
+                              None if x0 is None else ctypes.c_void_p(x0.ptr), _subspace_h(subspace), ctypes.byref(cfg),
                               ctypes.c_void_p(x.ptr), MEM_DEVICE, ctypes.byref(raw)))
     return _solution(raw, None)
 
@@ -1032,7 +1068,7 @@ def gmres_block(op: DenseMatrixOperator, B, config: GmresConfig, X0=None):
     X0v = None if X0 is None else np.ascontiguousarray(X0, dtype=np.complex128).reshape(n, k)
     raws = (_ffi.gmres_solution_t * k)()
     cfg = config._c()
-    _check(_lib().sbh_gmres_block(op.handle, _cptr(Bv), None if X0v is None else _cptr(X0v), k,
+    _check(_lib().sbh_gmres_block(_op_h(op), _cptr(Bv), None if X0v is None else _cptr(X0v), k,
                                   ctypes.byref(cfg), _cptr(X), MEM_HOST, raws))
     return X, [_solution(raws[c], X[:, c]) for c in range(k)]
 
@@ -1121,7 +1157,7 @@ def block_gmres_preconditioned_with_guess(op: DenseMatrixOperator, B, precond=No
     X0v = None if X0 is None else np.ascontiguousarray(X0, dtype=np.complex128).reshape(n, k)
     info = _ffi.block_gmres_info_t()
     res, tres, berr = (np.zeros(k) for _ in range(3))
-    _check(_lib().sbh_block_gmres(op.handle, None if precond is None else precond._h, _cptr(Bv),
+    _check(_lib().sbh_block_gmres(_op_h(op), _precond_h(precond), _cptr(Bv),
                                   None if X0v is None else _cptr(X0v), k, ctypes.byref(config._c()), _cptr(X),
                                   MEM_HOST, ctypes.byref(info), _cptr(res), _cptr(tres), _cptr(berr)))
     return _block_solution(info, X, res, tres, berr)
@@ -1140,7 +1176,7 @@ def block_gmres_device(op: DenseMatrixOperator, B: DeviceVector, k: int, X: Devi
     _block_vectors(op, B, X, k, X0)
     info = _ffi.block_gmres_info_t()
     res, tres, berr = (np.zeros(k) for _ in range(3))
-    _check(_lib().sbh_block_gmres(op.handle, None if precond is None else precond._h, ctypes.c_void_p(B.ptr),
+    _check(_lib().sbh_block_gmres(_op_h(op), _precond_h(precond), ctypes.c_void_p(B.ptr),
                                   None if X0 is None else ctypes.c_void_p(X0.ptr), k, ctypes.byref(config._c()),
                                   ctypes.c_void_p(X.ptr), MEM_DEVICE, ctypes.byref(info), _cptr(res), _cptr(tres),
                                   _cptr(berr)))
@@ -1161,7 +1197,7 @@ def gmres_block_device(op: DenseMatrixOperator, B: DeviceVector, k: int, X: Devi
     """gmres_block on device-resident row-major n x k blocks; X stays in HBM."""
     _block_vectors(op, B, X, k, X0)
     raws = (_ffi.gmres_solution_t * k)()
-    _check(_lib().sbh_gmres_block(op.handle, ctypes.c_void_p(B.ptr), None if X0 is None else ctypes.c_void_p(X0.ptr),
+    _check(_lib().sbh_gmres_block(_op_h(op), ctypes.c_void_p(B.ptr), None if X0 is None else ctypes.c_void_p(X0.ptr),
                                   k, ctypes.byref(config._c()), ctypes.c_void_p(X.ptr), MEM_DEVICE, raws))
     return [_solution(raws[c], None) for c in range(k)]
 
@@ -1176,7 +1212,7 @@ class LowpMatrix:
         self.system = system
         self.format = fmt
         h = ctypes.c_void_p()
-        _check(_lib().sbh_lowp_matrix_create(system.handle, LOWP_FORMATS[fmt], ctypes.byref(h)))
+        _check(_lib().sbh_lowp_matrix_create(_system_h(system), LOWP_FORMATS[fmt], ctypes.byref(h)))
         self._h = h
 
     @property
@@ -1266,7 +1302,7 @@ def gmres_ir(op: DenseMatrixOperator, lp: LowpMatrix, B, config: GmresIrConfig):
     X = np.zeros_like(Bv)
     raws = (_ffi.gmres_ir_status_t * k)()
     cfg = config._c()
-    _check(_lib().sbh_gmres_ir(op.handle, lp.handle, _cptr(Bv), k, ctypes.byref(cfg), _cptr(X), MEM_HOST, raws))
+    _check(_lib().sbh_gmres_ir(_op_h(op), _lowp_h(lp), _cptr(Bv), k, ctypes.byref(cfg), _cptr(X), MEM_HOST, raws))
     return X, _ir_statuses(raws, k)
 
 
@@ -1275,7 +1311,7 @@ def gmres_ir_device(op: DenseMatrixOperator, lp: LowpMatrix, B: DeviceVector, k:
     """gmres_ir on device-resident row-major n x k blocks; X stays in HBM."""
     _block_vectors(op, B, X, k)
     raws = (_ffi.gmres_ir_status_t * k)()
-    _check(_lib().sbh_gmres_ir(op.handle, lp.handle, ctypes.c_void_p(B.ptr), k, ctypes.byref(config._c()),
+    _check(_lib().sbh_gmres_ir(_op_h(op), _lowp_h(lp), ctypes.c_void_p(B.ptr), k, ctypes.byref(config._c()),
                                ctypes.c_void_p(X.ptr), MEM_DEVICE, raws))
     return _ir_statuses(raws, k)
 
@@ -1318,9 +1354,9 @@ class Batch:
     def __init__(self, ctx: Context, meshes, route_threads: int = 0):
         self.ctx = ctx
         self.meshes = list(meshes)
-        arr = (ctypes.c_void_p * len(self.meshes))(*[m.handle.value for m in self.meshes])
+        arr = (ctypes.c_void_p * len(self.meshes))(*[_mesh_h(m).value for m in self.meshes])
         h = ctypes.c_void_p()
-        _check(_lib().sbh_batch_create(ctx.handle, len(self.meshes), arr, int(route_threads), ctypes.byref(h)))
+        _check(_lib().sbh_batch_create(_ctx_h(ctx), len(self.meshes), arr, int(route_threads), ctypes.byref(h)))
         self._h = h
         self.num_rhs = None
 
@@ -1448,7 +1484,10 @@ class Batch:
     def learned_guesses(self, net, out: Optional[DeviceVector] = None) -> None:
         """The network's guesses for every column, computed on the device, into
         ``out`` (packed layout) or as the batch's initial guesses."""
-        _check(_lib().sbh_batch_learned_guesses(self._h, net._h, None if out is None else out.ptr))
+        from .warmstart import WarmStartMLP
+
+        _check(_lib().sbh_batch_learned_guesses(self._h, _handle_of(net, WarmStartMLP),
+                                                None if out is None else out.ptr))
 
     def solutions(self):
         """Every instance's solution block, in one download."""
@@ -1532,7 +1571,7 @@ def device_sincos(ctx: Context, x) -> tuple:
     xv = np.ascontiguousarray(x, dtype=np.float64)
     s = np.empty_like(xv)
     c = np.empty_like(xv)
-    _check(_lib().sbh_debug_device_sincos(ctx.handle, _cptr(xv), xv.size, _cptr(s), _cptr(c)))
+    _check(_lib().sbh_debug_device_sincos(_ctx_h(ctx), _cptr(xv), xv.size, _cptr(s), _cptr(c)))
     return s, c
 
 
@@ -1540,7 +1579,7 @@ def device_rsqrt(ctx: Context, x) -> np.ndarray:
     """The kernels' 1/sqrt evaluated on the device (test hook)."""
     xv = np.ascontiguousarray(x, dtype=np.float64)
     y = np.empty_like(xv)
-    _check(_lib().sbh_debug_device_rsqrt(ctx.handle, _cptr(xv), xv.size, _cptr(y)))
+    _check(_lib().sbh_debug_device_rsqrt(_ctx_h(ctx), _cptr(xv), xv.size, _cptr(y)))
     return y
 
 

@@ -18,7 +18,7 @@ from typing import Optional
 import numpy as np
 
 from . import _ffi
-from . import _check, _cptr, _lib, Context, DenseMatrixOperator, GmresConfig, gmres_with_guess, gmres
+from . import _check, _cptr, _ctx_h, _lib, Context, DenseMatrixOperator, GmresConfig, gmres_with_guess, gmres
 
 RAW = 10
 
@@ -74,7 +74,7 @@ class WarmStartMLP:
         self.ctx = ctx
         self.width = int(width)
         h = ctypes.c_void_p()
-        _check(_lib().sbh_mlp_create(ctx.handle, self.width, int(seed), ctypes.byref(h)))
+        _check(_lib().sbh_mlp_create(_ctx_h(ctx), self.width, int(seed), ctypes.byref(h)))
         self._h = h
         self.num_params = int(_lib().sbh_mlp_num_params(h))
 
