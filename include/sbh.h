@@ -846,6 +846,10 @@ sbh_status sbh_nc_project_surface_mesh(const sbh_nc_project* project, sbh_contex
 sbh_status sbh_debug_subelements(const double* source_point, const double* element_coords,
                                  double element_area, double* leaves_out, int* count);
 
+/* Test hook: writes `byte` over all work memory kept for the next call (see
+ * sbh_trim_idle_memory), so that a result that reads a part of its work memory
+ * before writing it changes. */
+sbh_status sbh_debug_fill_idle_memory(int byte, int64_t* bytes);
 /* Test hook: the device sin/cos used by the assembly kernels, evaluated at
  * host-supplied points (for accuracy checks against the C library). */
 sbh_status sbh_debug_device_sincos(sbh_context* ctx, const double* x, int64_t n, double* s, double* c);

@@ -1583,6 +1583,13 @@ def device_rsqrt(ctx: Context, x) -> np.ndarray:
     return y
 
 
+def debug_fill_idle_memory(byte: int) -> int:
+    """Writes ``byte`` over the work memory kept for the next call (test hook): the bytes written."""
+    n = ctypes.c_int64()
+    _check(_lib().sbh_debug_fill_idle_memory(int(byte), ctypes.byref(n)))
+    return int(n.value)
+
+
 def debug_subelements(source_point, element_coords, element_area: float) -> np.ndarray:
     """The host route builder's subdivision of one pair (test hook, no GPU)."""
     src = np.ascontiguousarray(source_point, dtype=np.float64).reshape(3)

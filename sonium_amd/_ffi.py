@@ -272,6 +272,7 @@ SIGNATURES = {
     "sbh_mlp_set_dataset": (_int, [_vp, _vp, _vp, _i64]),
     "sbh_mlp_train": (_int, [_vp, _i64, _i64, ctypes.c_double, ctypes.c_double, ctypes.c_uint64, _vp]),
     "sbh_mlp_predict": (_int, [_vp, _vp, _i64, _vp, _int]),
+    "sbh_debug_fill_idle_memory": (_int, [_int, ctypes.POINTER(_i64)]),
     "sbh_debug_subelements": (_int, [_vp, _vp, ctypes.c_double, _vp, ctypes.POINTER(_int)]),
     "sbh_debug_device_sincos": (_int, [_vp, _vp, _i64, _vp, _vp]),
     "sbh_debug_device_rsqrt": (_int, [_vp, _vp, _i64, _vp]),

@@ -1601,6 +1601,13 @@ sbh_status sbh_gmres_ir(sbh_operator* op, sbh_lowp_matrix* lp, const sbh_c64* B,
     });
 }
 
+sbh_status sbh_debug_fill_idle_memory(int byte, int64_t* bytes) {
+    return guard([&] {
+        const int64_t n = work_fill(byte);
+        if (bytes) *bytes = n;
+    });
+}
+
 sbh_status sbh_debug_subelements(const double* source_point, const double* element_coords,
                                  double element_area, double* leaves_out, int* count) {
     return guard([&] {

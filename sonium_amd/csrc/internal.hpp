@@ -106,6 +106,7 @@ struct IdleBytes {
 };
 IdleBytes work_trim();                // frees every idle block: the bytes freed
 int64_t work_idle_bytes(int device);  // device memory of the idle blocks
+int64_t work_fill(int byte);          // writes over every idle block: the bytes written
 
 // Owning block from the work pool: device memory, or pinned host memory.
 template <typename T, bool PINNED = false>

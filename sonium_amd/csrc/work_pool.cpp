@@ -3,6 +3,8 @@
 // runtime's allocation calls alone, so its rules are tested on the host against
 // a model of those calls.
 
+#include <cstring>
+
 #include "internal.hpp"
 
 namespace sbh {
@@ -76,6 +78,21 @@ int64_t work_idle_bytes(int device) {
     int64_t sum = 0;
     for (const WorkBlock& b : pool.idle)
         if (!b.pinned && b.device == device) sum += (int64_t)b.bytes;
+    return sum;
+}
+
+int64_t work_fill(int byte) {
+    WorkPool& pool = work_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    int64_t sum = 0;
+    for (const WorkBlock& b : pool.idle) {
+        if (b.pinned)
+            std::memset(b.ptr, byte, b.bytes);
+        else
+            SBH_HIP(hipMemset(b.ptr, byte, b.bytes));
+        sum += (int64_t)b.bytes;
+    }
+    SBH_HIP(hipDeviceSynchronize());
     return sum;
 }
 

@@ -56,6 +56,7 @@ hipError_t hipMalloc(void** p, size_t bytes) { return model_malloc(p, bytes, fal
 hipError_t hipFree(void* p) { return model_free(p, false); }
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { return model_malloc(p, bytes, true); }
 hipError_t hipHostFree(void* p) { return model_free(p, true); }
+hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }

@@ -2,8 +2,8 @@
 
 A block that a call gives back is handed to the next one with its old contents,
 on any thread, context or stream.  The answers may depend on neither: equal
-bits whatever ran before, also after blocks were left full of NaN, and equal
-bits from threads that exchange blocks while one of them captures a graph.
+bits whatever the idle blocks were filled with, and equal bits from threads
+that exchange blocks while one of them captures a graph.
 """
 
 from concurrent.futures import ThreadPoolExecutor
@@ -13,6 +13,7 @@ import pytest
 
 import sonium_amd as sa
 from sonium_amd.mesh import icosphere
+from sonium_amd.warmstart import WarmStartMLP
 
 pytestmark = pytest.mark.gpu
 
@@ -35,8 +36,8 @@ class Problem:
         self.batch.set_problem([k, 1.1 * k], [[(0.0, 0.0, 1.0)]] * 2)
         self.batch.assemble()
 
-    def answers(self, b=None, B=None):
-        b, B = self.b if b is None else b, self.B if B is None else B
+    def answers(self):
+        b, B = self.b, self.B
         plain = sa.GmresConfig(max_iterations=4, restart=30, tolerance=1e-8)
         block = sa.BlockGmresConfig(max_iterations=4, restart=30, tolerance=1e-8)
         ir = sa.GmresIrConfig(max_outer_iterations=6, outer_tolerance=1e-8, max_inner_iterations=20)
@@ -46,17 +47,71 @@ class Problem:
         return [np.asarray(x) for x in out + list(self.batch.solutions())]
 
 
+    def calls(self):
+        """Every kind of call that takes work blocks, each from nothing but its inputs."""
+        n, b, B = self.op.num_rows(), self.b, self.B
+        rng = np.random.default_rng(n + 1)
+        wide = rng.standard_normal((n, 40)) + 1j * rng.standard_normal((n, 40))
+        low = rng.standard_normal((48, 24)) @ rng.standard_normal((24, 48))
+        samples = rng.standard_normal((700, 10)).astype(np.float32)
+        values = rng.standard_normal((700, 2)).astype(np.float32)
+        points = 3.0 * rng.standard_normal((50, 3))
+        ph = sa.PhysicsParams.from_wavenumber(1.7)
+        field = sa.IncidentField.plane_wave_z()
+        block = lambda restart, cycles=4: sa.BlockGmresConfig(max_iterations=cycles, restart=restart, tolerance=1e-8)
+        ir = sa.GmresIrConfig(max_outer_iterations=6, outer_tolerance=1e-8, max_inner_iterations=20)
+
+        def batch():
+            self.batch.solve("fp64", restart=20, max_cycles=4, tolerance=1e-8, use_graph=True)
+            return self.batch.solutions()
+
+        def train():
+            net = WarmStartMLP(self.ctx, width=128, seed=3)
+            net.set_dataset(samples, values)
+            out = [net.train(6, batch=512), net.params(), net.predict(samples), net.predict_layered(samples)]
+            return out + [net.loss_and_gradients(samples[:256], values[:256])[1]]
+
+        def recycled():
+            sub = sa.GcroDrSubspace(self.ctx, n, 6)
+            cfg = sa.GcroDrConfig(max_iterations=40, restart=12, tolerance=1e-8)
+            return [sa.gcro_dr(self.op, v, None, sub, cfg).x for v in (b, B[:, 0])]
+
+        def spent():  # a basis beyond its space: the least squares grow
+            op = sa.CallbackOperator(self.ctx, 48, lambda x: low @ x)
+            return [sa.block_gmres(op, wide[:48, :3], block(30, 1)).x]
+
+        return {
+            "gmres": lambda: [sa.gmres(self.op, b, sa.GmresConfig(max_iterations=4, restart=30, tolerance=1e-8)).x],
+            "gmres restarts": lambda: [sa.gmres(self.op, b, sa.GmresConfig(max_iterations=9, restart=4,
+                                                                         tolerance=1e-8)).x],
+            "block": lambda: [sa.block_gmres(self.op, B, block(30)).x],
+            "wide block": lambda: [sa.block_gmres(self.op, wide, block(3)).x],
+            "deflated block": lambda: [sa.block_gmres(self.op, np.concatenate([B, B[:, :2]], 1), block(30)).x],
+            "spent block": spent,
+            "columns": lambda: [sa.gmres_block(self.op, B, sa.GmresConfig(max_iterations=4, restart=9,
+                                                                         tolerance=1e-8))[0]],
+            "refinement": lambda: [sa.gmres_ir(self.op, self.lp, B, ir)[0], sa.gmres_ir(self.op, self.lp, wide, ir)[0]],
+            "products": lambda: [self.op.apply(b), self.op.apply_block(wide), self.lp.apply(B)],
+            "batch": batch,
+            "recycled": recycled,
+            "field": lambda: [sa.compute_scattered_field(points, self.mesh, b, ph)],
+            "right-hand side": lambda: [field.compute_rhs_with_beta(self.mesh, ph, ph.burton_miller_beta())],
+            "network": train,
+        }
+
+
 def test_answers_do_not_depend_on_what_a_block_held():
+    """NaN, huge numbers (and as integers, minus one and far out of any range)
+    and zeros in every idle block before each call."""
     p = Problem(2)
-    want = p.answers()
+    calls = p.calls()
+    want = {name: [np.array(x) for x in call()] for name, call in calls.items()}
     held = sa.live_device_bytes()
-    for value in (np.nan, np.inf, 1e300):
-        try:
-            p.answers(np.full_like(p.b, value), np.full_like(p.B, value))
-        except sa.SbhError:
-            pass
-        for x, y in zip(p.answers(), want):
-            assert np.array_equal(x, y)
+    for byte in (0xFF, 0x7F, 0x00):
+        for name, call in calls.items():
+            assert sa.debug_fill_idle_memory(byte) > 0
+            for x, y in zip(call(), want[name]):
+                assert np.array_equal(x, y) and np.all(np.isfinite(y)), (name, byte)
     assert sa.live_device_bytes() == held, "idle blocks belong to nobody"
 
 
