@@ -196,8 +196,9 @@ struct FarPanel {
     double pad;
 };
 
-// Exact geometry for the near-pair and self-panel kernels, which evaluate in
-// the reference's operation order.
+// Exact geometry for the kernels that follow the reference's operation order:
+// self panels, right-hand sides of driven panels and the near pairs of a
+// frequency family.
 struct PanelGeom {
     double c[9];    // node coordinates, row-major (node, xyz)
     double nf[3];   // vertex-order unit normal (compute_parameters)
@@ -599,8 +600,6 @@ void zgemm_block(sbh_context* ctx, const double2* A, int64_t lda, int64_t n, con
 // Roofline ceiling probes (GB/s of a streaming read; FP64 FMA TFLOP/s).
 double probe_stream_read(sbh_context* ctx, const void* x, int64_t bytes, int reps, unsigned* sink);
 double probe_fma_rate(sbh_context* ctx, double* sink);
-// Partial sums for dot products <v_i, w> (i < nvec) and ||w||^2 in one launch;
-// out holds (nvec + 1) x chunks complex partials (the last row is the norm).
 // A whole Gram-Schmidt step in one workgroup (n <= ARNOLDI_MAX_N, at most
 // ARNOLDI_MAX_BASIS vectors): v_next = the normalised w, and into `out` (device
 // accessible host memory) nvec coefficients, ||w|| and whether the second pass ran.
@@ -608,6 +607,8 @@ constexpr int ARNOLDI_MAX_N = 2048;
 constexpr int ARNOLDI_MAX_BASIS = 256;
 void arnoldi_small(sbh_context* ctx, const double2* V, int64_t ldv, int nvec, const double2* w, int64_t n,
                    double2* vnext, double* out);
+// Partial sums for dot products <v_i, w> (i < nvec) and ||w||^2 in one launch;
+// out holds (nvec + 1) x chunks complex partials (the last row is the norm).
 int dots_and_norm_partials(sbh_context* ctx, const double2* V, int64_t ldv, int nvec,
                            const double2* w, int64_t n, double2* out);
 // s[v] = sum of the chunk partials of slot v (v < nv), in chunk order, on the device.

@@ -37,12 +37,6 @@ namespace {
 
 #include "lowp_common.hpp"
 
-__device__ __forceinline__ float wave_sumf(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 // Complex vectors are double2 (FP64) or float2 (FP32); ld2/st2 move them to
 // and from FP64 arithmetic (st2 rounds to nearest).
 __device__ __forceinline__ double2 ld2(double2 v) { return v; }
@@ -930,8 +924,10 @@ static size_t zgemm_partial_doubles(int64_t n, int64_t k) {
 }
 
 // Column tiles and K slices of one chunk of kc columns.  The chip holds 512
-// workgroups of this kernel (two per CU) and they all cost the same, so what
-// counts is the last round: 10240 rows make 80 row tiles, whose 640 workgroups
+// workgroups of this kernel, two per CU (the registers' limit from 17 columns
+// on and at 64 also that of the LDS; up to 16 columns three or four fit, which
+// the plan does not count), and they all cost the same, so what counts is the
+// last round: 10240 rows make 80 row tiles, whose 640 workgroups
 // at 8 slices took two rounds, 1.15 ms at 64 columns, and whose 480 at 6 take one,
 // 0.89 ms; 24 columns on 5056 rows take 124 us instead of 219.  The
 // slice count is the one with the least rounds x stages per workgroup, plus

@@ -287,11 +287,6 @@ __device__ inline void ref_point_t(const double pos[3], double wga, const double
     }
 }
 
-__device__ inline void ref_point(const double pos[3], double wga, const double src[3], const double srcn[3],
-                                 const double nf[3], double wavruim, double k2, Acc& r) {
-    ref_point_t<false>(pos, wga, src, srcn, nf, wavruim, k2, 0.0, 0.0, r, r);
-}
-
 // Shape-function position of local (s, t) (regular.rs:682-690).
 __device__ inline void shape_pos(const double* c, double s, double t, double p[3]) {
     double N0 = 1.0 - s - t;
@@ -1517,9 +1512,11 @@ __global__ void plane_wave_kernel(const Source* __restrict__ sources, int64_t n,
 // each member then needs only the phase advance (one complex product) and
 // its channel sums.  The members' own k_f enter the channel formulas; the
 // phase recurrence differs from a direct sincos(k_f r) by at most about
-// F ulp of the phase (F <= 16).  MODE 0 (velocity panels without
-// admittance): A_ij = H tau + E beta, the far_sums/velocity_coefficient
-// formulas of the single-frequency far kernel.
+// F ulp of the phase (F <= 16).  Velocity panels without admittance:
+// A_ij = H tau + E beta (velocity_coefficient) from separate sums of the H and E
+// channels per member, 15 FP64 instructions a member and evaluation, over the
+// distances of family_points; far_sums folds tau and beta into one weight and
+// takes its geometry and phases from the panel centre.
 constexpr int FAMILY_ROWS = 16;
 
 template <int F>
@@ -1609,7 +1606,7 @@ __global__ __launch_bounds__(256) void batch_far_family_kernel(const FreqFamily*
 }
 
 // Near pairs of a frequency family: the subdivided-leaf quadrature of each
-// pair (regular.rs:164-281, the rule of near_entry) with the point geometry
+// pair (regular.rs:164-281, the points of near_point) with the point geometry
 // formed once for all members.  Sixteen lanes take one pair (a wave four),
 // lanes over (leaf, point); per point the phase exp(i k0 r) and the step
 // exp(i dk r) come from two sincos evaluations and each member advances the
@@ -1714,7 +1711,8 @@ __global__ __launch_bounds__(256) void batch_near_family_kernel(const FreqFamily
 // their plane-wave right-hand sides; PHASE 1, launched after it, overwrites
 // the near pairs and the diagonal of those rows, which is the overwrite order
 // of the single-system launch.  The phases are separate kernels because the
-// near/self code needs about twice the registers of the far loop.
+// near/self code needs 201 registers, two waves to a SIMD, and the far loop 147,
+// three.
 template <int PHASE>
 __global__ __launch_bounds__(256) void batch_assemble_kernel(BatchAssemblyArgs args) {
     __shared__ int s_item;
