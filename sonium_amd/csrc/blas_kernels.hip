@@ -222,7 +222,8 @@ __global__ __launch_bounds__(BLOCK) void project_norm_kernel(const double2* __re
 // panels, most of it in the two round trips; this kernel takes 9 us there and
 // the host reads it behind the next step (a step is 18 us).  w stays in LDS; a wave takes every
 // 16th dot product, a thread one element of the projection.  Above
-// ARNOLDI_MAX_N one CU's share of the L2 is the slower way.
+// ARNOLDI_MAX_N rows, or ARNOLDI_MAX_ENTRIES of the basis, one CU's share of the
+// L2 is the slower way.
 constexpr int ARNOLDI_THREADS = 1024;
 
 __global__ __launch_bounds__(ARNOLDI_THREADS) void arnoldi_small_kernel(const double2* __restrict__ V, int64_t ldv,

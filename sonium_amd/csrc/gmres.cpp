@@ -12,7 +12,7 @@
 // The Krylov basis, the iterate and every vector operation stay on the
 // device; only the (j+1) Gram–Schmidt coefficients and norms come back to the
 // host each step, where the small Hessenberg recurrence runs in FP64.
-// Small dense systems (Krylov::small_steps) take a step's whole orthogonalisation
+// Small dense systems (Krylov::one_launch) take a step's whole orthogonalisation
 // in one launch and keep one step in flight while the host works on the last.
 
 #include <algorithm>
@@ -143,14 +143,16 @@ sbh_status run_gmres(sbh_operator* op, sbh_precond* M, const double2* d_b, const
         g[0] = cplx(beta, 0.0);
         bool inner_converged = false;
         bool restart_now = false;
-        if (small) K.queue_step(V.ptr, 0, w.ptr, opb.ptr);
+        // the basis grows past the range of the one-launch step within a cycle
+        auto one_launch = [&](int j) { return small && K.one_launch(j); };
+        if (one_launch(0)) K.queue_step(V.ptr, 0, w.ptr, opb.ptr);
         for (int j = 0; j < m; ++j) {
             total += 1;
             double wn;
-            if (small) {
+            if (one_launch(j)) {
                 // step j + 1 needs nothing of the host: it is queued before
                 // step j is read (and left unused when step j ends the cycle)
-                if (j + 1 < m) K.queue_step(V.ptr, j + 1, w.ptr, opb.ptr);
+                if (j + 1 < m && one_launch(j + 1)) K.queue_step(V.ptr, j + 1, w.ptr, opb.ptr);
                 bool again = false;
                 wn = K.wait_step(j, coeffs, &again);
                 for (int i = 0; i <= j; ++i) h(i, j) = coeffs[i];
@@ -175,7 +177,7 @@ sbh_status run_gmres(sbh_operator* op, sbh_precond* M, const double2* d_b, const
             h(j + 1, j) = cplx(wn, 0.0);
             if (wn < 1e-20) {
                 inner_converged = true;
-            } else if (!small) {
+            } else if (!one_launch(j)) {
                 scale_copy(ctx, w.ptr, 1.0 / wn, vec(j + 1), n);
             }
             for (int i = 0; i < j; ++i) {

@@ -603,8 +603,15 @@ double probe_fma_rate(sbh_context* ctx, double* sink);
 // A whole Gram-Schmidt step in one workgroup (n <= ARNOLDI_MAX_N, at most
 // ARNOLDI_MAX_BASIS vectors): v_next = the normalised w, and into `out` (device
 // accessible host memory) nvec coefficients, ||w|| and whether the second pass ran.
+// Its one CU reads the basis four times a step, and takes longer than the
+// separate launches over the whole chip from about 120000 (2048 rows), 155000
+// (1536) and 190000 entries (1280) of the vectors projected against on; beyond
+// ARNOLDI_MAX_ENTRIES of them a cycle goes on with those.  2048 rows, 256 steps:
+// 39.5 ms in one launch a step throughout, 25.9 in separate ones, 24.8 with the
+// change at 73 vectors; 640 rows, 200 steps: 10.0, 16.5, 10.0.
 constexpr int ARNOLDI_MAX_N = 2048;
 constexpr int ARNOLDI_MAX_BASIS = 256;
+constexpr int64_t ARNOLDI_MAX_ENTRIES = 150000;
 void arnoldi_small(sbh_context* ctx, const double2* V, int64_t ldv, int nvec, const double2* w, int64_t n,
                    double2* vnext, double* out);
 // Partial sums for dot products <v_i, w> (i < nvec) and ||w||^2 in one launch;

@@ -62,6 +62,8 @@ struct Krylov {
     bool small_steps(int m) const {
         return op->dense() && n <= ARNOLDI_MAX_N && m <= ARNOLDI_MAX_BASIS && (!M || M->kind <= 1);
     }
+    // Step j of a cycle with small_steps: j + 1 vectors within ARNOLDI_MAX_ENTRIES.
+    bool one_launch(int j) const { return (int64_t)(j + 1) * n <= ARNOLDI_MAX_ENTRIES; }
     void queue_step(double2* V, int j, double2* w, double2* tmp) {
         if (!M || M->kind == 0) {
             operator_apply_device(op, V + (size_t)j * n, w);

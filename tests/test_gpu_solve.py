@@ -215,3 +215,29 @@ def test_gmres_steps_at_the_edges_of_the_small_path(ctx, n_theta, n_phi, restart
     # the same steps in another summation order
     assert np.linalg.norm(sol.x - xr) <= 1e-10 * np.linalg.norm(xr)
     assert np.linalg.norm(b - op.apply(sol.x)) <= 1.01e-8 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("restart,jacobi", [(200, False), (100, False), (100, True)])
+def test_gmres_cycle_beyond_the_one_launch_step(ctx, restart, jacobi):
+    """A cycle that starts on the one-launch step and outgrows it (2048 rows: from
+    the 74th vector on), once and in every cycle: the oracle's steps, and an
+    error against LAPACK like the oracle's, whose iterate it is to rounding."""
+    from sonium_amd.mesh import Mesh, fibonacci_sphere
+
+    sphere = fibonacci_sphere(1.0, 33, 32)
+    m = Mesh(sphere.nodes * np.array([1.0, 0.3, 0.1]), sphere.triangles)  # thin and slow: 136 steps
+    ph = sa.PhysicsParams.from_wavenumber(0.02)
+    beta = ph.burton_miller_beta()
+    tm = sa.TbemMesh(ctx, m)
+    system = sa.build_tbem_system_with_beta(ctx, tm, ph, beta)
+    b = sa.IncidentField.plane_wave_z().compute_rhs_with_beta(tm, ph, beta)
+    op = sa.DenseMatrixOperator(system)
+    A = system.matrix
+    pre = sa.JacobiPreconditioner(op) if jacobi else None
+    sol = sa.gmres_preconditioned(op, pre, b, sa.GmresConfig(max_iterations=10, restart=restart, tolerance=1e-8))
+    xr, st = oracle.gmres(A, b, restart=restart, max_iterations=10, tol=1e-8, jacobi=jacobi)
+    assert sol.converged and st["converged"] and sol.iterations > 74
+    assert abs(sol.iterations - st["iterations"]) <= 1 and sol.restarts == st["restarts"]
+    assert np.linalg.norm(b - A @ sol.x) <= 1.01e-8 * np.linalg.norm(b)
+    xl = np.linalg.solve(A, b)
+    assert np.linalg.norm(sol.x - xl) <= 2.0 * np.linalg.norm(xr - xl) + 1e-12 * np.linalg.norm(xl)
