@@ -36,26 +36,26 @@ class BlockLeastSquares {
     // row-major) over the QR's factor.  Nothing is added where the Cholesky QR
     // did not hold; accept() follows where it did.
     void add(const void* chol, const void* chain, const double2* hacc, int sj);
-    void accept(int sj) {
-        done_ += 1;
-        cols_ += sj;
-    }
+    void accept(int sj);
     // Queues y (columns() x s, row-major) of the columns added.
     void solve(double2* y);
     int columns() const { return cols_; }
     const BlockStep& host() const { return *host_.ptr; }  // after a synchronization
 
    private:
+    bool joins(int sj) const;  // a step of sj columns fits the last group's window
+    static int64_t most_groups(int s, int64_t steps, int64_t cols);
     static int64_t room_bytes(int s, int64_t steps, int64_t cols);
     void make_room(int steps, int cols);
 
     sbh_context* ctx_;
     int64_t n_;
-    int s_, done_ = 0, cols_ = 0;
+    int s_, done_ = 0, cols_ = 0;          // steps and columns added
+    int ngroups_ = 0, open_ = 0;           // groups of steps, columns of the last
     int max_basis_, max_steps_;            // limits of a cycle
     int room_cols_ = 0, room_steps_ = 0;   // what the arrays hold
     int64_t ldg_ = 0;
-    WorkArray<int2> steps_;
+    WorkArray<int4> groups_;
     WorkArray<double2> refl_, qh_, R_, window_, g_, work_;
     WorkArray<BlockStep, true> host_;
 };

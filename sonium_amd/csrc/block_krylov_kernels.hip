@@ -29,6 +29,7 @@
 
 #include <cmath>
 #include <cstddef>
+#include <type_traits>
 
 #include "block_krylov.hpp"
 #include "internal.hpp"
@@ -830,15 +831,20 @@ __global__ __launch_bounds__(BK_THREADS) void bk_qr_project_kernel(QrArgs a, int
 // 614-664) solves with Givens rotations.  Step q holds columns and rows
 // [p_q, p_q + s_q); its columns reach s_{q+1} rows further, so its
 // transformation acts on the window [p_q, p_q + s_q + s_{q+1}), at most 2 * 64
-// rows: one or two (W) entries per lane of a wave.
+// rows: one or two (W) entries per lane of a wave.  Consecutive steps whose
+// windows fit one of 64 W rows together make one group with one unitary factor,
+// so the chain that a new column goes through is as long as the basis, not the
+// steps: with a group to each step, 200 steps of one column on 2048 rows took
+// 45.7 ms (40.0 with the rotations on the host), now 21.5; of 16 columns on 5120
+// rows 123 (175), now 101.
 //
 // On the host the rotations of a 24-column step took 350 us (half of it the
 // new block's own, in one thread), more than the device needs for the step,
 // and every Hessenberg block and every coefficient crossed the bus.
 struct LsState {
-    int2* steps;        // (p_q, s_q) of the factored steps
+    int4* groups;       // of steps: first row, columns, rows of the last step's QR after them
     double2* refl;      // the last step's column c: 64 W window entries of v, H = I - v v^H
-    double2* qh;        // step q: Q^H of its window, column by column, (64 W)^2 entries
+    double2* qh;        // group q: Q^H of its window, column by column, (64 W)^2 entries
     double2* R;         // packed columns of the triangle, column c from c(c+1)/2
     double2* window;    // the new columns' windows, 64 W entries each
     double2* g;         // transformed right-hand sides, column q from q * ldg
@@ -875,9 +881,9 @@ __device__ __forceinline__ void reflect(const double2 (&v)[W], double2 (&x)[W]) 
     }
 }
 
-// The `done` earlier steps' transformations on one new Hessenberg column per
+// The `done` groups' transformations on one new Hessenberg column per
 // workgroup: the finished entries go to R, the rest to its window.  Lane l of
-// wave w forms row l of a quarter of the product Q_q^H x, so a step costs two
+// wave w forms row l of a quarter of the product Q_q^H x, so a group costs two
 // barriers and a fourth of the window's multiplications in a row.  Reflector by
 // reflector, each with its dot product across a wave, the 265 of an average
 // step of a 24-column solve took 62 us; the products take 27, and Q^H 7 to form.
@@ -898,9 +904,9 @@ __global__ __launch_bounds__(256) void bk_ls_apply_kernel(LsState ls, LsQr qr, c
         if (row < p) return hacc[(int64_t)row * sj + c];
         return qr.entry(sj, c, row - p);
     };
-    // widths of the steps, read ahead as well
-    auto width = [&](int q) { return q < done ? ls.steps[q].y : q == done ? sj : s_next; };
-    int s0 = width(0), s1 = width(1), s2 = width(2);
+    // the groups, read ahead as well; after the last the new step's own window
+    auto group = [&](int q) { return q < done ? ls.groups[q] : make_int4(p_start, sj, s_next, 0); };
+    int4 now = group(0), next = group(1), third = group(2);
     int base = 0;
     double2 qh[AHEAD][W];
     auto load = [&](int q, int rows) {
@@ -916,16 +922,16 @@ __global__ __launch_bounds__(256) void bk_ls_apply_kernel(LsState ls, LsQr qr, c
         if (t < N && t >= from && t < from + count) fresh = entry(row0 + t);
     };
     if (done > 0) {
-        load(0, s0 + s1);
-        load_fresh(s0, s1, s2);
+        load(0, now.y + now.z);
+        load_fresh(now.y, now.z, next.y + next.z - now.z);
     }
-    if (t < N) x[t] = t < s0 + s1 ? entry(t) : make_double2(0.0, 0.0);
+    if (t < N) x[t] = t < now.y + now.z ? entry(t) : make_double2(0.0, 0.0);
     lds_barrier();
     const int64_t column = (int64_t)p_start + c;
     double2* Rc = ls.R + column * (column + 1) / 2;
     for (int q = 0; q < done; ++q) {
-        const int s3 = q + 1 < done ? width(q + 3) : 0;
-        const int rows = s0 + s1;
+        const int4 fourth = q + 1 < done ? group(q + 3) : now;
+        const int rows = now.y + now.z;
         const int quarter = (rows + 3) / 4;
         const int kbeg = wave * quarter, kend = min(rows, kbeg + quarter);
         double2 acc[W];
@@ -955,56 +961,60 @@ __global__ __launch_bounds__(256) void bk_ls_apply_kernel(LsState ls, LsQr qr, c
         for (int w = 0; w < W; ++w) sum[wave][lane + 64 * w] = acc[w];
         const double2 enters = fresh;
         if (q + 1 < done) {
-            load(q + 1, s1 + s2);
+            load(q + 1, next.y + next.z);
             fresh = make_double2(0.0, 0.0);
-            load_fresh(base + s0 + s1, s2, s3);
+            load_fresh(base + now.y + next.y, next.z, third.y + third.z - next.z);
         }
         lds_barrier();
         if (t < rows) {
             const double2 y = make_double2(((sum[0][t].x + sum[1][t].x) + sum[2][t].x) + sum[3][t].x,
                                            ((sum[0][t].y + sum[1][t].y) + sum[2][t].y) + sum[3][t].y);
-            // the first s0 rows are finished; the window moves on by them
-            if (t < s0)
+            // the group's own rows are finished; the window moves on by them
+            if (t < now.y)
                 Rc[base + t] = y;
             else
-                x[t - s0] = y;
+                x[t - now.y] = y;
         }
-        if (t < N && t >= s1) x[t] = enters;
+        if (t < N && t >= now.z) x[t] = enters;
         lds_barrier();
-        base += s0;
-        s0 = s1;
-        s1 = s2;
-        s2 = s3;
+        base += now.y;
+        now = next;
+        next = third;
+        third = fourth;
     }
     if (t < N) ls.window[(int64_t)c * N + t] = x[t];
 }
 
-// Column k = blockIdx.x of Q^H of the step just factored: its reflectors on e_k.
+// Column k = blockIdx.x of Q^H of group `group` with the step just factored, whose
+// rows start at `offset` in the group's window: the step's reflectors on the
+// column that the group had, or on e_k for the rows that are new to it.
 template <int W>
-__global__ __launch_bounds__(64) void bk_ls_form_kernel(LsState ls, LsQr qr, int sj, int done, int p_start) {
+__global__ __launch_bounds__(64) void bk_ls_form_kernel(LsState ls, LsQr qr, int sj, int group, int offset) {
     if (!qr.chain && qr.chol->ok == 0) return;
     constexpr int N = 64 * W;
     const int lane = threadIdx.x;
     const int k = blockIdx.x;
-    if (k >= sj + qr.next(sj)) return;
+    if (k >= offset + sj + qr.next(sj)) return;
+    double2* column = ls.qh + ((int64_t)group * N + k) * N + lane;
     double2 x[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) x[w] = make_double2(lane + 64 * w == k ? 1.0 : 0.0, 0.0);
-    const double2* refl = ls.refl + lane;
+    for (int w = 0; w < W; ++w)
+        x[w] = offset > 0 && k < offset + sj ? column[64 * w] : make_double2(lane + 64 * w == k ? 1.0 : 0.0, 0.0);
     for (int a = 0; a < sj; a += 8) {
         double2 v[8][W];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
 #pragma unroll
             for (int w = 0; w < W; ++w) {
-                const double2 y = refl[(int64_t)min(a + u, sj - 1) * N + 64 * w];
-                v[u][w] = a + u < sj ? y : make_double2(0.0, 0.0);  // past the last: no reflection
+                const int i = lane + 64 * w - offset;
+                const double2 y = ls.refl[(int64_t)min(a + u, sj - 1) * N + max(i, 0)];
+                v[u][w] = a + u < sj && i >= 0 ? y : make_double2(0.0, 0.0);  // past the last: no reflection
             }
 #pragma unroll
         for (int u = 0; u < 8; ++u) reflect<W>(v[u], x);
     }
 #pragma unroll
-    for (int w = 0; w < W; ++w) ls.qh[((int64_t)done * N + k) * N + lane + 64 * w] = x[w];
+    for (int w = 0; w < W; ++w) column[64 * w] = x[w];
 }
 
 // Householder QR of the new step's windows, its reflectors on the s
@@ -1016,8 +1026,8 @@ __global__ __launch_bounds__(64) void bk_ls_form_kernel(LsState ls, LsQr qr, int
 // barrier: the owner of the next one reflects it first and forms its reflector
 // while the others still apply the present one.
 template <int W>
-__global__ __launch_bounds__(1024) void bk_ls_factor_kernel(LsState ls, LsQr qr, int sj, int s, int done,
-                                                            int p_start) {
+__global__ __launch_bounds__(1024) void bk_ls_factor_kernel(LsState ls, LsQr qr, int sj, int s, int group,
+                                                            int offset, int p_start) {
     if (!qr.chain && qr.chol->ok == 0) {
         if (threadIdx.x == 0) ls.host->ok = 0;
         return;
@@ -1114,7 +1124,7 @@ __global__ __launch_bounds__(1024) void bk_ls_factor_kernel(LsState ls, LsQr qr,
     tail = sqrt(row_sum(tail));
     if (c < s && l == 0) ls.host->tail[c] = tail;
     if (threadIdx.x == 0) {
-        ls.steps[done] = make_int2(p_start, sj);
+        ls.groups[group] = make_int4(p_start - offset, offset + sj, s_next, 0);
         ls.host->next = s_next;
         ls.host->ok = 1;
     }
@@ -1393,10 +1403,16 @@ void BlockLeastSquares::allocate() {
     make_room((int)std::min<int64_t>(max_steps_, n_ + 1), (int)std::min<int64_t>(max_basis_, n_ + 2 * s_));
 }
 
+// A step opens a group where the last one has more than window - 2 s columns.
+int64_t BlockLeastSquares::most_groups(int s, int64_t steps, int64_t cols) {
+    return std::min(steps, cols / ((int64_t)bk_ls_window(s) - 2 * s + 1) + 1);
+}
+
 int64_t BlockLeastSquares::room_bytes(int s, int64_t steps, int64_t cols) {
     const int64_t window = (int64_t)bk_ls_window(s);
-    return (int64_t)sizeof(int2) * (steps + 1) +
-           (int64_t)sizeof(double2) * (steps * window * window + cols * (cols + 1) / 2 + 2 * (cols + s) * s);
+    const int64_t groups = most_groups(s, steps, cols);
+    return (int64_t)sizeof(int4) * groups +
+           (int64_t)sizeof(double2) * (groups * window * window + cols * (cols + 1) / 2 + 2 * (cols + s) * s);
 }
 
 int64_t BlockLeastSquares::device_bytes(int64_t n, int s, int64_t restart) {
@@ -1409,19 +1425,20 @@ int64_t BlockLeastSquares::device_bytes(int64_t n, int s, int64_t restart) {
 void BlockLeastSquares::make_room(int steps, int cols) {
     const size_t window = bk_ls_window(s_);
     const int64_t ldg = cols + s_;
-    WorkArray<int2> steps_new((size_t)steps + 1);
-    WorkArray<double2> qh((size_t)steps * window * window), R((size_t)cols * (cols + 1) / 2), g((size_t)ldg * s_),
+    const size_t most = (size_t)most_groups(s_, steps, cols);
+    WorkArray<int4> groups(most);
+    WorkArray<double2> qh(most * window * window), R((size_t)cols * (cols + 1) / 2), g((size_t)ldg * s_),
         work((size_t)ldg * s_);
     auto keep = [&](void* to, const void* from, size_t bytes) {
         if (bytes) SBH_HIP(hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToDevice, ctx_->stream));
     };
-    keep(steps_new.ptr, steps_.ptr, sizeof(int2) * done_);
-    keep(qh.ptr, qh_.ptr, sizeof(double2) * done_ * window * window);
+    keep(groups.ptr, groups_.ptr, sizeof(int4) * ngroups_);
+    keep(qh.ptr, qh_.ptr, sizeof(double2) * ngroups_ * window * window);
     keep(R.ptr, R_.ptr, sizeof(double2) * ((size_t)cols_ * (cols_ + 1) / 2));
     if (ldg_)
         SBH_HIP(hipMemcpy2DAsync(g.ptr, sizeof(double2) * ldg, g_.ptr, sizeof(double2) * ldg_, sizeof(double2) * ldg_,
                                  s_, hipMemcpyDeviceToDevice, ctx_->stream));
-    steps_.swap(steps_new);
+    groups_.swap(groups);
     qh_.swap(qh);
     R_.swap(R);
     g_.swap(g);
@@ -1432,8 +1449,9 @@ void BlockLeastSquares::make_room(int steps, int cols) {
 }
 
 namespace {
-LsState ls_state(int2* steps, double2* refl, double2* qh, double2* R, double2* window, double2* g, int64_t ldg, BlockStep* host) {
-    return LsState{steps, refl, qh, R, window, g, ldg, host};
+LsState ls_state(int4* groups, double2* refl, double2* qh, double2* R, double2* window, double2* g, int64_t ldg,
+                 BlockStep* host) {
+    return LsState{groups, refl, qh, R, window, g, ldg, host};
 }
 LsQr ls_qr(const void* chol, const void* chain) {
     return LsQr{static_cast<const CholState*>(chol), static_cast<const QrState*>(chain)};
@@ -1448,8 +1466,25 @@ void BlockLeastSquares::report(const void* chol, const void* chain, int sj) {
 void BlockLeastSquares::reset(const double2* c0, int s1) {
     done_ = 0;
     cols_ = 0;
+    ngroups_ = 0;
+    open_ = 0;
     hipLaunchKernelGGL(bk_ls_reset_kernel, dim3(1), dim3(BK_THREADS), 0, ctx_->stream, c0, s1, s_, g_.ptr, ldg_);
     SBH_HIP(hipGetLastError());
+}
+
+bool BlockLeastSquares::joins(int sj) const {
+    return ngroups_ > 0 && open_ + 2 * sj <= (int)bk_ls_window(s_);
+}
+
+void BlockLeastSquares::accept(int sj) {
+    if (joins(sj)) {
+        open_ += sj;
+    } else {
+        ngroups_ += 1;
+        open_ = sj;
+    }
+    done_ += 1;
+    cols_ += sj;
 }
 
 void BlockLeastSquares::add(const void* chol, const void* chain, const double2* hacc, int sj) {
@@ -1468,25 +1503,29 @@ void BlockLeastSquares::add(const void* chol, const void* chain, const double2* 
     }
     hipEvent_t ev;
     ctx_->begin_timed(SBH_KERNEL_KRYLOV_VECTOR, &ev);
-    const LsState st = ls_state(steps_.ptr, refl_.ptr, qh_.ptr, R_.ptr, window_.ptr, g_.ptr, ldg_, host_.ptr);
+    const LsState st = ls_state(groups_.ptr, refl_.ptr, qh_.ptr, R_.ptr, window_.ptr, g_.ptr, ldg_, host_.ptr);
     const LsQr qr = ls_qr(chol, chain);
     const unsigned threads = (unsigned)((s_ + 3) / 4 * 64);  // sixteen lanes to a column
-    if (bk_ls_window(s_) == 64) {
-        hipLaunchKernelGGL(bk_ls_apply_kernel<1>, dim3(sj), dim3(256), 0, ctx_->stream, st, qr, hacc, sj, done_, cols_);
-        hipLaunchKernelGGL(bk_ls_factor_kernel<1>, dim3(1), dim3(threads), 0, ctx_->stream, st, qr, sj, s_, done_, cols_);
-        hipLaunchKernelGGL(bk_ls_form_kernel<1>, dim3(2 * sj), dim3(64), 0, ctx_->stream, st, qr, sj, done_, cols_);
-    } else {
-        hipLaunchKernelGGL(bk_ls_apply_kernel<2>, dim3(sj), dim3(256), 0, ctx_->stream, st, qr, hacc, sj, done_, cols_);
-        hipLaunchKernelGGL(bk_ls_factor_kernel<2>, dim3(1), dim3(threads), 0, ctx_->stream, st, qr, sj, s_, done_, cols_);
-        hipLaunchKernelGGL(bk_ls_form_kernel<2>, dim3(2 * sj), dim3(64), 0, ctx_->stream, st, qr, sj, done_, cols_);
-    }
+    const int group = joins(sj) ? ngroups_ - 1 : ngroups_, offset = joins(sj) ? open_ : 0;
+    auto launch = [&](auto w) {
+        constexpr int W = decltype(w)::value;
+        hipLaunchKernelGGL(bk_ls_apply_kernel<W>, dim3(sj), dim3(256), 0, ctx_->stream, st, qr, hacc, sj, ngroups_, cols_);
+        hipLaunchKernelGGL(bk_ls_factor_kernel<W>, dim3(1), dim3(threads), 0, ctx_->stream, st, qr, sj, s_, group, offset,
+                           cols_);
+        hipLaunchKernelGGL(bk_ls_form_kernel<W>, dim3(offset + 2 * sj), dim3(64), 0, ctx_->stream, st, qr, sj, group,
+                           offset);
+    };
+    if (bk_ls_window(s_) == 64)
+        launch(std::integral_constant<int, 1>());
+    else
+        launch(std::integral_constant<int, 2>());
     SBH_HIP(hipGetLastError());
     ctx_->end_timed(SBH_KERNEL_KRYLOV_VECTOR, ev);
 }
 
 void BlockLeastSquares::solve(double2* y) {
     const size_t bytes = sizeof(double2) * (size_t)cols_;
-    const LsState st = ls_state(steps_.ptr, refl_.ptr, qh_.ptr, R_.ptr, window_.ptr, g_.ptr, ldg_, host_.ptr);
+    const LsState st = ls_state(groups_.ptr, refl_.ptr, qh_.ptr, R_.ptr, window_.ptr, g_.ptr, ldg_, host_.ptr);
     if (bytes <= (64u << 10))  // what a launch may ask for
         hipLaunchKernelGGL(bk_ls_solve_kernel<true>, dim3(s_), dim3(256), bytes, ctx_->stream, st, cols_, s_, work_.ptr, y);
     else

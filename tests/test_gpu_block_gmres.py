@@ -274,3 +274,29 @@ def test_block_gmres_basis_beyond_the_space(ctx, n, s, restart):
     assert np.all(np.isfinite(sol.x)) and np.all(np.isfinite(sol.true_residuals))
     assert np.all(sol.residuals == 0.0)  # as the reference reports a spent budget
     op.close()
+
+
+@pytest.mark.parametrize("sizes", [[150], [100, 101], [2, 5, 11, 24, 47, 90], [60] * 3 + [61], [30] * 16 + [9] * 9,
+                                   [10] * 12 + [25] * 12 + [40] * 16, [3] * 10 + [7] * 10 + [12] * 44])
+def test_block_gmres_deflates_within_a_cycle(ctx, sizes):
+    """A unitary operator that takes column c sizes[c] steps, and not one less, in
+    a space of its own, all hidden by a unitary basis and by mixed columns: the
+    block narrows whenever one of them is done, in groups of least-squares steps
+    of every width.  The last step solves all columns; with a condition of one
+    their errors are the rounding of some 100 projections, 1e-12 with room."""
+    rng = np.random.default_rng(len(sizes))
+    c = lambda *shape: rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    n, s, o = sum(sizes), len(sizes), 0
+    A, B = np.zeros((n, n), complex), np.zeros((n, s), complex)
+    for i, d in enumerate(sizes):
+        Q = np.linalg.qr(c(d, d))[0]
+        A[o:o + d, o:o + d] = (Q * np.exp(2j * np.pi * np.arange(d) / d)) @ Q.conj().T
+        B[o:o + d, i] = c(d)
+        o += d
+    P = np.linalg.qr(c(n, n))[0]
+    A, B = P @ A @ P.conj().T, P @ B @ c(s, s)
+    op = sa.CallbackOperator(ctx, n, lambda x: A @ x)
+    sol = sa.block_gmres(op, B, sa.BlockGmresConfig(max_iterations=1, restart=200, tolerance=1e-10))
+    assert sol.converged and sol.iterations == max(sizes) and sol.max_basis <= n
+    assert np.linalg.norm(sol.x - A.conj().T @ B) <= 1e-12 * np.linalg.norm(B)
+    op.close()
